@@ -6,7 +6,10 @@
 //     dS = P * (dO V^T - D)     dQ = scale * dS K     dK = scale * dS^T Q     dV = P^T dO     dbias = dS
 // Nothing is stored between forward and backward but O and LSE; P is recomputed per 32 x 32 tile.
 //
-// Two kernels, each the forward kernel's arrangement (see attention.hip) with one side held in registers:
+// For head dimensions up to 32 one kernel makes all four gradients in one pass over the score planes
+// (flash_attn_back_fused_kernel, below).  Larger heads, and long sequences in few planes (a work-group of that kernel
+// takes a whole plane), go in two kernels, each the forward kernel's arrangement (see attention.hip) with one side held
+// in registers:
 //   * rows kernel  (dQ, dbias): a wave owns 32 queries; scores and dO V^T are computed transposed, so a lane
 //     holds 16 keys of ITS query: D_i and LSE_i are per-lane scalars, dS is ready as the B operand of
 //     dQ^T += K^T dS, and dbias is written from the registers;
@@ -446,6 +449,423 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_cols_kernel(const Att
         }
 }
 
+// ------------------------------------------------------------------------------------------------------------
+// All four gradients in one pass over the score planes (d <= 32).  A work-group takes whole planes, one after the other,
+// each of its NW waves 32 keys of a plane (NW * 32 keys at a time, longer planes in several rounds), and all waves walk
+// over the query tiles together.  The columns kernel's arrangement -- S and dO V^T un-transposed, a lane holds 16 queries
+// of ITS key -- gives P and dS as B operands of dV^T and dK^T as they stand and reads the bias / writes dbias in whole
+// 128-byte row pieces; what it lacks is dQ^T += K^T dS^T, whose B operand wants a lane per QUERY.  dS, split once for dK,
+// goes through LDS as bf16 parts and comes back transposed by ds_read_b64_tr_b16; the waves' partial dQ tiles meet in LDS
+// and are added in wave order (no atomics: results do not depend on scheduling).  The same instruction reads Q and dO for
+// the gradients out of their row fragments, so no second arrangement of them is staged.  Against the two kernels above, S,
+// P and dO V^T are computed once instead of twice (60 MFMAs per 32 x 32 tile instead of 84) and the bias is read once.
+// One barrier per query tile: the next tile is staged into the other half of a double buffer from loads issued two tiles
+// ahead (across planes too), the partial tiles alternate between two regions.
+// A step is five phases of twelve MFMAs -- S, dO V^T, dV, dK, dQ -- each with the vector work that does not depend on it
+// placed between its MFMAs, and the fragments of a phase read during the one before: eight waves fill the registers and
+// the LDS of a CU, so nothing else hides that work.  Per-wave time stamps: a step takes 8200 cycles for the two waves of a
+// SIMD, 3840 of them MFMAs; what is left is the 32 accesses to bias and dbias (20 cycles each), LDS reads behind the
+// barrier, and a clock of 1.7 GHz.  Registers decide: a variant with one more fragment set or with a second copy of the
+// step (keys past the matrix handled apart) spilled inside the loop, and every reload waits for all stores in flight
+// (370 us instead of 162).
+// Measured, us, against the two kernels (dQ + dbias, dK + dV): 824 planes of 256 x 256, d 32, with bias 291 -> 162 (648 MB:
+// 4.0 TB/s), 412 of 103 x 103 46 -> 25, 824 of 64 x 64 40 -> 25, 16 of 256 x 256 47 -> 33.
+typedef short v4s __attribute__((ext_vector_type(4)));
+
+template <int NW> struct FusedBack {
+    // Row fragments of 32 rows x 32 features as in BackTiling, but with the halves (features 8 .. 15 of a chunk) 576 bytes
+    // apart: the transposing reads and the staging writes then touch every bank once.
+    static constexpr int HALF = 576, FRAG = 2 * HALF, CHUNK = 3 * FRAG;
+    static constexpr int TILE = 2 * CHUNK;
+    static constexpr int STAGE = 2 * TILE + 512;          // Q, dO, then LSE * log2(e) and D of the 32 queries, then 256 bytes nobody reads
+    static constexpr int NO_KEY = 256;                     // what a lane whose key lies past the matrix reads instead of those: +inf and 0
+    // A wave's dS parts ([key][query] of bf16, 64 bytes per key, its eight-byte pieces exchanged by key / 4 so that the
+    // writes of sixteen keys meet every bank once), then its partial dQ tile ([query][36] floats)
+    static constexpr int PART = 32 * 64;
+    static constexpr int REGION = 3 * PART;
+    static constexpr int QP = 36;
+    static constexpr size_t LDS = 2 * STAGE + 2 * NW * static_cast<size_t>(REGION) + NO_KEY;
+    static_assert(32 * QP * 4 <= REGION, "the partial tile takes the place of the parts");
+};
+
+// eight 16-bit elements of this lane's column, four rows at `at` and four at `at + step`, each piece transposed on the
+// way (a group of sixteen lanes names four rows of sixteen columns, four columns per lane)
+__device__ __forceinline__ v8bf read_transposed(const uint8_t* at, int step) {
+    typedef __attribute__((address_space(3))) v4s* lds_v4s;
+    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at));
+    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at + step));
+    return __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// DB: dbias not wanted / ordinary stores / streaming stores (rows of whole 128-byte lines)
+constexpr int DB_NONE = 0, DB_ORDINARY = 1, DB_STREAM = 2;
+
+// One MFMA, then up to `valu` vector instructions, `count` times over: a wave issues in order, so vector work hides behind
+// its own matrix work only where the two alternate in the program.
+template <int count, int valu> __device__ __forceinline__ void interleave() {
+#pragma unroll
+    for (int i = 0; i < count; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, valu, 0);
+    }
+}
+
+template <int NW, bool BIAS, int DB, bool CAUSAL>
+__global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const AttnBackParams p) {
+    using F = FusedBack<NW>;
+    extern __shared__ __attribute__((aligned(16))) uint8_t back_lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 31, half = lane >> 5;
+    const int L = p.L, d = p.d;
+    const int tiles = (L + 31) / 32;
+    uint8_t* const regions = back_lds + 2 * F::STAGE;
+    uint8_t* const no_key_lds = regions + 2 * NW * F::REGION;
+    if (tid < 64) reinterpret_cast<float*>(no_key_lds)[tid] = tid < 32 ? INFINITY : 0.0f;   // (read behind the first barrier)
+
+    const int64_t mat = static_cast<int64_t>(L) * d, square = static_cast<int64_t>(L) * L;
+    const uint32_t mat_bytes = static_cast<uint32_t>(L) * d * 4u, square_bytes = static_cast<uint32_t>(L) * L * 4u;
+    const auto rsrc = [](const float* base, uint32_t bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, static_cast<int>(bytes), 0x00020000);
+    };
+    const auto load4 = [](__amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0)); };
+    const auto load1 = [](__amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0)); };
+    constexpr uint32_t OUT = 0x80000000u;
+
+    // The work-group's sequence of steps: its planes, per plane the rounds of NW * 32 keys, per round the query tiles.
+    // Loads run ahead of the computation along this sequence, across rounds and planes.
+    struct Step { int plane, g0, t; };
+    const auto advance = [&](Step& s) {
+        if (++s.t < tiles) return;
+        s.t = 0;
+        s.g0 += NW * 32;
+        if (s.g0 < L) return;
+        s.g0 = 0;
+        s.plane += static_cast<int>(gridDim.x);
+    };
+
+    // ---- staging of a query tile: 256 items (row, four features) of Q and 256 of dO (with O, for D), shared out over
+    // the threads; rows and features past the matrix, and everything past the last plane, read as zeros
+    constexpr int NT = NW * 64, ITEMS = (512 + NT - 1) / NT;
+    v4f xs[ITEMS], xo[ITEMS];
+    float xl[ITEMS];
+    Step ahead{static_cast<int>(blockIdx.x), 0, 0};        // the tile whose loads are next (two steps ahead of the computation)
+    const auto stage_load = [&]() {
+        const bool there = ahead.plane < p.planes;
+        const int64_t po = there ? ahead.plane * mat : 0;
+        const uint32_t bytes = there ? mat_bytes : 0;
+        const __amdgpu_buffer_rsrc_t rlse = rsrc(p.LSE + (there ? static_cast<int64_t>(ahead.plane) * L : 0), there ? static_cast<uint32_t>(L) * 4u : 0);
+        const __amdgpu_buffer_rsrc_t ro = rsrc(p.O + po, bytes);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const bool is_do = (wave * 64 + i * NT) >= 256;          // (items of one kind per wave and turn)
+            const __amdgpu_buffer_rsrc_t rx = rsrc((is_do ? p.dO : p.Q) + po, bytes);
+            const int e = (tid + i * NT) & 255;
+            const int row = ahead.t * 32 + (e >> 3), c = (e & 7) * 4;
+            const uint32_t at = row < L && c < d ? (static_cast<uint32_t>(row) * d + c) * 4u : OUT;
+            xs[i] = load4(rx, at);
+            if (NT >= 512 || is_do) {
+                xo[i] = load4(ro, is_do ? at : OUT);
+                // (a row past the matrix: log of a sum of zero, which makes its probabilities zero)
+                xl[i] = load1(rlse, is_do && row < L ? static_cast<uint32_t>(row) * 4u : OUT);
+                xl[i] = row < L ? xl[i] : -INFINITY;
+            }
+        }
+        advance(ahead);
+    };
+    const auto stage_put = [&](int n) {
+        uint8_t* const stage = back_lds + (n & 1) * F::STAGE;
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const bool is_do = (wave * 64 + i * NT) >= 256;
+            const int e = (tid + i * NT) & 255;
+            const int row = e >> 3, c = (e & 7) * 4;
+            uint2 parts[3];
+            split4(xs[i], parts);
+            uint8_t* const dst = stage + (is_do ? F::TILE : 0) + (c >> 4) * F::CHUNK + ((c >> 3) & 1) * F::HALF + row * 16 + ((c >> 2) & 1) * 8;
+#pragma unroll
+            for (int part = 0; part < 3; ++part) *reinterpret_cast<uint2*>(dst + part * F::FRAG) = parts[part];
+            if (NT >= 512 || is_do) {
+                float sum = xs[i][0] * xo[i][0] + xs[i][1] * xo[i][1] + xs[i][2] * xo[i][2] + xs[i][3] * xo[i][3];
+                // the eight lanes of the row: neighbours, pairs, then the other four
+                sum += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, sum), 0xB1, 0xf, 0xf, true));
+                sum += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, sum), 0x4E, 0xf, 0xf, true));
+                sum += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, sum), 0x141, 0xf, 0xf, true));
+                // A row without any visible key (LSE = -inf) has no gradient: +inf makes every probability exp2(-inf) = 0.
+                // (Lanes that have nothing to write write where nobody reads: a branch here would cut the block in which
+                // this work hides behind the matrix pipe.)
+                float* const lse_at = reinterpret_cast<float*>(stage + 2 * F::TILE) + (c == 0 && is_do ? row : 64 + (lane & 31));
+                lse_at[0] = xl[i] > -INFINITY ? xl[i] * LOG2E : INFINITY;
+                lse_at[c == 0 && is_do ? 32 : 0] = sum;
+            }
+        }
+    };
+
+    // dQ of a tile: the waves' shares, in wave order
+    const auto add_shares = [&](const Step& s, int n) {
+        constexpr int W = NT >= 512 ? 2 : 4;               // floats per thread and turn
+        typedef float vw __attribute__((ext_vector_type(W)));
+#pragma unroll
+        for (int i = 0; i < (1024 / W + NT - 1) / NT; ++i) {
+            const int e = tid + i * NT;
+            const int row = s.t * 32 + e / (32 / W), c = e % (32 / W) * W;
+            if (row >= L || c >= d) continue;
+            const float* src = reinterpret_cast<const float*>(regions + (n & 1) * NW * F::REGION) + e / (32 / W) * F::QP + c;
+            vw x[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) x[w] = *reinterpret_cast<const vw*>(src + w * (F::REGION / 4));
+            vw sum = x[0];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) sum += x[w];
+            vw* const dst = reinterpret_cast<vw*>(p.dQ + s.plane * mat + static_cast<int64_t>(row) * d + c);
+            sum *= p.scale;
+            if (s.g0 > 0) sum += *dst;                     // (this thread wrote it in the round before)
+            *dst = sum;
+        }
+    };
+
+    // ---- The bias of this lane's key for its 16 queries of a tile (requested a step ahead) and dbias; rows and keys past
+    // the matrix fall outside the plane.
+    float bv[16];
+    const uint32_t row_bytes = static_cast<uint32_t>(L) * 4u;
+    const auto square_at = [&](const Step& s) {
+        const int key = s.g0 + wave * 32 + j;
+        return key < L ? static_cast<uint32_t>(key) * 4u + (static_cast<uint32_t>(s.t) * 32u + 4u * half) * row_bytes : OUT;
+    };
+    // from the row of accumulator register r to that of the next one; opaque, so that the sixteen offsets of a tile
+    // follow each other through one register instead of taking one each
+    const auto next_row = [&](uint32_t& at, int r) {
+        at += (r & 3) == 3 ? 5 * row_bytes : row_bytes;
+        asm volatile("" : "+v"(at));
+    };
+    const auto load_bias = [&](const Step& s) {
+        if (!BIAS) return;
+        const bool there = s.plane < p.planes;
+        const __amdgpu_buffer_rsrc_t rbias = rsrc(p.bias + (there ? s.plane * square : 0), there ? square_bytes : 0);
+        uint32_t at = square_at(s);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            bv[r] = load1(rbias, at);
+            next_row(at, r);
+        }
+    };
+    const auto store_dbias = [&](const Step& s, const v16f& x) {
+        if (DB == DB_NONE) return;
+        const __amdgpu_buffer_rsrc_t rdb = rsrc(p.dbias + s.plane * square, square_bytes);
+        uint32_t at = square_at(s);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float v = x[r];
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rdb, at, 0, DB == DB_STREAM ? 3 : 0);
+            next_row(at, r);
+        }
+    };
+
+    // this lane's place in the fragments: row reads; transposing reads (see read_transposed) of staged rows and of dS parts
+    const int grp = lane & 15;
+    const int row_at = (lane & 31) * 16 + half * F::HALF;
+    const int tr = ((lane >> 4) & 1) * F::CHUNK + ((grp >> 1) & 1) * F::HALF + (4 * half + (grp >> 2)) * 16 + (grp & 1) * 8;
+    const auto read_rows = [&](const uint8_t* tile, v8bf (&a)[2][3]) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int part = 0; part < 3; ++part) a[c][part] = *reinterpret_cast<const v8bf*>(tile + row_at + c * F::CHUNK + part * F::FRAG);
+    };
+    const auto read_columns = [&](const uint8_t* tile, v8bf (&a)[2][3]) {
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+            for (int part = 0; part < 3; ++part) a[ch][part] = read_transposed(tile + tr + part * F::FRAG + ch * 256, 128);
+    };
+    const auto contract = [](v16f& acc, const v8bf (&a)[2][3], const v8bf (&b)[2][3], bool from_zero) {
+        const v16f zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[c][SPLIT_TERMS[q][0]], b[c][SPLIT_TERMS[q][1]], from_zero && c == 0 && q == 0 ? zero : acc, 0, 0, 0);
+    };
+    const auto parts_of = [](const v4f& x0, const v4f& x1, v8bf (&out)[3]) {
+        uint2 lo[3], hi[3];
+        split4(x0, lo);
+        split4(x1, hi);
+#pragma unroll
+        for (int part = 0; part < 3; ++part) out[part] = pack_parts(lo[part], hi[part]);
+    };
+
+    v8bf kb[2][3], vb[2][3], kt[2][3], fs[2][3];
+    v16f acc_k, acc_v;
+
+    // One step of this wave: 32 queries, its 32 keys.  Fragments are read a phase ahead of their MFMAs.
+    const auto tile_step = [&](const Step& s, const Step& next, int n) {
+        const uint8_t* const stage = back_lds + (n & 1) * F::STAGE;
+        uint8_t* const region = regions + ((n & 1) * NW + wave) * F::REGION;
+        const bool no_key = s.g0 + wave * 32 + j >= L;
+        const float* const lse_at = reinterpret_cast<const float*>(no_key ? no_key_lds : stage + 2 * F::TILE) + 4 * half;
+        // ---- S[query][key]: this lane's key, 16 of the tile's queries; beside it, the next tile goes to LDS
+        v16f st, ds;
+        v8bf fd[2][3], fo[2][3], fq[2][3];
+        contract(st, fs, kb, true);
+        read_rows(stage + F::TILE, fd);
+        stage_put(n + 1);
+        stage_load();
+        interleave<12, 6>();
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- dO V^T; beside it, the probabilities and their parts
+        contract(ds, fd, vb, true);
+        read_columns(stage + F::TILE, fo);
+        if (BIAS)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) st[r] = __builtin_fmaf(bv[r], LOG2E, st[r]);
+        if (CAUSAL) {                                      // keys behind the query: P = 0
+            const int first = s.g0 + wave * 32 + j - s.t * 32 - 4 * half;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) st[r] = 8 * (r >> 2) + (r & 3) >= first ? st[r] : -INFINITY;
+        }
+        v8bf wp[2][3], wd[2][3];
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+#pragma unroll
+            for (int g = 2 * ch; g < 2 * ch + 2; ++g) {
+                const v4f lse4 = *reinterpret_cast<const v4f*>(lse_at + 8 * g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) st[4 * g + i] = __builtin_amdgcn_exp2f(st[4 * g + i] - lse4[i]);
+            }
+            parts_of(v4f{st[8 * ch], st[8 * ch + 1], st[8 * ch + 2], st[8 * ch + 3]}, v4f{st[8 * ch + 4], st[8 * ch + 5], st[8 * ch + 6], st[8 * ch + 7]}, wp[ch]);
+        }
+        interleave<12, 11>();
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- dV^T += dO^T . P; beside it, dS and its parts, which also go to LDS to be transposed
+        contract(acc_v, fo, wp, false);
+        int put_at = j * 64 + ((half ^ (j >> 2)) & 7) * 8; // (opaque: the four pieces' places are formed from this one, not held)
+        asm volatile("" : "+v"(put_at));
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+#pragma unroll
+            for (int g = 2 * ch; g < 2 * ch + 2; ++g) {
+                const v4f D4 = *reinterpret_cast<const v4f*>(lse_at + 32 + 8 * g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) ds[4 * g + i] = st[4 * g + i] * (ds[4 * g + i] - D4[i]);
+            }
+            parts_of(v4f{ds[8 * ch], ds[8 * ch + 1], ds[8 * ch + 2], ds[8 * ch + 3]}, v4f{ds[8 * ch + 4], ds[8 * ch + 5], ds[8 * ch + 6], ds[8 * ch + 7]}, wd[ch]);
+            // piece of eight bytes: queries 4 u .. 4 u + 3, u = 4 ch + half and two further on
+#pragma unroll
+            for (int part = 0; part < 3; ++part) {
+                const v4i x = __builtin_bit_cast(v4i, wd[ch][part]);
+                *reinterpret_cast<uint2*>(region + part * F::PART + (put_at ^ (32 * ch))) = uint2{static_cast<uint32_t>(x[0]), static_cast<uint32_t>(x[1])};
+                *reinterpret_cast<uint2*>(region + part * F::PART + (put_at ^ (32 * ch + 16))) = uint2{static_cast<uint32_t>(x[2]), static_cast<uint32_t>(x[3])};
+            }
+        }
+        interleave<12, 10>();
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- dK^T += Q^T . dS; beside it, dbias = dS and the next step's bias (into the registers read above)
+        read_columns(stage, fq);
+        contract(acc_k, fq, wd, false);
+        v8bf w[2][3];
+        // keys 16 ch + 4 half + grp / 4 and eight further on, pieces of four queries (queries from 16 * (lane / 16 % 2))
+        int get_at = (4 * half + (grp >> 2)) * 64 + ((4 * ((lane >> 4) & 1) + (grp & 3)) ^ half) * 8;
+        asm volatile("" : "+v"(get_at));
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+#pragma unroll
+            for (int part = 0; part < 3; ++part) {
+                typedef __attribute__((address_space(3))) v4s* lds_v4s;
+                const uint8_t* const at = region + part * F::PART + ch * 1024;
+                const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at + (get_at ^ (32 * ch))));
+                const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at + 512 + (get_at ^ (32 * ch + 16))));
+                w[ch][part] = __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+        }
+        load_bias(next);
+        store_dbias(s, ds);
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- this wave's share of dQ^T = K^T . dS^T: lane = query
+        v16f dq;
+        contract(dq, kt, w, true);
+        float* const part_at = reinterpret_cast<float*>(region) + j * F::QP + 4 * half;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) *reinterpret_cast<v4f*>(part_at + 8 * g) = v4f{dq[4 * g], dq[4 * g + 1], dq[4 * g + 2], dq[4 * g + 3]};
+    };
+
+    Step s{static_cast<int>(blockIdx.x), 0, 0};
+    stage_load();
+    load_bias(s);
+    stage_put(0);
+    stage_load();
+    __syncthreads();
+    read_rows(back_lds, fs);
+    int n = 0;                                             // steps so far: which half of the double buffers a step uses
+    while (s.plane < p.planes) {
+        // ---- a round begins: this wave's slices of K and V as B operands over the features, K^T as the A operand of
+        // dQ^T (lane = feature, its keys in the order of the transposed dS).  All loads before the first use: one round trip.
+        {
+            const __amdgpu_buffer_rsrc_t rk = rsrc(p.K + s.plane * mat, mat_bytes), rv = rsrc(p.V + s.plane * mat, mat_bytes);
+            const int k0w = s.g0 + wave * 32, key = k0w + j;
+            v4f xk[2][2], xv[2][2];
+            float xt[16];
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int e = 16 * c + 8 * half + 4 * i;
+                    const uint32_t at = key < L && e < d ? (static_cast<uint32_t>(key) * d + e) * 4u : OUT;
+                    xk[c][i] = load4(rk, at);
+                    xv[c][i] = load4(rv, at);
+                }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int kk = k0w + 8 * (i >> 2) + 4 * half + (i & 3);
+                xt[i] = load1(rk, kk < L && j < d ? (static_cast<uint32_t>(kk) * d + j) * 4u : OUT);
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                parts_of(xk[c][0] * (p.scale * LOG2E), xk[c][1] * (p.scale * LOG2E), kb[c]);
+                parts_of(xv[c][0], xv[c][1], vb[c]);
+                parts_of(v4f{xt[8 * c], xt[8 * c + 1], xt[8 * c + 2], xt[8 * c + 3]}, v4f{xt[8 * c + 4], xt[8 * c + 5], xt[8 * c + 6], xt[8 * c + 7]}, kt[c]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { acc_k[r] = 0.0f; acc_v[r] = 0.0f; }
+        const Step round = s;
+        for (int t = 0; t < tiles; ++t, ++n) {
+            Step next = s;
+            advance(next);
+            tile_step(s, next, n);
+            // the tile's shares are complete and the next tile is staged; the next write to this region is two steps away
+            __syncthreads();
+            read_rows(back_lds + ((n + 1) & 1) * F::STAGE, fs);
+            if (p.dQ) add_shares(s, n);
+            s = next;
+        }
+        const int key = round.g0 + wave * 32 + j;
+        if (key < L) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int dd = 8 * g + 4 * half;
+                if (dd >= d) continue;
+                const int64_t off = round.plane * mat + static_cast<int64_t>(key) * d + dd;
+                if (p.dK) *reinterpret_cast<v4f*>(p.dK + off) = v4f{acc_k[4 * g] * p.scale, acc_k[4 * g + 1] * p.scale, acc_k[4 * g + 2] * p.scale, acc_k[4 * g + 3] * p.scale};
+                if (p.dV) *reinterpret_cast<v4f*>(p.dV + off) = v4f{acc_v[4 * g], acc_v[4 * g + 1], acc_v[4 * g + 2], acc_v[4 * g + 3]};
+            }
+        }
+    }
+}
+
+template <int NW, bool BIAS, int DB, bool CAUSAL>
+int launch_fused(const AttnBackParams& p, hipStream_t stream) {
+    using F = FusedBack<NW>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_attn_back_fused_kernel<NW, BIAS, DB, CAUSAL>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(F::LDS));
+    if (attr != hipSuccess) {
+        (void)hipGetLastError();
+        set_error("flash_attn_backward_hip: cannot reserve the LDS of the one-pass kernel");
+        return RC_LAUNCH;
+    }
+    const int resident = device_cu_count() * (NW >= 8 ? 1 : 2);
+    hipLaunchKernelGGL((flash_attn_back_fused_kernel<NW, BIAS, DB, CAUSAL>), dim3(p.planes < resident ? p.planes : resident), dim3(NW * 64), F::LDS, stream, p);
+    return check_launch("flash_attn_back_fused_kernel");
+}
+
 template <int DP>
 int launch_back(AttnBackParams p, hipStream_t stream) {
     using T = BackTiling<DP>;
@@ -521,5 +941,21 @@ extern "C" int flash_attn_backward_hip(int B, int h, int L, int d, int causal, f
     p.stage_rows = 0;
     StatsScope stat("hip/flash_attn_back", static_cast<int64_t>(planes) * L, d, L, static_cast<hipStream_t>(stream));
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // One pass where a head fits one feature block.  Beyond 256 rows a work-group walks over a plane in rounds while the
+    // two kernels have a work-group per 128 rows: they stay the better choice until the planes alone fill the chip (us, one
+    // pass / two kernels: 64 planes of 384 rows 91 / 75, 128 of them 92 / 105; of 640 rows 217 / 162 and 233 / 290).  The
+    // choice does not look at which gradients are wanted: a subset has the bits of the whole.
+    if (d <= 32 && L < 16384 && (L <= 256 || planes * 8 >= 3 * device_cu_count())) {
+        const bool streaming = L % 32 == 0 && (reinterpret_cast<uintptr_t>(dbias) & 127) == 0;
+        const int db = !dbias ? DB_NONE : streaming ? DB_STREAM : DB_ORDINARY;
+        const int kt = (L + 31) / 32;
+#define PPML_BACK_DB(NW_, BIAS_, C_) (db == DB_NONE ? launch_fused<NW_, BIAS_, DB_NONE, C_>(p, s) : db == DB_STREAM ? launch_fused<NW_, BIAS_, DB_STREAM, C_>(p, s) : launch_fused<NW_, BIAS_, DB_ORDINARY, C_>(p, s))
+#define PPML_BACK_B(NW_, C_) (bias ? PPML_BACK_DB(NW_, true, C_) : PPML_BACK_DB(NW_, false, C_))
+#define PPML_BACK(NW_) (causal ? PPML_BACK_B(NW_, true) : PPML_BACK_B(NW_, false))
+        return kt <= 4 ? PPML_BACK(4) : PPML_BACK(8);
+#undef PPML_BACK
+#undef PPML_BACK_B
+#undef PPML_BACK_DB
+    }
     return d <= 32 ? launch_back<32>(p, s) : launch_back<64>(p, s);
 }

@@ -215,6 +215,37 @@ def test_flash_attn_backward_matches_oracle(ops, oracle, B, h, L, d, causal, use
         assert (np.triu(db[0, 0], 1) == 0).all()
 
 
+@pytest.mark.parametrize("planes,L,d,causal,use_bias", [
+    (2, 31, 32, False, True), (2, 32, 8, False, False), (3, 33, 32, True, True),      # one key tile, whole and ragged
+    (2, 129, 32, False, True), (2, 255, 24, False, True), (1, 256, 32, True, False),  # four waves' keys and one more, eight waves'
+    (100, 257, 4, False, True), (97, 288, 32, True, True),                            # a second round of keys (dQ added to), ragged and whole
+    (520, 40, 32, False, True),                                                       # more planes than work-groups: loads run on into the next plane
+])
+def test_flash_attn_backward_in_one_pass(ops, planes, L, d, causal, use_bias):
+    """The one-pass kernel at the edges of its key tiles, rounds and plane lists, against the same gradients in binary64."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(L * 7 + d)
+    q, k, v, do = (torch.randn(1, planes, L, d, device="cuda", generator=g) for _ in range(4))
+    bias = torch.randn(1, planes, L, L, device="cuda", generator=g) if use_bias else None
+    if use_bias:
+        bias[0, :, 1, :] -= 200.0                   # a row whose LSE lies far below zero: a key past the matrix must not see exp(0 - LSE)
+    o, lse = ops.flash_attn_forward(q, k, v, bias, causal=causal)
+    got = ops.flash_attn_backward(q, k, v, bias, o, do, lse, causal=causal)
+    Q, K, V, DO = (t[0].double() for t in (q, k, v, do))
+    s = torch.matmul(Q, K.transpose(1, 2).contiguous()) / np.sqrt(d)
+    if use_bias:
+        s = s + bias[0].double()
+    if causal:
+        s = s.masked_fill(torch.ones(L, L, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    p = torch.softmax(s, -1)
+    ds = p * (torch.matmul(DO, V.transpose(1, 2).contiguous()) - (DO * torch.matmul(p, V)).sum(-1, keepdim=True))
+    want = (torch.matmul(ds, K) / np.sqrt(d), torch.matmul(ds.transpose(1, 2).contiguous(), Q) / np.sqrt(d),
+            torch.matmul(p.transpose(1, 2).contiguous(), DO), ds)
+    for x, w, name in zip(got, want, ("dQ", "dK", "dV", "dbias")):
+        x, w = x[0].cpu().numpy(), w.cpu().numpy()
+        _check_grad(x, w, name)        # (logits near -200 carry 2^-16 of rounding, exp(LSE - ...) as much: 3e-5)
+
+
 def test_flash_attn_backward_subsets_and_determinism(ops, oracle):
     rng = np.random.default_rng(77)
     B, h, L, d = 1, 3, 90, 32
