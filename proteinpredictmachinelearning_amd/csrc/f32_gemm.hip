@@ -137,10 +137,10 @@ __device__ __forceinline__ void store_tile(float* __restrict__ lds, int tid, con
 
 // work-group -> (plane, tile row, tile col); bands of 8 tile rows keep operand panels in one L2
 template <int TILE_M = BM>
-__device__ __forceinline__ void tile_of_group(const GemmParams& p, int& plane, int& m0, int& n0) {
+__device__ __forceinline__ void tile_of_group(const GemmParams& p, int& plane, int& m0, int& n0, int group) {
     const int tiles = p.tiles_m * p.tiles_n;
     const int total = tiles * p.np2 * p.np3;
-    const int idx = xcd_contiguous_index(blockIdx.x, total);
+    const int idx = xcd_contiguous_index(group, total);
     plane = idx / tiles;
     int t = idx - plane * tiles;
     const int band_rows = 8;
@@ -151,6 +151,11 @@ __device__ __forceinline__ void tile_of_group(const GemmParams& p, int& plane, i
     const int tn = t / rows_here;
     m0 = tm * TILE_M;
     n0 = tn * BN;
+}
+
+template <int TILE_M = BM>
+__device__ __forceinline__ void tile_of_group(const GemmParams& p, int& plane, int& m0, int& n0) {
+    tile_of_group<TILE_M>(p, plane, m0, n0, static_cast<int>(blockIdx.x));
 }
 
 // The finished accumulators of one wave (TI x 2 tiles of 32 x 32) (rows from m_base, columns from n_base) go to C.
@@ -746,14 +751,14 @@ __global__ __launch_bounds__(256) void gemm_bf16x3_kernel(const GemmParams p) {
 // more tiles than CUs (26368 x 256 -> 256 and wider, the many-plane contractions) the work-groups of a CU overlap
 // each other anyway and the two forms measure the same: the launcher takes this one up to one tile per CU.
 constexpr int PC_AHEAD = 3;                       // chunks a producer wave has in flight
-template <int MODE, bool STREAM_C, bool K4, int BMODE = MODE>
-__global__ __launch_bounds__(512) void gemm_bf16x3_pc_kernel(const GemmParams p) {
+constexpr int PC_STAGE = 3 * SPLIT_PLANE;         // the three planes of one operand's chunk
+template <int MODE, bool STREAM_C, bool K4, int BMODE>
+__device__ __forceinline__ void pc_tile(const GemmParams& p, uint8_t (&lds_ab)[2][2 * PC_STAGE], int group) {
     // (MODE: how A lies; BMODE: how B lies -- the backward of the triangle multiplication contracts a gradient that is
     // contiguous in k with an operand that is contiguous in its rows)
     static_assert(MODE == LOAD_ROW_CONTIG || MODE == LOAD_K_CONTIG, "buffer addressing");
     static_assert(BMODE == LOAD_ROW_CONTIG || BMODE == LOAD_K_CONTIG, "buffer addressing");
-    constexpr int STAGE = 3 * SPLIT_PLANE;            // the three planes of one operand's chunk
-    __shared__ __attribute__((aligned(16))) uint8_t lds_ab[2][2 * STAGE];
+    constexpr int STAGE = PC_STAGE;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -764,7 +769,7 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_kernel(const GemmParams p)
     const int wm = (cw >> 1) * 64, wn = (cw & 1) * 64;
 
     int plane, m0, n0;
-    tile_of_group(p, plane, m0, n0);
+    tile_of_group(p, plane, m0, n0, group);
     const int p2 = plane % p.np2, p3 = plane / p.np2;
     const float* A = p.A + p2 * p.a_p2 + p3 * p.a_p3;
     const float* B = p.B + (p2 / p.b_div2) * p.b_p2 + (p3 / p.b_div3) * p.b_p3;
@@ -853,6 +858,25 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_kernel(const GemmParams p)
         const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(C, 0, static_cast<int>(p.M * p.c_mi * 4), 0x00020000);
         store_acc_buffer<STREAM_C>(rsrc_c, static_cast<uint32_t>(p.c_mi) * 4u, p.N, p.alpha, acc, m0 + wm, n0 + wn, lane);
     }
+}
+
+template <int MODE, bool STREAM_C, bool K4, int BMODE = MODE>
+__global__ __launch_bounds__(512) void gemm_bf16x3_pc_kernel(const GemmParams p) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds_ab[2][2 * PC_STAGE];
+    pc_tile<MODE, STREAM_C, K4, BMODE>(p, lds_ab, static_cast<int>(blockIdx.x));
+}
+
+// Two independent contractions of that kind in one launch (the two gradients of the triangle multiplication): the first
+// groups_a work-groups take the tiles of `a`, the others those of `b`.  With one tile per plane, as the pair tensor has up
+// to 128 residues, each of the two by itself leaves half of the CUs idle and is a single latency chain (load, split, seven
+// chunks, store) that the other has to wait for.  Either tile is what the launch for it alone computes: same bits.
+// Measured on 128 planes of 103 x 103 x 103: forward and both gradients 31.4 -> 23.0 us, the forward call's 9 in both.
+template <int MODE_A, int BMODE_A, int MODE_B, int BMODE_B, bool STREAM_C, bool K4>
+__global__ __launch_bounds__(512) void gemm_bf16x3_pc_pair_kernel(const GemmParams a, const GemmParams b, int groups_a) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds_ab[2][2 * PC_STAGE];
+    const int group = static_cast<int>(blockIdx.x);
+    if (group < groups_a) pc_tile<MODE_A, STREAM_C, K4, BMODE_A>(a, lds_ab, group);
+    else pc_tile<MODE_B, STREAM_C, K4, BMODE_B>(b, lds_ab, group - groups_a);
 }
 
 // gemm_bf16x3_pc_kernel for a few output tiles under a long K (a LinearLayer's weight gradient: 256 x 768 outputs over
@@ -2198,24 +2222,62 @@ bool try_pc_slices_done(const GemmParams& p, hipStream_t stream, const char* wha
     return rc >= 0;
 }
 
+// Streaming (non-temporal) stores where every store instruction writes whole 128-byte lines: dense rows of a
+// multiple of 32 floats, on a 128-byte boundary, in every plane.  Ordinary stores leave the output dirty in the
+// XCDs' L2s, which are written back when the kernel ends; streaming ones go out as they are issued.  Measured
+// on the attention-logit kernels (us, streaming / ordinary): 100 planes of 128 x 128  4.8 / 6.1, 400 of them
+// 8.0 / 10.9, 2000 of them 30.5 / 42.7, 824 planes of 256 x 256  49 / 54.  With rows that are not whole lines
+// it is the other way round at every size (412 planes of 103 x 103  12.3 / 10.0, 3200 of them 100 / 49:
+// partial lines are merged in L2 only by ordinary stores).  Outputs with compound addressing keep the older
+// rule (streaming from 128 MB on: 72 -> 63 us on the 216 MB logits at the time).
+bool streams_output(const GemmParams& p) {
+    const bool compound = !(p.c_lm >= p.M && p.c_ln >= p.N);
+    const bool planes_ok = (p.np2 == 1 || p.c_p2 % 32 == 0) && (p.np3 == 1 || p.c_p3 % 32 == 0);
+    const bool whole_lines = !compound && p.c_ni == 1 && p.c_mi % 32 == 0 && p.N % 32 == 0 && planes_ok &&
+                             (reinterpret_cast<uintptr_t>(p.C) & 127) == 0;
+    return compound ? static_cast<int64_t>(p.M) * p.N * p.np2 * p.np3 * 4 >= (128LL << 20) : whole_lines;
+}
+
+// Both gradients of the triangle multiplication in one launch (gemm_bf16x3_pc_pair_kernel); -1 when one of the two is not
+// of the kind that launch_gemm gives to gemm_bf16x3_pc_kernel with at most one tile per CU (beyond that each fills the
+// chip by itself) or the two do not lie as one of the two instances has them, and the caller launches them one by one.
+int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what) {
+    if (f32_arithmetic() == 1) return -1;
+    const auto kmode = [](int64_t rs, int64_t ks) { return ks == 1 ? LOAD_K_CONTIG : rs == 1 ? LOAD_ROW_CONTIG : LOAD_STRIDED; };
+    for (GemmParams* p : {&a, &b}) {
+        p->tiles_m = (p->M + BM - 1) / BM;
+        p->tiles_n = (p->N + BN - 1) / BN;
+        p->stream_c = streams_output(*p);
+        if (static_cast<int64_t>(p->tiles_m) * p->tiles_n * p->np2 * p->np3 > device_cu_count()) return -1;
+        if (p->M <= 32 || p->N <= 32 || p->K <= 3 * BK || p->np2 * p->np3 == 1 || p->bias || p->clamp || p->f16_in || p->a_lm > 0) return -1;
+        if (p->c_ni != 1 || p->c_lm < p->M || p->c_ln < p->N) return -1;
+        // buffer addressing: every plane below 2 GiB, and the launcher's bounds on the pitches
+        const auto reach = [&](int64_t rs, int64_t ks, int64_t rows) {
+            return ks == 1 ? ((rows - 1) * rs + p->K) * 4 < (1LL << 31) && rs < (1 << 22) : p->K * ks * 4 < (1LL << 31) && ks < (1 << 24);
+        };
+        if (!reach(p->a_rs, p->a_ks, p->M) || !reach(p->b_rs, p->b_ks, p->N)) return -1;
+        if (p->M * p->c_mi * 4 >= (1LL << 31) || p->c_mi >= (1 << 22)) return -1;
+    }
+    const int am = kmode(a.a_rs, a.a_ks), ab = kmode(a.b_rs, a.b_ks), bm = kmode(b.a_rs, b.a_ks), bb = kmode(b.b_rs, b.b_ks);
+    const bool outgoing = am == LOAD_K_CONTIG && ab == LOAD_ROW_CONTIG && bm == LOAD_ROW_CONTIG && bb == LOAD_ROW_CONTIG;
+    const bool incoming = am == LOAD_K_CONTIG && ab == LOAD_K_CONTIG && bm == LOAD_K_CONTIG && bb == LOAD_ROW_CONTIG;
+    if ((!outgoing && !incoming) || a.stream_c != b.stream_c) return -1;
+    const bool k4 = a.K % 4 == 0 && (outgoing || b.K % 4 == 0);      // (loads along k; the outgoing `b` has none)
+    const int groups_a = a.tiles_m * a.tiles_n * a.np2 * a.np3, groups_b = b.tiles_m * b.tiles_n * b.np2 * b.np3;
+    const dim3 grid(static_cast<unsigned>(groups_a + groups_b)), block(512);
+#define PPML_PAIR(AB_, BM_, STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_pc_pair_kernel<LOAD_K_CONTIG, AB_, BM_, LOAD_ROW_CONTIG, STREAM_, K4_>), grid, block, 0, stream, a, b, groups_a)
+#define PPML_PAIR_K4(AB_, BM_, STREAM_) do { if (k4) PPML_PAIR(AB_, BM_, STREAM_, true); else PPML_PAIR(AB_, BM_, STREAM_, false); } while (0)
+    if (outgoing) { if (a.stream_c) PPML_PAIR_K4(LOAD_ROW_CONTIG, LOAD_ROW_CONTIG, true); else PPML_PAIR_K4(LOAD_ROW_CONTIG, LOAD_ROW_CONTIG, false); }
+    else          { if (a.stream_c) PPML_PAIR_K4(LOAD_K_CONTIG, LOAD_K_CONTIG, true); else PPML_PAIR_K4(LOAD_K_CONTIG, LOAD_K_CONTIG, false); }
+#undef PPML_PAIR_K4
+#undef PPML_PAIR
+    return check_launch(what);
+}
+
 int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fixed_ws = nullptr, size_t fixed_cap = 0) {
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
-    // Streaming (non-temporal) stores where every store instruction writes whole 128-byte lines: dense rows of a
-    // multiple of 32 floats, on a 128-byte boundary, in every plane.  Ordinary stores leave the output dirty in the
-    // XCDs' L2s, which are written back when the kernel ends; streaming ones go out as they are issued.  Measured
-    // on the attention-logit kernels (us, streaming / ordinary): 100 planes of 128 x 128  4.8 / 6.1, 400 of them
-    // 8.0 / 10.9, 2000 of them 30.5 / 42.7, 824 planes of 256 x 256  49 / 54.  With rows that are not whole lines
-    // it is the other way round at every size (412 planes of 103 x 103  12.3 / 10.0, 3200 of them 100 / 49:
-    // partial lines are merged in L2 only by ordinary stores).  Outputs with compound addressing keep the older
-    // rule (streaming from 128 MB on: 72 -> 63 us on the 216 MB logits at the time).
-    {
-        const bool compound = !(p.c_lm >= p.M && p.c_ln >= p.N);
-        const bool planes_ok = (p.np2 == 1 || p.c_p2 % 32 == 0) && (p.np3 == 1 || p.c_p3 % 32 == 0);
-        const bool whole_lines = !compound && p.c_ni == 1 && p.c_mi % 32 == 0 && p.N % 32 == 0 && planes_ok &&
-                                 (reinterpret_cast<uintptr_t>(p.C) & 127) == 0;
-        p.stream_c = compound ? static_cast<int64_t>(p.M) * p.N * p.np2 * p.np3 * 4 >= (128LL << 20) : whole_lines;
-    }
+    p.stream_c = streams_output(p);
     const int64_t total = static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.np2 * p.np3;
     if (total <= 0 || total > 0x7fffffffLL) { set_error("%s: grid of %lld work-groups is out of range", what, (long long)total); return RC_BAD_ARGS; }
     const dim3 grid(static_cast<unsigned>(total)), block(256);
@@ -2753,10 +2815,9 @@ extern "C" int tri_mul_back_hip(const float* grad, const float* left, const floa
     //   outgoing  gleft[i][k]  = sum_j grad[i][j] * right[j][k]     gright[j][k] = sum_i grad[i][j] * left[i][k]
     //   incoming  gleft[k][i]  = sum_j grad[i][j] * right[k][j]     gright[k][j] = sum_i grad[i][j] * left[k][i]
     // Every one is a contraction with one stride per operand index, i.e. a launch of the strided kernel.
-    const auto launch = [&](const float* a, int64_t a_rs, int64_t a_ks, const float* b, int64_t b_rs, int64_t b_ks,
+    const auto contraction = [&](const float* a, int64_t a_rs, int64_t a_ks, const float* b, int64_t b_rs, int64_t b_ks,
                             float* c, int64_t c_mi, int64_t c_ni, int64_t M, int64_t N, int64_t Kc,
                             int64_t a_p3, int64_t b_p3, int64_t c_p3) {
-        StatsScope stat("hip/tri_mul_back", M, Kc, N, static_cast<hipStream_t>(stream));
         GemmParams p = plain_params();
         // an output whose ROW index runs along memory is the dense plane of the transposed product: the operands trade
         // places (the fast forms of the contraction store dense planes)
@@ -2770,15 +2831,35 @@ extern "C" int tri_mul_back_hip(const float* grad, const float* left, const floa
         p.a_p2 = 1; p.b_p2 = 1; p.c_p2 = 1;
         p.a_p3 = (swap ? b_p3 : a_p3) * B; p.b_p3 = (swap ? a_p3 : b_p3) * B; p.c_p3 = c_p3 * B;
         p.alpha = inv_L;
-        return launch_gemm(p, static_cast<hipStream_t>(stream), "tri_mul_back_hip");
+        return p;
     };
-    int rc = RC_OK;
+    GemmParams of_left{}, of_right{};
     if (outgoing) {
-        if (gleft)  rc = launch(grad, J, 1, right, 1, K, gleft, K, 1, I, K, J, I * J, J * K, I * K);
-        if (rc == RC_OK && gright) rc = launch(grad, 1, J, left, 1, K, gright, K, 1, J, K, I, I * J, I * K, J * K);
+        if (gleft)  of_left = contraction(grad, J, 1, right, 1, K, gleft, K, 1, I, K, J, I * J, J * K, I * K);
+        if (gright) of_right = contraction(grad, 1, J, left, 1, K, gright, K, 1, J, K, I, I * J, I * K, J * K);
     } else {
-        if (gleft)  rc = launch(grad, J, 1, right, J, 1, gleft, 1, I, I, K, J, I * J, K * J, K * I);
-        if (rc == RC_OK && gright) rc = launch(grad, 1, J, left, I, 1, gright, 1, J, J, K, I, I * J, K * I, K * J);
+        if (gleft)  of_left = contraction(grad, J, 1, right, J, 1, gleft, 1, I, I, K, J, I * J, K * J, K * I);
+        if (gright) of_right = contraction(grad, 1, J, left, I, 1, gright, 1, J, J, K, I, I * J, K * I, K * J);
+    }
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    // One launch for both, unless calls are being counted and timed (one row per contraction) or gright shares memory
+    // with what the first contraction reads or writes (in turn, it may).
+    const auto apart = [](const float* x, int64_t nx, const float* y, int64_t ny) {
+        const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+        return x0 + static_cast<uintptr_t>(nx) * 4 <= y0 || y0 + static_cast<uintptr_t>(ny) * 4 <= x0;
+    };
+    if (gleft && gright && !stats_enabled() && apart(gright, D * J * K * B, right, D * J * K * B) && apart(gright, D * J * K * B, gleft, D * I * K * B)) {
+        const int rc = try_pc_pair(of_left, of_right, s, "tri_mul_back_hip");
+        if (rc >= 0) return rc;
+    }
+    int rc = RC_OK;
+    if (gleft) {
+        StatsScope stat("hip/tri_mul_back", I, J, K, s);
+        rc = launch_gemm(of_left, s, "tri_mul_back_hip");
+    }
+    if (rc == RC_OK && gright) {
+        StatsScope stat("hip/tri_mul_back", J, I, K, s);
+        rc = launch_gemm(of_right, s, "tri_mul_back_hip");
     }
     return rc;
 }

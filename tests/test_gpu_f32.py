@@ -780,6 +780,25 @@ def test_tri_mul_back(ops, oracle, D, I, J, K, Bt, outgoing):
     assert none is None and np.array_equal(gr.cpu().numpy(), wr)
 
 
+# both gradients in one launch against each by itself, bit for bit: contractions of 49 (four 16-k chunks, the shortest) to
+# 200, whole and ragged lengths along k, rows of whole lines (streaming stores) and not, several tiles per plane, a total
+# just at and just above one tile per CU, and an operand the split cannot carry in one gradient's tile only
+@pytest.mark.parametrize("outgoing", [True, False])
+@pytest.mark.parametrize("D,I,J,K", [(2, 49, 49, 49), (4, 64, 96, 64), (3, 130, 51, 70), (2, 200, 52, 129), (128, 52, 50, 33), (129, 140, 50, 40),
+                                     (1, 60, 60, 60)])
+def test_tri_mul_back_pair(ops, D, I, J, K, outgoing):
+    rng = np.random.default_rng(D + I + J + K)
+    left, right, grad = (_dev(rng.standard_normal(n).astype(np.float32)) for n in (D * I * K, D * J * K, D * I * J))
+    right[5] = float("inf")                             # in plane 0 of the left gradient's operand alone
+    args = (D, I, J, K, 1, 3.0, outgoing)
+    gl, gr = ops.tri_mul_back(grad, left, right, *args)
+    one_l, _ = ops.tri_mul_back(grad, left, right, *args, want_right=False)
+    _, one_r = ops.tri_mul_back(grad, left, right, *args, want_left=False)
+    assert np.array_equal(gl.cpu().numpy(), one_l.cpu().numpy(), equal_nan=True)
+    assert np.array_equal(gr.cpu().numpy(), one_r.cpu().numpy(), equal_nan=True)
+    assert not np.isfinite(gl.cpu().numpy()).all() and np.isfinite(gr.cpu().numpy()).all()
+
+
 # (3, 4, 8), (8, 48, 64, 2): the generic kernel (a short pair tensor; a batch); the others: the gradient tensor split in
 # the tile loop -- runs of whole 16-k chunks (L a multiple of 16) and of any length (103, 50, 40), ragged rows (2176 =
 # 17 tiles) and columns, two to eight K slices, up to four column tiles
