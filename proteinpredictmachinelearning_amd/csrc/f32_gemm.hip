@@ -47,6 +47,7 @@ struct GemmParams {
     int64_t c_mo, c_mi, c_no, c_ni;
     int tiles_m, tiles_n;
     int stream_c;         // output larger than the last-level cache: write it with streaming stores
+    uint32_t c_span;      // compound output: bytes from C to behind a plane's last element where buffer addressing reaches them, else 0
     int f16_in;           // A and B hold IEEE halves (k contiguous); products and sums are binary32
     int clamp;            // finite guard in the epilogue (triangle multiplication)
     // LOAD_SPLIT_A: both indices of A are compound, A(m,k) = A[(m/a_lm)*a_mo + (m%a_lm)*a_mi + (k/a_lk)*a_ko + (k%a_lk)*a_ki]
@@ -204,6 +205,53 @@ __device__ __forceinline__ void store_acc(const GemmParams& p, float* __restrict
                 if (CLAMP) v = (v != v) ? 0.0f : (v > 1e4f ? 1e4f : (v < -1e4f ? -1e4f : v));
                 if (STREAM_C) __builtin_nontemporal_store(v, &C[roff + coff]);
                 else C[roff + coff] = v;
+            }
+        }
+    }
+}
+
+// The same for an output with compound addressing whose planes 32-bit byte offsets reach (p.c_span, set by the launcher:
+// below 2 GiB, row runs of at least 32).  The general form above spends 36 vector instructions per stored register on
+// 64-bit addresses, carries and bounds, in a phase without matrix work (a third of all issue cycles of the contraction of
+// 12288 x 12288 outputs over 256).  Here a tile of 32 rows that stays within one run and inside the matrix -- known per
+// wave -- takes its row steps from scalar registers: a product and a store.  Other tiles pick the run per row.  Measured,
+// with both gradients: 384 residues x 32 features x 256 sequences 1342 -> 1239 us, 103 residues 152 -> 145.
+template <bool STREAM_C, int TI>
+__device__ __forceinline__ void store_acc_compound_buffer(const GemmParams& p, float* __restrict__ C, const v16f (&acc)[TI][2],
+                                                          int m_base, int n_base, int lane) {
+    constexpr int AUX = STREAM_C ? 3 : 0;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(C, 0, static_cast<int>(p.c_span), 0x00020000);
+    const int j = lane & 31;
+    const int m_first = __builtin_amdgcn_readfirstlane(m_base);
+    const uint32_t mi_bytes = static_cast<uint32_t>(p.c_mi) * 4u;
+    const uint32_t carry = static_cast<uint32_t>(p.c_mo - p.c_lm * p.c_mi) * 4u;      // (modulo 2^32: only the sum has to be an offset)
+#pragma unroll
+    for (int ti = 0; ti < TI; ++ti) {
+        const int m0 = m_first + ti * 32;
+        const int q = m0 / p.c_lm, rem = m0 - q * p.c_lm;
+        const uint32_t row0 = static_cast<uint32_t>(q * p.c_mo + rem * p.c_mi) * 4u;
+        const bool whole = rem + 32 <= p.c_lm && m0 + 32 <= p.M;
+        const int own = 4 * (lane >> 5);               // this lane's first row of the tile
+#pragma unroll
+        for (int tj = 0; tj < 2; ++tj) {
+            const int n = n_base + tj * 32 + j;
+            if (n >= p.N) continue;
+            const int nq = n / p.c_ln;
+            const uint32_t base = row0 + own * mi_bytes + static_cast<uint32_t>(nq * p.c_no + (n - nq * p.c_ln) * p.c_ni) * 4u;
+            if (whole) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, acc[ti][tj][r] * p.alpha), rsrc, base,
+                                                          (8 * (r >> 2) + (r & 3)) * mi_bytes, AUX);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int step = 8 * (r >> 2) + (r & 3);
+                    uint32_t at = base + step * mi_bytes;
+                    if (rem + own + step >= p.c_lm) at += carry;                  // (at most one: the run is 32 or longer)
+                    if (m0 + own + step < p.M)
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, acc[ti][tj][r] * p.alpha), rsrc, at, 0, AUX);
+                }
             }
         }
     }
@@ -733,6 +781,7 @@ __global__ __launch_bounds__(256) void gemm_bf16x3_kernel(const GemmParams p) {
     }
 
     if (FAST_IO && !SPLIT_C) store_acc_buffer<STREAM_C>(rsrc_c, static_cast<uint32_t>(p.c_mi) * 4u, p.N, p.alpha, acc, m0 + wm, n0 + wn, lane);
+    else if (SPLIT_C && p.c_span) store_acc_compound_buffer<STREAM_C, 2>(p, C, acc, m0 + wm, n0 + wn, lane);
     else store_acc<SPLIT_C, STREAM_C, false, false>(p, C, acc, m0 + wm, n0 + wn, lane);
 }
 
@@ -2042,7 +2091,8 @@ __global__ __launch_bounds__(256, 2) void gemm_planes_kernel(const GemmParams p,
         plain_tile(p, p.A, p.B, p.C, m0, n0, PBM, BN, tid);
         return;
     }
-    store_acc<SPLIT_C, STREAM_C, false, false, 4>(p, p.C, acc, m0 + wm, n0 + wn, lane);
+    if (SPLIT_C && p.c_span) store_acc_compound_buffer<STREAM_C, 4>(p, p.C, acc, m0 + wm, n0 + wn, lane);
+    else store_acc<SPLIT_C, STREAM_C, false, false, 4>(p, p.C, acc, m0 + wm, n0 + wn, lane);
 }
 
 // C = alpha * (bias + sum over the K slices, in slice order) with the contraction's own output addressing
@@ -2282,6 +2332,11 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
     if (total <= 0 || total > 0x7fffffffLL) { set_error("%s: grid of %lld work-groups is out of range", what, (long long)total); return RC_BAD_ARGS; }
     const dim3 grid(static_cast<unsigned>(total)), block(256);
     const bool split = !(p.c_lm >= p.M && p.c_ln >= p.N);
+    if (split && p.c_lm >= 32) {
+        const int64_t last_m = std::min(p.c_lm, p.M) - 1, last_n = std::min(p.c_ln, p.N) - 1;
+        const int64_t span = (p.M - 1) / p.c_lm * p.c_mo + last_m * p.c_mi + (p.N - 1) / p.c_ln * p.c_no + last_n * p.c_ni + 1;
+        p.c_span = span * 4 < (1LL << 31) ? static_cast<uint32_t>(span * 4) : 0;
+    }
     int mode = LOAD_STRIDED;
     if (p.a_ks == 1 && p.b_ks == 1) mode = LOAD_K_CONTIG;
     else if (p.a_rs == 1 && p.b_rs == 1) mode = LOAD_ROW_CONTIG;

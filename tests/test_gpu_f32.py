@@ -655,6 +655,17 @@ def test_split_ahead_workspace_on_two_streams(ops):
         assert torch.equal(o, want1 if which == 1 else want2)
 
 
+# runs of one row tile (32), one more (33: every tile but the first crosses), ragged (47), several whole tiles (64, 96), a
+# batch; 2048 columns a side and more through the operands split ahead (whole tiles there, 99: crossing ones), and the
+# shortest run that keeps the general form (31)
+@pytest.mark.parametrize("D,L,N,B", [(5, 32, 32, 1), (5, 33, 32, 1), (9, 47, 16, 1), (4, 64, 16, 2), (3, 96, 16, 1), (5, 31, 16, 1), (48, 128, 8, 1), (60, 99, 8, 1)])
+def test_outer_prod_mean_compound_store(ops, oracle, D, L, N, B):
+    rng = np.random.default_rng(D * L)
+    l, r = (rng.integers(-3, 4, size=D * L * N * B).astype(np.float32) for _ in range(2))
+    got = ops.outer_product_mean(_dev(l), _dev(r), D, L, N, B).cpu().numpy()
+    assert np.array_equal(got, oracle.outer_prod_mean(l, r, D, L, N, B))
+
+
 def test_outer_product_mean_graph_form_large(ops, oracle):
     # D * L = 5888 rows a side: the graph form through the split-ahead path, compound output index
     D, L, N, B = 32, 184, 8, 1
