@@ -1278,7 +1278,10 @@ __global__ __launch_bounds__(512, 2) void gemm_bf16x3_half_split_kernel(const Ge
                 const uint32_t here = kd < nruns ? static_cast<uint32_t>(static_cast<int64_t>(kd) * p.a_ko + static_cast<int64_t>(kr) * p.a_ki) * 4u : NO_RUN;
                 const uint32_t next = kd + 1 < nruns ? static_cast<uint32_t>(static_cast<int64_t>(kd + 1) * p.a_ko + static_cast<int64_t>(kr - p.a_lk) * p.a_ki) * 4u : NO_RUN;
                 const int left = p.a_lk - kr;             // elements of the chunk that lie in this run
-                if (AMODE == HS_KRUN) {
+                if (AMODE == HS_KRUN && left >= BK && kd < nruns) {       // a chunk inside one run: as in the other form
+#pragma unroll
+                    for (int it = 0; it < 2; ++it) x[it] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, roff[it] + here, 0, 0));
+                } else if (AMODE == HS_KRUN) {
                     const int u0 = (ptid & 3) * 4;
 #pragma unroll
                     for (int it = 0; it < 2; ++it)
