@@ -161,6 +161,22 @@ def test_softmax_at_the_configured_attention_shapes_in_full(ops, oracle):
         np.testing.assert_allclose(got.sum(-1), 1.0, rtol=2e-6)
 
 
+# four rows per wave from 16384 rows on: the bits of the same rows taken in calls too small for that form, for every number
+# of rows in the last wave, rows of one and two pieces a lane and of whole sixteen-byte pieces, bias rows that end inside a wave
+@pytest.mark.parametrize("D,rest", [(1, 0), (63, 1), (65, 2), (103, 3), (127, 5), (4, 1), (128, 2), (256, 3)])
+def test_softmax_of_many_rows_has_the_bits_of_few(ops, D, rest):
+    rng = np.random.default_rng(D)
+    rows = 16384 + rest
+    x = _dev((3 * rng.standard_normal((rows, D))).astype(np.float32))
+    parts = torch.cat([ops.softmax(c.clone()) for c in x.split(5000)])
+    assert torch.equal(ops.softmax(x).view(torch.int32), parts.view(torch.int32))
+    for brows in (rows, next(d for d in range(7, 0, -1) if rows % d == 0)):
+        b = _dev((2 * rng.standard_normal((brows, D))).astype(np.float32))
+        two = ops.bcast_elemwise(x, b, "add")
+        want = torch.cat([ops.softmax(c.clone()) for c in two.split(5000)])
+        assert torch.equal(ops.softmax(x, bias=b).view(torch.int32), want.view(torch.int32)), brows
+
+
 @pytest.mark.parametrize("D", [1, 3, 64, 103, 256, 257, 512, 513, 2048, 2049, 5000])
 def test_softmax_with_the_bias_add_folded_in_has_the_bits_of_the_two_nodes(ops, oracle, D):
     rng = np.random.default_rng(D + 1)
