@@ -77,6 +77,35 @@ __global__ __launch_bounds__(256) void repeat_back_kernel(const RepeatBackJob jb
     jb.out[idx * jb.slices + slice] = sum;              // an element's runs side by side, for the wave that adds them
 }
 
+// The same sums where every copy of the destination is one contiguous stretch and the copies lie evenly (a bias gradient:
+// the rows of [rows][features]), in pieces of sixteen bytes: term k of element j at src[k * step + j].  A thread takes four
+// neighbouring elements, sixteen terms in flight, without the counters.  The runs and the order within them are those of
+// the general kernel: same bits.  (26368 x 768, 81 MB: 21.6 us at 3.7 TB/s, four bytes a lane
+// and the counters' branches between the loads; 16.7 us at 4.9 TB/s this way.)
+__global__ __launch_bounds__(256) void repeat_back_rows_kernel(const RepeatBackJob jb, int64_t step) {
+    const int64_t quads = jb.total / 4;
+    const int64_t gidx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (gidx >= quads * jb.slices) return;
+    const int64_t slice = gidx / quads;
+    const int64_t j = (gidx - slice * quads) * 4;
+    const int64_t begin = slice * jb.per_slice;
+    const int64_t end = begin + jb.per_slice < jb.reps ? begin + jb.per_slice : jb.reps;
+    const float* at = jb.src + begin * step + j;
+    v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    int64_t term = begin;
+    for (; term + 16 <= end; term += 16) {
+        v4f v[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const v4f*>(at + i * step);
+        at += 16 * step;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum += v[i];
+    }
+    for (; term < end; ++term) { sum += *reinterpret_cast<const v4f*>(at); at += step; }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) jb.out[(j + c) * jb.slices + slice] = sum[c];
+}
+
 // The runs of one destination element, added by one wave: lane l takes runs l, l + 64, ... in their order, then the
 // lanes' sums meet in a fixed butterfly -- a fixed function of the shapes, like everything else here.  (One thread
 // per element walking its runs one load at a time took longer than the sums themselves: 341 runs for a bias
@@ -153,7 +182,11 @@ extern "C" int repeat_back_hip(const float* src, float* dst,
     }
     jb.out = partial ? partial : dst;
     jb.slices = slices;
-    hipLaunchKernelGGL(repeat_back_kernel, dim3(static_cast<unsigned>((jb.total * slices + 255) / 256)), dim3(256), 0, s, jb);
+    // one stretch per copy: only dimension 1 repeats, over whole rows of a destination of one row
+    const bool rows = d1 == 1 && d2 == 1 && d3 == 1 && r0 == 1 && r2 == 1 && r3 == 1 && d0 % 4 == 0 && s0 % 4 == 0 &&
+                      (reinterpret_cast<uintptr_t>(src) & 15) == 0;
+    if (rows) hipLaunchKernelGGL(repeat_back_rows_kernel, dim3(static_cast<unsigned>((jb.total / 4 * slices + 255) / 256)), dim3(256), 0, s, jb, s0);
+    else hipLaunchKernelGGL(repeat_back_kernel, dim3(static_cast<unsigned>((jb.total * slices + 255) / 256)), dim3(256), 0, s, jb);
     int rc = check_launch("repeat_back_kernel");
     if (partial) {
         if (rc == RC_OK) {

@@ -90,3 +90,14 @@ def test_sizes_whose_products_would_wrap_are_refused(ops):
     assert lib.repeat_back_hip(p, p, big, big, 4, 1, big, big, 4, 1, 1, 1, 1, 1, None) == 1
     # a plain case still runs
     assert lib.repeat_back_hip(p, p, 16, 1, 1, 1, 4, 1, 1, 1, 4, 1, 1, 1, None) == 0
+
+
+# rows in pieces of sixteen bytes against the same rows behind an odd offset (the general kernel): same bits.  One run and
+# many, fewer than sixteen terms, remainders of a run
+@pytest.mark.parametrize("rows,n", [(1, 4), (15, 8), (63, 12), (64, 4), (1000, 132), (26368, 256)])
+def test_rows_in_pieces_have_the_bits_of_the_general_form(ops, rows, n):
+    rng = np.random.default_rng(rows + n)
+    a = torch.from_numpy(rng.standard_normal(1 + rows * n).astype(np.float32)).cuda()
+    odd = a[1:].view(rows, n)
+    assert odd.data_ptr() % 16 == 4
+    assert torch.equal(ops.repeat_back(odd.clone(), (n,)), ops.repeat_back(odd, (n,)))
