@@ -38,7 +38,7 @@ typedef float v2f __attribute__((ext_vector_type(2)));
 template <int DP, int NW> struct AttnTiling {
     // keys staged in LDS at a time: 36 KB per four-wave work-group (four of them share a CU and its
     // 160 KB; 128 keys would leave room for three, measured 64.7 against 61.2 us at the MSA shape)
-    static constexpr int CH = DP <= 32 ? (NW == 4 ? 96 : 192) : (NW == 4 ? 64 : 128);
+    static constexpr int CH = DP <= 32 ? (NW == 4 ? 96 : 128) : (NW == 4 ? 64 : 128);
     static constexpr int NC = DP / 16;                // 16-feature chunks of the score contraction
     // a 32-key tile of K in LDS: one 1 KB MFMA operand fragment per (chunk, bf16 part), [half][key][8 bf16]
     static constexpr int KT_BYTES = NC * 3 * 1024;
@@ -375,7 +375,9 @@ int launch_flash(AttnParams p, hipStream_t stream) {
     using T = AttnTiling<DP, NW>;
     auto kernel = &flash_attn_forward_kernel<DP, NW, PF>;
     const int l32 = (p.L + 31) / 32 * 32;
-    p.stage_rows = l32 < T::CH ? l32 : T::CH;
+    // stages of even size: 103 keys go 64 + 64, not 96 + 32 (412 planes with bias 16.1 -> 15.7 us)
+    const int stages = (l32 + T::CH - 1) / T::CH;
+    p.stage_rows = (l32 / 32 + stages - 1) / stages * 32;
     const size_t lds = static_cast<size_t>(p.stage_rows / 32) * (T::KT_BYTES + T::VT_BYTES);
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(T::lds_bytes));
@@ -428,10 +430,15 @@ extern "C" int flash_attn_forward_ex_hip(int B, int h, int L, int d, int causal,
     p.out_ld = (layout >> 1) & 1;
     StatsScope stat("hip/flash_attn", static_cast<int64_t>(planes) * L, d, L, static_cast<hipStream_t>(stream));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // Four-wave work-groups (128 queries): 824 planes of 256 queries make 1648 of them, which spread over
-    // 256 CUs more evenly than 824 eight-wave ones (6.4 per CU against 3.2, each rounded up).
+    // Four-wave work-groups (128 queries), eight-wave ones where they hold a whole plane that four-wave ones share between
+    // two: K and V are then staged and split once per plane, not twice (us, four / eight waves, 32 features with bias: 824
+    // planes of 160 44.0 / 37.7, 224 59.7 / 57.6, 256 91 / 88; 200 of 256 26.8 / 24.3, 64 of 256 21.0 / 20.4).  Beyond 256
+    // a plane does not end with its last work-group: 400 planes of 320 62 / 78, 400 of 384 95 / 112.
     const bool short_rows = L <= 128;
-    if (d <= 32) return short_rows ? launch_flash<32, 4, true>(p, s) : launch_flash<32, 4, false>(p, s);
+    if (d <= 32) {
+        if (short_rows) return launch_flash<32, 4, true>(p, s);
+        return L <= 256 ? launch_flash<32, 8, false>(p, s) : launch_flash<32, 4, false>(p, s);
+    }
     return short_rows ? launch_flash<64, 4, true>(p, s) : launch_flash<64, 4, false>(p, s);
 }
 

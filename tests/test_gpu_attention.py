@@ -75,6 +75,15 @@ def test_flash_attn_forward_matches_oracle(ops, oracle, B, h, L, d, causal, use_
     _check(got_o, got_lse, want_o, want_lse)
 
 
+# eight waves on a plane of 129 to 256: waves without queries, tiles past the last key, stages of 96 and 128 keys
+@pytest.mark.parametrize("L,d,causal", [(130, 24, False), (161, 32, True), (193, 8, False), (224, 32, False), (255, 32, True), (257, 32, False)])
+def test_flash_attn_forward_whole_planes(ops, oracle, L, d, causal):
+    rng = np.random.default_rng(L)
+    q, k, v = [rng.standard_normal((1, 3, L, d)).astype(np.float32) for _ in range(3)]
+    bias = (2 * rng.standard_normal((1, 3, L, L))).astype(np.float32)
+    _check(*_run(ops, q, k, v, bias, causal=causal), *oracle.flash_attn_forward(q, k, v, bias, causal=causal))
+
+
 def test_reference_golden_vectors(ops):
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "flash_attn_forward.json")
     with open(path) as f:
