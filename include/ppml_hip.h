@@ -266,6 +266,9 @@ int flash_attn_forward_ex_hip(int B, int h, int L, int d, int causal, float scal
  * mathematics of flash_attn_backward_cpu (src/ops/FlashAttn.cpp:140-210): from dO and the forward's O and LSE,
  *     P = exp(S - LSE),  D_i = sum_d dO_id O_id,  dS = P (dO V^T - D),
  *     dQ = scale dS K,   dK = scale dS^T Q,   dV = P^T dO,   dbias = dS  (0 at masked positions)
+ * causal: contractions go by tiles of 32 queries x 32 keys, and a tile none of whose queries sees a key is left out.  A
+ * row of K or V that is not finite reaches dQ and dbias of no query in an earlier tile, one of Q or dO reaches dK and dV
+ * of no key in a later one; within a tile on the diagonal a masked pair is a product with zero, which NaN and inf survive.
  * Layouts as in flash_attn_forward_hip; dQ, dK, dV, dbias may each be NULL (not all).  Every output element is
  * written (rows with LSE = -inf as zeros), nothing needs clearing beforehand, and there are no atomics: results
  * do not depend on scheduling.  d <= 64 and a multiple of 4 (the reference's CUDA path stops at 32).

@@ -276,8 +276,8 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_rows_kernel(const Att
                 const int key = key0 + 8 * (r >> 2) + 4 * half + (r & 3);
                 float s2 = st[r];
                 if (bias_row) s2 = __builtin_fmaf(bv[r], LOG2E, s2);
-                const float pr = key < row_keys ? __builtin_amdgcn_exp2f(s2 - lse2) : 0.0f;
-                st[r] = pr * (dp[r] - D_i);            // dS
+                // dS (chosen behind the product: 0 * NaN is not 0)
+                st[r] = key < row_keys ? __builtin_amdgcn_exp2f(s2 - lse2) * (dp[r] - D_i) : 0.0f;
             }
             // the bias registers are free again: the next tile's values travel during the rest of this tile
             // and the first contractions of the next (the tiles follow each other across the stages)
@@ -470,6 +470,11 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_cols_kernel(const Att
 // (370 us instead of 162).
 // Measured, us, against the two kernels (dQ + dbias, dK + dV): 824 planes of 256 x 256, d 32, with bias 291 -> 162 (648 MB:
 // 4.0 TB/s), 412 of 103 x 103 46 -> 25, 824 of 64 x 64 40 -> 25, 16 of 256 x 256 47 -> 33.
+// Causal: a wave none of whose keys the tile's queries see leaves the five phases out (staging, zeros for dbias and dQ, and
+// the barrier remain), and a round starts at its first visible tile; the tiles before it only have their dbias cleared.
+// With all tiles contracted and P = 0 at masked pairs, one NaN behind a query reached its gradients as 0 * NaN.  With bias,
+// us, contracted / left out / the two kernels: 412 planes of 256 72 / 67 / 152, 412 of 192 54 / 47 / 101, 412 of 257
+// 162 / 101 / 208, 128 of 640 238 / 148 / 260; of 103, where every wave has a diagonal tile, 24.6 / 23.0 / 41.
 typedef short v4s __attribute__((ext_vector_type(4)));
 
 template <int NW> struct FusedBack {
@@ -532,16 +537,24 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
     const auto load1 = [](__amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0)); };
     constexpr uint32_t OUT = 0x80000000u;
 
-    // The work-group's sequence of steps: its planes, per plane the rounds of NW * 32 keys, per round the query tiles.
-    // Loads run ahead of the computation along this sequence, across rounds and planes.
+    // The work-group's sequence of steps: its planes, per plane the rounds of NW * 32 keys, per round the query tiles
+    // (causal: from the first one that sees a key of the round).  Loads run ahead of the computation along this sequence,
+    // across rounds and planes.
     struct Step { int plane, g0, t; };
     const auto advance = [&](Step& s) {
         if (++s.t < tiles) return;
-        s.t = 0;
         s.g0 += NW * 32;
-        if (s.g0 < L) return;
-        s.g0 = 0;
-        s.plane += static_cast<int>(gridDim.x);
+        if (s.g0 >= L) {
+            s.g0 = 0;
+            s.plane += static_cast<int>(gridDim.x);
+        }
+        s.t = CAUSAL ? s.g0 / 32 : 0;
+    };
+    // Causal: no query of the tile sees a key of this wave (or it has none).  Such a wave contracts nothing: P = 0 there,
+    // but 0 * NaN is not, and what lies behind a query has no part in its gradients.
+    const auto hidden = [&](const Step& s) {
+        const int k0 = s.g0 + wave * 32;
+        return CAUSAL && (s.t * 32 + 31 < k0 || k0 >= L);
     };
 
     // ---- staging of a query tile: 256 items (row, four features) of Q and 256 of dO (with O, for D), shared out over
@@ -642,7 +655,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
         if (!BIAS) return;
         const bool there = s.plane < p.planes;
         const __amdgpu_buffer_rsrc_t rbias = rsrc(p.bias + (there ? s.plane * square : 0), there ? square_bytes : 0);
-        uint32_t at = square_at(s);
+        uint32_t at = hidden(s) ? OUT : square_at(s);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             bv[r] = load1(rbias, at);
@@ -700,6 +713,16 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
     const auto tile_step = [&](const Step& s, const Step& next, int n) {
         const uint8_t* const stage = back_lds + (n & 1) * F::STAGE;
         uint8_t* const region = regions + ((n & 1) * NW + wave) * F::REGION;
+        float* const part_at = reinterpret_cast<float*>(region) + j * F::QP + 4 * half;
+        if (hidden(s)) {
+            stage_put(n + 1);
+            stage_load();
+            load_bias(next);
+            store_dbias(s, v16f{});
+#pragma unroll
+            for (int g = 0; g < 4; ++g) *reinterpret_cast<v4f*>(part_at + 8 * g) = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            return;
+        }
         const bool no_key = s.g0 + wave * 32 + j >= L;
         const float* const lse_at = reinterpret_cast<const float*>(no_key ? no_key_lds : stage + 2 * F::TILE) + 4 * half;
         // ---- S[query][key]: this lane's key, 16 of the tile's queries; beside it, the next tile goes to LDS
@@ -717,11 +740,9 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
         if (BIAS)
 #pragma unroll
             for (int r = 0; r < 16; ++r) st[r] = __builtin_fmaf(bv[r], LOG2E, st[r]);
-        if (CAUSAL) {                                      // keys behind the query: P = 0
-            const int first = s.g0 + wave * 32 + j - s.t * 32 - 4 * half;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) st[r] = 8 * (r >> 2) + (r & 3) >= first ? st[r] : -INFINITY;
-        }
+        // causal: accumulator register r holds a query that does not lie before this lane's key
+        const int first = s.g0 + wave * 32 + j - s.t * 32 - 4 * half;
+        const auto seen = [&](int r) { return !CAUSAL || 8 * (r >> 2) + (r & 3) >= first; };
         v8bf wp[2][3], wd[2][3];
 #pragma unroll
         for (int ch = 0; ch < 2; ++ch) {
@@ -729,7 +750,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
             for (int g = 2 * ch; g < 2 * ch + 2; ++g) {
                 const v4f lse4 = *reinterpret_cast<const v4f*>(lse_at + 8 * g);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) st[4 * g + i] = __builtin_amdgcn_exp2f(st[4 * g + i] - lse4[i]);
+                for (int i = 0; i < 4; ++i) st[4 * g + i] = seen(4 * g + i) ? __builtin_amdgcn_exp2f(st[4 * g + i] - lse4[i]) : 0.0f;
             }
             parts_of(v4f{st[8 * ch], st[8 * ch + 1], st[8 * ch + 2], st[8 * ch + 3]}, v4f{st[8 * ch + 4], st[8 * ch + 5], st[8 * ch + 6], st[8 * ch + 7]}, wp[ch]);
         }
@@ -745,7 +766,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
             for (int g = 2 * ch; g < 2 * ch + 2; ++g) {
                 const v4f D4 = *reinterpret_cast<const v4f*>(lse_at + 32 + 8 * g);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) ds[4 * g + i] = st[4 * g + i] * (ds[4 * g + i] - D4[i]);
+                for (int i = 0; i < 4; ++i) ds[4 * g + i] = seen(4 * g + i) ? st[4 * g + i] * (ds[4 * g + i] - D4[i]) : 0.0f;
             }
             parts_of(v4f{ds[8 * ch], ds[8 * ch + 1], ds[8 * ch + 2], ds[8 * ch + 3]}, v4f{ds[8 * ch + 4], ds[8 * ch + 5], ds[8 * ch + 6], ds[8 * ch + 7]}, wd[ch]);
             // piece of eight bytes: queries 4 u .. 4 u + 3, u = 4 ch + half and two further on
@@ -782,7 +803,6 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
         // ---- this wave's share of dQ^T = K^T . dS^T: lane = query
         v16f dq;
         contract(dq, kt, w, true);
-        float* const part_at = reinterpret_cast<float*>(region) + j * F::QP + 4 * half;
 #pragma unroll
         for (int g = 0; g < 4; ++g) *reinterpret_cast<v4f*>(part_at + 8 * g) = v4f{dq[4 * g], dq[4 * g + 1], dq[4 * g + 2], dq[4 * g + 3]};
     };
@@ -827,7 +847,9 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
 #pragma unroll
         for (int r = 0; r < 16; ++r) { acc_k[r] = 0.0f; acc_v[r] = 0.0f; }
         const Step round = s;
-        for (int t = 0; t < tiles; ++t, ++n) {
+        if (CAUSAL)                                        // the tiles before the round's first one see none of its keys
+            for (int t = 0; t < round.t; ++t) store_dbias(Step{round.plane, round.g0, t}, v16f{});
+        for (int t = round.t; t < tiles; ++t, ++n) {
             Step next = s;
             advance(next);
             tile_step(s, next, n);

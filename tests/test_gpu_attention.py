@@ -255,6 +255,37 @@ def test_flash_attn_backward_in_one_pass(ops, planes, L, d, causal, use_bias):
         _check_grad(x, w, name)        # (logits near -200 carry 2^-16 of rounding, exp(LSE - ...) as much: 3e-5)
 
 
+# one pass and two kernels (few long planes, 64 features), one round of keys and two, whole and ragged tiles
+@pytest.mark.parametrize("planes,L,d,use_bias", [(2, 70, 32, True), (3, 160, 24, False), (2, 256, 32, True), (97, 300, 32, True), (97, 288, 8, False),
+                                                 (2, 300, 32, True), (2, 150, 64, True)])
+def test_causal_backward_keeps_what_a_query_does_not_see_out_of_its_gradients(ops, planes, L, d, use_bias):
+    """A position whose operands are not finite: the tiles of 32 rows before it (K, V: queries that do not see it) and
+    behind it (Q, dO: keys it does not see) keep the bits of the clean call."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(L + d)
+    q, k, v, do = (torch.randn(1, planes, L, d, device="cuda", generator=g) for _ in range(4))
+    bias = torch.randn(1, planes, L, L, device="cuda", generator=g) if use_bias else None
+    o, lse = ops.flash_attn_forward(q, k, v, bias, causal=True)
+    clean = ops.flash_attn_backward(q, k, v, bias, o, do, lse, causal=True)
+    masked = torch.ones(L, L, dtype=torch.bool, device="cuda").triu(1)
+    for at in (L - 2, 40):
+        first, behind = at // 32 * 32, at // 32 * 32 + 32
+        for name in ("q", "k", "v", "do"):
+            for value in (float("nan"), float("inf")):
+                x = dict(q=q, k=k, v=v, do=do)
+                x[name] = x[name].clone()
+                x[name][:, :, at] = value
+                o2, lse2 = ops.flash_attn_forward(x["q"], x["k"], x["v"], bias, causal=True)
+                dq, dk, dv, db = ops.flash_attn_backward(x["q"], x["k"], x["v"], bias, o2, x["do"], lse2, causal=True)
+                what = f"{name} = {value} at {at}"
+                if name in ("k", "v"):
+                    assert torch.equal(dq[:, :, :first], clean[0][:, :, :first]), what
+                else:
+                    assert torch.equal(dk[:, :, behind:], clean[1][:, :, behind:]) and torch.equal(dv[:, :, behind:], clean[2][:, :, behind:]), what
+                if use_bias:
+                    assert torch.equal(db[:, :, :first], clean[3][:, :, :first]) and not db[:, :, masked].any(), what
+
+
 def test_flash_attn_backward_subsets_and_determinism(ops, oracle):
     rng = np.random.default_rng(77)
     B, h, L, d = 1, 3, 90, 32
