@@ -271,7 +271,8 @@ int flash_attn_forward_ex_hip(int B, int h, int L, int d, int causal, float scal
  * of no key in a later one; within a tile on the diagonal a masked pair is a product with zero, which NaN and inf survive.
  * Layouts as in flash_attn_forward_hip; dQ, dK, dV, dbias may each be NULL (not all).  Every output element is
  * written (rows with LSE = -inf as zeros), nothing needs clearing beforehand, and there are no atomics: results
- * do not depend on scheduling.  d <= 64 and a multiple of 4 (the reference's CUDA path stops at 32).
+ * do not depend on scheduling, and a call for some of the gradients has the bits of the call for all of them.
+ * d <= 64 and a multiple of 4 (the reference's CUDA path stops at 32).
  * returns 0 = ran, 1 = refused, 6 = launch error. */
 int flash_attn_backward_hip(int B, int h, int L, int d, int causal, float scale,
                             const float *Q, const float *K, const float *V, const float *bias,

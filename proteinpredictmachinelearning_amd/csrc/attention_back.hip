@@ -7,8 +7,8 @@
 // Nothing is stored between forward and backward but O and LSE; P is recomputed per 32 x 32 tile.
 //
 // For head dimensions up to 32 one kernel makes all four gradients in one pass over the score planes
-// (flash_attn_back_fused_kernel, below).  Larger heads, and long sequences in few planes (a work-group of that kernel
-// takes a whole plane), go in two kernels, each the forward kernel's arrangement (see attention.hip) with one side held
+// (flash_attn_back_fused_kernel, below).  Larger heads, long sequences in few planes (a work-group of that kernel takes a
+// whole plane) and calls for dQ and dbias or for dK and dV alone go in two kernels, each the forward kernel's arrangement (see attention.hip) with one side held
 // in registers:
 //   * rows kernel  (dQ, dbias): a wave owns 32 queries; scores and dO V^T are computed transposed, so a lane
 //     holds 16 keys of ITS query: D_i and LSE_i are per-lane scalars, dS is ready as the B operand of
@@ -114,10 +114,10 @@ __device__ __forceinline__ void put_fragments(const v4f& x, int row, int c, uint
 }
 
 // Stages rows r0 .. r0+rows-1 (at most MAXROWS) of two [L][d] matrices into LDS as fragments (zeros past `valid`
-// rows and past d).  Every load of the stage is issued before the first value is used: a work-group waits for
+// rows and past d); SCALED: the first one's row fragments times a_factor.  Every load of the stage is issued before the first value is used: a work-group waits for
 // one memory round trip per stage, not one per loop iteration.
-template <int DP, int NT, int MAXROWS>
-__device__ __forceinline__ void stage_two(const float* a, uint8_t* a_row, uint8_t* a_col,
+template <int DP, int NT, int MAXROWS, bool SCALED>
+__device__ __forceinline__ void stage_two(const float* a, uint8_t* a_row, uint8_t* a_col, float a_factor,
                                           const float* b, uint8_t* b_row, uint8_t* b_col,
                                           int r0, int rows, int valid, int d, int tid) {
     constexpr int NI = (MAXROWS * (DP / 4) + NT - 1) / NT;
@@ -139,15 +139,21 @@ __device__ __forceinline__ void stage_two(const float* a, uint8_t* a_row, uint8_
         const int idx = tid + i * NT;
         const int row = idx / (DP / 4), c = (idx % (DP / 4)) * 4;
         if (row < rows) {
-            put_fragments<DP>(xa[i], row, c, a_row, a_col);
+            if (SCALED) {
+                put_fragments<DP>(xa[i] * a_factor, row, c, a_row, nullptr);
+                put_fragments<DP>(xa[i], row, c, nullptr, a_col);
+            } else {
+                put_fragments<DP>(xa[i], row, c, a_row, a_col);
+            }
             put_fragments<DP>(xb[i], row, c, b_row, b_col);
         }
     }
 }
 
 // acc(32 x 32) = tile(32 rows x DP, row fragments in LDS, rows = accumulator rows) . slice^T (this lane's column);
-// `frags` points at this lane's 16 bytes of the tile's first fragment
-template <int DP>
+// `frags` points at this lane's 16 bytes of the tile's first fragment.  SWAP: the partial products in the order of the
+// transposed product (the bits of slice . tile^T)
+template <int DP, bool SWAP = false>
 __device__ __forceinline__ v16f tile_times_slice(const uint8_t* frags, const v8bf (&slice)[DP / 16][3]) {
     v16f acc;
 #pragma unroll
@@ -159,7 +165,7 @@ __device__ __forceinline__ v16f tile_times_slice(const uint8_t* frags, const v8b
         for (int t = 0; t < 6; ++t) {
             // the first product starts from the constant zero: no registers to clear
             const v16f zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[SPLIT_TERMS[t][0]], slice[c][SPLIT_TERMS[t][1]], (c == 0 && t == 0) ? zero : acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[SPLIT_TERMS[t][SWAP]], slice[c][SPLIT_TERMS[t][!SWAP]], (c == 0 && t == 0) ? zero : acc, 0, 0, 0);
         }
     }
     return acc;
@@ -167,7 +173,8 @@ __device__ __forceinline__ v16f tile_times_slice(const uint8_t* frags, const v8b
 
 // out^T(DP features x 32 columns) += tile^T . w, contracting the 32 rows of the tile in the order in which the
 // accumulator registers of `w` hold them; `frags` points at this lane's 16 bytes of the tile's first column fragment.
-template <int DP>
+// FROM_ZERO: without what `out` held (the constant zero as the first product's addend: no registers to clear).
+template <int DP, bool FROM_ZERO = false>
 __device__ __forceinline__ void accumulate_transposed(v16f (&out)[DP / 32], const uint8_t* frags, const v16f& w) {
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch) {
@@ -184,17 +191,27 @@ __device__ __forceinline__ void accumulate_transposed(v16f (&out)[DP / 32], cons
             for (int part = 0; part < 3; ++part) a[part] = *reinterpret_cast<const v8bf*>(frags + ((b * 2 + ch) * 3 + part) * 1024);
 #pragma unroll
             for (int t = 0; t < 6; ++t)
-                out[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[SPLIT_TERMS[t][0]], wb[SPLIT_TERMS[t][1]], out[b], 0, 0, 0);
+                out[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[SPLIT_TERMS[t][0]], wb[SPLIT_TERMS[t][1]], FROM_ZERO && ch == 0 && t == 0 ? v16f{} : out[b], 0, 0, 0);
         }
     }
 }
 
+constexpr int TWIN_KEYS = 256;                        // keys whose shares of dQ are added up before the scale (eight waves' of the one-pass kernel)
+
 // ------------------------------------------------------------------------------------------------------------
 // dQ and dbias: a wave owns 32 queries and walks over the keys.
-template <int DP, int NW>
-__global__ __launch_bounds__(NW * 64) void flash_attn_back_rows_kernel(const AttnBackParams p) {
+// TWIN (one block of features): the bits of the one-pass kernel, for calls whose full set of gradients goes there.  K
+// carries the scale of the scores, the partial products come in the un-transposed order, D is summed as a butterfly over
+// the eight quads of features, and dQ is the sum of its tiles' shares, 256 keys at a time.  The price is a second split of
+// K and sixteen additions per tile that wait for their products; LATE adds a tile's share behind the next tile's products
+// instead, in sixteen more registers.  Against the form that owes nobody its bits, us: dQ of 8 planes of 256 without bias
+// 17.1 / 17.0 (18.3 not late), of 824 planes 76 / 77; with bias, 412 planes of 192, dQ and dbias 51.2 / 52.0 (54.4 not late).
+// BIAS: a compile-time property for the registers of its prefetch.
+template <int DP, int NW, bool TWIN, bool BIAS, bool LATE>
+__global__ __launch_bounds__(NW * 64, !TWIN ? 1 : BIAS && LATE ? 2 : 3) void flash_attn_back_rows_kernel(const AttnBackParams p) {
     using T = BackTiling<DP>;
     constexpr int NB = T::NB, NC = T::NC;
+    static_assert(TWIN ? (NB == 1 && NC == 2) : !LATE, "the one-pass kernel's features");
     extern __shared__ __attribute__((aligned(16))) uint8_t back_lds[];
     const int tiles_staged = p.stage_rows / 32;
     uint8_t* lds_k_row = back_lds;                                  // K by rows: S^T = K . Q^T
@@ -209,10 +226,10 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_rows_kernel(const Att
     const int64_t po = static_cast<int64_t>(plane) * L * d;
 
     v8bf qb[NC][3], dob[NC][3];
-    load_slice_parts<DP>(p.Q + po, q, L, d, half, p.scale * LOG2E, qb);
+    load_slice_parts<DP>(p.Q + po, q, L, d, half, TWIN ? 1.0f : p.scale * LOG2E, qb);
     load_slice_parts<DP>(p.dO + po, q, L, d, half, 1.0f, dob);
     // D_i = sum_d dO_id * O_id: this lane's half of the features, then the other half from lane j + 32
-    float D_i = 0.0f;
+    float D_i = 0.0f, D_c[NC] = {};
     if (q < L) {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
@@ -221,16 +238,23 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_rows_kernel(const Att
                 if (e >= d) continue;
                 const v4f a = *reinterpret_cast<const v4f*>(p.dO + po + static_cast<int64_t>(q) * d + e);
                 const v4f o = *reinterpret_cast<const v4f*>(p.O + po + static_cast<int64_t>(q) * d + e);
-                D_i += a[0] * o[0] + a[1] * o[1] + a[2] * o[2] + a[3] * o[3];
+                const float quad = a[0] * o[0] + a[1] * o[1] + a[2] * o[2] + a[3] * o[3];
+                D_i += quad;
+                D_c[c] += quad;
             }
     }
-    D_i += lane_xor32(D_i);
+    if (TWIN) {
+        D_i = D_c[0] + lane_xor32(D_c[0]);
+        if (NC > 1) D_i += D_c[NC - 1] + lane_xor32(D_c[NC - 1]);
+    } else {
+        D_i += lane_xor32(D_i);
+    }
     const float lse = q < L ? p.LSE[static_cast<int64_t>(plane) * L + q] : -INFINITY;
     // a row without any visible key (LSE = -inf) has no gradient: +inf makes every probability exp2(-inf) = 0
     const float lse2 = lse > -INFINITY ? lse * LOG2E : INFINITY;
     const int row_keys = p.causal ? (q + 1 < L ? q + 1 : L) : L;
     const int wave_keys = p.causal ? (q0 + 32 < L ? q0 + 32 : L) : L;
-    const float* bias_row = p.bias ? p.bias + (static_cast<int64_t>(plane) * L + (q < L ? q : L - 1)) * L : nullptr;
+    const float* bias_row = BIAS && p.bias ? p.bias + (static_cast<int64_t>(plane) * L + (q < L ? q : L - 1)) * L : nullptr;
     float* dbias_row = p.dbias ? p.dbias + (static_cast<int64_t>(plane) * L + (q < L ? q : L - 1)) * L : nullptr;
 
     v16f acc_q[NB];
@@ -238,11 +262,28 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_rows_kernel(const Att
     for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc_q[b][r] = 0.0f;
+    v16f late = {};                                    // LATE: the last tile's share of dQ, not yet in acc_q
+    // acc_q times the scale to this lane's query, or added to what it stored there before
+    const auto store_dq = [&](bool add) {
+        if (q >= L || !p.dQ) return;
+        float* row = p.dQ + po + static_cast<int64_t>(q) * d;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int dd = b * 32 + 8 * g + 4 * half;
+                if (dd >= d) continue;
+                v4f* const dst = reinterpret_cast<v4f*>(row + dd);
+                v4f x = v4f{acc_q[b][4 * g], acc_q[b][4 * g + 1], acc_q[b][4 * g + 2], acc_q[b][4 * g + 3]} * p.scale;
+                if (add) x += *dst;
+                *dst = x;
+            }
+    };
 
     // Bias of this lane's 16 keys of the tile that starts at key0 (zeros past L), 16 bytes at a time.
     float bv[16];
     const auto load_bias = [&](int key0) {
-        if (!bias_row) return;
+        if (!BIAS || !bias_row) return;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const int key = key0 + 8 * g + 4 * half;
@@ -262,20 +303,20 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_rows_kernel(const Att
         __syncthreads();
         const int ckeys = L - c0 < stage ? L - c0 : stage;
         const int rows = (ckeys + 31) / 32 * 32;
-        stage_two<DP, NW * 64, T::CH_ROWS>(p.K + po, lds_k_row, lds_k_col, p.V + po, lds_v_row, nullptr, c0, rows, ckeys, d, tid);
+        stage_two<DP, NW * 64, T::CH_ROWS, TWIN>(p.K + po, lds_k_row, lds_k_col, p.scale * LOG2E, p.V + po, lds_v_row, nullptr, c0, rows, ckeys, d, tid);
         __syncthreads();
         if (!wave_active) continue;
         for (int kt = 0; kt < rows / 32; ++kt) {
             const int key0 = c0 + kt * 32;
             // ---- probabilities of this lane's query for its 16 keys of the tile (their bias was requested a
             // tile ago, see below)
-            v16f st = tile_times_slice<DP>(lds_k_row + kt * T::ROW_BYTES + lane * 16, qb);
-            v16f dp = tile_times_slice<DP>(lds_v_row + kt * T::ROW_BYTES + lane * 16, dob);
+            v16f st = tile_times_slice<DP, TWIN>(lds_k_row + kt * T::ROW_BYTES + lane * 16, qb);
+            v16f dp = tile_times_slice<DP, TWIN>(lds_v_row + kt * T::ROW_BYTES + lane * 16, dob);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int key = key0 + 8 * (r >> 2) + 4 * half + (r & 3);
                 float s2 = st[r];
-                if (bias_row) s2 = __builtin_fmaf(bv[r], LOG2E, s2);
+                if (BIAS && bias_row) s2 = __builtin_fmaf(bv[r], LOG2E, s2);
                 // dS (chosen behind the product: 0 * NaN is not 0)
                 st[r] = key < row_keys ? __builtin_amdgcn_exp2f(s2 - lse2) * (dp[r] - D_i) : 0.0f;
             }
@@ -297,20 +338,26 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_rows_kernel(const Att
             }
             if (key0 >= wave_keys) continue;           // causal: no query of the wave sees this tile (dS = 0)
             // ---- dQ^T += K^T . dS
-            if (p.dQ) accumulate_transposed<DP>(acc_q, lds_k_col + kt * T::COL_BYTES + lane * 16, st);
+            if (!p.dQ) continue;
+            if (TWIN) {
+                if (key0 > 0 && key0 % TWIN_KEYS == 0) {
+                    if (LATE) acc_q[0] += late;
+                    store_dq(key0 > TWIN_KEYS);
+                    acc_q[0] = late = v16f{};
+                }
+                v16f share[NB];
+                if (LATE) acc_q[0] += late;
+                accumulate_transposed<DP, true>(share, lds_k_col + kt * T::COL_BYTES + lane * 16, st);
+                if (LATE) late = share[0];
+                else acc_q[0] += share[0];
+            } else {
+                accumulate_transposed<DP>(acc_q, lds_k_col + kt * T::COL_BYTES + lane * 16, st);
+            }
         }
     }
-    if (!wave_active || q >= L || !p.dQ) return;
-    float* row = p.dQ + po + static_cast<int64_t>(q) * d;
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int dd = b * 32 + 8 * g + 4 * half;
-            if (dd < d)
-                *reinterpret_cast<v4f*>(row + dd) = v4f{acc_q[b][4 * g] * p.scale, acc_q[b][4 * g + 1] * p.scale,
-                                                        acc_q[b][4 * g + 2] * p.scale, acc_q[b][4 * g + 3] * p.scale};
-        }
+    if (!wave_active) return;
+    if (LATE) acc_q[0] += late;
+    store_dq(TWIN && wave_keys > TWIN_KEYS);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -543,12 +590,12 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
     struct Step { int plane, g0, t; };
     const auto advance = [&](Step& s) {
         if (++s.t < tiles) return;
+        s.t = 0;
         s.g0 += NW * 32;
-        if (s.g0 >= L) {
-            s.g0 = 0;
-            s.plane += static_cast<int>(gridDim.x);
-        }
-        s.t = CAUSAL ? s.g0 / 32 : 0;
+        if (CAUSAL && s.g0 < L) s.t = s.g0 / 32;
+        if (s.g0 < L) return;
+        s.g0 = 0;
+        s.plane += static_cast<int>(gridDim.x);
     };
     // Causal: no query of the tile sees a key of this wave (or it has none).  Such a wave contracts nothing: P = 0 there,
     // but 0 * NaN is not, and what lies behind a query has no part in its gradients.
@@ -713,8 +760,8 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
     const auto tile_step = [&](const Step& s, const Step& next, int n) {
         const uint8_t* const stage = back_lds + (n & 1) * F::STAGE;
         uint8_t* const region = regions + ((n & 1) * NW + wave) * F::REGION;
-        float* const part_at = reinterpret_cast<float*>(region) + j * F::QP + 4 * half;
         if (hidden(s)) {
+            float* const part_at = reinterpret_cast<float*>(region) + j * F::QP + 4 * half;
             stage_put(n + 1);
             stage_load();
             load_bias(next);
@@ -803,6 +850,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
         // ---- this wave's share of dQ^T = K^T . dS^T: lane = query
         v16f dq;
         contract(dq, kt, w, true);
+        float* const part_at = reinterpret_cast<float*>(region) + j * F::QP + 4 * half;
 #pragma unroll
         for (int g = 0; g < 4; ++g) *reinterpret_cast<v4f*>(part_at + 8 * g) = v4f{dq[4 * g], dq[4 * g + 1], dq[4 * g + 2], dq[4 * g + 3]};
     };
@@ -849,7 +897,7 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
         const Step round = s;
         if (CAUSAL)                                        // the tiles before the round's first one see none of its keys
             for (int t = 0; t < round.t; ++t) store_dbias(Step{round.plane, round.g0, t}, v16f{});
-        for (int t = round.t; t < tiles; ++t, ++n) {
+        for (int t = CAUSAL ? round.t : 0; t < tiles; ++t, ++n) {
             Step next = s;
             advance(next);
             tile_step(s, next, n);
@@ -888,25 +936,44 @@ int launch_fused(const AttnBackParams& p, hipStream_t stream) {
     return check_launch("flash_attn_back_fused_kernel");
 }
 
-template <int DP>
+template <int DP, bool TWIN, bool BIAS, bool LATE>
+int launch_rows(AttnBackParams p, hipStream_t stream) {
+    using T = BackTiling<DP>;
+    constexpr int NW = 4;
+    const int l32 = (p.L + 31) / 32 * 32;
+    p.stage_rows = l32 < T::CH_ROWS ? l32 : T::CH_ROWS;
+    const size_t lds = static_cast<size_t>(p.stage_rows / 32) * (2 * T::ROW_BYTES + T::COL_BYTES);
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_attn_back_rows_kernel<DP, NW, TWIN, BIAS, LATE>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       (T::CH_ROWS / 32) * (2 * T::ROW_BYTES + T::COL_BYTES));
+    if (attr != hipSuccess) {
+        (void)hipGetLastError();
+        set_error("flash_attn_backward_hip: cannot reserve the LDS of the rows kernel");
+        return RC_LAUNCH;
+    }
+    hipLaunchKernelGGL((flash_attn_back_rows_kernel<DP, NW, TWIN, BIAS, LATE>), dim3((p.L + 32 * NW - 1) / (32 * NW), p.planes), dim3(NW * 64), lds, stream, p);
+    return check_launch("flash_attn_back_rows_kernel");
+}
+
+template <int DP, bool TWIN>
 int launch_back(AttnBackParams p, hipStream_t stream) {
     using T = BackTiling<DP>;
     constexpr int NW = 4;
     const int l32 = (p.L + 31) / 32 * 32;
-    const dim3 grid((p.L + 32 * NW - 1) / (32 * NW), p.planes), block(NW * 64);
     if (p.dQ || p.dbias) {
-        p.stage_rows = l32 < T::CH_ROWS ? l32 : T::CH_ROWS;
-        const size_t lds = static_cast<size_t>(p.stage_rows / 32) * (2 * T::ROW_BYTES + T::COL_BYTES);
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_attn_back_rows_kernel<DP, NW>),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                           (T::CH_ROWS / 32) * (2 * T::ROW_BYTES + T::COL_BYTES));
-        if (attr != hipSuccess) {
-            (void)hipGetLastError();
-            set_error("flash_attn_backward_hip: cannot reserve the LDS of the rows kernel");
-            return RC_LAUNCH;
+        int rc;
+        if constexpr (TWIN) {
+            // With a bias the late form's registers leave room for two work-groups per CU instead of three: taken where its
+            // rounds over the chip still come no dearer.  dQ and dbias, us, late / not: 8 planes of 256 20.8 / 22.9, 412 of
+            // 192 51.2 / 54.4, 412 of 103 21.1 / 22.4; 300 of 256 (600 work-groups) 55.8 / 49.4.
+            const int64_t groups = static_cast<int64_t>((p.L + 127) / 128) * p.planes, cus = device_cu_count();
+            const bool late = (groups + 2 * cus - 1) / (2 * cus) * 2 <= (groups + 3 * cus - 1) / (3 * cus) * 3;
+            rc = !p.bias ? launch_rows<DP, true, false, true>(p, stream)
+                 : late  ? launch_rows<DP, true, true, true>(p, stream)
+                         : launch_rows<DP, true, true, false>(p, stream);
+        } else {
+            rc = launch_rows<DP, false, true, false>(p, stream);
         }
-        hipLaunchKernelGGL((flash_attn_back_rows_kernel<DP, NW>), grid, block, lds, stream, p);
-        const int rc = check_launch("flash_attn_back_rows_kernel");
         if (rc != RC_OK) return rc;
     }
     if (p.dK || p.dV) {
@@ -921,7 +988,7 @@ int launch_back(AttnBackParams p, hipStream_t stream) {
             set_error("flash_attn_backward_hip: cannot reserve the LDS of the columns kernel");
             return RC_LAUNCH;
         }
-        hipLaunchKernelGGL((flash_attn_back_cols_kernel<DP, NW>), grid, block, lds, stream, p);
+        hipLaunchKernelGGL((flash_attn_back_cols_kernel<DP, NW>), dim3((p.L + 32 * NW - 1) / (32 * NW), p.planes), dim3(NW * 64), lds, stream, p);
         return check_launch("flash_attn_back_cols_kernel");
     }
     return RC_OK;
@@ -963,11 +1030,27 @@ extern "C" int flash_attn_backward_hip(int B, int h, int L, int d, int causal, f
     p.stage_rows = 0;
     StatsScope stat("hip/flash_attn_back", static_cast<int64_t>(planes) * L, d, L, static_cast<hipStream_t>(stream));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // One pass where a head fits one feature block.  Beyond 256 rows a work-group walks over a plane in rounds while the
-    // two kernels have a work-group per 128 rows: they stay the better choice until the planes alone fill the chip (us, one
-    // pass / two kernels: 64 planes of 384 rows 91 / 75, 128 of them 92 / 105; of 640 rows 217 / 162 and 233 / 290).  The
-    // choice does not look at which gradients are wanted: a subset has the bits of the whole.
-    if (d <= 32 && L < 16384 && (L <= 256 || planes * 8 >= 3 * device_cu_count())) {
+    // One pass or two kernels, for head dimensions of one feature block (all figures us, one pass / two kernels).
+    // A call that wants gradients on both sides (dQ or dbias, dK or dV): one pass up to 256 rows.  Beyond, a work-group walks
+    // over a plane in rounds while the two kernels have one per 128 rows, and the planes alone have to occupy the chip -- from
+    // 3/8 of the CUs on if causal (96 planes of 384 62 / 91) or, up to 512 rows, with a bias (of 384 97 / 108; 64 planes
+    // 91 / 73), half of them with a bias beyond (128 of 640 236 / 273, 96 of them 220 / 193), and without either only where the
+    // rounds over the chip are 3/5 full (160 of 512 112 / 159, 128 of 320 72 / 73, 300 of them 144 / 132).
+    // A call that wants one side only would have the one-pass kernel contract for the other as well; for it the two kernels'
+    // half is the rule (8 planes of 256, dQ 29 / 17, dK and dV 29 / 23; 128 of 640, dbias 201 / 147), and the exceptions need
+    // rounds 3/4 full and a side's pair (dbias with the bias its kernel would read a lane per row): causal from 129 rows on
+    // (412 of 256, dQ and dbias 65 / 87), not causal from 129 to 256 rows in at most two rounds (256 of 160, dK and dV 22 / 26),
+    // or with a bias from 385 to 512 (200 of 448, dQ and dbias 117 / 142).
+    // Either way the bits are the same: where the whole set goes in one pass, the two kernels compute as it does.
+    const int64_t cus = device_cu_count(), slots = (planes + cus - 1) / cus * cus;
+    const bool rows = dQ || dbias, cols = dK || dV;
+    const bool whole = d <= 32 && L < 16384 &&
+                       (L <= 256 || (causal || (bias && L <= 512) ? 8 * planes >= 3 * cus : bias ? 2 * planes >= cus : 5 * planes >= 3 * slots));
+    const bool pair = (dK && dV) || (dbias && bias);
+    const bool one_side = pair && L > 128 && 4 * planes >= 3 * slots &&
+                          (causal ? bias || planes <= 2 * cus
+                                  : L <= 256 ? planes <= 2 * cus && (cols || dQ) : bias && L > 384 && L <= 512);
+    if (whole && ((rows && cols) || one_side)) {
         const bool streaming = L % 32 == 0 && (reinterpret_cast<uintptr_t>(dbias) & 127) == 0;
         const int db = !dbias ? DB_NONE : streaming ? DB_STREAM : DB_ORDINARY;
         const int kt = (L + 31) / 32;
@@ -979,5 +1062,5 @@ extern "C" int flash_attn_backward_hip(int B, int h, int L, int d, int causal, f
 #undef PPML_BACK_B
 #undef PPML_BACK_DB
     }
-    return d <= 32 ? launch_back<32>(p, s) : launch_back<64>(p, s);
+    return d > 32 ? launch_back<64, false>(p, s) : whole ? launch_back<32, true>(p, s) : launch_back<32, false>(p, s);
 }

@@ -255,6 +255,40 @@ def test_flash_attn_backward_in_one_pass(ops, planes, L, d, causal, use_bias):
         _check_grad(x, w, name)        # (logits near -200 carry 2^-16 of rounding, exp(LSE - ...) as much: 3e-5)
 
 
+# beyond 256 rows in few planes: two kernels; either side of the numbers of planes from which one pass takes over (3/8 and
+# 1/2 of 256 CUs with a bias, 3/5 of them without)
+@pytest.mark.parametrize("planes,L,d,causal,use_bias", [
+    (2, 257, 32, False, True), (2, 300, 20, True, True), (3, 300, 32, False, False), (1, 520, 32, True, False),
+    (95, 257, 32, False, True), (96, 257, 32, False, True), (95, 260, 8, True, False), (96, 260, 8, True, False),
+    (153, 257, 16, False, False), (154, 257, 16, False, False), (127, 513, 8, False, True), (128, 513, 8, False, True),
+])
+def test_flash_attn_backward_of_long_planes(ops, planes, L, d, causal, use_bias):
+    test_flash_attn_backward_in_one_pass(ops, planes, L, d, causal, use_bias)
+
+
+# one pass for the whole set, two kernels for most of the others: rounds of 256 keys, ragged tiles, the features' remainder,
+# and enough planes for the exceptions (256 x 150, 200 x 260 causal, 200 x 400)
+@pytest.mark.parametrize("planes,L,d,causal,use_bias", [
+    (2, 31, 32, False, True), (3, 103, 20, True, True), (2, 128, 4, False, False), (2, 160, 32, False, True), (2, 255, 24, True, False),
+    (256, 150, 32, False, True), (200, 260, 32, True, True), (200, 400, 12, False, True), (160, 300, 32, False, False),
+    (300, 256, 32, False, True), (130, 520, 32, False, True), (2, 300, 32, False, True),
+])
+def test_flash_attn_backward_subsets_have_the_bits_of_the_whole(ops, planes, L, d, causal, use_bias):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3 * L + d)
+    q, k, v, do = (torch.randn(1, planes, L, d, device="cuda", generator=g) for _ in range(4))
+    bias = torch.randn(1, planes, L, L, device="cuda", generator=g) if use_bias else None
+    o, lse = ops.flash_attn_forward(q, k, v, bias, causal=causal)
+    names = ("dq", "dk", "dv", "dbias")
+    whole = ops.flash_attn_backward(q, k, v, bias, o, do, lse, causal=causal, want=names)
+    for mask in range(1, 15):
+        want = tuple(n for i, n in enumerate(names) if mask >> i & 1)
+        got = ops.flash_attn_backward(q, k, v, bias, o, do, lse, causal=causal, want=want)
+        for n, x, w in zip(names, got, whole):
+            assert (x is not None) == (n in want)
+            assert x is None or torch.equal(x, w), (want, n)
+
+
 # one pass and two kernels (few long planes, 64 features), one round of keys and two, whole and ragged tiles
 @pytest.mark.parametrize("planes,L,d,use_bias", [(2, 70, 32, True), (3, 160, 24, False), (2, 256, 32, True), (97, 300, 32, True), (97, 288, 8, False),
                                                  (2, 300, 32, True), (2, 150, 64, True)])
