@@ -1033,13 +1033,13 @@ extern "C" int flash_attn_backward_hip(int B, int h, int L, int d, int causal, f
     // One pass or two kernels, for head dimensions of one feature block (all figures us, one pass / two kernels).
     // A call that wants gradients on both sides (dQ or dbias, dK or dV): one pass up to 256 rows.  Beyond, a work-group walks
     // over a plane in rounds while the two kernels have one per 128 rows, and the planes alone have to occupy the chip -- from
-    // 3/8 of the CUs on if causal (96 planes of 384 62 / 91) or, up to 512 rows, with a bias (of 384 97 / 108; 64 planes
-    // 91 / 73), half of them with a bias beyond (128 of 640 236 / 273, 96 of them 220 / 193), and without either only where the
-    // rounds over the chip are 3/5 full (160 of 512 112 / 159, 128 of 320 72 / 73, 300 of them 144 / 132).
+    // 3/8 of the CUs on if causal (96 planes of 384 62 / 90) or, up to 512 rows, with a bias (of 384 90 / 101; 64 planes
+    // 89 / 72), half of them with a bias beyond (128 of 640 245 / 295, 96 of them 220 / 198), and without either only where the
+    // rounds over the chip are 3/5 full (160 of 512 113 / 160, 128 of 320 73 / 73, 300 of them 144 / 133).
     // A call that wants one side only would have the one-pass kernel contract for the other as well; for it the two kernels'
-    // half is the rule (8 planes of 256, dQ 29 / 17, dK and dV 29 / 23; 128 of 640, dbias 201 / 147), and the exceptions need
+    // half is the rule (8 planes of 256, dQ 29 / 17, dK and dV 29 / 23; 128 of 640, dbias 215 / 149), and the exceptions need
     // rounds 3/4 full and a side's pair (dbias with the bias its kernel would read a lane per row): causal from 129 rows on
-    // (412 of 256, dQ and dbias 65 / 87), not causal from 129 to 256 rows in at most two rounds (256 of 160, dK and dV 22 / 26),
+    // (412 of 256, dQ and dbias 62 / 83), not causal from 129 to 256 rows in at most two rounds (256 of 160, dK and dV 22 / 26),
     // or with a bias from 385 to 512 (200 of 448, dQ and dbias 117 / 142).
     // Either way the bits are the same: where the whole set goes in one pass, the two kernels compute as it does.
     const int64_t cus = device_cu_count(), slots = (planes + cus - 1) / cus * cus;
