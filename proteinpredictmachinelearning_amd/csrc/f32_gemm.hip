@@ -2905,13 +2905,15 @@ extern "C" int tri_mul_back_hip(const float* grad, const float* left, const floa
         if (gright) of_right = contraction(grad, 1, J, left, I, 1, gright, 1, J, J, K, I, I * J, K * I, K * J);
     }
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    // One launch for both, unless calls are being counted and timed (one row per contraction) or gright shares memory
-    // with what the first contraction reads or writes (in turn, it may).
+    // One launch for both, unless what one of them writes shares memory with what the other reads or writes (in turn, it
+    // may: gleft is complete before left is read, right has been read before gright is written).
     const auto apart = [](const float* x, int64_t nx, const float* y, int64_t ny) {
         const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
         return x0 + static_cast<uintptr_t>(nx) * 4 <= y0 || y0 + static_cast<uintptr_t>(ny) * 4 <= x0;
     };
-    if (gleft && gright && !stats_enabled() && apart(gright, D * J * K * B, right, D * J * K * B) && apart(gright, D * J * K * B, gleft, D * I * K * B)) {
+    const int64_t n_grad = D * I * J * B, n_left = D * I * K * B, n_right = D * J * K * B;
+    if (gleft && gright && !stats_enabled() && apart(gright, n_right, right, n_right) && apart(gright, n_right, gleft, n_left) &&
+        apart(gright, n_right, grad, n_grad) && apart(gleft, n_left, left, n_left) && apart(gleft, n_left, grad, n_grad)) {
         const int rc = try_pc_pair(of_left, of_right, s, "tri_mul_back_hip");
         if (rc >= 0) return rc;
     }

@@ -810,6 +810,38 @@ def test_tri_mul_back_pair(ops, D, I, J, K, outgoing):
     assert not np.isfinite(gl.cpu().numpy()).all() and np.isfinite(gr.cpu().numpy()).all()
 
 
+# outputs on the memory of what the other gradient's contraction reads or writes: the two run in turn, the left one first
+@pytest.mark.parametrize("outgoing", [True, False])
+def test_tri_mul_back_outputs_on_other_operands(ops, outgoing):
+    from proteinpredictmachinelearning_amd import cabi
+
+    D, L = 16, 64
+    rng = np.random.default_rng(5)
+    left, right, grad = (_dev(rng.standard_normal(D * L * L).astype(np.float32)) for _ in range(3))
+    want_l, want_r = ops.tri_mul_back(grad, left, right, D, L, L, L, 1, 3.0, outgoing)
+    _, want_r_of_gl = ops.tri_mul_back(grad, want_l, right, D, L, L, L, 1, 3.0, outgoing, want_left=False)
+
+    def call(g, l, r, gl, gr):
+        rc = cabi.load().tri_mul_back_hip(g.data_ptr(), l.data_ptr(), r.data_ptr(), gl.data_ptr(), gr.data_ptr(), D, L, L, L, 1,
+                                          1.0 / 3.0, 1 if outgoing else 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+
+    g, l, r, out = grad.clone(), left.clone(), right.clone(), torch.empty_like(left)
+    call(g, l, r, out, r)                               # gright on right, which gleft's contraction has read by then
+    assert torch.equal(out, want_l) and torch.equal(r, want_r)
+    g, l, r = grad.clone(), left.clone(), right.clone()
+    call(g, l, r, l, out)                               # gleft on left: gright is that of the left gradient
+    assert torch.equal(l, want_l) and torch.equal(out, want_r_of_gl)
+    g, l, r = grad.clone(), left.clone(), right.clone()
+    call(g, l, r, out, out)                             # gright on gleft: the later one stays
+    assert torch.equal(out, want_r)
+    # one contiguous buffer, side by side without sharing a byte: either order of the two
+    both = torch.empty(2 * D * L * L, device="cuda")
+    for gl, gr in ((both[: D * L * L], both[D * L * L:]), (both[D * L * L:], both[: D * L * L])):
+        call(grad, left, right, gl, gr)
+        assert torch.equal(gl, want_l) and torch.equal(gr, want_r)
+
+
 # (3, 4, 8), (8, 48, 64, 2): the generic kernel (a short pair tensor; a batch); the others: the gradient tensor split in
 # the tile loop -- runs of whole 16-k chunks (L a multiple of 16) and of any length (103, 50, 40), ragged rows (2176 =
 # 17 tiles) and columns, two to eight K slices, up to four column tiles
