@@ -2299,7 +2299,8 @@ bool streams_output(const GemmParams& p) {
 // Both gradients of the triangle multiplication in one launch (gemm_bf16x3_pc_pair_kernel); -1 when one of the two is not
 // of the kind that launch_gemm gives to gemm_bf16x3_pc_kernel with at most one tile per CU (beyond that each fills the
 // chip by itself) or the two do not lie as one of the two instances has them, and the caller launches them one by one.
-int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what) {
+// I, J, K: the statistics' row, which is that of the left gradient's contraction.
+int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what, int64_t I, int64_t J, int64_t K) {
     if (f32_arithmetic() == 1) return -1;
     const auto kmode = [](int64_t rs, int64_t ks) { return ks == 1 ? LOAD_K_CONTIG : rs == 1 ? LOAD_ROW_CONTIG : LOAD_STRIDED; };
     for (GemmParams* p : {&a, &b}) {
@@ -2323,6 +2324,7 @@ int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what
     const bool k4 = a.K % 4 == 0 && (outgoing || b.K % 4 == 0);      // (loads along k; the outgoing `b` has none)
     const int groups_a = a.tiles_m * a.tiles_n * a.np2 * a.np3, groups_b = b.tiles_m * b.tiles_n * b.np2 * b.np3;
     const dim3 grid(static_cast<unsigned>(groups_a + groups_b)), block(512);
+    StatsScope stat("hip/tri_mul_back_pair", I, J, K, stream);
 #define PPML_PAIR(AB_, BM_, STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_pc_pair_kernel<LOAD_K_CONTIG, AB_, BM_, LOAD_ROW_CONTIG, STREAM_, K4_>), grid, block, 0, stream, a, b, groups_a)
 #define PPML_PAIR_K4(AB_, BM_, STREAM_) do { if (k4) PPML_PAIR(AB_, BM_, STREAM_, true); else PPML_PAIR(AB_, BM_, STREAM_, false); } while (0)
     if (outgoing) { if (a.stream_c) PPML_PAIR_K4(LOAD_ROW_CONTIG, LOAD_ROW_CONTIG, true); else PPML_PAIR_K4(LOAD_ROW_CONTIG, LOAD_ROW_CONTIG, false); }
@@ -2912,9 +2914,9 @@ extern "C" int tri_mul_back_hip(const float* grad, const float* left, const floa
         return x0 + static_cast<uintptr_t>(nx) * 4 <= y0 || y0 + static_cast<uintptr_t>(ny) * 4 <= x0;
     };
     const int64_t n_grad = D * I * J * B, n_left = D * I * K * B, n_right = D * J * K * B;
-    if (gleft && gright && !stats_enabled() && apart(gright, n_right, right, n_right) && apart(gright, n_right, gleft, n_left) &&
+    if (gleft && gright && apart(gright, n_right, right, n_right) && apart(gright, n_right, gleft, n_left) &&
         apart(gright, n_right, grad, n_grad) && apart(gleft, n_left, left, n_left) && apart(gleft, n_left, grad, n_grad)) {
-        const int rc = try_pc_pair(of_left, of_right, s, "tri_mul_back_hip");
+        const int rc = try_pc_pair(of_left, of_right, s, "tri_mul_back_hip", I, J, K);
         if (rc >= 0) return rc;
     }
     int rc = RC_OK;

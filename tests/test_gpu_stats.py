@@ -58,3 +58,27 @@ def test_calls_and_milliseconds_per_shape(oracle, capfd):
         ops.mulmat_stats_enable(before)
     ops.mul_mat(x, w)
     assert ops.mulmat_stats_rows() == []
+
+
+def test_both_triangle_gradients_in_one_launch_are_one_row():
+    from proteinpredictmachinelearning_amd import cabi, ops
+
+    lib = cabi.load()
+    g = torch.Generator(device="cuda").manual_seed(2)
+    before = ops.mulmat_stats_enable(True)
+    try:
+        for D, I, J, K, paths in ((4, 64, 96, 60, {("hip/tri_mul_back_pair", 64, 96, 60)}),                            # one launch
+                                  (4, 40, 40, 40, {("hip/tri_mul_back", 40, 40, 40)}),                                 # too short a contraction: two
+                                  (300, 60, 52, 56, {("hip/tri_mul_back", 60, 52, 56), ("hip/tri_mul_back", 52, 60, 56)})):     # more tiles than CUs: two
+            lib.ppml_hip_mulmat_stats_reset()
+            left, right, grad = (torch.randn(D * n, device="cuda", generator=g) for n in (I * K, J * K, I * J))
+            counted = ops.tri_mul_back(grad, left, right, D, I, J, K, 1, 2.0)
+            rows = {(r["path"], r["M"], r["K"], r["N"]): r for r in ops.mulmat_stats_rows()}
+            assert set(rows) == paths and all(0.0 < r["ms"] < 200.0 for r in rows.values())
+            assert sum(r["calls"] for r in rows.values()) == (1 if "pair" in next(iter(paths))[0] else 2)
+            ops.mulmat_stats_enable(False)
+            assert all(torch.equal(a, b) for a, b in zip(counted, ops.tri_mul_back(grad, left, right, D, I, J, K, 1, 2.0)))
+            ops.mulmat_stats_enable(True)
+        lib.ppml_hip_mulmat_stats_reset()
+    finally:
+        ops.mulmat_stats_enable(before)
