@@ -691,7 +691,12 @@ __device__ __forceinline__ void store_acc_buffer(const __amdgpu_buffer_rsrc_t rs
     }
 }
 
-template <int MODE, bool SPLIT_C, bool STREAM_C, bool FAST_IO = false, bool K4 = true>
+// SPLIT_C of the kernels below: how the output is addressed.  The two compound forms are instances of their own: with both
+// stores in one kernel, chosen by p.c_span as it ran, the general one cost 1 to 2.5 us more per launch (32 features x 24
+// residues x 8 sequences 14.0 -> 16.5 us, the value form at 8 x 8 x 33 13.5 -> 15.6).
+constexpr int C_DENSE = 0, C_COMPOUND = 1, C_COMPOUND_BUFFER = 2;
+
+template <int MODE, int SPLIT_C, bool STREAM_C, bool FAST_IO = false, bool K4 = true>
 __global__ __launch_bounds__(256) void gemm_bf16x3_kernel(const GemmParams p) {
     // (FAST_IO with SPLIT_C: buffer-addressed loads, the output by its compound addressing)
     static_assert(!FAST_IO || MODE == LOAD_ROW_CONTIG || MODE == LOAD_K_CONTIG, "buffer addressing: rows contiguous in themselves or in k");
@@ -786,8 +791,8 @@ __global__ __launch_bounds__(256) void gemm_bf16x3_kernel(const GemmParams p) {
     }
 
     if (FAST_IO && !SPLIT_C) store_acc_buffer<STREAM_C>(rsrc_c, static_cast<uint32_t>(p.c_mi) * 4u, p.N, p.alpha, acc, m0 + wm, n0 + wn, lane);
-    else if (SPLIT_C && p.c_span) store_acc_compound_buffer<STREAM_C, 2>(p, C, acc, m0 + wm, n0 + wn, lane);
-    else store_acc<SPLIT_C, STREAM_C, false, false>(p, C, acc, m0 + wm, n0 + wn, lane);
+    else if (SPLIT_C == C_COMPOUND_BUFFER) store_acc_compound_buffer<STREAM_C, 2>(p, C, acc, m0 + wm, n0 + wn, lane);
+    else store_acc<SPLIT_C == C_COMPOUND, STREAM_C, false, false>(p, C, acc, m0 + wm, n0 + wn, lane);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1997,7 +2002,7 @@ constexpr int PBM = 256;
 constexpr int PLANES_MIN_TILES = 8;              // 128-wide tiles per side from which the operands are split ahead ...
 constexpr int PLANES_MIN_GROUPS = 512;           // ... if that leaves two 256 x 128 work-groups for every CU
 constexpr int PLANES_MIN_SLICE_CHUNKS = 16;      // a K slice is at least 256 long
-template <bool SPLIT_C, bool STREAM_C>
+template <int SPLIT_C, bool STREAM_C>
 __global__ __launch_bounds__(256, 2) void gemm_planes_kernel(const GemmParams p, const uint8_t* __restrict__ wa,
                                                              const uint8_t* __restrict__ wb, int chunks, int ma_pad, int nb_pad,
                                                              int slice_chunks, float* __restrict__ partial,
@@ -2099,8 +2104,8 @@ __global__ __launch_bounds__(256, 2) void gemm_planes_kernel(const GemmParams p,
         plain_tile(p, p.A, p.B, p.C, m0, n0, PBM, BN, tid);
         return;
     }
-    if (SPLIT_C && p.c_span) store_acc_compound_buffer<STREAM_C, 4>(p, p.C, acc, m0 + wm, n0 + wn, lane);
-    else store_acc<SPLIT_C, STREAM_C, false, false, 4>(p, p.C, acc, m0 + wm, n0 + wn, lane);
+    if (SPLIT_C == C_COMPOUND_BUFFER) store_acc_compound_buffer<STREAM_C, 4>(p, p.C, acc, m0 + wm, n0 + wn, lane);
+    else store_acc<SPLIT_C == C_COMPOUND, STREAM_C, false, false, 4>(p, p.C, acc, m0 + wm, n0 + wn, lane);
 }
 
 // C = alpha * (bias + sum over the K slices, in slice order) with the contraction's own output addressing
@@ -2413,10 +2418,11 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
             if (rc == RC_OK) rc = launch_split(jb, stream);
             if (rc == RC_OK) {
                 const bool stream_c = p.stream_c && !partial;
-                if (split && !partial) { if (stream_c) hipLaunchKernelGGL((gemm_planes_kernel<true, true>), pgrid, block, 0, stream, q, ws, ws + a_bytes, chunks, ma_pad, nb_pad, slice_chunks, partial, fired_a, fired_b);
-                                         else hipLaunchKernelGGL((gemm_planes_kernel<true, false>), pgrid, block, 0, stream, q, ws, ws + a_bytes, chunks, ma_pad, nb_pad, slice_chunks, partial, fired_a, fired_b); }
-                else                   { if (stream_c) hipLaunchKernelGGL((gemm_planes_kernel<false, true>), pgrid, block, 0, stream, q, ws, ws + a_bytes, chunks, ma_pad, nb_pad, slice_chunks, partial, fired_a, fired_b);
-                                         else hipLaunchKernelGGL((gemm_planes_kernel<false, false>), pgrid, block, 0, stream, q, ws, ws + a_bytes, chunks, ma_pad, nb_pad, slice_chunks, partial, fired_a, fired_b); }
+#define PPML_PLANES(C_, STREAM_) hipLaunchKernelGGL((gemm_planes_kernel<C_, STREAM_>), pgrid, block, 0, stream, q, ws, ws + a_bytes, chunks, ma_pad, nb_pad, slice_chunks, partial, fired_a, fired_b)
+                if (!split || partial) { if (stream_c) PPML_PLANES(C_DENSE, true); else PPML_PLANES(C_DENSE, false); }
+                else if (p.c_span)     { if (stream_c) PPML_PLANES(C_COMPOUND_BUFFER, true); else PPML_PLANES(C_COMPOUND_BUFFER, false); }
+                else                   { if (stream_c) PPML_PLANES(C_COMPOUND, true); else PPML_PLANES(C_COMPOUND, false); }
+#undef PPML_PLANES
                 rc = check_launch(what);
             }
             if (rc == RC_OK && partial) {
@@ -2438,6 +2444,12 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
         if (p.stream_c) hipLaunchKernelGGL((gemm_bf16x3_kernel<MODE, SPLIT, true>), grid, block, 0, stream, p);  \
         else hipLaunchKernelGGL((gemm_bf16x3_kernel<MODE, SPLIT, false>), grid, block, 0, stream, p); \
     } while (0)
+#define PPML_LAUNCH_BF16_C(MODE)                                                                      \
+    do {                                                                                              \
+        if (!split) PPML_LAUNCH_BF16(MODE, C_DENSE);                                                  \
+        else if (p.c_span) PPML_LAUNCH_BF16(MODE, C_COMPOUND_BUFFER);                                 \
+        else PPML_LAUNCH_BF16(MODE, C_COMPOUND);                                                      \
+    } while (0)
 #define PPML_LAUNCH_F32(MODE, SPLIT)                                                                  \
     do {                                                                                              \
         if (p.stream_c) hipLaunchKernelGGL((gemm_f32_kernel<MODE, SPLIT, true>), grid, block, 0, stream, p);  \
@@ -2446,7 +2458,7 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
     if (p.a_lm > 0) {
         if (split || p.f16_in || p.clamp) { set_error("%s: no split-operand instance for this addressing", what); return RC_BAD_ARGS; }
         if (fp32_pipe) PPML_LAUNCH_F32(LOAD_SPLIT_A, false);
-        else PPML_LAUNCH_BF16(LOAD_SPLIT_A, false);
+        else PPML_LAUNCH_BF16(LOAD_SPLIT_A, C_DENSE);
     }
     else if (!p.clamp && !p.f16_in && fp32_pipe) {
         if (mode == LOAD_K_CONTIG)        { if (split) PPML_LAUNCH_F32(LOAD_K_CONTIG, true);   else PPML_LAUNCH_F32(LOAD_K_CONTIG, false); }
@@ -2512,8 +2524,8 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
             if (p.stream_c) hipLaunchKernelGGL((gemm_bf16x3_pc_kernel<LOAD_ROW_CONTIG, true, true>), grid, dim3(512), 0, stream, p);
             else hipLaunchKernelGGL((gemm_bf16x3_pc_kernel<LOAD_ROW_CONTIG, false, true>), grid, dim3(512), 0, stream, p);
         }
-        else if (p.stream_c) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_ROW_CONTIG, false, true, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_ROW_CONTIG, false, false, true>), grid, block, 0, stream, p);
+        else if (p.stream_c) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_ROW_CONTIG, C_DENSE, true, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_ROW_CONTIG, C_DENSE, false, true>), grid, block, 0, stream, p);
     }
     else if (!p.clamp && !p.f16_in) {
         // binary32 operands without the finite guard: the contraction runs on the bf16 matrix pipe
@@ -2545,7 +2557,7 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
 #undef PPML_KPC
         }
         else if (k_fast) {
-#define PPML_KFAST(STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_K_CONTIG, false, STREAM_, true, K4_>), grid, block, 0, stream, p)
+#define PPML_KFAST(STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_K_CONTIG, C_DENSE, STREAM_, true, K4_>), grid, block, 0, stream, p)
             if (p.K % 4 == 0) { if (p.stream_c) PPML_KFAST(true, true); else PPML_KFAST(false, true); }
             else              { if (p.stream_c) PPML_KFAST(true, false); else PPML_KFAST(false, false); }
 #undef PPML_KFAST
@@ -2554,15 +2566,19 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
         // below 2 GiB that are contiguous in k or in their rows: buffer-addressed loads, the generic store
         else if (split && p.a_lm == 0 && mode == LOAD_K_CONTIG && ((p.M - 1) * p.a_rs + p.K) * 4 < (1LL << 31) &&
                  ((p.N - 1) * p.b_rs + p.K) * 4 < (1LL << 31) && p.a_rs < (1 << 22) && p.b_rs < (1 << 22)) {
-#define PPML_KFAST_SPLIT(STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_K_CONTIG, true, STREAM_, true, K4_>), grid, block, 0, stream, p)
-            if (p.K % 4 == 0) { if (p.stream_c) PPML_KFAST_SPLIT(true, true); else PPML_KFAST_SPLIT(false, true); }
-            else              { if (p.stream_c) PPML_KFAST_SPLIT(true, false); else PPML_KFAST_SPLIT(false, false); }
+#define PPML_KFAST_SPLIT(C_, STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_K_CONTIG, C_, STREAM_, true, K4_>), grid, block, 0, stream, p)
+#define PPML_KFAST_SPLIT_K4(C_, STREAM_) do { if (p.K % 4 == 0) PPML_KFAST_SPLIT(C_, STREAM_, true); else PPML_KFAST_SPLIT(C_, STREAM_, false); } while (0)
+            if (p.c_span) { if (p.stream_c) PPML_KFAST_SPLIT_K4(C_COMPOUND_BUFFER, true); else PPML_KFAST_SPLIT_K4(C_COMPOUND_BUFFER, false); }
+            else          { if (p.stream_c) PPML_KFAST_SPLIT_K4(C_COMPOUND, true); else PPML_KFAST_SPLIT_K4(C_COMPOUND, false); }
+#undef PPML_KFAST_SPLIT_K4
 #undef PPML_KFAST_SPLIT
         }
         else if (split && p.a_lm == 0 && mode == LOAD_ROW_CONTIG && p.K * p.a_ks * 4 < (1LL << 31) && p.K * p.b_ks * 4 < (1LL << 31) &&
                  p.a_ks < (1 << 24) && p.b_ks < (1 << 24)) {
-            if (p.stream_c) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_ROW_CONTIG, true, true, true>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_ROW_CONTIG, true, false, true>), grid, block, 0, stream, p);
+#define PPML_RFAST_SPLIT(C_, STREAM_) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_ROW_CONTIG, C_, STREAM_, true>), grid, block, 0, stream, p)
+            if (p.c_span) { if (p.stream_c) PPML_RFAST_SPLIT(C_COMPOUND_BUFFER, true); else PPML_RFAST_SPLIT(C_COMPOUND_BUFFER, false); }
+            else          { if (p.stream_c) PPML_RFAST_SPLIT(C_COMPOUND, true); else PPML_RFAST_SPLIT(C_COMPOUND, false); }
+#undef PPML_RFAST_SPLIT
         }
         // A contiguous in k, B contiguous in its rows, dense output planes below 2 GiB (the backward of the triangle
         // multiplication): the loading / contracting form with a loader per operand, whatever the number of tiles
@@ -2574,9 +2590,9 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
             else              { if (p.stream_c) PPML_MIXED(true, false); else PPML_MIXED(false, false); }
 #undef PPML_MIXED
         }
-        else if (mode == LOAD_K_CONTIG)   { if (split) PPML_LAUNCH_BF16(LOAD_K_CONTIG, true);   else PPML_LAUNCH_BF16(LOAD_K_CONTIG, false); }
-        else if (mode == LOAD_ROW_CONTIG) { if (split) PPML_LAUNCH_BF16(LOAD_ROW_CONTIG, true); else PPML_LAUNCH_BF16(LOAD_ROW_CONTIG, false); }
-        else                              { if (split) PPML_LAUNCH_BF16(LOAD_STRIDED, true);    else PPML_LAUNCH_BF16(LOAD_STRIDED, false); }
+        else if (mode == LOAD_K_CONTIG)   PPML_LAUNCH_BF16_C(LOAD_K_CONTIG);
+        else if (mode == LOAD_ROW_CONTIG) PPML_LAUNCH_BF16_C(LOAD_ROW_CONTIG);
+        else                              PPML_LAUNCH_BF16_C(LOAD_STRIDED);
     }
     else if (p.clamp) {
         if (split || p.f16_in) { set_error("%s: no clamped instance for this addressing", what); return RC_BAD_ARGS; }
@@ -2608,6 +2624,7 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
         else if (p.stream_c) hipLaunchKernelGGL((gemm_f16_kernel<true>), grid, block, 0, stream, p);
         else hipLaunchKernelGGL((gemm_f16_kernel<false>), grid, block, 0, stream, p);
     }
+#undef PPML_LAUNCH_BF16_C
 #undef PPML_LAUNCH_BF16
 #undef PPML_LAUNCH_F32
     return check_launch(what);
