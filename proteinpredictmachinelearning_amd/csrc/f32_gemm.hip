@@ -633,14 +633,15 @@ __device__ __forceinline__ void load_rows8_buffer(const __amdgpu_buffer_rsrc_t r
 }
 
 // two rows (tid / 4 and tid / 4 + 64 of the tile), four consecutive k each, of an operand plane whose rows are
-// contiguous in k: A(row, k) = plane[row * rs + k].  K4 (K a multiple of four): a piece of sixteen bytes never runs
-// over the end of its row, so it is one load; otherwise so is every piece of a chunk that ends inside K, and the last
+// contiguous in k: A(row, k) = plane[row * rs + k].  K4 = 1 (K a multiple of four): a piece of sixteen bytes never runs
+// over the end of its row, so it is one load; otherwise (0) so is every piece of a chunk that ends inside K, and the last
 // chunk goes element by element (a test that is the same for the work-group; element by element throughout, 412 planes of
-// 103 x 103 times 103 x 32 in the default attention took 37.3 us with its logits and softmax, 35.7 this way).  No branch
-// that lanes take differently: the generic form
+// 103 x 103 times 103 x 32 in the default attention took 37.3 us with its logits and softmax, 35.7 this way).  2: element
+// by element throughout, for a K of one whole chunk at most under few columns, where the test and the second form cost
+// what they give (51 x 21 -> 32 5.1 us against 5.4; 408 x 31 -> 256 6.4 against 6.1).  No branch that lanes take differently: the generic form
 // of this load sits inside tests of the row and of the row's end, and the compiler waits for every load at the end of
 // its branch (26368 x 256 -> 256: 29 us, the waves waiting 38 % of it; 25 us with this form).
-template <bool K4>
+template <int K4>
 __device__ __forceinline__ void load_kcontig_buffer(const __amdgpu_buffer_rsrc_t rsrc, uint32_t rs_bytes, int row0, int nrows, int k0, int K,
                                                     int tid, v4f (&reg)[2]) {
     const int k = k0 + (tid & 3) * 4;
@@ -648,10 +649,10 @@ __device__ __forceinline__ void load_kcontig_buffer(const __amdgpu_buffer_rsrc_t
     for (int it = 0; it < 2; ++it) {
         const int row = row0 + (tid >> 2) + it * 64;
         const uint32_t at = row < nrows ? static_cast<uint32_t>(row) * rs_bytes + static_cast<uint32_t>(k) * 4u : OUTSIDE;
-        if (K4) {
+        if (K4 == 1) {
             const v4i raw = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, k < K ? at : OUTSIDE, 0, 0));
             reg[it] = __builtin_bit_cast(v4f, raw);
-        } else if (k0 + BK <= K) {
+        } else if (K4 == 0 && k0 + BK <= K) {
             reg[it] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, 0));
         } else {
 #pragma unroll
@@ -696,7 +697,7 @@ __device__ __forceinline__ void store_acc_buffer(const __amdgpu_buffer_rsrc_t rs
 // residues x 8 sequences 14.0 -> 16.5 us, the value form at 8 x 8 x 33 13.5 -> 15.6).
 constexpr int C_DENSE = 0, C_COMPOUND = 1, C_COMPOUND_BUFFER = 2;
 
-template <int MODE, int SPLIT_C, bool STREAM_C, bool FAST_IO = false, bool K4 = true>
+template <int MODE, int SPLIT_C, bool STREAM_C, bool FAST_IO = false, int K4 = 1>
 __global__ __launch_bounds__(256) void gemm_bf16x3_kernel(const GemmParams p) {
     // (FAST_IO with SPLIT_C: buffer-addressed loads, the output by its compound addressing)
     static_assert(!FAST_IO || MODE == LOAD_ROW_CONTIG || MODE == LOAD_K_CONTIG, "buffer addressing: rows contiguous in themselves or in k");
@@ -2558,8 +2559,9 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
         }
         else if (k_fast) {
 #define PPML_KFAST(STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_K_CONTIG, C_DENSE, STREAM_, true, K4_>), grid, block, 0, stream, p)
-            if (p.K % 4 == 0) { if (p.stream_c) PPML_KFAST(true, true); else PPML_KFAST(false, true); }
-            else              { if (p.stream_c) PPML_KFAST(true, false); else PPML_KFAST(false, false); }
+            if (p.K % 4 == 0) { if (p.stream_c) PPML_KFAST(true, 1); else PPML_KFAST(false, 1); }
+            else if (p.K < 2 * BK && p.N <= 64) { if (p.stream_c) PPML_KFAST(true, 2); else PPML_KFAST(false, 2); }
+            else              { if (p.stream_c) PPML_KFAST(true, 0); else PPML_KFAST(false, 0); }
 #undef PPML_KFAST
         }
         // an output with compound addressing (the outer-product-mean in its graph and value forms) over operand planes
@@ -2567,7 +2569,7 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
         else if (split && p.a_lm == 0 && mode == LOAD_K_CONTIG && ((p.M - 1) * p.a_rs + p.K) * 4 < (1LL << 31) &&
                  ((p.N - 1) * p.b_rs + p.K) * 4 < (1LL << 31) && p.a_rs < (1 << 22) && p.b_rs < (1 << 22)) {
 #define PPML_KFAST_SPLIT(C_, STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_K_CONTIG, C_, STREAM_, true, K4_>), grid, block, 0, stream, p)
-#define PPML_KFAST_SPLIT_K4(C_, STREAM_) do { if (p.K % 4 == 0) PPML_KFAST_SPLIT(C_, STREAM_, true); else PPML_KFAST_SPLIT(C_, STREAM_, false); } while (0)
+#define PPML_KFAST_SPLIT_K4(C_, STREAM_) do { if (p.K % 4 == 0) PPML_KFAST_SPLIT(C_, STREAM_, 1); else PPML_KFAST_SPLIT(C_, STREAM_, 0); } while (0)
             if (p.c_span) { if (p.stream_c) PPML_KFAST_SPLIT_K4(C_COMPOUND_BUFFER, true); else PPML_KFAST_SPLIT_K4(C_COMPOUND_BUFFER, false); }
             else          { if (p.stream_c) PPML_KFAST_SPLIT_K4(C_COMPOUND, true); else PPML_KFAST_SPLIT_K4(C_COMPOUND, false); }
 #undef PPML_KFAST_SPLIT_K4

@@ -655,6 +655,17 @@ def test_split_ahead_workspace_on_two_streams(ops):
         assert torch.equal(o, want1 if which == 1 else want2)
 
 
+# k of less than a chunk, one chunk and one with a remainder, either side of the columns up to which it is loaded element by
+# element; integer operands: the sums are exact
+@pytest.mark.parametrize("K", [1, 5, 15, 17, 31, 33])
+@pytest.mark.parametrize("M,N", [(51, 64), (51, 65), (200, 33), (130, 128)])
+def test_mul_mat_short_k(ops, oracle, M, K, N):
+    rng = np.random.default_rng(K * N)
+    a, b = rng.integers(-9, 10, size=(M, K)).astype(np.float32), rng.integers(-9, 10, size=(N, K)).astype(np.float32)
+    bias = rng.integers(-9, 10, size=N).astype(np.float32)
+    assert np.array_equal(ops.mul_mat(_dev(a), _dev(b), _dev(bias)).cpu().numpy(), oracle.mul_mat_f32(a, b, bias))
+
+
 # runs of one row tile (32), one more (33: every tile but the first crosses), ragged (47), several whole tiles (64, 96), a
 # batch; 2048 columns a side and more through the operands split ahead (whole tiles there, 99: crossing ones), and the
 # shortest run that keeps the general form (31)
