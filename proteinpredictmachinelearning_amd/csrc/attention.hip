@@ -430,14 +430,22 @@ extern "C" int flash_attn_forward_ex_hip(int B, int h, int L, int d, int causal,
     p.out_ld = (layout >> 1) & 1;
     StatsScope stat("hip/flash_attn", static_cast<int64_t>(planes) * L, d, L, static_cast<hipStream_t>(stream));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // Four-wave work-groups (128 queries), eight-wave ones where they hold a whole plane that four-wave ones share between
-    // two: K and V are then staged and split once per plane, not twice (us, four / eight waves, 32 features with bias: 824
-    // planes of 160 44.0 / 37.7, 224 59.7 / 57.6, 256 91 / 88; 200 of 256 26.8 / 24.3, 64 of 256 21.0 / 20.4).  Beyond 256
-    // a plane does not end with its last work-group: 400 planes of 320 62 / 78, 400 of 384 95 / 112.
+    // Four-wave work-groups (128 queries).  From 129 to 256 rows an eight-wave one can hold the whole plane, so that K and V
+    // are staged and split once per plane, not twice.  It takes 1.5 to 1.8 times as long as one of the two that it replaces:
+    // worth it where those would queue for the CUs -- more than half as many planes as CUs -- and, but for up to 160 rows,
+    // not where a CU gets two of it in place of three (planes between one and one and a half times the CUs).  us, four /
+    // eight waves, 32 features, bias unless said: 64 planes of 176 14.0 / 15.4, 128 of 256 without 16.1 / 17.5; 200 of 256
+    // 25.8 / 23.5, 420 of 160 26.9 / 20.5; 300 of 240 31.4 / 33.6 (of 160 22.0 / 19.5); 824 of 160 43.8 / 37.4, of 256 83 / 83,
+    // without 58 / 57, 1024 of 256 103 / 97.  Causal, the second of two four-wave work-groups has most of the keys: eight
+    // waves win there from 193 rows on (300 of 240 29.3 / 28.9, without bias 26.2 / 24.3), and below that lose wherever the
+    // four-wave ones' rounds are odd (824 of 176 36.7 / 39.2).  The bits do not depend on it.  Beyond 256 rows a plane does
+    // not end with its last work-group: 400 planes of 320 62 / 78, 400 of 384 95 / 112.
     const bool short_rows = L <= 128;
+    const int64_t cus = device_cu_count(), rounds = (2 * planes + cus - 1) / cus;
+    const bool whole = L > 128 && L <= 256 && 2 * planes > cus && (L <= 160 || (causal ? L > 192 || rounds % 2 == 0 : rounds != 3));
     if (d <= 32) {
         if (short_rows) return launch_flash<32, 4, true>(p, s);
-        return L <= 256 ? launch_flash<32, 8, false>(p, s) : launch_flash<32, 4, false>(p, s);
+        return whole ? launch_flash<32, 8, false>(p, s) : launch_flash<32, 4, false>(p, s);
     }
     return short_rows ? launch_flash<64, 4, true>(p, s) : launch_flash<64, 4, false>(p, s);
 }

@@ -75,13 +75,29 @@ def test_flash_attn_forward_matches_oracle(ops, oracle, B, h, L, d, causal, use_
     _check(got_o, got_lse, want_o, want_lse)
 
 
-# eight waves on a plane of 129 to 256: waves without queries, tiles past the last key, stages of 96 and 128 keys
+# planes of 129 to 256: waves without queries, tiles past the last key
 @pytest.mark.parametrize("L,d,causal", [(130, 24, False), (161, 32, True), (193, 8, False), (224, 32, False), (255, 32, True), (257, 32, False)])
 def test_flash_attn_forward_whole_planes(ops, oracle, L, d, causal):
     rng = np.random.default_rng(L)
     q, k, v = [rng.standard_normal((1, 3, L, d)).astype(np.float32) for _ in range(3)]
     bias = (2 * rng.standard_normal((1, 3, L, L))).astype(np.float32)
     _check(*_run(ops, q, k, v, bias, causal=causal), *oracle.flash_attn_forward(q, k, v, bias, causal=causal))
+
+
+# four-wave and eight-wave work-groups on either side of the numbers of planes between which the choice changes: same bits
+@pytest.mark.parametrize("planes", [129, 300, 400])
+@pytest.mark.parametrize("L,d,causal,use_bias", [(129, 32, False, True), (161, 24, True, True), (176, 32, False, False), (224, 8, True, False),
+                                                 (255, 32, False, True), (256, 32, True, True)])
+def test_flash_attn_forward_has_the_bits_of_fewer_planes(ops, planes, L, d, causal, use_bias):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(planes + L)
+    q, k, v = (torch.randn(1, planes, L, d, device="cuda", generator=g) for _ in range(3))
+    bias = torch.randn(1, planes, L, L, device="cuda", generator=g) if use_bias else None
+    o, lse = ops.flash_attn_forward(q, k, v, bias, causal=causal)
+    for p0 in range(0, planes, 100):
+        part = [None if t is None else t[:, p0:p0 + 100].contiguous() for t in (q, k, v, bias)]
+        o1, lse1 = ops.flash_attn_forward(*part, causal=causal)
+        assert torch.equal(o[:, p0:p0 + 100], o1) and torch.equal(lse[:, p0:p0 + 100], lse1)
 
 
 def test_reference_golden_vectors(ops):
