@@ -177,6 +177,14 @@ def test_softmax_of_many_rows_has_the_bits_of_few(ops, D, rest):
         assert torch.equal(ops.softmax(x, bias=b).view(torch.int32), want.view(torch.int32)), brows
 
 
+# rows of 161 to 256 in pieces of sixteen bytes: four a wave from 131072 on, either side of that number and of 160 elements
+@pytest.mark.parametrize("rows,D", [(131071, 192), (131073, 164), (131074, 256), (16385, 160), (16387, 164)])
+def test_softmax_of_very_many_rows_has_the_bits_of_few(ops, rows, D):
+    g = torch.Generator(device="cuda").manual_seed(rows + D)
+    x = 3 * torch.randn(rows, D, device="cuda", generator=g)
+    assert torch.equal(ops.softmax(x), torch.cat([ops.softmax(c.clone()) for c in x.split(16000)]))
+
+
 @pytest.mark.parametrize("D", [1, 3, 64, 103, 256, 257, 512, 513, 2048, 2049, 5000])
 def test_softmax_with_the_bias_add_folded_in_has_the_bits_of_the_two_nodes(ops, oracle, D):
     rng = np.random.default_rng(D + 1)
