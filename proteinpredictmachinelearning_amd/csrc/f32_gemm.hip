@@ -1057,7 +1057,7 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_slices_kernel(const GemmPa
 // mat_transpose(Q)), 256 x 32 per plane under K = 256), buffer addressing, same products in the same order as the other
 // forms: same bits.
 constexpr int SIDE_M = 1, SIDE_N = 2;
-template <int MODE, int SIDE, bool STREAM_C, bool K4>
+template <int MODE, int SIDE, bool STREAM_C, int K4>
 __global__ __launch_bounds__(512) void gemm_bf16x3_pc_narrow_kernel(const GemmParams p) {
     static_assert(SIDE == SIDE_M || SIDE == SIDE_N, "which operand is the narrow one");
     static_assert(MODE == LOAD_ROW_CONTIG || MODE == LOAD_K_CONTIG, "buffer addressing");
@@ -1107,7 +1107,7 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_narrow_kernel(const GemmPa
                     const int k = c * BK + (ptid & 3) * 4;
                     const int row = ptid >> 2;
                     const uint32_t at = row < narrow_rows ? static_cast<uint32_t>(row) * narrow_rs + static_cast<uint32_t>(k) * 4u : OUTSIDE;
-                    if (K4) {
+                    if (K4 == 1) {
                         xn[0] = __builtin_bit_cast(v4f, __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_narrow, k < p.K ? at : OUTSIDE, 0, 0)));
                     } else {
 #pragma unroll
@@ -2515,7 +2515,7 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
             const int64_t tiles_long = side_n ? p.tiles_m : p.tiles_n;
             if (side_n) p.tiles_n = 1; else p.tiles_m = 1;
             const dim3 ngrid(static_cast<unsigned>(tiles_long * p.np2 * p.np3));
-#define PPML_RNARROW(SIDE_, STREAM_) hipLaunchKernelGGL((gemm_bf16x3_pc_narrow_kernel<LOAD_ROW_CONTIG, SIDE_, STREAM_, true>), ngrid, dim3(512), 0, stream, p)
+#define PPML_RNARROW(SIDE_, STREAM_) hipLaunchKernelGGL((gemm_bf16x3_pc_narrow_kernel<LOAD_ROW_CONTIG, SIDE_, STREAM_, 1>), ngrid, dim3(512), 0, stream, p)
             if (side_n) { if (p.stream_c) PPML_RNARROW(SIDE_N, true); else PPML_RNARROW(SIDE_N, false); }
             else        { if (p.stream_c) PPML_RNARROW(SIDE_M, true); else PPML_RNARROW(SIDE_M, false); }
 #undef PPML_RNARROW
@@ -2544,11 +2544,13 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
             if (side_n) p.tiles_n = 1; else p.tiles_m = 1;
             const dim3 ngrid(static_cast<unsigned>(tiles_long * p.np2 * p.np3));
 #define PPML_KNARROW(SIDE_, STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_pc_narrow_kernel<LOAD_K_CONTIG, SIDE_, STREAM_, K4_>), ngrid, dim3(512), 0, stream, p)
-            const bool k4 = p.K % 4 == 0;
-            if (side_n) { if (k4) { if (p.stream_c) PPML_KNARROW(SIDE_N, true, true); else PPML_KNARROW(SIDE_N, false, true); }
-                          else    { if (p.stream_c) PPML_KNARROW(SIDE_N, true, false); else PPML_KNARROW(SIDE_N, false, false); } }
-            else        { if (k4) { if (p.stream_c) PPML_KNARROW(SIDE_M, true, true); else PPML_KNARROW(SIDE_M, false, true); }
-                          else    { if (p.stream_c) PPML_KNARROW(SIDE_M, true, false); else PPML_KNARROW(SIDE_M, false, false); } }
+#define PPML_KNARROW_K4(SIDE_, STREAM_) do { if (k4 == 1) PPML_KNARROW(SIDE_, STREAM_, 1); else if (k4 == 2) PPML_KNARROW(SIDE_, STREAM_, 2); else PPML_KNARROW(SIDE_, STREAM_, 0); } while (0)
+            // (four chunks under more tiles than two per CU: the three whole ones gain less than their test costs.  us, by
+            // chunks / by elements, 51 x 51 times 51 x 8: 824 planes 11.3 / 10.5, 412 planes 6.8 / 6.9)
+            const int k4 = p.K % 4 == 0 ? 1 : p.K <= 4 * BK && ngrid.x > 2 * static_cast<unsigned>(device_cu_count()) ? 2 : 0;
+            if (side_n) { if (p.stream_c) PPML_KNARROW_K4(SIDE_N, true); else PPML_KNARROW_K4(SIDE_N, false); }
+            else        { if (p.stream_c) PPML_KNARROW_K4(SIDE_M, true); else PPML_KNARROW_K4(SIDE_M, false); }
+#undef PPML_KNARROW_K4
 #undef PPML_KNARROW
         }
         else if (k_fast && two_sets) {

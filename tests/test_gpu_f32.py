@@ -666,6 +666,18 @@ def test_mul_mat_short_k(ops, oracle, M, K, N):
     assert np.array_equal(ops.mul_mat(_dev(a), _dev(b), _dev(bias)).cpu().numpy(), oracle.mul_mat_f32(a, b, bias))
 
 
+# one narrow side under a k of four chunks, more tiles than two per CU and fewer: same bits; integer operands, exact sums
+@pytest.mark.parametrize("K", [49, 51, 63])
+@pytest.mark.parametrize("rows,cols", [(51, 8), (40, 30), (7, 60)])
+def test_out_prod_tt_narrow_in_many_planes(ops, K, rows, cols):
+    rng = np.random.default_rng(K + rows)
+    planes = 600
+    a, b = (rng.integers(-9, 10, size=(planes, n, K)).astype(np.float32) for n in (rows, cols))
+    got = ops.out_prod_tt(_dev(a), _dev(b)).view(planes, cols, rows)
+    few = torch.cat([ops.out_prod_tt(_dev(a[i:i + 200]), _dev(b[i:i + 200])).view(-1, cols, rows) for i in range(0, planes, 200)])
+    assert torch.equal(got, few) and np.array_equal(got.cpu().numpy(), np.matmul(b, a.transpose(0, 2, 1)))
+
+
 # runs of one row tile (32), one more (33: every tile but the first crosses), ragged (47), several whole tiles (64, 96), a
 # batch; 2048 columns a side and more through the operands split ahead (whole tiles there, 99: crossing ones), and the
 # shortest run that keeps the general form (31)
