@@ -420,7 +420,7 @@ def main() -> int:
                 keep.append(sets)
                 return fn, ns
             return make
-        # flops: five 2*L*L*D contractions per plane in exact terms (S, dP, dQ, dK, dV); S and dP are computed twice
+        # flops: five 2*L*L*D contractions per plane (S, dP, dQ, dK, dV)
         f32_case(attention_back(824, 256, 32), (8 * 824 * 256 * 32 + 824 * 256 + 2 * 824 * 256 * 256) * 4,
                  10.0 * 824 * 256 * 256 * 32, "fused_attention_backward_msa_824x256x32_bias", pipe="bf16x3")
 

@@ -55,7 +55,7 @@ struct AttnParams {
     int causal;
     float scale, eps;
     int head;            // keys of the reference's first block: min(Bc, keys of the row)
-    int stage_rows;      // keys staged in LDS at a time: min(CH, L rounded up to 32)
+    int stage_rows;      // keys staged in LDS at a time: at most CH, L's tiles of 32 shared out evenly
     int in_ld;           // Q, K, V are [B][h][d][L] (the graph's [L, D, h, B] tensors, not yet permuted)
     int out_ld;          // O is written as [B][h][d][L]
 };

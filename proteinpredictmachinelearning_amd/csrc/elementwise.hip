@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void softmax_rows_kernel(const float* __restri
     const int lane = threadIdx.x & 63;
     const int64_t row0 = (static_cast<int64_t>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * ROWS;
     if (row0 >= rows) return;
-    const int64_t left = rows - row0;                   // (rows past the last one are computed as the last one, not stored)
+    const int64_t left = rows - row0;                   // (rows past the last one are computed as the wave's first, not stored)
     int64_t brow = 0;
     if (HAS_BIAS) brow = rows < (1LL << 31) ? static_cast<int64_t>(static_cast<uint32_t>(row0) % static_cast<uint32_t>(bias_rows)) : row0 % bias_rows;
     constexpr int W = VEC ? 4 : 1;
