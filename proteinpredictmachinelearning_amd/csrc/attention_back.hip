@@ -1041,13 +1041,16 @@ extern "C" int flash_attn_backward_hip(int B, int h, int L, int d, int causal, f
     // rounds 3/4 full and a side's pair (dbias with the bias its kernel would read a lane per row): causal from 129 rows on
     // (412 of 256, dQ and dbias 62 / 83), not causal from 129 to 256 rows in at most two rounds (256 of 160, dK and dV 22 / 26),
     // or with a bias from 385 to 512 (200 of 448, dQ and dbias 117 / 142).
+    // dQ on the memory of Q, dO or O, which such a call may have (the rows kernel reads a query's row before it writes it),
+    // rules out rounds: they read those again.
     // Either way the bits are the same: where the whole set goes in one pass, the two kernels compute as it does.
     const int64_t cus = device_cu_count(), slots = (planes + cus - 1) / cus * cus;
     const bool rows = dQ || dbias, cols = dK || dV;
     const bool whole = d <= 32 && L < 16384 &&
                        (L <= 256 || (causal || (bias && L <= 512) ? 8 * planes >= 3 * cus : bias ? 2 * planes >= cus : 5 * planes >= 3 * slots));
     const bool pair = (dK && dV) || (dbias && bias);
-    const bool one_side = pair && L > 128 && 4 * planes >= 3 * slots &&
+    const bool in_place = dQ && (dQ == Q || dQ == dO || dQ == O);
+    const bool one_side = pair && L > 128 && !(in_place && L > 256) && 4 * planes >= 3 * slots &&
                           (causal ? bias || planes <= 2 * cus
                                   : L <= 256 ? planes <= 2 * cus && (cols || dQ) : bias && L > 384 && L <= 512);
     if (whole && ((rows && cols) || one_side)) {

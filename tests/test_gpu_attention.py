@@ -305,6 +305,28 @@ def test_flash_attn_backward_subsets_have_the_bits_of_the_whole(ops, planes, L, 
             assert x is None or torch.equal(x, w), (want, n)
 
 
+# dQ and dbias on the memory of Q (dO, O) and the bias: a query's row and a pair's bias are read before they are written, in
+# one round of keys (256 x 150), in rounds (causal 200 x 260, 200 x 400) and where the rows kernel is the rule (3 x 300)
+@pytest.mark.parametrize("planes,L,d,causal", [(256, 150, 32, False), (200, 260, 32, True), (200, 400, 16, False), (3, 300, 32, True)])
+def test_flash_attn_backward_rows_in_place(ops, planes, L, d, causal):
+    from proteinpredictmachinelearning_amd import cabi
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(L)
+    q, k, v, do = (torch.randn(1, planes, L, d, device="cuda", generator=g) for _ in range(4))
+    bias = torch.randn(1, planes, L, L, device="cuda", generator=g)
+    o, lse = ops.flash_attn_forward(q, k, v, bias, causal=causal)
+    dq, _, _, db = ops.flash_attn_backward(q, k, v, bias, o, do, lse, causal=causal, want=("dq", "dbias"))
+    for name in ("q", "o", "do"):
+        x = dict(q=q.clone(), o=o.clone(), do=do.clone())
+        out_b = bias.clone()
+        rc = cabi.load().flash_attn_backward_hip(1, planes, L, d, int(causal), 0.0, x["q"].data_ptr(), k.data_ptr(), v.data_ptr(),
+                                                 out_b.data_ptr(), x["o"].data_ptr(), x["do"].data_ptr(), lse.data_ptr(),
+                                                 x[name].data_ptr(), None, None, out_b.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        assert torch.equal(x[name], dq) and torch.equal(out_b, db), name
+
+
 # one pass and two kernels (few long planes, 64 features), one round of keys and two, whole and ragged tiles
 @pytest.mark.parametrize("planes,L,d,use_bias", [(2, 70, 32, True), (3, 160, 24, False), (2, 256, 32, True), (97, 300, 32, True), (97, 288, 8, False),
                                                  (2, 300, 32, True), (2, 150, 64, True)])
