@@ -2125,7 +2125,18 @@ __global__ __launch_bounds__(256) void reduce_slices_kernel(const GemmParams p, 
         for (int c = 0; c < 4; ++c) if (n4 + c < p.N) sum[c] = p.bias[n4 + c];
     }
     const float* src = partial + static_cast<size_t>(m) * nb_pad + n4;          // nb_pad is a multiple of 128
-    for (int s = 0; s < slices; ++s) sum += *reinterpret_cast<const v4f*>(src + static_cast<size_t>(s) * ma_pad * nb_pad);
+    // in slice order; eight loads in flight at a time (one after the other the kernel waited a memory round trip per slice: the
+    // weight gradient of 32768 x 64 -> 64, 89 slices, 44.6 -> 22.7 us, of 26368 x 300 -> 100 42.8 -> 24.0)
+    const size_t step = static_cast<size_t>(ma_pad) * nb_pad;
+    int s = 0;
+    for (; s + 8 <= slices; s += 8) {
+        v4f x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = *reinterpret_cast<const v4f*>(src + (s + i) * step);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum += x[i];
+    }
+    for (; s < slices; ++s) sum += *reinterpret_cast<const v4f*>(src + s * step);
     // operands the split could not carry: these four again, the reference's way -- by the flags of the splits, or
     // (callers that pass none) wherever the slices' sum is NaN, which is what a slice leaves for such a tile
     if (fired_a ? (fired_a[m >> 5] | fired_b[n4 >> 5]) != 0 : (sum[0] != sum[0] || sum[1] != sum[1] || sum[2] != sum[2] || sum[3] != sum[3])) {
