@@ -14,7 +14,7 @@
 // pipe unchanged (gemm_f16_kernel).  The clamped contraction of the triangle multiplication, whose
 // result depends on how infinities propagate, stays on the fp32 pipe (gemm_f32_kernel:
 // v_mfma_f32_32x32x2_f32, k ascending two at a time).
-#include "common.hpp"
+#include "gemm.hpp"
 
 #include <atomic>
 #include <type_traits>
@@ -29,31 +29,6 @@ constexpr int BM = 128, BN = 128, BK = 16;
 constexpr int LDS_LD = BM + 4;        // row pitch of the k-major LDS tiles (floats)
 
 enum LoadMode { LOAD_K_CONTIG = 0, LOAD_ROW_CONTIG = 1, LOAD_STRIDED = 2, LOAD_SPLIT_A = 4 };
-
-struct GemmParams {
-    const float* A;       // rows m: A(m,k) = A[m*a_rs + k*a_ks]
-    const float* B;       // cols n: B(n,k) = B[n*b_rs + k*b_ks]
-    float* C;
-    const float* bias;    // [N] or null
-    int M, N, K;
-    int64_t a_rs, a_ks, b_rs, b_ks;
-    // planes: p = p3*np2 + p2
-    int np2, np3;
-    int64_t a_p2, a_p3, b_p2, b_p3, c_p2, c_p3;
-    int b_div2, b_div3;   // B-side plane index = p / div (out_prod's src0 broadcast)
-    float alpha;
-    // C(m,n) = C[(m/c_lm)*c_mo + (m%c_lm)*c_mi + (n/c_ln)*c_no + (n%c_ln)*c_ni]
-    int c_lm, c_ln;
-    int64_t c_mo, c_mi, c_no, c_ni;
-    int tiles_m, tiles_n;
-    int stream_c;         // output larger than the last-level cache: write it with streaming stores
-    uint32_t c_span;      // compound output: bytes from C to behind a plane's last element where buffer addressing reaches them, else 0
-    int f16_in;           // A and B hold IEEE halves (k contiguous); products and sums are binary32
-    int clamp;            // finite guard in the epilogue (triangle multiplication)
-    // LOAD_SPLIT_A: both indices of A are compound, A(m,k) = A[(m/a_lm)*a_mo + (m%a_lm)*a_mi + (k/a_lk)*a_ko + (k%a_lk)*a_ki]
-    int a_lm, a_lk;
-    int64_t a_mo, a_mi, a_ko, a_ki;
-};
 
 // 16 x 128 tile of one operand -> two v4f per thread
 template <int MODE>
@@ -205,53 +180,6 @@ __device__ __forceinline__ void store_acc(const GemmParams& p, float* __restrict
                 if (CLAMP) v = (v != v) ? 0.0f : (v > 1e4f ? 1e4f : (v < -1e4f ? -1e4f : v));
                 if (STREAM_C) __builtin_nontemporal_store(v, &C[roff + coff]);
                 else C[roff + coff] = v;
-            }
-        }
-    }
-}
-
-// The same for an output with compound addressing whose planes 32-bit byte offsets reach (p.c_span, set by the launcher:
-// below 2 GiB, row runs of at least 32).  The general form above spends 36 vector instructions per stored register on
-// 64-bit addresses, carries and bounds, in a phase without matrix work (a third of all issue cycles of the contraction of
-// 12288 x 12288 outputs over 256).  Here a tile of 32 rows that stays within one run and inside the matrix -- known per
-// wave -- takes its row steps from scalar registers: a product and a store.  Other tiles pick the run per row.  Measured,
-// with both gradients: 384 residues x 32 features x 256 sequences 1342 -> 1239 us, 103 residues 152 -> 145.
-template <bool STREAM_C, int TI>
-__device__ __forceinline__ void store_acc_compound_buffer(const GemmParams& p, float* __restrict__ C, const v16f (&acc)[TI][2],
-                                                          int m_base, int n_base, int lane) {
-    constexpr int AUX = STREAM_C ? 3 : 0;
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(C, 0, static_cast<int>(p.c_span), 0x00020000);
-    const int j = lane & 31;
-    const int m_first = __builtin_amdgcn_readfirstlane(m_base);
-    const uint32_t mi_bytes = static_cast<uint32_t>(p.c_mi) * 4u;
-    const uint32_t carry = static_cast<uint32_t>(p.c_mo - p.c_lm * p.c_mi) * 4u;      // (modulo 2^32: only the sum has to be an offset)
-#pragma unroll
-    for (int ti = 0; ti < TI; ++ti) {
-        const int m0 = m_first + ti * 32;
-        const int q = m0 / p.c_lm, rem = m0 - q * p.c_lm;
-        const uint32_t row0 = static_cast<uint32_t>(q * p.c_mo + rem * p.c_mi) * 4u;
-        const bool whole = rem + 32 <= p.c_lm && m0 + 32 <= p.M;
-        const int own = 4 * (lane >> 5);               // this lane's first row of the tile
-#pragma unroll
-        for (int tj = 0; tj < 2; ++tj) {
-            const int n = n_base + tj * 32 + j;
-            if (n >= p.N) continue;
-            const int nq = n / p.c_ln;
-            const uint32_t base = row0 + own * mi_bytes + static_cast<uint32_t>(nq * p.c_no + (n - nq * p.c_ln) * p.c_ni) * 4u;
-            if (whole) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, acc[ti][tj][r] * p.alpha), rsrc, base,
-                                                          (8 * (r >> 2) + (r & 3)) * mi_bytes, AUX);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int step = 8 * (r >> 2) + (r & 3);
-                    uint32_t at = base + step * mi_bytes;
-                    if (rem + own + step >= p.c_lm) at += carry;                  // (at most one: the run is 32 or longer)
-                    if (m0 + own + step < p.M)
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, acc[ti][tj][r] * p.alpha), rsrc, at, 0, AUX);
-                }
             }
         }
     }
@@ -482,38 +410,6 @@ int launch_f32_midk(const GemmParams& p, hipStream_t stream, const char* what) {
 constexpr int SPLIT_PITCH = 48;                   // bytes per tile row in a plane: 16 bf16, then 16 bytes of padding
 constexpr int SPLIT_PLANE = BM * SPLIT_PITCH;     // one of the three bf16 planes of a 128 x 16 operand tile
 
-// One output the reference's way (src/backend/CPUKernels.cpp:763-771, 836-884, 1006-1028): from the bias (or zero),
-// one product at a time, k ascending, every product and every sum rounded to binary32 on its own (this file is
-// compiled without contraction).  A and B are the plane's bases.
-__device__ __forceinline__ float plain_dot(const GemmParams& p, const float* __restrict__ A, const float* __restrict__ B, int m, int n) {
-    float s = p.bias ? p.bias[n] : 0.0f;
-    const int64_t ra = p.a_lm > 0 ? static_cast<int64_t>(m / p.a_lm) * p.a_mo + static_cast<int64_t>(m % p.a_lm) * p.a_mi
-                                  : static_cast<int64_t>(m) * p.a_rs;
-    const float* b = B + static_cast<int64_t>(n) * p.b_rs;
-    for (int k = 0; k < p.K; ++k) {
-        const float a = p.a_lm > 0 ? A[ra + static_cast<int64_t>(k / p.a_lk) * p.a_ko + static_cast<int64_t>(k % p.a_lk) * p.a_ki]
-                                   : A[ra + static_cast<int64_t>(k) * p.a_ks];
-        const float prod = a * b[static_cast<int64_t>(k) * p.b_ks];
-        s = s + prod;
-    }
-    return s;
-}
-
-// A whole tile of the output (rows x cols from (m0, n0) of the plane whose bases are A, B, C) by plain_dot, written
-// straight to C with the contraction's own output addressing: what a work-group does INSTEAD of storing its
-// accumulators when a SplitGuard fired for the tile.  One loop, no use of the accumulators: the ordinary path pays
-// nothing for it but the test.
-__device__ __forceinline__ void plain_tile(const GemmParams& p, const float* __restrict__ A, const float* __restrict__ B,
-                                           float* __restrict__ C, int m0, int n0, int rows, int cols, int tid) {
-    for (int e = tid; e < rows * cols; e += 256) {
-        const int m = m0 + e / cols, n = n0 + e % cols;
-        if (m >= p.M || n >= p.N) continue;
-        const float v = plain_dot(p, A, B, m, n) * p.alpha;
-        C[static_cast<int64_t>(m / p.c_lm) * p.c_mo + static_cast<int64_t>(m % p.c_lm) * p.c_mi +
-          static_cast<int64_t>(n / p.c_ln) * p.c_no + static_cast<int64_t>(n % p.c_ln) * p.c_ni] = v;
-    }
-}
-
 // The same for the kernels whose operands have contiguous rows (A(m, k) = A[k * a_ks + m]) and whose output plane is
 // dense (C[m * ldc + n]), without bias: it names nothing that those kernels do not hold already.
 __device__ __forceinline__ void plain_tile_rows(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
@@ -618,7 +514,6 @@ __device__ __forceinline__ void load_rows8(const float* __restrict__ base, int64
 // takes both over: the address is one 32-bit add per access, and an access whose offset is not inside the
 // plane is dropped (stores) or returns zero (loads) in hardware.  Lanes whose row or column lies outside the
 // matrix carry an offset of 2^31, which no plane reaches.
-constexpr uint32_t OUTSIDE = 0x80000000u;
 
 // one row, eight consecutive k of an operand plane [K][ks] whose rows are contiguous: A(row, k) = plane[k * ks + row]
 __device__ __forceinline__ void load_rows8_buffer(const __amdgpu_buffer_rsrc_t rsrc, uint32_t ks_bytes, int row0, int nrows, int k0,
@@ -691,11 +586,6 @@ __device__ __forceinline__ void store_acc_buffer(const __amdgpu_buffer_rsrc_t rs
         }
     }
 }
-
-// SPLIT_C of the kernels below: how the output is addressed.  The two compound forms are instances of their own: with both
-// stores in one kernel, chosen by p.c_span as it ran, the general one cost 1 to 2.5 us more per launch (32 features x 24
-// residues x 8 sequences 14.0 -> 16.5 us, the value form at 8 x 8 x 33 13.5 -> 15.6).
-constexpr int C_DENSE = 0, C_COMPOUND = 1, C_COMPOUND_BUFFER = 2;
 
 template <int MODE, int SPLIT_C, bool STREAM_C, bool FAST_IO = false, int K4 = 1>
 __global__ __launch_bounds__(256) void gemm_bf16x3_kernel(const GemmParams p) {
@@ -1686,7 +1576,6 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16x3_shortk_kernel(const GemmPa
 // into a binary32 accumulator, which is the reference's arithmetic (src/backend/CPUKernels.cpp:763-771
 // with half operands converted on load) up to the order of the additions; the bias joins the finished
 // sum, as the CPU branch of the reference does.
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 // eight consecutive halves (16 bytes) of row `row`, zeros past the matrix
 __device__ __forceinline__ v4i load_halves8(const uint16_t* __restrict__ base, int64_t rs, int row, int nrows, int k, int K) {
@@ -2182,22 +2071,6 @@ int f32_arithmetic() {
 // `fixed_ws` / `fixed_cap`: a workspace the caller brings (the static array of the entry point that allocates
 // nothing).  With one, the pool is never touched: a contraction that wants more workspace than `fixed_cap`
 // is refused, one that wants none runs as it always does.
-// How many K slices make `groups` output tiles come out even over the CUs (a CU's rate does not depend on how many
-// work-groups it holds): the smallest count within 2 % of the best, slices of at least `least_chunks` chunks.
-int even_slices(int groups, int chunks, int most_slices, int least_chunks = PLANES_MIN_SLICE_CHUNKS) {
-    const int cus = device_cu_count();
-    int most = chunks / least_chunks < most_slices ? chunks / least_chunks : most_slices;
-    if (most < 1) most = 1;
-    int slices = 1;
-    double best = 1e30;
-    for (int sl = 1; sl <= most; ++sl) {
-        const int64_t wgs = static_cast<int64_t>(groups) * sl;
-        const double waste = static_cast<double>((wgs + cus - 1) / cus * cus) / static_cast<double>(wgs);
-        if (waste < best - 0.02) { best = waste; slices = sl; }
-    }
-    return slices;
-}
-
 // gemm_bf16x3_half_split_kernel for a single-plane contraction whose tall operand A has compound indices; -1 when the
 // contraction is not of that kind (the caller goes on to the other forms).  p.tiles_m / p.tiles_n / p.stream_c are set.
 int try_half_split(const GemmParams& p, hipStream_t stream, const char* what) {
@@ -2212,7 +2085,7 @@ int try_half_split(const GemmParams& p, hipStream_t stream, const char* what) {
     if (p.a_mo < 0 || p.a_mi < 0 || p.a_ko < 0 || p.a_ki < 0 || a_span * 4 >= (1LL << 31) || (gen && a_span * 4 > (1LL << 30))) return -1;
     const int chunks = (p.K + BK - 1) / BK;
     const int groups = p.tiles_m * p.tiles_n;
-    int slices = even_slices(groups, chunks, 16);
+    int slices = even_slices(groups, chunks, 16, PLANES_MIN_SLICE_CHUNKS);
     const int slice_chunks = (chunks + slices - 1) / slices;
     slices = (chunks + slice_chunks - 1) / slice_chunks;
     const int ma_pad = p.tiles_m * BM, nb_pad = p.tiles_n * BN;
@@ -2387,6 +2260,10 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
     }
     const bool planes_fit = slices > 1 ? planes_groups * slices >= PLANES_MIN_GROUPS / 2 && static_cast<int64_t>(p.M) * p.N >= (1 << 20)
                                        : p.tiles_m >= PLANES_MIN_TILES && p.tiles_n >= PLANES_MIN_TILES && planes_groups >= PLANES_MIN_GROUPS;
+    if (!fp32_pipe && !fixed_ws) {
+        const int rc = try_f16x2(p, stream, what, nullptr, 0);
+        if (rc >= 0) return rc;
+    }
     if (!fp32_pipe && !fixed_ws && p.a_lm > 0) {
         const int rc = try_half_split(p, stream, what);
         if (rc >= 0) return rc;
@@ -2408,6 +2285,8 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
                 set_error("%s: this contraction needs %zu bytes of workspace, the static one holds %zu", what, ws_bytes, fixed_cap);
                 return RC_BAD_ARGS;
             }
+            const int rc = try_f16x2(p, stream, what, fixed_ws, fixed_cap);
+            if (rc >= 0) return rc;
             ws = fixed_ws;
         } else {
             held = workspace_take(ws_bytes, stream);
@@ -2644,6 +2523,33 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
 #undef PPML_LAUNCH_F32
     return check_launch(what);
 }
+
+}  // namespace
+
+// How many K slices make `groups` output tiles come out even over the CUs (a CU's rate does not depend on how many
+// work-groups it holds): the smallest count within 2 % of the best, slices of at least `least_chunks` chunks.
+int even_slices(int groups, int chunks, int most_slices, int least_chunks) {
+    const int cus = device_cu_count();
+    int most = chunks / least_chunks < most_slices ? chunks / least_chunks : most_slices;
+    if (most < 1) most = 1;
+    int slices = 1;
+    double best = 1e30;
+    for (int sl = 1; sl <= most; ++sl) {
+        const int64_t wgs = static_cast<int64_t>(groups) * sl;
+        const double waste = static_cast<double>((wgs + cus - 1) / cus * cus) / static_cast<double>(wgs);
+        if (waste < best - 0.02) { best = waste; slices = sl; }
+    }
+    return slices;
+}
+
+int launch_reduce_slices(const GemmParams& p, hipStream_t stream, const char* what, const float* partial, int slices, int ma_pad, int nb_pad) {
+    const int64_t threads = static_cast<int64_t>(p.M) * ((p.N + 3) / 4);
+    hipLaunchKernelGGL((reduce_slices_kernel<false>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, p, partial, slices,
+                       ma_pad, nb_pad, static_cast<const int*>(nullptr), static_cast<const int*>(nullptr));
+    return check_launch(what);
+}
+
+namespace {
 
 GemmParams plain_params() {
     GemmParams p{};

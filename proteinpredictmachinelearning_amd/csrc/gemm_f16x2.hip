@@ -1,0 +1,736 @@
+// Large binary32 contractions on the f16 matrix pipe.
+//
+// A binary32 number times a power of two that brings the largest element of its row near 2^12 .. 2^15 is, to within 2^-24
+// of itself, the sum of two halves: h = f16(x), l = f16(x - h), eleven significant bits each with the sign of l for one
+// more.  Three products -- h h, h l, l h -- are kept (l l lies below 2^-24 of |a||b|); the matrix pipe forms each exactly
+// and adds it into a binary32 accumulator, and the powers of two leave again by ldexp, exactly.  Against the exact split into three
+// bf16 parts with its six products (gemm_bf16x3_kernel) that is half the matrix work, a third less LDS traffic and less
+// than half the vector work (two v_fma_mixlo/hi per element); and, with half as many additions into the accumulator, half
+// the error.  What it asks for is the scale: a half has five bits of exponent.  One power of two per ROW of either operand
+// and K slice -- not per operand, whose rows may differ by anything -- keeps every element above 2^-17 of its row's largest
+// whole, and smaller ones to 2^-40 of that largest: an error of 2^-40 max_k|a| sum_k|b| at most, far below the binary32
+// rounding of the sum unless the row's largest elements meet only zeros.
+//
+// B (the smaller operand as a rule: a weight, an alignment's projection) is split ahead by split_f16x2_kernel, which sees a
+// whole row of the slice and knows its maximum.  A is split in the tile loop by the loading waves, whose scale
+// follows the data: a row starts at the scale of its first nonzero stage with three bits of room, and a stage with a larger element moves it
+// and leaves a factor by which the contracting waves multiply what they hold (a branch that is taken once in a row's life
+// as a rule).
+//
+// What no power of two can bring into range -- infinities, NaN, rows whose largest element lies below 2^-111 -- is noticed
+// with the maxima (v_maximum3_f32 passes NaN on), and the outputs concerned are redone in plain binary32 arithmetic, one
+// product at a time (plain_dot), as everywhere in this library.
+#include "gemm.hpp"
+
+#include <algorithm>
+
+namespace ppmlhip {
+namespace {
+
+constexpr int HX_M = 128;                          // rows of A per tile
+constexpr int HX_K = 32;                           // k per stage
+// A stage of A in LDS: 32 rows x 16 k of one part are two halves (k 0 .. 7, 8 .. 15) of 32 rows x 16 bytes, as the MFMA reads
+// them.  The paddings put the eight-byte pieces that sixteen lanes write (two rows, 32 k) into sixteen different banks' pairs.
+constexpr int HX_HALF = 576, HX_FRAG = 2 * HX_HALF, HX_STEP = 4 * HX_FRAG + 32, HX_PART = 2 * HX_STEP, HX_STAGE = 2 * HX_PART;
+constexpr int HX_BUFS = 3;                         // stages in LDS: one being written, one contracted, one peeked into
+constexpr int HX_AHEAD = 3;                        // stages a loading wave has in flight
+constexpr int HX_EXPS = 4;                         // items whose row exponents are kept (see lds_exp)
+constexpr int HX_BAD = 0x10000;                    // exponent of a row that the split cannot carry
+constexpr uint32_t HX_FIRST_SCALE = (127u + 126u) << 23;      // before a row's first nonzero element: 2^126
+constexpr int HX_KC = 0, HX_RC = 1, HX_KRUN = 2, HX_RRUN = 3; // how A lies: contiguous in k / in its rows; compound indices with runs along k / the rows
+constexpr int HX_PARTIAL = 0, HX_DENSE = 1, HX_COMPOUND = 2;  // where the sums go: the slices' workspace, a dense C, a compound C
+
+struct F16x2Job {
+    const uint8_t* wb;        // B's fragments: [stage][part][16-k step][tile of 32 columns][1 KB]
+    const int* eb;            // [slice][nb_pad]: exponent of B's column in the slice, HX_BAD where the split cannot carry it
+    float* partial;           // [slice][ma_pad][nb_pad]
+    int nb_pad, ma_pad;
+    int chunks, slice_chunks; // stages in all and per slice: even numbers
+    int slices, items;
+    uint32_t a_span;          // bytes of A from its base to behind its last element
+};
+
+// two halves of four consecutive elements times s
+__device__ __forceinline__ void split4_f16(const v4f& x, float s, uint2 (&out)[2]) {
+    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+    v4h h, l;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        h[c] = static_cast<_Float16>(__builtin_fmaf(x[c], s, 0.0f));
+        l[c] = static_cast<_Float16>(__builtin_fmaf(x[c], s, -static_cast<float>(h[c])));       // (the difference is exact)
+    }
+    out[0] = __builtin_bit_cast(uint2, h);
+    out[1] = __builtin_bit_cast(uint2, l);
+}
+
+// the largest magnitude, NaN if there is one
+__device__ __forceinline__ float max4(float m, const v4f& x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(x[0])), __builtin_fabsf(x[1]));
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(x[2])), __builtin_fabsf(x[3]));
+#else
+    return m + x[0];
+#endif
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// B ahead of the contraction.  A work-group takes 32 rows of B (columns of the product) and one slice of K: maxima, scale,
+// parts.  A round covers 256 k; a slice of up to eight rounds stays in registers between the two passes.
+constexpr int HX_SPLIT_ROUNDS = 8;
+struct F16x2Split {
+    const float* src;
+    uint8_t* dst;
+    int* exps;
+    int rows, rows_pad, K, chunks, slice_chunks;
+    int64_t rs, ks;
+};
+
+template <bool KS1>
+__global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) {
+    __shared__ uint32_t lds_max[32][33];
+    const int tid = threadIdx.x;
+    // (row of the 32, octet of k within a round): lanes along k or along the rows, as the operand lies
+    const int row = KS1 ? tid >> 5 : tid & 31, oct = KS1 ? tid & 31 : tid >> 5;
+    const int r = blockIdx.x * 32 + row;
+    const int c_begin = blockIdx.y * jb.slice_chunks;
+    const int c_end = c_begin + jb.slice_chunks < jb.chunks ? c_begin + jb.slice_chunks : jb.chunks;
+    const int k_begin = c_begin * HX_K, k_end = c_end * HX_K;
+    const int rounds = (k_end - k_begin + 255) / 256;
+    const float* src = jb.src + static_cast<int64_t>(r) * jb.rs;
+    const auto load = [&](int i, v4f (&v)[2]) {
+        const int kb = k_begin + i * 256 + oct * 8;
+        v[0] = v[1] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (r >= jb.rows || kb >= k_end) return;
+        if (KS1 && kb + 7 < jb.K) {
+            v[0] = *reinterpret_cast<const v4f_u*>(src + kb);
+            v[1] = *reinterpret_cast<const v4f_u*>(src + kb + 4);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) if (kb + c < jb.K) v[c >> 2][c & 3] = src[static_cast<int64_t>(kb + c) * (KS1 ? 1 : jb.ks)];
+        }
+    };
+    const bool kept = rounds <= HX_SPLIT_ROUNDS;
+    v4f held[HX_SPLIT_ROUNDS][2];
+    uint32_t top = 0;
+    const auto see = [&](const v4f (&v)[2]) {
+        const uint32_t b = __float_as_uint(max4(max4(0.0f, v[0]), v[1]));
+        top = b > top ? b : top;
+    };
+    if (kept) {
+#pragma unroll
+        for (int i = 0; i < HX_SPLIT_ROUNDS; ++i) load(i, held[i]);
+#pragma unroll
+        for (int i = 0; i < HX_SPLIT_ROUNDS; ++i) see(held[i]);
+    } else {
+        for (int i = 0; i < rounds; i += 2) {
+            v4f a[2], b[2];
+            load(i, a);
+            load(i + 1, b);
+            see(a);
+            see(b);
+        }
+    }
+    lds_max[row][oct] = top;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 32; ++i) { const uint32_t o = lds_max[row][i]; top = o > top ? o : top; }
+    // the largest element goes to 2^14 .. 2^15; an all-zero row needs no scale
+    const int e = static_cast<int>(top >> 23) & 0xff;
+    const bool bad = top >= 0x7f800000u || (e < 14 && top != 0);
+    const int scale_exp = top == 0 || bad ? 127 : 268 - e;          // biased exponent of the scale
+    const float scale = __uint_as_float(static_cast<uint32_t>(scale_exp) << 23);
+    if (oct == 0) jb.exps[static_cast<int64_t>(blockIdx.y) * jb.rows_pad + r] = bad ? HX_BAD : scale_exp - 127;
+    const auto put = [&](int i, const v4f (&v)[2]) {
+        const int kb = k_begin + i * 256 + oct * 8;
+        if (kb >= k_end) return;
+        uint2 lo[2], hi[2];
+        split4_f16(v[0], scale, lo);
+        split4_f16(v[1], scale, hi);
+        // [stage][part][16-k step][tile][half][row]
+        uint8_t* dst = jb.dst + ((static_cast<int64_t>(kb >> 5) * 2 * 2 + ((kb >> 4) & 1)) * jb.rows_pad + blockIdx.x * 32) * 32 + ((kb >> 3) & 1) * 512 + row * 16;
+        const int64_t part = static_cast<int64_t>(jb.rows_pad) * 64;
+        *reinterpret_cast<uint4*>(dst) = uint4{lo[0].x, lo[0].y, hi[0].x, hi[0].y};
+        *reinterpret_cast<uint4*>(dst + part) = uint4{lo[1].x, lo[1].y, hi[1].x, hi[1].y};
+    };
+    if (kept) {
+#pragma unroll
+        for (int i = 0; i < HX_SPLIT_ROUNDS; ++i) put(i, held[i]);
+    } else {
+        for (int i = 0; i < rounds; i += 2) {
+            v4f a[2], b[2];
+            load(i, a);
+            load(i + 1, b);
+            put(i, a);
+            put(i + 1, b);
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// The contraction.  One work-group of eight waves per CU walks a list of items (128 x 128 TJ tiles, times the slices of K).
+// Waves 4 .. 7 load A three stages ahead, find the rows' maxima, scale, split and write the stage to LDS; they run on into
+// the next item while waves 0 .. 3 store the finished one.  A contracting wave takes all 128 rows and 32 TJ columns: B's
+// fragments belong to it alone and come straight from memory (L2), two stages ahead; A's come from LDS one step ahead of
+// their six MFMAs.  Barrier i + 1 says "stages up to i + 1 are in LDS" and "stage i - 1 has been read".
+template <int AMODE, bool GEN, int TJ, int OUT, bool STREAM>
+__global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const GemmParams p, const F16x2Job jb) {
+    constexpr bool KLOAD = AMODE == HX_KC || AMODE == HX_KRUN;
+    constexpr bool RUNS = AMODE == HX_KRUN || AMODE == HX_RRUN;
+    constexpr int NR = KLOAD ? 4 : 1;                  // rows of A a loading lane has a share of
+    __shared__ __attribute__((aligned(16))) uint8_t lds_a[HX_BUFS * HX_STAGE];
+    __shared__ __attribute__((aligned(16))) float lds_factor[HX_BUFS][HX_M];
+    __shared__ __attribute__((aligned(16))) int lds_mark[HX_BUFS][4];
+    // exponents of the rows' scales, per item: written with an item's last stage, read behind it, by when the loading waves
+    // are at most two stages (two items, were an item one stage) further
+    __shared__ __attribute__((aligned(16))) int lds_exp[HX_EXPS][HX_M];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles = p.tiles_m * p.tiles_n;
+
+    // this work-group's items: first, first + step, ...; an XCD's are consecutive ones
+    const int xcd = blockIdx.x & 7, step = gridDim.x >> 3;
+    const int lo = static_cast<int>(static_cast<int64_t>(jb.items) * xcd / 8);
+    const int hi = static_cast<int>(static_cast<int64_t>(jb.items) * (xcd + 1) / 8);
+    const int first = lo + static_cast<int>(blockIdx.x >> 3);
+    const int my_items = first < hi ? (hi - first + step - 1) / step : 0;
+    if (my_items == 0) return;                          // (the whole work-group: no barrier is left behind)
+    struct Item { int m0, n0, slice, c_begin, nch; };
+    const auto item_at = [&](int i) {
+        Item it;
+        int t = first + i * step;
+        it.slice = t / tiles;
+        t -= it.slice * tiles;
+        const int band_rows = 8;
+        const int band = t / (band_rows * p.tiles_n);
+        t -= band * band_rows * p.tiles_n;
+        const int rows_here = (p.tiles_m - band * band_rows) < band_rows ? (p.tiles_m - band * band_rows) : band_rows;
+        it.m0 = (band * band_rows + t % rows_here) * HX_M;
+        it.n0 = (t / rows_here) * (128 * TJ);
+        it.c_begin = it.slice * jb.slice_chunks;
+        it.nch = jb.chunks - it.c_begin < jb.slice_chunks ? jb.chunks - it.c_begin : jb.slice_chunks;
+        return it;
+    };
+    int total = 0;                                      // stages of this work-group
+    for (int i = 0; i < my_items; ++i) total += item_at(i).nch;
+    const int padded = (total + HX_AHEAD - 1) / HX_AHEAD * HX_AHEAD;
+
+    if (wave >= 4) {
+        const int w = wave - 4;                         // this wave's 32 rows
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A), 0, static_cast<int>(jb.a_span), 0x00020000);
+        // (A with runs of whole stages is read once, by one column of tiles as a rule, and is larger than the caches: it goes past
+        // L2, where B's fragments stay; 384 residues x 32 features x 256 sequences, one gradient: 262 -> 254 us.  Stages that
+        // begin inside a line share it with the next one's: those stay in L2, 211 residues 115 us past it)
+        constexpr int AUX = RUNS && !GEN ? 2 : 0;
+        const auto load4 = [&](uint32_t at) { return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, AUX)); };
+        const auto load1 = [&](uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at, 0, AUX)); };
+        // KLOAD: rows 8 i + r0, four k from u0 on; otherwise row r0, sixteen k from u0 on
+        const int r0 = KLOAD ? lane >> 3 : lane & 31;
+        const int u0 = KLOAD ? (lane & 7) * 4 : (lane >> 5) * 16;
+        const uint32_t k_step = static_cast<uint32_t>(RUNS ? p.a_ki : p.a_ks) * 4u;        // bytes from k to k + 1
+        uint32_t roff[NR];
+        Item load_item = item_at(0);
+        int li = 0, lc = 0, kd = 0, kr = 0;
+        const auto open = [&]() {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const int row = load_item.m0 + w * 32 + 8 * i + r0;
+                const int64_t el = RUNS ? static_cast<int64_t>(row / p.a_lm) * p.a_mo + static_cast<int64_t>(row % p.a_lm) * p.a_mi
+                                        : static_cast<int64_t>(row) * p.a_rs;
+                roff[i] = row < p.M ? static_cast<uint32_t>(el) * 4u + u0 * k_step : OUTSIDE;
+            }
+            if (RUNS) { kd = load_item.c_begin * HX_K / p.a_lk; kr = load_item.c_begin * HX_K - kd * p.a_lk; }
+        };
+        open();
+        const int nruns = RUNS ? p.K / p.a_lk : 0;
+        // requests the next stage; past the last item every offset is outside (the loads are still made: the count of loads
+        // in flight that the wait for a stage names is then the same in every iteration)
+        const auto request = [&](v4f (&x)[4]) {
+            const bool live = li < my_items;
+            const int k0 = (load_item.c_begin + lc) * HX_K;
+            if (AMODE == HX_KC) {
+                const uint32_t koff = static_cast<uint32_t>(k0) * 4u;
+                if (!GEN) {                             // K a multiple of four: a piece lies inside its row or behind it
+                    const bool in = live && k0 + u0 < p.K;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] = load4(in ? roff[i] + koff : OUTSIDE);
+                } else if (live && k0 + HX_K <= p.K) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] = load4(roff[i] + koff);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) x[i][c] = load1(live && k0 + u0 + c < p.K ? roff[i] + koff + 4u * c : OUTSIDE);
+                }
+            } else if (AMODE == HX_RC) {                // (k behind K: behind the end of the plane)
+                const uint32_t base = (live ? roff[0] : OUTSIDE) + static_cast<uint32_t>(k0) * k_step;
+#pragma unroll
+                for (int c = 0; c < 16; ++c) x[c >> 2][c & 3] = load1(base + c * k_step);
+            } else if (!GEN) {                          // runs of whole stages
+                const bool in = live && kd < nruns;
+                const uint32_t koff = static_cast<uint32_t>(static_cast<int64_t>(kd) * p.a_ko + static_cast<int64_t>(kr) * p.a_ki) * 4u;
+                if (KLOAD) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] = load4(in ? roff[i] + koff : OUTSIDE);
+                } else {
+                    const uint32_t base = in ? roff[0] + koff : OUTSIDE;
+#pragma unroll
+                    for (int c = 0; c < 16; ++c) x[c >> 2][c & 3] = load1(base + c * k_step);
+                }
+            } else {
+                // element u places behind the stage's first k lies in this run while kr + u < run length, else in the next one
+                // (a run is at least a stage long: the launcher's rule); a run behind the last one is outside: 2^30, which with
+                // the operand's span (at most 2^30 bytes in this form) and with a row's 2^31 stays outside
+                constexpr uint32_t NO_RUN = 0x40000000u;
+                const uint32_t here = live && kd < nruns ? static_cast<uint32_t>(static_cast<int64_t>(kd) * p.a_ko + static_cast<int64_t>(kr) * p.a_ki) * 4u : NO_RUN;
+                const uint32_t next = live && kd + 1 < nruns ? static_cast<uint32_t>(static_cast<int64_t>(kd + 1) * p.a_ko + static_cast<int64_t>(kr - p.a_lk) * p.a_ki) * 4u : NO_RUN;
+                const int left = p.a_lk - kr;
+                if (KLOAD && left >= HX_K) {            // a stage inside one run
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] = load4(roff[i] + here);
+                } else if (KLOAD) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) x[i][c] = load1(roff[i] + (u0 + c < left ? here : next) + 4u * c);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 16; ++c) x[c >> 2][c & 3] = load1(roff[0] + (u0 + c < left ? here : next) + c * k_step);
+                }
+            }
+            if (RUNS) { kr += HX_K; if (kr >= p.a_lk) { kr -= p.a_lk; ++kd; } }
+            if (++lc == load_item.nch) {
+                lc = 0;
+                if (++li < my_items) { load_item = item_at(li); open(); }
+            }
+        };
+
+        float scale[NR];
+        uint32_t seen[NR];                              // OR of the maxima's bits; the sign bit: infinite or NaN
+        int pi = 0, pc = 0, p_nch = load_item.nch, buf = 0;
+        // splits the next stage into LDS
+        const auto place = [&](const v4f (&x)[4]) {
+            if (pc == 0) {
+#pragma unroll
+                for (int i = 0; i < NR; ++i) { scale[i] = __uint_as_float(HX_FIRST_SCALE); seen[i] = 0; }
+            }
+            uint32_t top[NR];
+            bool over = false;
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                float m = max4(0.0f, x[i]);
+                if (!KLOAD) m = max4(max4(max4(m, x[1]), x[2]), x[3]);
+                uint32_t b = __float_as_uint(m);
+                const auto meet = [&](uint32_t o) { b = o > b ? o : b; };
+                if (KLOAD) {                            // the eight lanes of the row: neighbours, pairs, then the other four
+                    meet(__builtin_amdgcn_mov_dpp(b, 0xB1, 0xf, 0xf, true));
+                    meet(__builtin_amdgcn_mov_dpp(b, 0x4E, 0xf, 0xf, true));
+                    meet(__builtin_amdgcn_mov_dpp(b, 0x141, 0xf, 0xf, true));
+                } else {
+                    meet(__shfl_xor(b, 32, 64));
+                }
+                top[i] = b;
+                seen[i] |= b;
+                over |= !(__uint_as_float(b) * scale[i] < 32768.0f);
+            }
+            int mark = 0;
+            if (__builtin_amdgcn_ballot_w64(over) != 0) {
+#pragma unroll
+                for (int i = 0; i < NR; ++i) {
+                    float factor = 1.0f;
+                    if (!(__uint_as_float(top[i]) * scale[i] < 32768.0f)) {
+                        if (top[i] >= 0x7f800000u) {
+                            seen[i] |= 0x80000000u;
+                        } else {
+                            const int e = static_cast<int>(top[i] >> 23);                    // (at least 16: the first scale is 2^126)
+                            const int was = static_cast<int>(__float_as_uint(scale[i]) >> 23), now = 266 - e;
+                            const int f = now - was + 127;
+                            factor = f > 0 ? __uint_as_float(static_cast<uint32_t>(f) << 23) : 0.0f;
+                            scale[i] = __uint_as_float(static_cast<uint32_t>(now) << 23);
+                        }
+                    }
+                    if (u0 == 0) lds_factor[buf][w * 32 + 8 * i + r0] = factor;
+                }
+                mark = 1;
+            }
+            if (lane == 0) lds_mark[buf][w] = mark;
+            uint8_t* const stage = lds_a + buf * HX_STAGE + w * HX_FRAG;
+            if (KLOAD) {
+                uint8_t* const dst = stage + (u0 >> 4) * HX_STEP + ((u0 >> 3) & 1) * HX_HALF + ((u0 >> 2) & 1) * 8 + r0 * 16;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    uint2 parts[2];
+                    split4_f16(x[i], scale[i % NR], parts);
+                    *reinterpret_cast<uint2*>(dst + i * 128) = parts[0];
+                    *reinterpret_cast<uint2*>(dst + HX_PART + i * 128) = parts[1];
+                }
+            } else {
+                uint8_t* const dst = stage + (u0 >> 4) * HX_STEP + r0 * 16;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    uint2 a[2], b[2];
+                    split4_f16(x[2 * h], scale[0], a);
+                    split4_f16(x[2 * h + 1], scale[0], b);
+                    *reinterpret_cast<uint4*>(dst + h * HX_HALF) = uint4{a[0].x, a[0].y, b[0].x, b[0].y};
+                    *reinterpret_cast<uint4*>(dst + HX_PART + h * HX_HALF) = uint4{a[1].x, a[1].y, b[1].x, b[1].y};
+                }
+            }
+            if (++pc == p_nch) {
+                if (pi < my_items && u0 == 0) {
+#pragma unroll
+                    for (int i = 0; i < NR; ++i) {
+                        const uint32_t s = __float_as_uint(scale[i]);
+                        const bool untouched = s == HX_FIRST_SCALE;         // a row of zeros, or of elements below 2^-111
+                        const bool bad = (seen[i] & 0x80000000u) != 0 || (untouched && seen[i] != 0);
+                        lds_exp[pi & (HX_EXPS - 1)][w * 32 + 8 * i + r0] = bad ? HX_BAD : untouched ? 0 : static_cast<int>(s >> 23) - 127;
+                    }
+                }
+                pc = 0;
+                if (++pi < my_items) p_nch = item_at(pi).nch;
+            }
+            buf = buf == HX_BUFS - 1 ? 0 : buf + 1;
+        };
+
+        v4f x[HX_AHEAD][4];
+#pragma unroll
+        for (int d = 0; d < HX_AHEAD; ++d) { request(x[d]); __builtin_amdgcn_sched_barrier(0); }
+        for (int g = 0; g < padded; g += HX_AHEAD) {
+#pragma unroll
+            for (int d = 0; d < HX_AHEAD; ++d) {
+                place(x[d]);
+                request(x[d]);
+                __syncthreads();
+            }
+        }
+        __syncthreads();
+        return;
+    }
+
+    // ---- contracting waves
+    const int j = lane & 31, hh = lane >> 5;
+    const int wn = wave * 32 * TJ;
+    v8h fb[2][TJ][2][2];                                // [stage parity][tile column][16-k step][part]
+    Item b_item = item_at(0);
+    int bi = 0, bc = 0;
+    const size_t b_unit = static_cast<size_t>(jb.nb_pad) * 32;
+    // the fragments of the next stage of the sequence (behind the last item: of that item's first stages again)
+    const auto load_b = [&](v8h (&f)[TJ][2][2]) {
+        const uint8_t* src = jb.wb + static_cast<size_t>(b_item.c_begin + bc) * 4 * b_unit + static_cast<size_t>(b_item.n0 + wn) * 32 + lane * 16;
+#pragma unroll
+        for (int part = 0; part < 2; ++part)
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int tj = 0; tj < TJ; ++tj) f[tj][ks][part] = *reinterpret_cast<const v8h*>(src + (part * 2 + ks) * b_unit + tj * 1024);
+        if (++bc == b_item.nch) {
+            bc = 0;
+            if (bi + 1 < my_items) b_item = item_at(++bi);
+        }
+    };
+    load_b(fb[0]);
+    load_b(fb[1]);
+    const uint8_t* const frag = lds_a + hh * HX_HALF + j * 16;
+    v8h fa[2][2];                                       // the step at hand and the next
+    int buf = 0;
+    __syncthreads();
+    __syncthreads();                                    // stages 0 and 1 are in LDS
+#pragma unroll
+    for (int part = 0; part < 2; ++part) fa[0][part] = *reinterpret_cast<const v8h*>(frag + part * HX_PART);
+    v4i mark = *reinterpret_cast<const v4i*>(lds_mark[0]);
+    v16f acc[4][TJ];
+    int g = 0;
+    for (int i = 0; i < my_items; ++i) {
+        const Item it = item_at(i);
+        int eb[TJ];
+#pragma unroll
+        for (int tj = 0; tj < TJ; ++tj) eb[tj] = jb.eb[static_cast<size_t>(it.slice) * jb.nb_pad + it.n0 + wn + tj * 32 + j];
+#pragma unroll
+        for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < TJ; ++tj)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[ti][tj][r] = 0.0f;
+        const auto chunk = [&](v8h (&f)[TJ][2][2], int k0, bool fresh) {
+            if (!fresh && __builtin_amdgcn_readfirstlane(mark[0] | mark[1] | mark[2] | mark[3]) != 0) {
+                // some rows' scales have moved: what their sums hold so far moves with them
+#pragma unroll
+                for (int ti = 0; ti < 4; ++ti) {
+                    if (__builtin_amdgcn_readfirstlane(mark[ti]) == 0) continue;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const v4f fac = *reinterpret_cast<const v4f*>(&lds_factor[buf][ti * 32 + 8 * q + 4 * hh]);
+#pragma unroll
+                        for (int tj = 0; tj < TJ; ++tj)
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) acc[ti][tj][4 * q + c] *= fac[c];
+                    }
+                }
+            }
+            const uint8_t* const here = frag + buf * HX_STAGE;
+            buf = buf == HX_BUFS - 1 ? 0 : buf + 1;
+            const uint8_t* const next = frag + buf * HX_STAGE;
+            // (16-k steps behind K are left out: K padded to whole pairs of stages would be contracted in full)
+            const int steps = (p.K - k0 + 15) / 16;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                if (ks >= steps) {
+                    if (ks == 0 || steps == 1) {
+#pragma unroll
+                        for (int part = 0; part < 2; ++part) fa[0][part] = *reinterpret_cast<const v8h*>(next + part * HX_PART);
+                    }
+                    break;
+                }
+#pragma unroll
+                for (int ti = 0; ti < 4; ++ti) {
+                    const int s = ks * 4 + ti;
+                    const uint8_t* const at = s < 7 ? here + ((s + 1) >> 2) * HX_STEP + ((s + 1) & 3) * HX_FRAG : next;
+                    fa[(s + 1) & 1][0] = *reinterpret_cast<const v8h*>(at);
+                    fa[(s + 1) & 1][1] = *reinterpret_cast<const v8h*>(at + HX_PART);
+                    __builtin_amdgcn_sched_barrier(0);  // (left to itself the scheduler reads a fragment where it is needed)
+                    const v8h (&a)[2] = fa[s & 1];
+                    // smallest first: l h, h l, h h
+#pragma unroll
+                    for (int tj = 0; tj < TJ; ++tj) acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], f[tj][ks][0], acc[ti][tj], 0, 0, 0);
+#pragma unroll
+                    for (int tj = 0; tj < TJ; ++tj) acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], f[tj][ks][1], acc[ti][tj], 0, 0, 0);
+#pragma unroll
+                    for (int tj = 0; tj < TJ; ++tj) acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], f[tj][ks][0], acc[ti][tj], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            mark = *reinterpret_cast<const v4i*>(lds_mark[buf]);
+            load_b(f);
+            ++g;
+            if (g < total) __syncthreads();             // stage g - 1 has been read; stage g + 1 is in LDS
+        };
+        for (int c = 0; c < it.nch; c += 2) {
+            chunk(fb[0], (it.c_begin + c) * HX_K, c == 0);
+            chunk(fb[1], (it.c_begin + c + 1) * HX_K, false);
+        }
+
+        // ---- the scales leave, the sums go out
+        const int (&ea)[HX_M] = lds_exp[i & (HX_EXPS - 1)];
+        int worst = ea[lane] > ea[lane + 64] ? ea[lane] : ea[lane + 64];
+#pragma unroll
+        for (int tj = 0; tj < TJ; ++tj) worst = eb[tj] > worst ? eb[tj] : worst;
+        const bool any_bad = __builtin_amdgcn_ballot_w64(worst >= HX_BAD / 2) != 0;
+        if (OUT != HX_PARTIAL && any_bad) {
+            // operands of this wave's columns that the split could not carry: all of them again, the reference's way
+            plain_tile(p, p.A, p.B, p.C, it.m0, it.n0 + wn, HX_M, 32 * TJ, lane, 64);
+            continue;
+        }
+        if (OUT == HX_PARTIAL && any_bad) {             // NaN: reduce_slices_kernel redoes those
+#pragma unroll
+            for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+#pragma unroll
+                    for (int tj = 0; tj < TJ; ++tj)
+                        if (ea[ti * 32 + 8 * (r >> 2) + 4 * hh + (r & 3)] + eb[tj] >= HX_BAD / 2) acc[ti][tj][r] = __builtin_nanf("");
+        }
+        // (one tile row at a time: with all sixty-four exponents read ahead the kernel spills)
+        const auto unscale = [&](int ti) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const v4i e4 = *reinterpret_cast<const v4i*>(&ea[ti * 32 + 8 * q + 4 * hh]);
+#pragma unroll
+                for (int tj = 0; tj < TJ; ++tj)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) acc[ti][tj][4 * q + c] = ldexpf(acc[ti][tj][4 * q + c], -(e4[c] + eb[tj]));
+            }
+        };
+        if constexpr (OUT == HX_COMPOUND) {
+#pragma unroll
+            for (int ti = 0; ti < 4; ++ti) {
+                unscale(ti);
+                store_tile_compound_buffer<STREAM, TJ>(p, p.C, acc[ti], it.m0 + ti * 32, it.n0 + wn, lane);
+            }
+        } else {
+            constexpr bool part = OUT == HX_PARTIAL;
+            const uint32_t ld = part ? static_cast<uint32_t>(jb.nb_pad) * 4u : static_cast<uint32_t>(p.c_mi) * 4u;
+            float* const base = part ? jb.partial + static_cast<size_t>(it.slice) * jb.ma_pad * jb.nb_pad : p.C;
+            // rows past the matrix fall outside the plane by themselves
+            const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>((part ? jb.ma_pad : p.M) * ld), 0x00020000);
+            float tail[TJ];
+            uint32_t col[TJ];
+#pragma unroll
+            for (int tj = 0; tj < TJ; ++tj) {
+                const int n = it.n0 + wn + tj * 32 + j;
+                tail[tj] = !part && p.bias && n < p.N ? p.bias[n] : 0.0f;
+                col[tj] = part || n < p.N ? static_cast<uint32_t>(n) * 4u : OUTSIDE;
+            }
+            uint32_t row = static_cast<uint32_t>(it.m0 + 4 * hh) * ld;
+#pragma unroll
+            for (int ti = 0; ti < 4; ++ti) {
+                unscale(ti);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+#pragma unroll
+                    for (int tj = 0; tj < TJ; ++tj) {
+                        float v = acc[ti][tj][r];
+                        if (!part) v = (v + tail[tj]) * p.alpha;
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc_c, row + col[tj], 0, STREAM ? 3 : 0);
+                    }
+                    // to the next row (opaque: one offset that moves on, not sixty-four at once)
+                    row += (r & 3) == 3 ? 5 * ld : ld;
+                    asm volatile("" : "+v"(row));
+                }
+            }
+        }
+    }
+    for (; g < padded; ++g) __syncthreads();
+}
+
+}  // namespace
+
+int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap) {
+    GemmParams p = p0;
+    if (p.np2 * p.np3 != 1 || p.clamp || p.f16_in) return -1;
+    if (p.K < 64 || p.N <= 32) return -1;
+    const bool compound = !(p.c_lm >= p.M && p.c_ln >= p.N);
+    const int cus = device_cu_count() / 8 * 8;
+    // matrix work: 16-k steps of 128 x 128 tiles per CU
+    const int64_t tiles128 = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + 127) / 128);
+    const int64_t load = tiles128 * ((p.K + 15) / 16) / cus;
+    // few tiles under a long K (a LinearLayer's weight gradient): slices of K, and the smaller operand is split ahead
+    const bool sliced = !compound && p.a_lm == 0 && tiles128 * 2 <= cus;
+    if (sliced && p.M < p.N && !p.bias) {
+        std::swap(p.A, p.B);
+        std::swap(p.M, p.N);
+        std::swap(p.a_rs, p.b_rs);
+        std::swap(p.a_ks, p.b_ks);
+        std::swap(p.c_mi, p.c_ni);
+    }
+    if (p.M < 128) return -1;
+    // how A lies, and 32-bit byte offsets into it
+    int amode;
+    bool gen = false;
+    int64_t span;
+    if (p.a_lm > 0) {
+        if (p.a_lk < HX_K || p.K % p.a_lk != 0 || p.a_mo < 0 || p.a_mi < 0 || p.a_ko < 0 || p.a_ki < 0) return -1;
+        amode = p.a_ki == 1 ? HX_KRUN : p.a_mi == 1 ? HX_RRUN : -1;
+        gen = p.a_lk % HX_K != 0;
+        span = static_cast<int64_t>((p.M - 1) / p.a_lm) * p.a_mo + static_cast<int64_t>(std::min(p.a_lm, p.M) - 1) * p.a_mi +
+               static_cast<int64_t>((p.K - 1) / p.a_lk) * p.a_ko + static_cast<int64_t>(p.a_lk - 1) * p.a_ki + 1;
+        if (gen && span * 4 > (1LL << 30)) return -1;
+    } else if (p.a_ks == 1) {
+        amode = HX_KC;
+        gen = p.K % 4 != 0;
+        span = static_cast<int64_t>(p.M - 1) * p.a_rs + p.K;
+        if (p.a_rs < p.K) return -1;
+    } else if (p.a_rs == 1) {
+        amode = HX_RC;
+        span = static_cast<int64_t>(p.K) * p.a_ks;
+        if (p.a_ks < p.M || (span + 128 * p.a_ks) * 4 >= (1LL << 31)) return -1;
+    } else {
+        return -1;
+    }
+    if (amode < 0 || span * 4 >= (1LL << 31) - 65536) return -1;
+    // the output (slices: any strides)
+    if (compound ? p.c_span == 0 : (p.c_ni != 1 && !sliced) || static_cast<int64_t>(p.M + HX_M) * p.c_mi * 4 >= (1LL << 31)) return -1;
+
+    // Where the lines lie (us, the other forms / this one; `load` in steps).  The split ahead and a deeper pipeline cost 5 us
+    // before the first tile, so the contraction has to be worth it:
+    //   * compound A (outer-product-mean backward), one gradient: 2480 x 2480 x 245 (load 24) 34 / 32, 1984 x 1984 x 241 (15)
+    //     30 / 33, 4000 x 4000 x 135 56 / 42, 12288 x 12288 x 256 412 / 245;
+    //   * compound C (its forward): 3136 x 106 x 3136 (17) 25 / 32, 4464 x 123 x 4464 (38) 59 / 43, 7808 x 202 x 7808 242 / 165;
+    //   * slices: 888 x 3490 x 504 (24) 29 / 29, 832 x 8990 x 304 (46) 42 / 38, 768 x 26368 x 256 (77) 61 / 52; with few rows the
+    //     split of the other operand weighs more: 464 x 12651 x 392 (49) 42 / 43, 564 x 26377 x 197 (64) 51 / 52;
+    //   * otherwise: 10609 x 176 -> 532 (18) 20 / 21, 26368 x 256 -> 256 (26) 25 / 21, 26368 x 512 -> 1024 (206) 189 / 101.
+    // A K below 128 stays with the form that splits in the tile loop at any size (the bits of a contraction that is cut
+    // out of a larger one then do not depend on the size).
+    if (p.a_lm > 0) { if (load < 22) return -1; }
+    else if (compound) { if (load < 30) return -1; }
+    else if (sliced) { if (load < 42 || (p.M < 700 && load < 66) || p.K < 128) return -1; }
+    else if (load < 24 || p.K < 128) return -1;
+    // Tiles of 128 x 256 by one work-group per CU, or of 128 x 128 by two, which store while the other contracts but read A
+    // twice as often: where 256 columns would be half empty, where the wide tiles' last round leaves more than half of the CUs idle (26368 x 256 -> 768: 51.4
+    // / 48.8 us; 32768 x 512 -> 1024, whole rounds, 110 / 118), and for compound rows that are not whole lines, whose stores
+    // take as long as the products (7808 x 202 x 7808: 196 / 165; 12288 x 256 x 12288, whole lines, 288 / 314).
+    const int tn = (p.N + 127) / 128;
+    int tj = 2;
+    if (compound) {
+        if (p.c_lm % 32 != 0 || tn == 1) tj = 1;
+    } else if (tn == 1 || (tn == 3 && p.a_lm == 0)) {
+        tj = 1;
+    } else if (p.a_lm == 0 && !sliced) {
+        const int64_t wide = static_cast<int64_t>((p.M + HX_M - 1) / HX_M) * ((tn + 1) / 2);
+        if (wide > cus && wide % cus != 0 && wide % cus * 2 < cus) tj = 1;
+    }
+    const int nt = 128 * tj;
+    p.tiles_m = (p.M + HX_M - 1) / HX_M;
+    p.tiles_n = (p.N + nt - 1) / nt;
+    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
+    const int chunks = ((p.K + HX_K - 1) / HX_K + 1) / 2 * 2;
+    int slices = 1;
+    if (!compound && tiles * 4 < 3 * cus) {
+        slices = even_slices(static_cast<int>(tiles), chunks / 2, 128, 4);      // (whole pairs of stages, at least 256 k)
+    }
+    if (tiles > (1 << 24) || tiles * slices < 32 || (compound && p.c_ni <= 0)) return -1;
+    const int slice_chunks = (chunks / 2 + slices - 1) / slices * 2;
+    slices = (chunks + slice_chunks - 1) / slice_chunks;
+    const int ma_pad = p.tiles_m * HX_M, nb_pad = p.tiles_n * nt;
+    const size_t b_bytes = static_cast<size_t>(chunks) * 128 * nb_pad;
+    const size_t e_bytes = (static_cast<size_t>(slices) * nb_pad * 4 + 255) / 256 * 256;
+    const bool partial = slices > 1 || p.a_lm > 0 || p.c_ni != 1;     // (no direct instances for a compound A)
+    const size_t part_bytes = partial ? static_cast<size_t>(slices) * ma_pad * nb_pad * 4 : 0;
+    if (static_cast<size_t>(ma_pad) * nb_pad * 4 >= (1ull << 31) && partial) return -1;
+    const size_t need = b_bytes + e_bytes + part_bytes;
+    uint8_t* ws = fixed_ws;
+    Workspace held;
+    if (fixed_ws) {
+        if (need > fixed_cap) return -1;
+    } else {
+        held = workspace_take(need, stream);
+        ws = held.ptr;
+        if (!ws) return -1;
+    }
+    F16x2Job jb{};
+    jb.wb = ws;
+    int* const exps = reinterpret_cast<int*>(ws + b_bytes);
+    jb.eb = exps;
+    jb.partial = reinterpret_cast<float*>(ws + b_bytes + e_bytes);
+    jb.nb_pad = nb_pad; jb.ma_pad = ma_pad;
+    jb.chunks = chunks; jb.slice_chunks = slice_chunks; jb.slices = slices;
+    jb.items = static_cast<int>(tiles) * slices;
+    jb.a_span = static_cast<uint32_t>(span * 4);
+    const F16x2Split sp{p.B, ws, exps, p.N, nb_pad, p.K, chunks, slice_chunks, p.b_rs, p.b_ks};
+    const dim3 sgrid(nb_pad / 32, slices);
+    if (p.b_ks == 1) hipLaunchKernelGGL((split_f16x2_kernel<true>), sgrid, dim3(1024), 0, stream, sp);
+    else             hipLaunchKernelGGL((split_f16x2_kernel<false>), sgrid, dim3(1024), 0, stream, sp);
+    int rc = check_launch(what);
+    if (rc == RC_OK) {
+        const int wgs = std::min<int64_t>((jb.items + 7) / 8 * 8, tj == 1 ? 2 * cus : cus);
+        const int out = partial ? HX_PARTIAL : compound ? HX_COMPOUND : HX_DENSE;
+        const bool stream_c = p.stream_c && !partial;
+#define PPML_HX(A_, G_, T_, O_, S_) hipLaunchKernelGGL((gemm_f16x2_kernel<A_, G_, T_, O_, S_>), dim3(wgs), dim3(512), 0, stream, p, jb)
+#define PPML_HX_T(A_, G_, O_, S_) do { if (tj == 1) PPML_HX(A_, G_, 1, O_, S_); else PPML_HX(A_, G_, 2, O_, S_); } while (0)
+#define PPML_HX_O(A_, G_)                                                                                         \
+    do {                                                                                                          \
+        if (out == HX_PARTIAL) PPML_HX_T(A_, G_, HX_PARTIAL, false);                                              \
+        else if (stream_c) PPML_HX_T(A_, G_, HX_DENSE, true);                                                     \
+        else PPML_HX_T(A_, G_, HX_DENSE, false);                                                                  \
+    } while (0)
+#define PPML_HX_C(A_, G_) do { if (stream_c) PPML_HX_T(A_, G_, HX_COMPOUND, true); else PPML_HX_T(A_, G_, HX_COMPOUND, false); } while (0)
+        if (out == HX_COMPOUND) {
+            if (amode == HX_KC) { if (gen) PPML_HX_C(HX_KC, true); else PPML_HX_C(HX_KC, false); }
+            else                PPML_HX_C(HX_RC, false);
+        }
+        else if (amode == HX_KC)   { if (gen) PPML_HX_O(HX_KC, true); else PPML_HX_O(HX_KC, false); }
+        else if (amode == HX_RC)   PPML_HX_O(HX_RC, false);
+        else if (amode == HX_KRUN) { if (gen) PPML_HX_T(HX_KRUN, true, HX_PARTIAL, false); else PPML_HX_T(HX_KRUN, false, HX_PARTIAL, false); }
+        else                       { if (gen) PPML_HX_T(HX_RRUN, true, HX_PARTIAL, false); else PPML_HX_T(HX_RRUN, false, HX_PARTIAL, false); }
+#undef PPML_HX_C
+#undef PPML_HX_O
+#undef PPML_HX_T
+#undef PPML_HX
+        rc = check_launch(what);
+    }
+    if (rc == RC_OK && partial) rc = launch_reduce_slices(p, stream, what, jb.partial, slices, ma_pad, nb_pad);
+    if (!fixed_ws) workspace_give(held, stream);
+    return rc;
+}
+
+}  // namespace ppmlhip

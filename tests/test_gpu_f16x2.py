@@ -1,0 +1,109 @@
+"""Large contractions in two f16 parts (csrc/gemm_f16x2.hip) against binary64: every way the first operand may lie (contiguous in
+k with whole and ragged pieces, contiguous in its rows, runs of the outer-product-mean's gradient that are whole stages and
+that are not), both tile widths, every kind of output, and what the scales have to follow: rows that differ by 2^80, rows
+that grow along k, rows of zeros, and rows that no scale can bring into range.
+
+The bound: a product of two parts each is within 3 * 2^-24 of |a||b| (two splits, the dropped product), a sum of K terms in
+binary32 within K * 2^-24 of sum |a||b|: (K + 4) * 2^-24 together, for every output by itself.  An element far below the
+largest of its row (2^-17 of it) is kept to 2^-40 of that largest, which these operands never come near."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    assert torch.cuda.is_available(), "GPU tests need a device"
+    from proteinpredictmachinelearning_amd import ops as _ops
+
+    return _ops
+
+
+def _within(got, a, b, scale=1.0, add=None):
+    """got against scale * a @ b.T (+ add), all in binary64"""
+    K = a.shape[1]
+    want = scale * (a @ b.t())
+    size = scale * (a.abs() @ b.abs().t())
+    if add is not None:
+        want, size = want + add, size + add.abs()
+    bad = ~((got.double() - want).abs() <= (K + 4) * 2.0 ** -24 * size + 1e-45)
+    assert not bool(bad.any()), float(((got.double() - want).abs() / size)[bad].max())
+
+
+def _operand(g, rows, K, kind):
+    x = torch.randn(rows, K, device="cuda", generator=g)
+    if kind == "ranges":                                # rows of very different sizes, some of them zero
+        x *= torch.exp2(torch.randint(-40, 41, (rows, 1), device="cuda", generator=g).float())
+        x[::17] = 0
+    elif kind == "growing":                             # every stage's elements larger than the last one's: the scale moves on
+        x *= torch.exp2(torch.arange(K, device="cuda").float() * (60.0 / K) - 30)
+        x[5::7, :K // 2] = 0                            # (rows whose first half is zero)
+    return x
+
+
+# (M, K, N): ragged in every dimension; K of whole stages, of an odd number of them, of a 16-k step more, not a multiple of
+# four; tiles of 256 columns, of 128, and an empty second half of the last one; 6000 x 128 x 1024: rows of whole lines
+@pytest.mark.parametrize("kind", ["plain", "ranges", "growing"])
+@pytest.mark.parametrize("M,K,N", [(20011, 136, 516), (26368, 256, 200), (9001, 403, 390), (6000, 128, 1024), (13000, 165, 768), (4100, 320, 1031)])
+def test_linear(ops, M, K, N, kind):
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    a, b = _operand(g, M, K, kind), _operand(g, N, K, "plain" if kind == "growing" else kind) * 0.1
+    bias = torch.randn(N, device="cuda", generator=g) if kind == "plain" else None
+    got = ops.mul_mat(a, b, bias)
+    _within(got, a.double(), b.double(), 1.0, bias.double() if bias is not None else None)
+    # the same contraction on operands that are contiguous in their rows: the same parts, the same bits
+    if bias is None:
+        assert torch.equal(got.view(torch.int32), ops.mul_mat_tn(a.t().contiguous(), b.t().contiguous()).view(torch.int32))
+
+
+# slices of a long K, the smaller operand first and second
+@pytest.mark.parametrize("kind", ["plain", "ranges", "growing"])
+@pytest.mark.parametrize("M,K,N", [(768, 26368, 256), (200, 26367, 900), (1024, 4100, 1030), (900, 10609, 321)])
+def test_slices(ops, M, K, N, kind):
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    a, b = _operand(g, M, K, kind), _operand(g, N, K, "plain")
+    got = ops.mul_mat_tn(a.t().contiguous(), b.t().contiguous(), 0.5)
+    _within(got, a.double(), b.double(), 0.5)
+    assert torch.equal(ops.mul_mat_tn(a.t().contiguous(), b.t().contiguous()), ops.mul_mat(a, b))
+
+
+# residues of whole stages and ragged ones, one and two tiles of features
+@pytest.mark.parametrize("D,L,N", [(32, 96, 256), (32, 103, 130), (32, 128, 100), (8, 390, 72)])
+def test_outer_product_mean(ops, D, L, N):
+    g = torch.Generator(device="cuda").manual_seed(D + L + N)
+    left, right = _operand(g, D * L, N, "ranges"), _operand(g, D * L, N, "plain")
+    l64, r64 = left.double(), right.double()
+    out = ops.outer_product_mean(left.reshape(-1), right.reshape(-1), D, L, N, 1)
+    _within(out.reshape(D, D, L, L).permute(0, 2, 1, 3).reshape(D * L, D * L), l64, r64, 1.0 / N)
+    grad = _operand(g, D * L, D * L, "ranges")          # rows (d1, i), columns (d2, j)
+    g4 = grad.reshape(D, L, D, L).permute(0, 2, 1, 3).contiguous()
+    gl, gr = ops.outer_prod_mean_back(g4.reshape(-1), left.reshape(-1), right.reshape(-1), D, L, N, 1)
+    _within(gl.reshape(D * L, N), grad.double(), r64.t().contiguous(), 1.0 / N)
+    _within(gr.reshape(D * L, N), grad.double().t().contiguous(), l64.t().contiguous(), 1.0 / N)
+
+
+# Infinities, NaN and rows below 2^-111: those outputs the reference's way, the others what they are without them
+@pytest.mark.parametrize("M,K,N", [(20011, 136, 516), (768, 26368, 256)])
+def test_operands_no_scale_brings_into_range(ops, M, K, N):
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g)
+    clean = ops.mul_mat(a, b)
+    a[7, K - 1] = float("inf")
+    a[300, 0] = float("nan")
+    a[600] *= 2.0 ** -130
+    b[3, 5] = -float("inf")
+    b[70] *= 2.0 ** 100
+    got = ops.mul_mat(a, b)
+    want = a.double() @ b.double().t()
+    size = torch.nan_to_num((a.double().abs() @ b.double().abs().t()), nan=0.0, posinf=0.0)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    inf = want.isinf()
+    assert torch.equal(got[inf].double(), want[inf])
+    fin = want.isfinite()
+    assert bool(((got.double() - want).abs()[fin] <= ((K + 4) * 2.0 ** -24 * size + K * 1e-45)[fin]).all())
+    far = torch.ones(M, dtype=torch.bool, device="cuda")          # tiles of rows that hold none of the planted elements
+    for m in (7, 300, 600):
+        far[m // 128 * 128:m // 128 * 128 + 128] = False
+    assert torch.equal(got[far][:, 128:], clean[far][:, 128:])
