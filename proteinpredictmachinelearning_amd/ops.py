@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
+import os
 
 import torch
 
@@ -19,22 +20,30 @@ QK = 32
 BLOCK_BYTES = 34
 WTYPE_Q8_0, WTYPE_Q8_1, WTYPE_Q8_0R, WTYPE_Q8_0M = 0, 1, 2, 3
 
-_initialised = set()
+# What a call asks of torch beside its kernel -- the current device, its stream, the addresses -- costs more than a small
+# kernel: a projection of 408 x 256 -> 256, whose kernel takes 3.7 us, took 10.3 through this module with torch's public
+# forms (a stream object alone 2.7 us, is_available and current_device 0.8) and 6.1 with the functions beneath them.
+_current_device = torch._C._cuda_getDevice if hasattr(torch._C, "_cuda_getDevice") else torch.cuda.current_device
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
+
+_initialised = set()                                  # devices ppml_hip_init has run on in this process
+os.register_at_fork(after_in_child=_initialised.clear)      # (torch refuses the GPU in a forked child: the long way round says so)
 
 
 def _lib():
+    if _initialised and _current_device() in _initialised:
+        return cabi.load()
     lib = cabi.load()
     if not torch.cuda.is_available():
         raise RuntimeError("the gfx950 backend needs a GPU; there is no CPU path")
     dev = torch.cuda.current_device()
-    if dev not in _initialised:
-        cabi.check("ppml_hip_init", lib.ppml_hip_init(dev))
-        _initialised.add(dev)
+    cabi.check("ppml_hip_init", lib.ppml_hip_init(dev))
+    _initialised.add(dev)
     return lib
 
 
-def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream() -> int:
+    return _raw_stream(_current_device())
 
 
 def _dev_f32(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -43,8 +52,8 @@ def _dev_f32(t: torch.Tensor, name: str) -> torch.Tensor:
     return t.contiguous()
 
 
-def _ptr(t) -> C.c_void_p:
-    return C.c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t):
+    return None if t is None else t.data_ptr()
 
 
 Q8_PATH_NAMES = {0: "general", 1: "weight-stationary", 2: "low-latency", 3: "tiled"}
@@ -507,9 +516,8 @@ def mul_mat_q8(w: Q8Weight, x: torch.Tensor, c_trans: int = 1, relu: bool = Fals
         raise ValueError(f"mul_mat_q8: out must be a contiguous f32 tensor of shape {shape} on {x.device}")
     lib = _lib()
     if not dump and not relu and act == "q8_0" and path == "auto":
-        path = C.c_int(0)
         cabi.check("mul_mat_q8_hip", lib.mul_mat_q8_hip(_ptr(w.data), _ptr(x), _ptr(out), M, N, K, w.wtype,
-                                                         c_trans, C.byref(path), _stream()))
+                                                         c_trans, None, _stream()))
         return out
     xq = sums = None
     if dump:
