@@ -183,6 +183,8 @@ public:
     //               reference, src/core/ComputeGraphHelper.cpp:700-729).
     void set_fuse_add_into_soft_max(bool v) { fuse_add_into_soft_max_ = v; }
     bool fuse_add_into_soft_max() const { return fuse_add_into_soft_max_; }
+    // With all three on, a chain nobody else looks into -- no second reader, no output flag, no storage of its own -- over at
+    // least 32 planes of at most 128 rows and 32 features goes in one launch, again with the same bits.
     void set_fuse_permutes_into_out_prod(bool v) { fuse_permutes_into_out_prod_ = v; }
     bool fuse_permutes_into_out_prod() const { return fuse_permutes_into_out_prod_; }
     // The same for the weight gradient of a LinearLayer, dW = mul_mat(mat_transpose(grad), mat_transpose(x))
@@ -250,6 +252,7 @@ private:
     bool fuse_permutes_into_mul_mat_ = true;
     size_t nodes_fused_away_ = 0;
     int attn_layout_ = 0;                                // layout bits of the attention node being dispatched
+    bool attn_nodes_ = false;                            // ... which stands for the default chain, with its nodes' bits
     bool relu_in_quantizer_ = false;                     // the matmul being dispatched applies a fused-away ReLU
     float out_prod_alpha_ = 1.0f;                        // scale of a fused-away OP_SCALE behind the out_prod being dispatched
     bool out_prod_scaled_ = false;

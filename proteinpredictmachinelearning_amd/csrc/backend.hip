@@ -26,6 +26,7 @@
 #include "../../include/ppml_hip.h"
 #include "../../include/ppml_hip_backend.h"
 #include "../../include/ppml_hip_backend.hpp"
+#include "common.hpp"
 
 namespace ppmlhip {
 
@@ -464,6 +465,13 @@ Status HipBackend::kernel_flash_attn_ext(Tensor* node) {
     Tensor* lse = node->src[4];
     if (lse && lse->numel() != B * h * L) return fail(Status::NOT_SUPPORTED, "flash_attn_ext: LSE is not [L, h, B]");
     if (lse && !lse->data) return fail(Status::NOT_SUPPORTED, "flash_attn_ext: LSE buffer is unbound");
+    if (attn_nodes_) {
+        const int rc = attention_chain(static_cast<const float*>(q->data), static_cast<const float*>(k->data), static_cast<const float*>(v->data),
+                                       bias ? static_cast<const float*>(bias->data) : nullptr, static_cast<float*>(node->data), B * h,
+                                       static_cast<int>(L), static_cast<int>(d), node->param_f32(0), nullptr);
+        if (rc != 0) return fail(status_of_rc(rc), std::string("attention chain: ") + ppml_hip_last_error());
+        return Status::SUCCESS;
+    }
     const int rc = flash_attn_forward_ex_hip(static_cast<int>(B), static_cast<int>(h), static_cast<int>(L), static_cast<int>(d),
                                              node->op_params[1] != 0, node->param_f32(0), node->param_f32(2), node->op_params[4],
                                              static_cast<const float*>(q->data), static_cast<const float*>(k->data),
@@ -709,7 +717,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         Tensor* out_prod = nullptr;         // OP_SCALE node that runs as the (skipped) out_prod it reads, scaled
         Tensor* added = nullptr;            // OP_SOFT_MAX node that adds the second operand of this (skipped) OP_ADD on its way in
         bool transposed = false;            // OP_OUT_PROD / OP_MUL_MAT that reads the sources of its two (skipped) {1,0,2,3} permutations
-        bool chain = false;                 // out_prod(attn_t, V_t) that runs as the whole attention chain
+        bool chain = false;                 // out_prod(attn_t, V_t) that runs as the whole attention chain ...
+        bool chain_bits = false;            // ... with the bits of its nodes (attention_chain)
         Tensor *q = nullptr, *k = nullptr, *v = nullptr, *bias = nullptr;
         float scale = 1.0f;
     };
@@ -765,8 +774,30 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
             }
         }
 
-        // (2) the reference's default attention chain (src/modules/Attention.cpp:264-281) as one fused launch
-        if (fuse_attention_chain_) {
+        // (2) the reference's default attention chain (src/modules/Attention.cpp:264-281) as one launch: the fused attention
+        // where the caller asked for it, otherwise (with the three passes below on, whose launches it replaces) the one that has
+        // the bits of the nodes, for planes of up to 128 rows.  Fewer than 32 planes stay three launches, as they were.
+        const int arithmetic_here = f32_arithmetic_ >= 0 ? f32_arithmetic_ : ppml_hip_set_f32_arithmetic(-1);
+        const bool chain_bits = !fuse_attention_chain_ && fuse_scale_into_out_prod_ && fuse_add_into_soft_max_ &&
+                                fuse_permutes_into_out_prod_ && arithmetic_here != 1;
+        // a tensor's memory as far as it is settled before the graph runs (what is not gets memory of its own)
+        struct Range { uintptr_t lo = 0, hi = 0; };
+        const auto memory_of = [](const Tensor* t) {
+            const Tensor* r = t;
+            size_t offs = 0;
+            for (int guard = 0; guard < 64 && r && !r->data; ++guard) {
+                offs += r->view_offs;
+                r = r->view_src ? r->view_src : (r->op == OP_VIEW || r->op == OP_RESHAPE) ? r->src[0] : nullptr;
+            }
+            Range m;
+            if (r && r->data) { m.lo = reinterpret_cast<uintptr_t>(r->data) + offs; m.hi = m.lo + t->nbytes(); }
+            return m;
+        };
+        const auto meet = [&](const Tensor* a, const Tensor* b) {
+            const Range x = memory_of(a), y = memory_of(b);
+            return x.lo < y.hi && y.lo < x.hi;
+        };
+        if (fuse_attention_chain_ || chain_bits) {
             for (Tensor* n : *graph) {
                 if (!n || n->op != OP_OUT_PROD || n->type != TENSOR_TYPE_F32 || n->ndim != 4) continue;
                 Tensor* attn_t = n->src[0];
@@ -795,10 +826,33 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 const int64_t L = q->dims[0], D = q->dims[1];
                 bool same = true;
                 for (int d = 0; d < 4; ++d) same = same && k->dims[d] == q->dims[d] && v->dims[d] == q->dims[d];
-                if (!same || D <= 0 || D > 64 || (D % 4) != 0) continue;           // the fused kernel's own range
+                if (!same || D <= 0 || (!chain_bits && (D > 64 || (D % 4) != 0))) continue;       // the fused kernel's own range
                 if (n->numel() != q->numel() || scores->numel() != L * L * q->dims[2] * q->dims[3]) continue;
+                if (chain_bits) {
+                    const int64_t planes = q->dims[2] * q->dims[3];
+                    if (planes < 32 || !attention_chain_fits(planes, L, D) || attn->dims[0] != L || scores->dims[0] != L || scores->dims[1] != L ||
+                        n->dims[0] != L || n->dims[1] != D || (bias && bias->dims[0] != L) || !node_supported(n)) continue;
+                    // every node would have run, and none of those that the three passes do write has memory somebody gave it
+                    bool free = true;
+                    for (const Tensor* t : {static_cast<const Tensor*>(scores), static_cast<const Tensor*>(x), static_cast<const Tensor*>(added),
+                                            static_cast<const Tensor*>(attn), static_cast<const Tensor*>(attn_t), static_cast<const Tensor*>(v_t)})
+                        if (t) free = free && node_supported(t) && !t->data && !t->buffer;
+                    // Q, K and the bias are read when the last node runs: nothing in between may write there, nor that node itself
+                    for (const Tensor* r : {static_cast<const Tensor*>(q), static_cast<const Tensor*>(k), static_cast<const Tensor*>(v), static_cast<const Tensor*>(bias)})
+                        if (r) free = free && !meet(n, r);
+                    for (Tensor* m : *graph) {
+                        if (!free) break;
+                        if (m == x || m == added || m == attn || m == attn_t || m == v_t || !before(scores, m) || !before(m, n)) continue;
+                        if (m->op == OP_NONE || m->op == OP_VIEW || m->op == OP_RESHAPE) continue;
+                        free = (m->op == OP_MUL_MAT || m->op == OP_OUT_PROD || m->op == OP_PERMUTE || m->op == OP_TRANSPOSE || m->op == OP_ADD ||
+                                m->op == OP_SCALE || m->op == OP_UNARY || m->op == OP_SOFT_MAX) &&
+                               !meet(m, q) && !meet(m, k) && !(bias && meet(m, bias));
+                    }
+                    if (!free) continue;
+                }
                 Plan c;
                 c.chain = true;
+                c.chain_bits = chain_bits;
                 c.q = q; c.k = k; c.v = v; c.bias = bias;
                 c.scale = x->param_f32(0);
                 plans[n] = c;
@@ -930,6 +984,7 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         Tensor* exec = node;
         Tensor* storage = node;
         attn_layout_ = 0;
+        attn_nodes_ = false;
         relu_in_quantizer_ = false;
         out_prod_scaled_ = false;
         out_prod_transposed_ = false;
@@ -991,6 +1046,7 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 rewired.set_param_f32(2, 1e-9f);        // kernel_softmax's 1 / (sum + 1e-9), CPUKernels.cpp:1463
                 rewired.op_params[4] = 64;
                 attn_layout_ = 3;                       // inputs [L, D, h, B] as they are, result [L, D, h, B]
+                attn_nodes_ = pl.chain_bits;
             }
         }
         resolve_views(exec);
@@ -1037,6 +1093,7 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
 
         const Status st = dispatch_node(exec);
         attn_layout_ = 0;
+        attn_nodes_ = false;
         relu_in_quantizer_ = false;
         out_prod_scaled_ = false;
         out_prod_transposed_ = false;

@@ -49,6 +49,10 @@ Workspace workspace_take(size_t bytes, hipStream_t stream);
 void workspace_give(const Workspace& ws, hipStream_t stream);
 int noalloc_scratch_setup(uint8_t** out);   // address of the no-allocation entry point's static workspace on the current device
 int device_cu_count();
+// The default attention's nodes in one launch (attention_chain.hip): Q, K, V, O [planes][d][L], bias [planes][L][L] or null
+bool attention_chain_fits(int64_t planes, int64_t L, int64_t d);
+int attention_chain(const float* Q, const float* K, const float* V, const float* bias, float* O, int64_t planes, int L, int d, float scale,
+                    hipStream_t stream);
 void set_q8_path(int path);              // what ppml_hip_q8_last_path() reports for the calling thread
 
 typedef int   v4i  __attribute__((ext_vector_type(4)));
@@ -130,6 +134,58 @@ __device__ __forceinline__ void split4(const v4f& v, uint2 (&out)[3], SplitGuard
     g.sum3 = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, out[2].y), ones, g.sum3, false);
 #endif
 }
+
+// op over all 64 lanes, with the partners of a butterfly over lane ^ 32, 16, 8, 4, 2, 1 -- and so its bits, for a commutative
+// op.  No step goes through LDS: the halves and the rows of sixteen lanes change places by v_permlane32_swap / 16_swap (both
+// operands the value: one comes back as the even halves or rows twice over, the other as the odd ones), within a row the
+// moves are DPP operands (once lanes eight apart agree, four places round the row is lane ^ 4).
+template <class Op>
+__device__ __forceinline__ float row16_butterfly(float v, Op op) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#define PPML_DPP(CTRL) op(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true)))
+    v = PPML_DPP(0x128);                                // row_ror:8
+    v = PPML_DPP(0x124);                                // row_ror:4
+    v = PPML_DPP(0x4e);                                 // quad_perm [2, 3, 0, 1]
+    v = PPML_DPP(0xb1);                                 // quad_perm [1, 0, 3, 2]
+#undef PPML_DPP
+#endif
+    return v;
+}
+// a's lanes l and l ^ 32 (l ^ 16) combined in the even halves (rows of sixteen), b's in the odd ones
+template <class Op>
+__device__ __forceinline__ float fold32(float a, float b, Op op) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+#else
+    return op(a, b);
+#endif
+}
+template <class Op>
+__device__ __forceinline__ float fold16(float a, float b, Op op) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+#else
+    return op(a, b);
+#endif
+}
+template <class Op>
+__device__ __forceinline__ float wave_butterfly(float v, Op op) {
+    v = fold32(v, v, op);
+    return row16_butterfly(fold16(v, v, op), op);
+}
+// Four values at once: the two swaps hand half of the lanes to the next value instead of doing their work twice, so that four
+// reductions take the steps of one and a half.  Value i's result stands in the sixteen lanes from FOLD4_LANE[i] on.
+constexpr int FOLD4_LANE[4] = {0, 32, 16, 48};
+template <class Op>
+__device__ __forceinline__ float wave_butterfly4(const float (&v)[4], Op op) {
+    return row16_butterfly(fold16(fold32(v[0], v[1], op), fold32(v[2], v[3], op), op), op);
+}
+__device__ __forceinline__ float lane_value(float v, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
+
+__device__ __forceinline__ float wave_max(float v) { return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); }); }
+__device__ __forceinline__ float wave_sum(float v) { return wave_butterfly(v, [](float a, float b) { return a + b; }); }
 
 // XCD-aware work-group numbering.  Consecutive work-group ids go round-robin over the 8 XCDs, each
 // with its own L2.  This maps id -> a logical index such that every XCD walks one contiguous

@@ -92,31 +92,6 @@ __global__ __launch_bounds__(256) void bcast_kernel(const float* __restrict__ a,
     }
 }
 
-// op over all 64 lanes, with the partners of a butterfly over lane ^ 32, 16, 8, 4, 2, 1 -- and so its bits, for a commutative
-// op -- with a shuffle's LDS round trip in the first two steps only: within a row of sixteen lanes the moves are DPP operands
-// (once lanes eight apart agree, four places round the row is lane ^ 4).
-template <class Op>
-__device__ __forceinline__ float wave_butterfly(float v, Op op) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    v = op(v, __shfl_xor(v, 32, 64));
-    v = op(v, __shfl_xor(v, 16, 64));
-#define PPML_DPP(CTRL) op(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true)))
-    v = PPML_DPP(0x128);                                // row_ror:8
-    v = PPML_DPP(0x124);                                // row_ror:4
-    v = PPML_DPP(0x4e);                                 // quad_perm [2, 3, 0, 1]
-    v = PPML_DPP(0xb1);                                 // quad_perm [1, 0, 3, 2]
-#undef PPML_DPP
-#endif
-    return v;
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-    return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); });
-}
-__device__ __forceinline__ float wave_sum(float v) {
-    return wave_butterfly(v, [](float a, float b) { return a + b; });
-}
-
 // One wave per row, the row held in registers between the three passes (maximum, sum of exponentials, quotient):
 // it is read once and written once.  PIECES 16-byte pieces (VEC) or single elements per lane.  The reference starts
 // its maximum from the first element and moves it with `>` only, so a NaN there stays the maximum; elsewhere a NaN

@@ -1,7 +1,7 @@
 // What the binary32 contractions of this library share: the description of a contraction, the reference's own loop for
 // outputs whose operands a split cannot carry, and the stores of compound outputs.
 #pragma once
-#include "common.hpp"
+#include "split.hpp"
 
 namespace ppmlhip {
 
@@ -29,8 +29,6 @@ struct GemmParams {
     int a_lm, a_lk;
     int64_t a_mo, a_mi, a_ko, a_ki;
 };
-
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 // gemm_f16x2.hip: a large single-plane contraction in two f16 parts; -1 when the contraction is not of the kind that form is
 // for or no workspace is to be had.  `fixed_ws` / `fixed_cap`: a workspace the caller brings.

@@ -21,6 +21,7 @@
 // with the maxima (v_maximum3_f32 passes NaN on), and the outputs concerned are redone in plain binary32 arithmetic, one
 // product at a time (plain_dot), as everywhere in this library.
 #include "gemm.hpp"
+#include "split.hpp"
 
 #include <algorithm>
 
@@ -49,19 +50,6 @@ struct F16x2Job {
     int slices, items;
     uint32_t a_span;          // bytes of A from its base to behind its last element
 };
-
-// two halves of four consecutive elements times s
-__device__ __forceinline__ void split4_f16(const v4f& x, float s, uint2 (&out)[2]) {
-    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-    v4h h, l;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        h[c] = static_cast<_Float16>(__builtin_fmaf(x[c], s, 0.0f));
-        l[c] = static_cast<_Float16>(__builtin_fmaf(x[c], s, -static_cast<float>(h[c])));       // (the difference is exact)
-    }
-    out[0] = __builtin_bit_cast(uint2, h);
-    out[1] = __builtin_bit_cast(uint2, l);
-}
 
 // the largest magnitude, NaN if there is one
 __device__ __forceinline__ float max4(float m, const v4f& x) {

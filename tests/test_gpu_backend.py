@@ -848,3 +848,122 @@ def test_bias_add_and_permutations_stay_nodes_when_somebody_else_needs_them(be, 
     assert be.nodes_fused_away == 0
     ref = oracle.softmax(oracle.bcast_elemwise(small, oracle.out_prod(k, q), "add"))
     np.testing.assert_allclose(be.download(attn).reshape(ref.shape), ref, rtol=2e-5, atol=1e-30)
+
+
+# rows of one tile and of four, either side of a whole tile, of a whole chunk of keys and of 64 (one and two elements per
+# lane), a multiple of four and not; features of one chunk, of two, and not a multiple of four
+@pytest.mark.parametrize("with_bias", [True, False])
+@pytest.mark.parametrize("L,D,H,Bt", [(103, 32, 4, 40), (24, 8, 4, 8), (31, 16, 2, 16), (33, 32, 4, 9), (64, 24, 4, 8), (65, 32, 4, 8),
+                                      (96, 20, 1, 40), (113, 30, 4, 8), (128, 32, 4, 70), (1, 4, 4, 8), (17, 32, 4, 50)])
+def test_attention_chain_in_one_launch_has_the_bits_of_its_nodes(be, oracle, L, D, H, Bt, with_bias):
+    """At least 32 planes of at most 128 rows: the default chain as one launch, against the three launches (an
+    intermediate flagged as an output keeps them) bit for bit, and against the oracle; non-finite and sub-range operands
+    and masked rows end where the nodes put them."""
+    rng = np.random.default_rng(L * 7 + D)
+    k, q, v = (rng.standard_normal((Bt, H, D, L)).astype(np.float32) for _ in range(3))
+    bias = rng.standard_normal((Bt, H, L, L)).astype(np.float32) if with_bias else None
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(D)))
+
+    def run(k, q, v, bias, one):
+        kl, ql, vl = _leaf(be, k), _leaf(be, q), _leaf(be, v)
+        bl = _leaf(be, bias) if bias is not None else None
+        graph, out = _attention_chain_graph(be, kl, ql, vl, bl, L, D, H, Bt, scale)
+        if not one:
+            graph[-4].set_flag(B.FLAG_OUTPUT)                         # the probabilities
+        assert be.graph_compute(graph) == B.SUCCESS, be.last_error
+        assert be.nodes_fused_away == (5 if one else 3) + (1 if bias is not None else 0)
+        return be.download(out).reshape(Bt, H, D, L)
+
+    def want(k, q, v, bias):
+        with np.errstate(invalid="ignore", over="ignore"):
+            x = oracle.scale(oracle.out_prod(k, q), scale)
+            if bias is not None:
+                x = oracle.bcast_elemwise(x, bias, "add")
+            return oracle.out_prod(oracle.permute(oracle.softmax(x), (1, 0, 2, 3)), oracle.permute(v, (1, 0, 2, 3)))
+
+    got = run(k, q, v, bias, True)
+    assert np.array_equal(got.view(np.uint32), run(k, q, v, bias, False).view(np.uint32))
+    ref = want(k, q, v, bias)
+    np.testing.assert_allclose(got, ref, rtol=0, atol=1e-4 * np.abs(ref).max())
+    # one plane each: an infinite key, query and value, a NaN, elements below the split's range, a masked row and keys
+    k[0, 0, D // 2, L // 3] = np.inf
+    q[1, 0, 0, L - 1] = -np.inf
+    v[2, 0, D - 1, L // 2] = np.inf
+    k[3, 0, 0, 0] = np.nan
+    q[4, 0] *= np.float32(2.0 ** -130)
+    v[5, 0] *= np.float32(2.0 ** -130)
+    if bias is not None:
+        bias[6, 0, L // 2, :] = -np.inf
+        bias[7, 0, :, :L // 2] = -np.inf
+    got, ref = run(k, q, v, bias, True), want(k, q, v, bias)
+    nodes = run(k, q, v, bias, False)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isnan(nodes), np.isnan(ref))
+    assert np.array_equal(np.isinf(got), np.isinf(ref)) and np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    fin = np.isfinite(ref)
+    np.testing.assert_allclose(got[fin], ref[fin], rtol=0, atol=1e-4 * np.abs(ref[fin]).max())
+    np.testing.assert_allclose(got[5, 0], ref[5, 0], rtol=1e-4, atol=1e-4 * float(np.abs(np.nan_to_num(ref[5, 0])).max()))
+
+
+def test_attention_chain_in_one_launch_only_where_nothing_can_tell(be):
+    """Intermediates with storage of their own, a result that lies on an operand, a node in between that writes one, a pass
+    switched off, the fp32 pipe, few planes, long rows: the nodes run as they did."""
+    L, D, H, Bt = 40, 16, 4, 8
+    rng = np.random.default_rng(3)
+    k, q, v = (rng.standard_normal((Bt, H, D, L)).astype(np.float32) for _ in range(3))
+
+    def graph_of(L=L, Bt=Bt, k=k, q=q, v=v):
+        kl, ql, vl = _leaf(be, k), _leaf(be, q), _leaf(be, v)
+        nodes, out = _attention_chain_graph(be, kl, ql, vl, None, L, D, H, Bt, 0.25)
+        return nodes, out, (kl, ql, vl)
+
+    nodes, out, keep = graph_of()
+    assert be.graph_compute(nodes) == B.SUCCESS and be.nodes_fused_away == 5
+    want = be.download(out)
+
+    def same(count):
+        assert be.nodes_fused_away == count
+        assert np.array_equal(be.download(out).view(np.uint32), want.view(np.uint32))
+
+    for setter, left in ((be.set_fuse_scale_into_out_prod, 2), (be.set_fuse_permutes_into_out_prod, 1)):
+        setter(False)
+        try:
+            nodes, out, keep = graph_of()
+            assert be.graph_compute(nodes) == B.SUCCESS
+            same(left)
+        finally:
+            setter(True)
+    # the probabilities on memory of their own: written
+    nodes, out, keep = graph_of()
+    attn = nodes[2]
+    import torch
+    held = torch.full((Bt, H, L, L), float("nan"), device="cuda")
+    attn.bind(held.data_ptr())
+    assert be.graph_compute(nodes) == B.SUCCESS
+    same(3)
+    assert bool(held.isfinite().all())
+    # the result on the memory of the queries
+    nodes, out, keep = graph_of()
+    qt = torch.from_numpy(q).cuda()
+    keep[1].bind(qt.data_ptr())
+    out.bind(qt.data_ptr())
+    assert be.graph_compute(nodes) == B.SUCCESS
+    be.synchronize()
+    assert be.nodes_fused_away == 3 and np.array_equal(qt.cpu().numpy().reshape(-1).view(np.uint32), want.view(np.uint32))
+    # a node between the logits and the weighted sum that writes the keys
+    nodes, out, keep = graph_of()
+    kt = torch.from_numpy(k).cuda()
+    keep[0].bind(kt.data_ptr())
+    other = B.Tensor((L, D, H, Bt), B.F32, B.OP_SCALE, [keep[2]]).set_param(0, 2.0)
+    other.bind(kt.data_ptr())
+    assert be.graph_compute(nodes[:2] + [other] + nodes[2:]) == B.SUCCESS
+    same(3)
+    be.set_f32_arithmetic("fp32")
+    try:
+        nodes, out, keep = graph_of()
+        assert be.graph_compute(nodes) == B.SUCCESS and be.nodes_fused_away == 3
+    finally:
+        be.set_f32_arithmetic(None)
+    for L2, B2 in ((40, 7), (129, 8)):
+        k2, q2, v2 = (rng.standard_normal((B2, H, D, L2)).astype(np.float32) for _ in range(3))
+        nodes, out, keep = graph_of(L2, B2, k2, q2, v2)
+        assert be.graph_compute(nodes) == B.SUCCESS and be.nodes_fused_away == 3
