@@ -71,6 +71,7 @@ struct F16x2Split {
     int* exps;
     int rows, rows_pad, K, chunks, slice_chunks;
     int64_t rs, ks;
+    int64_t span;             // elements from src to behind the last one: below 2^29, any 32 rows' offsets too
 };
 
 template <bool KS1>
@@ -84,17 +85,24 @@ __global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) 
     const int c_end = c_begin + jb.slice_chunks < jb.chunks ? c_begin + jb.slice_chunks : jb.chunks;
     const int k_begin = c_begin * HX_K, k_end = c_end * HX_K;
     const int rounds = (k_end - k_begin + 255) / 256;
-    const float* src = jb.src + static_cast<int64_t>(r) * jb.rs;
+    // through a buffer resource from the work-group's first row on (outside: zero): loads under conditions are waited for one
+    // after the other (256 columns x 12288 14.2 us, this way 11.4; 256 x 26368 13.6 / 12.7, 768 x 256 5.6 / 5.3)
+    const int64_t span = jb.span - static_cast<int64_t>(blockIdx.x) * 32 * jb.rs;       // elements from there to the operand's end
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(jb.src + static_cast<int64_t>(blockIdx.x) * 32 * jb.rs), 0,
+                                                                          static_cast<int>(span > 0 ? span * 4 : 0), 0x00020000);
+    const uint32_t row_at = r < jb.rows ? static_cast<uint32_t>(row * jb.rs) * 4u : OUTSIDE;
+    const uint32_t k_step = static_cast<uint32_t>(KS1 ? 1 : jb.ks) * 4u;
     const auto load = [&](int i, v4f (&v)[2]) {
         const int kb = k_begin + i * 256 + oct * 8;
-        v[0] = v[1] = v4f{0.f, 0.f, 0.f, 0.f};
-        if (r >= jb.rows || kb >= k_end) return;
-        if (KS1 && kb + 7 < jb.K) {
-            v[0] = *reinterpret_cast<const v4f_u*>(src + kb);
-            v[1] = *reinterpret_cast<const v4f_u*>(src + kb + 4);
+        const uint32_t at = row_at + static_cast<uint32_t>(kb) * k_step;
+        const int k_last = k_end < jb.K ? k_end : jb.K;
+        if (KS1 && k_begin + (i + 1) * 256 <= k_last) {          // (the same for the work-group)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[h] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at + 16u * h, 0, 0));
         } else {
 #pragma unroll
-            for (int c = 0; c < 8; ++c) if (kb + c < jb.K) v[c >> 2][c & 3] = src[static_cast<int64_t>(kb + c) * (KS1 ? 1 : jb.ks)];
+            for (int c = 0; c < 8; ++c)
+                v[c >> 2][c & 3] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, kb + c < k_last ? at + c * k_step : OUTSIDE, 0, 0));
         }
     };
     const bool kept = rounds <= HX_SPLIT_ROUNDS;
@@ -106,9 +114,9 @@ __global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) 
     };
     if (kept) {
 #pragma unroll
-        for (int i = 0; i < HX_SPLIT_ROUNDS; ++i) load(i, held[i]);
+        for (int i = 0; i < HX_SPLIT_ROUNDS; ++i) if (i < rounds) load(i, held[i]);
 #pragma unroll
-        for (int i = 0; i < HX_SPLIT_ROUNDS; ++i) see(held[i]);
+        for (int i = 0; i < HX_SPLIT_ROUNDS; ++i) if (i < rounds) see(held[i]);
     } else {
         for (int i = 0; i < rounds; i += 2) {
             v4f a[2], b[2];
@@ -616,6 +624,9 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
         return -1;
     }
     if (amode < 0 || span * 4 >= (1LL << 31) - 65536) return -1;
+    // B by 32-bit byte offsets as well
+    const int64_t b_span = static_cast<int64_t>(p.N - 1) * p.b_rs + static_cast<int64_t>(p.K - 1) * p.b_ks + 1;
+    if (p.b_rs <= 0 || p.b_ks <= 0 || b_span * 4 >= (1LL << 31) || (static_cast<int64_t>(p.K) + 64) * p.b_ks * 4 + 32 * p.b_rs * 4 >= (1LL << 31)) return -1;
     // the output (slices: any strides)
     if (compound ? p.c_span == 0 : (p.c_ni != 1 && !sliced) || static_cast<int64_t>(p.M + HX_M) * p.c_mi * 4 >= (1LL << 31)) return -1;
 
@@ -626,13 +637,13 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     //   * compound C (its forward): 3136 x 106 x 3136 (17) 25 / 32, 4464 x 123 x 4464 (38) 59 / 43, 7808 x 202 x 7808 242 / 165;
     //   * slices: 888 x 3490 x 504 (24) 29 / 29, 832 x 8990 x 304 (46) 42 / 38, 768 x 26368 x 256 (77) 61 / 52; with few rows the
     //     split of the other operand weighs more: 464 x 12651 x 392 (49) 42 / 43, 564 x 26377 x 197 (64) 51 / 52;
-    //   * otherwise: 10609 x 176 -> 532 (18) 20 / 21, 26368 x 256 -> 256 (26) 25 / 21, 26368 x 512 -> 1024 (206) 189 / 101.
+    //   * otherwise: 10609 x 176 -> 532 (15) 20 / 21, 26368 x 256 -> 256 (26) 25 / 21, 26368 x 512 -> 1024 (206) 189 / 101.
     // A K below 128 stays with the form that splits in the tile loop at any size (the bits of a contraction that is cut
     // out of a larger one then do not depend on the size).
     if (p.a_lm > 0) { if (load < 22) return -1; }
     else if (compound) { if (load < 30) return -1; }
     else if (sliced) { if (load < 42 || (p.M < 700 && load < 66) || p.K < 128) return -1; }
-    else if (load < 24 || p.K < 128) return -1;
+    else if (p.K < 128 || static_cast<double>(p.M) * p.N * p.K < 20.0 * 128 * 128 * 16 * cus) return -1;      // (without the padding: 30001 x 131 -> 260 25.8 / 29.7)
     // Tiles of 128 x 256 by one work-group per CU, or of 128 x 128 by two, which store while the other contracts but read A
     // twice as often: where 256 columns would be half empty, where the wide tiles' last round leaves more than half of the CUs idle (26368 x 256 -> 768: 51.4
     // / 48.8 us; 32768 x 512 -> 1024, whole rounds, 110 / 118), and for compound rows that are not whole lines, whose stores
@@ -684,7 +695,7 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     jb.chunks = chunks; jb.slice_chunks = slice_chunks; jb.slices = slices;
     jb.items = static_cast<int>(tiles) * slices;
     jb.a_span = static_cast<uint32_t>(span * 4);
-    const F16x2Split sp{p.B, ws, exps, p.N, nb_pad, p.K, chunks, slice_chunks, p.b_rs, p.b_ks};
+    const F16x2Split sp{p.B, ws, exps, p.N, nb_pad, p.K, chunks, slice_chunks, p.b_rs, p.b_ks, b_span};
     const dim3 sgrid(nb_pad / 32, slices);
     if (p.b_ks == 1) hipLaunchKernelGGL((split_f16x2_kernel<true>), sgrid, dim3(1024), 0, stream, sp);
     else             hipLaunchKernelGGL((split_f16x2_kernel<false>), sgrid, dim3(1024), 0, stream, sp);
