@@ -816,6 +816,126 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_kernel(const GemmParams p)
     pc_tile<MODE, STREAM_C, K4, BMODE>(p, lds_ab, static_cast<int>(blockIdx.x));
 }
 
+// The same on tiles of 64 x 64 with two chunks per barrier, for a LinearLayer's contraction that leaves most CUs without a
+// 128 x 128 tile: what bounds such a call is one work-group's chain of load, split and products, and a quarter of the products per
+// wave, half of the barriers and four times the work-groups shorten it.  Operands contiguous in k; same products in the same
+// order: same bits.  Measured, us, 128 x 128 tiles / this: 2601 x 128 -> 132
+// 8.5 / 5.1, 408 x 256 -> 256 12.2 / 7.0, 51 x 64 -> 64 5.9 / 3.5, 2601 x 512 -> 512 (328 of these) 20.1 / 15.9.  Beyond two per
+// CU (they hold 74 KB each) the larger tiles win: 10609 x 500 -> 130 (498) 23.7 / 17.1, 20000 x 128 -> 128 (626) 8.9 / 9.5.
+constexpr int PC64_AHEAD = 4;                     // stages of 32 k in flight
+constexpr int PC64_PLANE = 64 * SPLIT_PITCH;      // one of the three planes of 64 rows x 16 k
+constexpr int PC64_OPERAND = 2 * 3 * PC64_PLANE;  // [16 k][plane][row]
+template <bool STREAM_C, bool K4>
+__global__ __launch_bounds__(512) void gemm_bf16x3_pc64_kernel(const GemmParams p) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds_ab[2][2 * PC64_OPERAND];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles_n = (p.N + 63) / 64, tiles_m = (p.M + 63) / 64;
+    const int tile = xcd_contiguous_index(blockIdx.x, tiles_m * tiles_n);
+    const int m0 = tile / tiles_n * 64, n0 = tile % tiles_n * 64;
+    const int stages = (p.K + 31) / 32;
+
+    // (barriers: stages + 1 in either loop, as in gemm_bf16x3_pc_kernel)
+    int fired = 0;
+    if (wave >= 4) {
+        const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A), 0, static_cast<int>(((p.M - 1) * p.a_rs + p.K) * 4), 0x00020000);
+        const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.B), 0, static_cast<int>(((p.N - 1) * p.b_rs + p.K) * 4), 0x00020000);
+        // a thread: row (tid % 256) / 4 of either tile, four k of each chunk of the stage
+        const int ptid = tid & 255, row = ptid >> 2, kq = (ptid & 3) * 4;
+        const uint32_t a_at = m0 + row < p.M ? static_cast<uint32_t>(m0 + row) * static_cast<uint32_t>(p.a_rs) * 4u : OUTSIDE;
+        const uint32_t b_at = n0 + row < p.N ? static_cast<uint32_t>(n0 + row) * static_cast<uint32_t>(p.b_rs) * 4u : OUTSIDE;
+        const auto load = [&](const __amdgpu_buffer_rsrc_t r, uint32_t at, int stage, v4f (&x)[2]) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int k = stage * 32 + c * 16 + kq;
+                if (K4 || stage * 32 + 32 <= p.K) {     // (a piece lies inside its row or behind it)
+                    x[c] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, k < p.K ? at + 4u * k : OUTSIDE, 0, 0));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[c][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, k + e < p.K ? at + 4u * (k + e) : OUTSIDE, 0, 0));
+                }
+            }
+        };
+        v4f xa[PC64_AHEAD][2], xb[PC64_AHEAD][2];
+#pragma unroll
+        for (int d = 0; d < PC64_AHEAD; ++d)
+            if (d < stages) { load(rsrc_a, a_at, d, xa[d]); load(rsrc_b, b_at, d, xb[d]); }
+        SplitGuard guard;
+        for (int g = 0; g < stages; g += PC64_AHEAD) {
+#pragma unroll
+            for (int d = 0; d < PC64_AHEAD; ++d) {
+                const int s = g + d;
+                if (s >= stages) break;                 // uniform
+                uint8_t* const dst = lds_ab[s & 1] + row * SPLIT_PITCH + kq * 2;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    uint2 a[3], b[3];
+                    split4(xa[d][c], a, guard);
+                    split4(xb[d][c], b, guard);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) {
+                        *reinterpret_cast<uint2*>(dst + (c * 3 + q) * PC64_PLANE) = a[q];
+                        *reinterpret_cast<uint2*>(dst + PC64_OPERAND + (c * 3 + q) * PC64_PLANE) = b[q];
+                    }
+                }
+                if (s + PC64_AHEAD < stages) { load(rsrc_a, a_at, s + PC64_AHEAD, xa[d]); load(rsrc_b, b_at, s + PC64_AHEAD, xb[d]); }
+                __syncthreads();
+            }
+        }
+        __syncthreads();
+        fired = guard.fired() ? 1 : 0;
+    }
+
+    v16f acc;
+    const int j = lane & 31, hh = lane >> 5;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    if (wave < 4) {
+        const float b0 = p.bias && n0 + wn + j < p.N ? p.bias[n0 + wn + j] : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = b0;
+        const int at = j * SPLIT_PITCH + hh * 16;
+        __syncthreads();                                // stage 0 is in LDS
+        for (int s = 0; s < stages; ++s) {
+            const uint8_t* const fa = lds_ab[s & 1] + at + wm * SPLIT_PITCH;
+            const uint8_t* const fb = lds_ab[s & 1] + at + wn * SPLIT_PITCH + PC64_OPERAND;
+            v8bf a[2][3], b[2][3];
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    a[c][q] = *reinterpret_cast<const v8bf*>(fa + (c * 3 + q) * PC64_PLANE);
+                    b[c][q] = *reinterpret_cast<const v8bf*>(fb + (c * 3 + q) * PC64_PLANE);
+                }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                if (c == 1 && s * 32 + 16 >= p.K) break;        // (the other forms have no chunk there: zeros would make -0 +0)
+#pragma unroll
+                for (int q = 0; q < 6; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[c][SPLIT_TERMS[q][0]], b[c][SPLIT_TERMS[q][1]], acc, 0, 0, 0);
+            }
+            __syncthreads();
+        }
+    }
+    // an operand of this tile that the split could not carry: the whole tile again, the reference's way
+    if (__syncthreads_or(fired)) {
+        if (tid < 256) plain_tile(p, p.A, p.B, p.C, m0, n0, 64, 64, tid);
+        return;
+    }
+    if (wave < 4) {
+        const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(p.C, 0, static_cast<int>(p.M * p.c_mi * 4), 0x00020000);
+        const uint32_t ld = static_cast<uint32_t>(p.c_mi) * 4u;
+        const int n = n0 + wn + j;
+        // rows past the matrix fall outside the plane by themselves (offset >= M * ld bytes)
+        const uint32_t base = n < p.N ? static_cast<uint32_t>(m0 + wm + 4 * hh) * ld + static_cast<uint32_t>(n) * 4u : OUTSIDE;
+        const bool scale = p.alpha != 1.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float v = acc[r];
+            if (scale) v *= p.alpha;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc_c, base + (8 * (r >> 2) + (r & 3)) * ld, 0, STREAM_C ? 3 : 0);
+        }
+    }
+}
+
 // Two independent contractions of that kind in one launch (the two gradients of the triangle multiplication): the first
 // groups_a work-groups take the tiles of `a`, the others those of `b`.  With one tile per plane, as the pair tensor has up
 // to 128 residues, each of the two by itself leaves half of the CUs idle and is a single latency chain (load, split, seven
@@ -2442,6 +2562,13 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
             else        { if (p.stream_c) PPML_KNARROW_K4(SIDE_M, true); else PPML_KNARROW_K4(SIDE_M, false); }
 #undef PPML_KNARROW_K4
 #undef PPML_KNARROW
+        }
+        else if (k_fast && p.K > 3 * BK && p.np2 * p.np3 == 1 && p.M > 32 && p.N > 32 && (static_cast<int64_t>((p.M + 63) / 64) * ((p.N + 63) / 64) <= 2 * device_cu_count())) {
+            const dim3 g64(static_cast<unsigned>((p.M + 63) / 64 * ((p.N + 63) / 64)));
+#define PPML_KPC64(STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_pc64_kernel<STREAM_, K4_>), g64, dim3(512), 0, stream, p)
+            if (p.K % 4 == 0) { if (p.stream_c) PPML_KPC64(true, true); else PPML_KPC64(false, true); }
+            else              { if (p.stream_c) PPML_KPC64(true, false); else PPML_KPC64(false, false); }
+#undef PPML_KPC64
         }
         else if (k_fast && two_sets) {
 #define PPML_KPC(STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_pc_kernel<LOAD_K_CONTIG, STREAM_, K4_>), grid, dim3(512), 0, stream, p)

@@ -1,0 +1,41 @@
+"""mul_mat on tiles of 64 x 64 (gemm_bf16x3_pc64_kernel): up to two of them per CU, K above 48."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    assert torch.cuda.is_available(), "GPU tests need a device"
+    from proteinpredictmachinelearning_amd import ops as _ops
+
+    return _ops
+
+
+# either side of a tile in both directions; K of 49 (a stage and a half-empty one), whole stages, one chunk more, four and
+# five of the stages in flight, not a multiple of four; the most work-groups the form is for, and one row more
+@pytest.mark.parametrize("M,N", [(33, 33), (64, 64), (65, 127), (2601, 132), (16384, 128), (1, 1000), (1000, 33)])
+@pytest.mark.parametrize("K", [49, 64, 80, 101, 128, 160, 333])
+def test_small_linear(ops, M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g)
+    bias = torch.randn(N, device="cuda", generator=g)
+    got = ops.mul_mat(a, b, bias)
+    want = a.double() @ b.double().t() + bias.double()
+    bound = (K + 2) * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t() + bias.double().abs())
+    assert bool(((got.double() - want).abs() <= bound).all())
+    # rows of a contraction too large for the form (tiles of 128 x 128): the same products in the same order
+    if M <= 2601 and N > 32 and K <= 160:
+        many = torch.randn(40000, K, device="cuda", generator=g)
+        many[:M] = a
+        if K < 128:                                     # (from 128 on so large a one goes in two f16 parts)
+            assert torch.equal(ops.mul_mat(many, b, bias)[:M], got)
+    # an infinite operand, a NaN and one below the split's range: the reference's infinities in that tile, the others untouched
+    if M > 64:
+        a[M - 1, K - 1] = float("inf")
+        b[N - 1, 0] = 1e-42
+        hot = ops.mul_mat(a, b, bias)
+        assert torch.equal(hot.isinf(), (a.double() @ b.double().t()).isinf())
+        assert torch.equal(hot[:(M - 1) // 64 * 64, :(N - 1) // 64 * 64], got[:(M - 1) // 64 * 64, :(N - 1) // 64 * 64])
