@@ -279,38 +279,30 @@ __global__ __launch_bounds__(256) void gemm_f32_midk_kernel(const GemmParams p, 
     const float* B = p.B + (p2 / p.b_div2) * p.b_p2 + (p3 / p.b_div3) * p.b_p3;
     float* C = p.C + p2 * p.c_p2 + p3 * p.c_p3;
 
-    // ---- both panels, all of K, in flight at once
+    // ---- both panels, all of K, in flight at once: through a buffer resource over the operand's plane (outside: zero).  Loads
+    // under conditions are waited for where the condition ends, sixteen memory round trips one after the other (128 planes
+    // of 103 x 103 x 103: 11.1 us)
     v4f ra[8], rb[8];
     const auto load_panel = [&](const float* __restrict__ base, int64_t rs, int64_t ks, int row0, int nrows, v4f (&reg)[8]) {
+        const int64_t span = MODE == LOAD_K_CONTIG ? (nrows - 1) * rs + p.K : (p.K - 1) * ks + nrows;
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, static_cast<int>(span * 4), 0x00020000);
+        const uint32_t step = static_cast<uint32_t>(MODE == LOAD_K_CONTIG ? rs : ks) * 4u;
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
-            v4f v = {0.f, 0.f, 0.f, 0.f};
             if (MODE == LOAD_K_CONTIG) {
-                // sixteen lanes along 64 k of a row, four rows per wave instruction
+                // sixteen lanes along 64 k of a row, four rows per wave instruction; what a row's last piece reads of the next row is zeroed below
                 const int row = row0 + (tid >> 4) + 16 * (it & 3);
                 const int k = (tid & 15) * 4 + 64 * (it >> 2);
-                if (row < nrows && k < p.K) {
-                    const float* src = base + static_cast<int64_t>(row) * rs + k;
-                    if (k + 3 < p.K) v = *reinterpret_cast<const v4f_u*>(src);
-                    else {
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) if (k + c < p.K) v[c] = src[c];
-                    }
-                }
+                const uint32_t at = row < nrows && k < p.K ? static_cast<uint32_t>(row) * step + static_cast<uint32_t>(k) * 4u : OUTSIDE;
+                reg[it] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, 0));
             } else {
-                // sixteen lanes along the 64 rows of one k, four k per wave instruction
+                // sixteen lanes along the 64 rows of one k, four k per wave instruction (rows past the matrix: whatever lies there, for
+                // outputs that are not stored)
                 const int k = (tid >> 4) + 16 * it;
                 const int row = row0 + (tid & 15) * 4;
-                if (k < p.K && row < nrows) {
-                    const float* src = base + static_cast<int64_t>(k) * ks + row;
-                    if (row + 3 < nrows) v = *reinterpret_cast<const v4f_u*>(src);
-                    else {
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) if (row + c < nrows) v[c] = src[c];
-                    }
-                }
+                const uint32_t at = k < p.K && row < nrows ? static_cast<uint32_t>(k) * step + static_cast<uint32_t>(row) * 4u : OUTSIDE;
+                reg[it] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, 0));
             }
-            reg[it] = v;
         }
     };
     const auto park_panel = [&](float* __restrict__ lds, const v4f (&reg)[8]) {
@@ -320,7 +312,7 @@ __global__ __launch_bounds__(256) void gemm_f32_midk_kernel(const GemmParams p, 
                 const int row = (tid >> 4) + 16 * (it & 3);
                 const int k = (tid & 15) * 4 + 64 * (it >> 2);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) if (k + c < kp) lds[(k + c) * LD + row] = reg[it][c];
+                for (int c = 0; c < 4; ++c) if (k + c < kp) lds[(k + c) * LD + row] = k + c < p.K ? reg[it][c] : 0.0f;
             } else {
                 const int k = (tid >> 4) + 16 * it;
                 if (k < kp) *reinterpret_cast<v4f*>(lds + k * LD + (tid & 15) * 4) = reg[it];
@@ -2620,7 +2612,10 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
         p.stream_c = 0;                                // (the clamped instances store the ordinary way, whatever the size)
         // planes of small contractions that leave most CUs without a 128 x 128 tile: 64 x 64 tiles, whole K at once
         const int64_t tiles64 = static_cast<int64_t>((p.M + 63) / 64) * ((p.N + 63) / 64) * p.np2 * p.np3;
-        if (p.K <= MIDK_MAX && !p.bias && static_cast<int64_t>(grid.x) < 2 * device_cu_count() && tiles64 <= 0x7fffffffLL) {
+        // (32-bit byte offsets within a plane of either operand)
+        const auto reach = [&](int64_t rs, int64_t ks, int64_t rows) { return rs > 0 && ks > 0 && ((rows - 1) * rs + (p.K - 1) * ks + 1) * 4 < (1LL << 31); };
+        if (p.K <= MIDK_MAX && !p.bias && static_cast<int64_t>(grid.x) < 2 * device_cu_count() && tiles64 <= 0x7fffffffLL &&
+            reach(p.a_rs, p.a_ks, p.M) && reach(p.b_rs, p.b_ks, p.N)) {
             if (mode == LOAD_K_CONTIG) return launch_f32_midk<LOAD_K_CONTIG, true>(p, stream, what);
             if (mode == LOAD_ROW_CONTIG) return launch_f32_midk<LOAD_ROW_CONTIG, true>(p, stream, what);
         }
