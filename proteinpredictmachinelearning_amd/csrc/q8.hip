@@ -1367,15 +1367,17 @@ int try_q8_linear_ws(const void* W, const float* X, float* C, int M, int N, int 
 //
 // Blocks ascend per output and every settlement is the same fma as everywhere else: same bits.
 // ------------------------------------------------------------------------------------------
-template <int TOK, int NBLK, int CPW, bool DUMP, bool Q81>
+template <int TOK, int NBLK, int CPW, bool DUMP, bool Q81, bool RT>
 __device__ __forceinline__ void q8_linear_ll_body(
     const uint8_t* __restrict__ W, const float* __restrict__ X, float* __restrict__ C,
-    int M, int N, int relu, uint8_t* __restrict__ xq_dump, int32_t* __restrict__ sums_dump) {
+    int M, int N, int nblk_rt, int relu, uint8_t* __restrict__ xq_dump, int32_t* __restrict__ sums_dump) {
     static_assert(TOK == 8 || TOK == 16 || TOK == 32, "token rows per work-group");
     static_assert(NBLK % 2 == 0, "blocks are taken in pairs");
     static_assert(CPW * NBLK <= 16, "the wave's weight fragments stay in 64 registers");
     constexpr int NW = 4;
-    constexpr int K = NBLK * QK;
+    static_assert(!RT || !DUMP, "the diagnostic buffers of these shapes are the general kernel's");
+    const int nblk = RT ? nblk_rt : NBLK;              // RT: NBLK - 1 or NBLK blocks
+    const int K = nblk * QK;
     constexpr int NUNITS = (TOK / 8) * (NBLK / 2);     // (8 rows) x (2 blocks) each: one wave-wide load pair
     constexpr int UPW = (NUNITS + NW - 1) / NW;
     constexpr int RV = TOK / 2;                        // accumulator registers that hold real tokens
@@ -1388,6 +1390,7 @@ __device__ __forceinline__ void q8_linear_ll_body(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 31;
     const int tok0 = blockIdx.x * TOK;
+    const int ct0 = RT ? static_cast<int>(blockIdx.y) * (NW * CPW) : 0;
     const int mct = (M + 31) / 32;
     const int mct_pad = packed_tiles(M);
     const int grp = lane >> 2, c4 = lane & 3;
@@ -1402,7 +1405,7 @@ __device__ __forceinline__ void q8_linear_ll_body(
         const int bl = (u / (TOK / 8)) * 2 + ublk;
         int t = tok0 + (u % (TOK / 8)) * 8 + urow;
         t = t < N ? t : N - 1;                         // rows past the end repeat the last row; never stored
-        const float* src = X + static_cast<int64_t>(t) * K + bl * QK + c4 * 8;
+        const float* src = X + static_cast<int64_t>(t) * K + (RT && bl >= nblk ? nblk - 1 : bl) * QK + c4 * 8;
         xv[s][0] = *reinterpret_cast<const v4f_u*>(src);
         xv[s][1] = *reinterpret_cast<const v4f_u*>(src + 4);
     }
@@ -1410,17 +1413,17 @@ __device__ __forceinline__ void q8_linear_ll_body(
     v4i wq[CPW][NBLK];
     uint16_t wd[CPW][NBLK / 2];                        // parked in LDS once they have arrived: read back pair by pair
     {
-        const uint16_t* dplane = reinterpret_cast<const uint16_t*>(W + static_cast<size_t>(mct_pad) * NBLK * 1024);
+        const uint16_t* dplane = reinterpret_cast<const uint16_t*>(W + static_cast<size_t>(mct_pad) * nblk * 1024);
 #pragma unroll
         for (int t = 0; t < CPW; ++t) {
-            int ct = wave + t * NW;
+            int ct = ct0 + wave + t * NW;
             ct = ct < mct_pad ? ct : mct_pad - 1;      // tiles past the end repeat the last one; never stored
-            const size_t frag = static_cast<size_t>(ct) * NBLK;
+            const size_t frag = static_cast<size_t>(ct) * nblk;
 #pragma unroll
-            for (int b = 0; b < NBLK; ++b) wq[t][b] = *reinterpret_cast<const v4i*>(W + ((frag + b) * 64 + lane) * 16);
+            for (int b = 0; b < NBLK; ++b) wq[t][b] = *reinterpret_cast<const v4i*>(W + ((frag + (RT && b >= nblk ? nblk - 1 : b)) * 64 + lane) * 16);
 #pragma unroll
             for (int pr = 0; pr < NBLK / 2; ++pr)      // lanes 0..31: columns of block 2 pr, 32..63: of block 2 pr + 1
-                wd[t][pr] = dplane[(frag + 2 * pr) * 32 + lane];
+                wd[t][pr] = dplane[(frag + 2 * pr) * 32 + (RT && 2 * pr + 1 >= nblk ? j : lane)];
         }
     }
 
@@ -1435,7 +1438,7 @@ __device__ __forceinline__ void q8_linear_ll_body(
         const BlockQuant bq = relu ? quantize_block_lane<Q81, true>(x0, x1) : quantize_block_lane<Q81, false>(x0, x1);
         uint2* dst = reinterpret_cast<uint2*>(lds_a) + ((bl * 64 + (c4 >> 1) * 32 + row) * 2 + (c4 & 1));
         *dst = uint2{bq.q_lo, bq.q_hi};
-        if (c4 == 0) lds_d[bl * 32 + row] = uint2{bq.d_bits, 0u};
+        if (c4 == 0) lds_d[bl * 32 + row] = uint2{RT && bl >= nblk ? 0u : bq.d_bits, 0u};
         if (DUMP && xq_dump) {
             const int t = tok0 + row;
             if (t < N) store_block_part(xq_dump + (static_cast<int64_t>(t) * NBLK + bl) * Q8_0_BYTES, c4, bq);
@@ -1445,7 +1448,7 @@ __device__ __forceinline__ void q8_linear_ll_body(
 #pragma unroll
     for (int t = 0; t < CPW; ++t)
 #pragma unroll
-        for (int pr = 0; pr < NBLK / 2; ++pr) my_wd[(t * (NBLK / 2) + pr) * 64] = wd[t][pr];   // written and read by this wave only
+        for (int pr = 0; pr < NBLK / 2; ++pr) my_wd[(t * (NBLK / 2) + pr) * 64] = RT && 2 * pr + (lane >> 5) >= nblk ? 0 : wd[t][pr];   // written and read by this wave only
     __syncthreads();
 
     // ---- column tiles of this wave, blocks ascending.  (The block sums are converted on the vector pipe here: the
@@ -1476,7 +1479,7 @@ __device__ __forceinline__ void q8_linear_ll_body(
         // it: left alone, the compiler issues every MFMA of the unrolled code up front and keeps all of
         // their results alive at once
         if (!opaque_one()) continue;
-        const int ct = wave + t * NW;
+        const int ct = ct0 + wave + t * NW;
         if (ct >= mct) break;                          // wave-uniform
         const int m = ct * 32 + j;                     // this lane's output feature
         float acc[RV];
@@ -1533,13 +1536,25 @@ template <int TOK, int NBLK, int CPW, bool DUMP, bool Q81>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void q8_linear_ll_kernel(
     const uint8_t* __restrict__ W, const float* __restrict__ X, float* __restrict__ C,
     int M, int N, int relu, uint8_t* __restrict__ xq_dump, int32_t* __restrict__ sums_dump) {
-    q8_linear_ll_body<TOK, NBLK, CPW, DUMP, Q81>(W, X, C, M, N, relu, xq_dump, sums_dump);
+    q8_linear_ll_body<TOK, NBLK, CPW, DUMP, Q81, false>(W, X, C, M, N, NBLK, relu, xq_dump, sums_dump);
 }
 template <int TOK, int NBLK, int CPW, bool DUMP, bool Q81>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void q8_linear_ll2_kernel(
     const uint8_t* __restrict__ W, const float* __restrict__ X, float* __restrict__ C,
     int M, int N, int relu, uint8_t* __restrict__ xq_dump, int32_t* __restrict__ sums_dump) {
-    q8_linear_ll_body<TOK, NBLK, CPW, DUMP, Q81>(W, X, C, M, N, relu, xq_dump, sums_dump);
+    q8_linear_ll_body<TOK, NBLK, CPW, DUMP, Q81, false>(W, X, C, M, N, NBLK, relu, xq_dump, sums_dump);
+}
+
+// The same body for the numbers of blocks that the forms above have no instance for, NBLK - 1 or NBLK, and any number of columns: four column tiles a work-group, one per wave, as many
+// work-groups side by side (blockIdx.y) as that takes.  A missing last block has scales of zero on both sides, which adds
+// +0 to sums that are never -0 (a product of two halves does not underflow): the bits are those of the blocks there are.
+// Bound by latency like the others, one chain of load, quantize, NBLK / 2 pairs, store.  us, the general or tiled kernel /
+// this one: 51 x 480 -> 768  20.2 / 4.0, 408 x 160 -> 256  7.2 / 4.0, 408 x 480 -> 128  13.1 / 4.1, 408 x 512 -> 1024  10.3 /
+// 5.3, 2601 x 288 -> 320  11.1 / 5.1, 10609 x 192 -> 128  8.3 / 4.6, 10609 x 480 -> 64  13.6 / 7.5.
+template <int TOK, int NBLK, bool Q81>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void q8_linear_ll_any_kernel(
+    const uint8_t* __restrict__ W, const float* __restrict__ X, float* __restrict__ C, int M, int N, int nblk, int relu) {
+    q8_linear_ll_body<TOK, NBLK, 1, false, Q81, true>(W, X, C, M, N, nblk, relu, nullptr, nullptr);
 }
 
 template <int TOK, int NBLK, int CPW, bool Q81>
@@ -1562,6 +1577,33 @@ int launch_q8_linear_ll(const void* W, const float* X, float* C, int M, int N, i
     return check_launch("q8_linear_ll_kernel");
 }
 
+// Unit size (8 or 16 tokens) of q8_linear_ll_any_kernel for a call, 0 where it does not take it: five to sixteen blocks,
+// for which the other two forms have no instance, while all work-groups are resident at once (three per CU; every shape
+// measured inside that line gained, the least of them 1.2 times).  Fewer blocks: the general kernel's chain is as short.
+int q8_ll_any_units(int M, int N, int nblk, int c_trans) {
+    const int mct = (M + 31) / 32;
+    if (!c_trans || nblk < 5 || nblk > 16 || nblk == 8 || (nblk == 16 && mct <= 8)) return 0;
+    const int64_t parts = (mct + 3) / 4, resident = 3 * device_cu_count();
+    return (N + 7) / 8 * parts <= resident ? 8 : (N + 15) / 16 * parts <= resident ? 16 : 0;
+}
+
+template <bool Q81>
+int try_q8_linear_ll_any(const void* W, const float* X, float* C, int M, int N, int nblk, int c_trans, int relu, hipStream_t stream) {
+    const int tok = q8_ll_any_units(M, N, nblk, c_trans);
+    if (tok == 0) return -1;
+    const dim3 grid((N + tok - 1) / tok, ((M + 31) / 32 + 3) / 4), block(256);
+#define PPML_LLA(NBLK) \
+    case NBLK: \
+        if (tok == 8) hipLaunchKernelGGL((q8_linear_ll_any_kernel<8, NBLK, Q81>), grid, block, 0, stream, static_cast<const uint8_t*>(W), X, C, M, N, nblk, relu); \
+        else hipLaunchKernelGGL((q8_linear_ll_any_kernel<16, NBLK, Q81>), grid, block, 0, stream, static_cast<const uint8_t*>(W), X, C, M, N, nblk, relu); \
+        break;
+    switch ((nblk + 1) & ~1) {
+        PPML_LLA(6) PPML_LLA(8) PPML_LLA(10) PPML_LLA(12) PPML_LLA(14) PPML_LLA(16)
+    }
+#undef PPML_LLA
+    return check_launch("q8_linear_ll_any_kernel");
+}
+
 // Shape gate of the low-latency kernel; returns -1 when the weight-stationary kernel (or the general one)
 // should take the call.  `force` = 8 or 16 picks that unit size whatever the gate says (measurements).
 template <bool Q81>
@@ -1570,6 +1612,10 @@ int try_q8_linear_ll(const void* W, const float* X, float* C, int M, int N, int 
     if (!c_trans) return -1;
     const int mct = (M + 31) / 32;
     const int cpw = nblk == 16 ? 1 : nblk == 8 ? 2 : nblk == 4 ? 4 : 0;
+    if (force == 0 && !xq_dump && !sums_dump) {
+        const int rc = try_q8_linear_ll_any<Q81>(W, X, C, M, N, nblk, c_trans, relu, stream);
+        if (rc >= 0) return rc;
+    }
     if (cpw == 0 || mct > 4 * cpw) return -1;          // the wave's share of the weight must fit 64 registers
     int tok = force;
     if (tok == 0) {
@@ -1686,22 +1732,22 @@ constexpr uint32_t QT_OUTSIDE = 0x80000000u;               // an offset no buffe
 // One wave per (token tile, its upper or lower sixteen tokens, block): four lanes hold a block in element order.
 template <bool Q81>
 __global__ __launch_bounds__(256) void q8_quantize_fragments_kernel(const float* __restrict__ X, uint8_t* __restrict__ xq,
-                                                                    uint16_t* __restrict__ xd, int N, int nblk, int relu, int total_waves) {
+                                                                    uint16_t* __restrict__ xd, int N, int nblk, int nblk_pad, int relu, int total_waves) {
     const int lane = threadIdx.x & 63;
     const int gw = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x >> 6));
     if (gw >= total_waves) return;                      // wave-uniform
-    const int b = gw % nblk, rest = gw / nblk;
+    const int b = gw % nblk_pad, rest = gw / nblk_pad;
     const int half = rest & 1, tile = rest >> 1;
     const int c4 = lane & 3, r = half * 16 + (lane >> 2);
     const int row = tile * 32 + r;
     v4f x0 = {0.f, 0.f, 0.f, 0.f}, x1 = {0.f, 0.f, 0.f, 0.f};
-    if (row < N) {
+    if (row < N && b < nblk) {
         const float* src = X + (static_cast<int64_t>(row) * nblk + b) * QK + c4 * 8;
         x0 = *reinterpret_cast<const v4f_u*>(src);
         x1 = *reinterpret_cast<const v4f_u*>(src + 4);
     }
     const BlockQuant bq = (relu & 1) ? quantize_block_lane<Q81, true>(x0, x1) : quantize_block_lane<Q81, false>(x0, x1);
-    const size_t frag = static_cast<size_t>(tile) * nblk + b;
+    const size_t frag = static_cast<size_t>(tile) * nblk_pad + b;
     *reinterpret_cast<uint2*>(xq + (frag << 10) + (((c4 >> 1) * 32 + r) << 4) + ((c4 & 1) << 3)) = uint2{bq.q_lo, bq.q_hi};
     if (c4 == 0) xd[frag * 32 + r] = bq.d_bits;
 }
@@ -1730,24 +1776,25 @@ __global__ __launch_bounds__(512) void q8_tiled_kernel(const uint8_t* __restrict
         tile_c = t / rows_here;
     }
     const int tt0 = tile_t * QT_TOK_TILES, ct0 = tile_c * T::COL_TILES;
-    const int stages = nblk / 2;
+    // stages are pairs of blocks; behind an odd number of them the activations hold a block of zeros with scale zero
+    const int stages = (nblk + 1) / 2, nblk_pad = 2 * stages;
 
-    const __amdgpu_buffer_rsrc_t rsrc_xq = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(xq), 0, ntt_pad * nblk * 1024, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsrc_xd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xd), 0, ntt_pad * nblk * 64, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_xq = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(xq), 0, ntt_pad * nblk_pad * 1024, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_xd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xd), 0, ntt_pad * nblk_pad * 64, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_wq = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(W), 0, mct_pad * nblk * 1024, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_wd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(W) + static_cast<size_t>(mct_pad) * nblk * 1024, 0,
                                                                              mct_pad * nblk * 64, 0x00020000);
     // this thread's shares of a stage (the two blocks of a pair lie side by side in memory: 2 KB of fragments, 128
     // bytes of scales per tile).  Column tiles past the weight's padded end repeat the last one; never stored.
     const auto col_tile = [&](int c) { return c < mct_pad ? c : mct_pad - 1; };
-    uint32_t a_off = static_cast<uint32_t>((tt0 + (tid >> 7)) * nblk) * 1024u + static_cast<uint32_t>(tid & 127) * 16u;
+    uint32_t a_off = static_cast<uint32_t>((tt0 + (tid >> 7)) * nblk_pad) * 1024u + static_cast<uint32_t>(tid & 127) * 16u;
     uint32_t w_off[TJ];
 #pragma unroll
     for (int i = 0; i < TJ; ++i) w_off[i] = static_cast<uint32_t>(col_tile(ct0 + (tid >> 7) + 4 * i) * nblk) * 1024u + static_cast<uint32_t>(tid & 127) * 16u;
     // scales: threads 0..31 the activations' (four tiles x 128 bytes), threads 64 .. 63 + 32 TJ the weight's (128 bytes
     // per column tile); the others request nothing (an offset outside), so every wave counts the same loads
     const bool dw_thread = tid >= 64 && tid < 64 + 32 * TJ;
-    uint32_t da_off = tid < 32 ? static_cast<uint32_t>((tt0 + (tid >> 3)) * nblk) * 64u + static_cast<uint32_t>(tid & 7) * 16u : QT_OUTSIDE;
+    uint32_t da_off = tid < 32 ? static_cast<uint32_t>((tt0 + (tid >> 3)) * nblk_pad) * 64u + static_cast<uint32_t>(tid & 7) * 16u : QT_OUTSIDE;
     uint32_t dw_off = dw_thread ? static_cast<uint32_t>(col_tile(ct0 + ((tid - 64) >> 3)) * nblk) * 64u + static_cast<uint32_t>(tid & 7) * 16u
                                                : QT_OUTSIDE;
     v4i ra, rw[TJ], rda, rdw;
@@ -1758,7 +1805,10 @@ __global__ __launch_bounds__(512) void q8_tiled_kernel(const uint8_t* __restrict
 #pragma unroll
         for (int i = 0; i < TJ; ++i) rw[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_wq, live ? w_off[i] + fo : QT_OUTSIDE, 0, 0));
         rda = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_xd, (live && tid < 32) ? da_off + so : QT_OUTSIDE, 0, 0));
-        rdw = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_wd, (live && dw_thread) ? dw_off + so : QT_OUTSIDE, 0, 0));
+        // (the scales of a block that is not there are zeros too, so that whatever lies behind the tile's last block -- the
+        // next tile's first one -- meets nothing but zeros)
+        const bool dw_there = dw_thread && 2 * s + ((tid >> 2) & 1) < nblk;
+        rdw = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_wd, (live && dw_there) ? dw_off + so : QT_OUTSIDE, 0, 0));
     };
     const auto deposit = [&](uint8_t* stage) {
         *reinterpret_cast<v4i*>(stage + tid * 16) = ra;
@@ -1900,7 +1950,19 @@ __global__ __launch_bounds__(512) void q8_tiled_kernel(const uint8_t* __restrict
 // 4096 in 10 us, against the 700 us that the general kernel loses on such a weight).
 template <bool Q81>
 int try_q8_tiled(const void* W, int wtype, const float* X, float* C, int M, int N, int nblk, int c_trans, int relu, hipStream_t stream) {
-    if (nblk % 2 != 0) return -1;                       // stages are pairs of blocks
+    const int nblk_pad = (nblk + 1) & ~1;               // stages are pairs of blocks
+    // An odd number of blocks wastes half a stage; the general kernel keeps what it is measured to do as well or better
+    // (us, general / this one): three blocks below 512 features, 26368 x 96 -> 128  8.9 / 9.5 (from there on 10.7 / 7.8 at
+    // 5000 x 96 -> 768); up to eight blocks of up to 128 features, where the quantized copy of the activations is most of
+    // the traffic, 26368 x 160 -> 128  10.6 / 11.6, 26368 x 192 -> 64  9.1 / 11.1; middling widths of many tokens, whose
+    // last round of tiles is thin, 26368 x 480 -> 320  32.1 / 34.3 (2601 x 480 -> 768  21.3 / 12.2, 10609 x 288 -> 320
+    // 14.6 / 11.8, 26368 x 480 -> 128  23.8 / 20.5 for the others).  Beyond 31 blocks odd numbers stay with the general one.
+    if (nblk % 2 != 0 && nblk > 31) return -1;
+    if (wtype == PPML_WTYPE_Q8_0M) {
+        if (nblk == 3 && M < 512) return -1;
+        if (nblk >= 5 && nblk <= (M <= 64 ? 9 : 8) && M <= 128) return -1;
+        if (nblk % 2 != 0 && N > 16384 && M > 128 && M < 768) return -1;
+    }
     const int ntt = (N + 31) / 32, ntt_pad = (ntt + QT_TOK_TILES - 1) / QT_TOK_TILES * QT_TOK_TILES;
     const int mct = (M + 31) / 32, mct_pad = packed_tiles(M);
     const int tiles_t = ntt_pad / QT_TOK_TILES;
@@ -1922,7 +1984,7 @@ int try_q8_tiled(const void* W, int wtype, const float* X, float* C, int M, int 
     // 116 / 108.
     if (M < 64 || static_cast<int64_t>(tiles_t) * tiles_c < 16) return -1;
     // 32-bit byte offsets everywhere: the fragments of both operands and C with the rows of its last, ragged tile
-    const int64_t xq_bytes = static_cast<int64_t>(ntt_pad) * nblk * 1024, xd_bytes = static_cast<int64_t>(ntt_pad) * nblk * 64;
+    const int64_t xq_bytes = static_cast<int64_t>(ntt_pad) * nblk_pad * 1024, xd_bytes = static_cast<int64_t>(ntt_pad) * nblk_pad * 64;
     const int64_t wq_bytes = static_cast<int64_t>(mct_pad) * nblk * 1024;
     const int64_t c_reach = c_trans ? static_cast<int64_t>(ntt_pad * 32 + 4) * M * 4 : static_cast<int64_t>(tiles_c * ctiles * 32 + 4) * N * 4;
     if (xq_bytes >= 0x7fff0000LL || wq_bytes >= 0x7fff0000LL || c_reach >= 0x7fff0000LL) return -1;
@@ -1938,9 +2000,9 @@ int try_q8_tiled(const void* W, int wtype, const float* X, float* C, int M, int 
         rc = q8_weight_pack_hip(W, wtype, M, nblk * QK, wp, stream);
         W = wp;
     }
-    const int total_waves = ntt_pad * 2 * nblk;
+    const int total_waves = ntt_pad * 2 * nblk_pad;
     if (rc == RC_OK) {
-        hipLaunchKernelGGL((q8_quantize_fragments_kernel<Q81>), dim3((total_waves + 3) / 4), dim3(256), 0, stream, X, xq, xd, N, nblk, relu, total_waves);
+        hipLaunchKernelGGL((q8_quantize_fragments_kernel<Q81>), dim3((total_waves + 3) / 4), dim3(256), 0, stream, X, xq, xd, N, nblk, nblk_pad, relu, total_waves);
         rc = check_launch("q8_quantize_fragments_kernel");
     }
     if (rc == RC_OK) {
@@ -2019,27 +2081,45 @@ extern "C" int mul_mat_q8_ex_hip(const void* W, const float* X, float* C, int M,
     };
     // A weight in one of the reference's own layouts (include/ppml/QuantBlocks.h:33-41, 123-133) need not wait for its
     // owner to adopt the packed one.  Beyond what stays resident it takes the tiled kernel, which packs it into its
-    // workspace on the way.  Up to that size it is packed into the stream's workspace here (one launch: 3.7 us more
+    // workspace on the way.  Up to that size it is packed into the stream's workspace here (one launch: 2 to 4 us more
     // than the call on a packed weight) and served by the kernels of the packed layout, wherever that launch costs less
-    // than the general kernel loses: from 2^27 products on, and for weights of 64 Ki elements with K >= 512 or 768
+    // than the general kernel loses: from 2^27 products on, and for K >= 512 or weights of 64 Ki elements with 768
     // features whatever the token count.  us on a Q8_0 weight, general kernel / this way: 26368 x 256 -> 768  60 / 22.9
     // (20.8 on a weight packed at load), 26368 x 256 -> 256  26.8 / 12.3, 105472 x 64 -> 256  39.6 / 21.9, 10609 x 64 ->
-    // 256  8.1 / 7.1, 2601 x 256 -> 256  8.4 / 7.0, 64 x 512 -> 128  14.0 / 7.8, 128 x 256 -> 768  16.7 / 9.8; below the
-    // rule: 5000 x 64 -> 256  5.5 / 6.9, 26368 x 64 -> 64  6.6 / 7.2, 1024 x 128 -> 128  5.6 / 7.8.  No workspace (a stream
-    // under capture): the general kernel, as before.
+    // 256  8.1 / 7.1, 2601 x 256 -> 256  8.4 / 7.0, 64 x 512 -> 128  14.0 / 6.3, 51 x 512 -> 12  13.5 / 6.2, 128 x 256 -> 768  16.7 / 9.8; below the
+    // rule: 5000 x 64 -> 256  5.5 / 6.9, 26368 x 64 -> 64  6.6 / 7.2, 1024 x 128 -> 128  5.6 / 7.8.
+    // Where no such kernel has an instance nothing is packed for it.  The numbers of blocks that the low-latency kernel
+    // takes one tile per wave are packed for it from six blocks or 256 features on (us on a Q8_0 weight, general / this
+    // way: 408 x 288 -> 128  9.9 / 6.3, 51 x 480 -> 768  44.8 / 6.6, 408 x 192 -> 64  6.8 / 6.3; below: 51 x 160 -> 64  6.3 /
+    // 6.3); beyond its range the tiled kernel, whose workspace holds the packed weight, from 2^28 products of 512 features
+    // on and from 2^29 of more than 128 or more than eight blocks (2601 x 160 -> 768  15.8 / 9.9, 10609 x 480 -> 320  41.7 /
+    // 17.9, 26368 x 64 -> 768  28.6 / 22, 26368 x 480 -> 768  165.7 / 53.5; below: 5000 x 160 -> 320  10.4 / 10.2, 26368 x 192
+    // -> 128  14.0 / 14).
+    // No workspace (a stream under capture): the general kernel.
     if (wtype == PPML_WTYPE_Q8_0 || wtype == PPML_WTYPE_Q8_1 || wtype == PPML_WTYPE_Q8_0R) {
-        if (static_cast<int64_t>(M) * K > (256 << 10)) {
+        const int64_t weight = static_cast<int64_t>(M) * K, products = weight * N;
+        const bool large = weight > (256 << 10);
+        if (large) {
             const int rt = tiled();
             if (rt >= 0) return rt;
-        } else if ((static_cast<int64_t>(N) * M * K >= (1LL << 27) || (static_cast<int64_t>(M) * K >= (64 << 10) && (K >= 512 || M >= 768))) &&
-                   !xq_dump && !sums_dump &&
-                   (flags & (PPML_Q8_FLAG_NO_LOW_LATENCY | PPML_Q8_FLAG_NO_WEIGHT_STATIONARY)) != (PPML_Q8_FLAG_NO_LOW_LATENCY | PPML_Q8_FLAG_NO_WEIGHT_STATIONARY)) {
+        }
+        const int mct = (M + 31) / 32;
+        const bool instance = nblk == 4 || nblk == 8 || ((nblk == 2 || nblk == 16) && mct <= 8);
+        const int any_units = (flags & PPML_Q8_FLAG_NO_LOW_LATENCY) ? 0 : q8_ll_any_units(M, N, nblk, c_trans);
+        const bool pack = any_units ? nblk >= 6 || M >= 256
+                                    : instance && !large && (products >= (1LL << 27) || K >= 512 || (weight >= (64 << 10) && M >= 768));
+        if (pack && !xq_dump && !sums_dump &&
+            (flags & (PPML_Q8_FLAG_NO_LOW_LATENCY | PPML_Q8_FLAG_NO_WEIGHT_STATIONARY)) != (PPML_Q8_FLAG_NO_LOW_LATENCY | PPML_Q8_FLAG_NO_WEIGHT_STATIONARY)) {
             const Workspace held = workspace_take(q8_weight_packed_bytes_hip(M, K), s);
             if (held.ptr) {
                 const int rc = q8_weight_pack_hip(W, wtype, M, K, held.ptr, stream) == RC_OK ? resident_families(held.ptr) : -1;
                 workspace_give(held, s);
                 if (rc >= 0) return rc;
             }
+        }
+        if (!large && !any_units && !instance && nblk <= 16 && (M > 128 || nblk > 8) && products >= (M >= 512 ? 1LL << 28 : 1LL << 29)) {
+            const int rt = tiled();
+            if (rt >= 0) return rt;
         }
     }
     switch (wtype) {

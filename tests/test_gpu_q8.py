@@ -764,3 +764,38 @@ def test_fused_linear_with_q8_1_activations(ops, oracle, wname, N, K, M, c_trans
             assert ops.last_q8_path() == _FAMILY_PATH[fam]
             assert (y3 == want).all(), fam
     assert (ops.mul_mat_q8(W, _dev(x), c_trans=c_trans).cpu().numpy() != want).any()
+
+
+@pytest.mark.parametrize("N,K,M,want_path", [
+    (1, 160, 4, "low-latency"), (33, 480, 300, "low-latency"), (2049, 192, 130, "low-latency"),   # 5 and 15 blocks: the last pair is half empty
+    (120, 224, 256, "low-latency"), (77, 320, 100, "low-latency"), (409, 352, 64, "low-latency"),
+    (300, 416, 96, "low-latency"), (63, 448, 31, "low-latency"), (95, 512, 288, "low-latency"),   # 9 to 14 blocks; 16 where nothing else fits
+    (700, 96, 520, "tiled"), (3001, 288, 1000, "tiled"), (600, 992, 600, "tiled"),                # odd numbers of blocks: half a stage of zeros
+    (17000, 160, 96, "general")])
+def test_row_lengths_between_the_powers_of_two(ops, oracle, N, K, M, want_path):
+    """Every number of blocks has a kernel beside the general one; same block sums, same settlement, blocks ascending,
+    so the oracle's bits, whatever stands behind the last block of a row (here: scales that are not finite)."""
+    x, w = _inputs(5 * N + K + M, N, K, M)
+    x[N // 2, -32:] = 0.0
+    wq = oracle.quantize_q8_0(w).copy()
+    rows = wq.reshape(M, K // 32, 34)
+    rows[M // 2, 0, :2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)   # one row only: what follows its predecessor's last block
+    keep = np.arange(M) != M // 2
+    W = ops.Q8Weight(_dev(wq.reshape(-1)), M, K, ops.WTYPE_Q8_0)
+    Wp = W.pack()
+    for relu in (False, True):
+        xr = np.maximum(x, 0.0) if relu else x
+        want = oracle.mul_mat_q8(wq, xr, wtype=0, c_trans=1, fma=1)
+        got = ops.mul_mat_q8(Wp, _dev(x), relu=relu)
+        assert ops.last_q8_path() == want_path
+        assert (got.cpu().numpy()[:, keep] == want[:, keep]).all()
+        assert not np.isfinite(got.cpu().numpy()[:, ~keep]).all()
+        assert (ops.mul_mat_q8(Wp, _dev(x), relu=relu, c_trans=0).cpu().numpy().T[:, keep] == want[:, keep]).all()
+        for wtype, data in ((ops.WTYPE_Q8_0, wq.reshape(-1)), (ops.WTYPE_Q8_0R, oracle.repack_q8_0(wq))):
+            got = ops.mul_mat_q8(ops.Q8Weight(_dev(data), M, K, wtype), _dev(x), relu=relu).cpu().numpy()
+            assert (got[:, keep] == want[:, keep]).all(), wtype
+    got = ops.mul_mat_q8(Wp, _dev(x), act="q8_1").cpu().numpy()
+    assert (got[:, keep] == oracle.mul_mat_q8_act(wq, x, act=1, c_trans=1)[:, keep]).all()
+    buf = torch.full((N * M + 2048,), 7.5, device="cuda")
+    ops.mul_mat_q8(Wp, _dev(x), out=buf[1024:1024 + N * M].view(N, M))
+    assert (buf[:1024] == 7.5).all() and (buf[1024 + N * M:] == 7.5).all()
