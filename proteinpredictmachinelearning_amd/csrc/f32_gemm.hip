@@ -1785,12 +1785,16 @@ __global__ __launch_bounds__(256) void gemm_f16_kernel(const GemmParams p) {
 // store), and a CU holds two such work-groups.  Tiles go to the XCDs in eight contiguous ranges, inside a range in
 // bands of eight tile rows, so that the work-groups resident on an XCD at one time share operand panels in its L2.
 // Same fragments, same order of the products, zero start and bias last as in gemm_f16_kernel: same bits.
-// Conditions (the launcher's): K, both row pitches and both base addresses multiples of eight halves -- every load
-// is sixteen bytes that lie inside one row or entirely past K --, operands and the dense output each below 2 GiB
-// (buffer addressing: what lies outside reads as zero and is not stored), a grid that is a multiple of eight.
+// Conditions (the launcher's): operands and the dense output each below 2 GiB (buffer addressing: what lies outside
+// reads as zero and is not stored), a grid that is a multiple of eight.  Without ANY also K, both row pitches and both
+// base addresses multiples of eight halves: every load is sixteen bytes that lie inside one row or entirely past K.
+// ANY: rows may start on any half.  A piece comes as the five whole words around its sixteen bytes, shifted by the half
+// that its row is off, and what its last stage holds past K is cut off before it goes to LDS: 408 x 197 -> 256 24.0 -> 7.9
+// us, 10609 x 197 -> 256 24.5 -> 8.6, 26368 x 197 -> 1024 112.5 -> 35.4 against the form of one work-group per tile, whose
+// loads of single halves were waited for one after the other.
 constexpr int F16P_AHEAD = 2;    // (three measured the same or 0.5 us slower: a longer start and end per work-group)
 constexpr int F16P_STAGE = (BM + BN) * F16_PITCH;     // A's tile, then B's
-template <bool STREAM_C>
+template <bool STREAM_C, bool ANY>
 __global__ __launch_bounds__(512, 2) void gemm_f16_pc_kernel(const GemmParams p, int total_tiles) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[2][F16P_STAGE];
 
@@ -1818,10 +1822,14 @@ __global__ __launch_bounds__(512, 2) void gemm_f16_pc_kernel(const GemmParams p,
 
     // Both kinds of wave pass padded + 1 barriers: barrier g + 1 says "stage g is in LDS" and "stage g - 1 has been read".
     if (producer) {
+        // (ANY: from the word that the first half lies in to the end of the word that the last one lies in)
+        const uint32_t a_odd = ANY ? static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p.A) & 2) : 0;
+        const uint32_t b_odd = ANY ? static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p.B) & 2) : 0;
+        const int a_bytes = static_cast<int>(((p.M - 1) * p.a_rs + p.K) * 2 + a_odd), b_bytes = static_cast<int>(((p.N - 1) * p.b_rs + p.K) * 2 + b_odd);
         const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(p.A), 0, static_cast<int>(((p.M - 1) * p.a_rs + p.K) * 2), 0x00020000);
+            reinterpret_cast<uint8_t*>(const_cast<float*>(p.A)) - a_odd, 0, ANY ? (a_bytes + 3) & ~3 : a_bytes, 0x00020000);
         const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(p.B), 0, static_cast<int>(((p.N - 1) * p.b_rs + p.K) * 2), 0x00020000);
+            reinterpret_cast<uint8_t*>(const_cast<float*>(p.B)) - b_odd, 0, ANY ? (b_bytes + 3) & ~3 : b_bytes, 0x00020000);
         const uint32_t a_rs_bytes = static_cast<uint32_t>(p.a_rs) * 2u, b_rs_bytes = static_cast<uint32_t>(p.b_rs) * 2u;
         // a thread's share of a stage: rows ptid / 8 + 32 i of both tiles, eight halves from k = 8 (ptid % 8) on --
         // eight lanes read a row's 128 bytes
@@ -1829,23 +1837,39 @@ __global__ __launch_bounds__(512, 2) void gemm_f16_pc_kernel(const GemmParams p,
         const int prow = ptid >> 3, pk = (ptid & 7) * 8;
         const int put = prow * F16_PITCH + pk * 2;
         v4i ra[F16P_AHEAD][4], rb[F16P_AHEAD][4];
+        int ea[F16P_AHEAD][4], eb[F16P_AHEAD][4];       // ANY: the word behind each piece ...
+        uint32_t da[F16P_AHEAD], db[F16P_AHEAD];        // ... where the pieces start in their first words, a bit each ...
+        int left[F16P_AHEAD];                           // ... and how many halves from k on are inside the rows
         int it = 0, ic = 0, m0 = 0, n0 = 0;             // the next stage to request: tile `it` of mine, stage ic of it
         if (my_tiles > 0) tile_origin(first, m0, n0);
         // (Past the last stage a request asks for nothing -- every offset outside -- but is still made: the count of
         // loads in flight that the wait for a stage names is then the same in every iteration, and the compiler
         // waits for that stage alone -- vmcnt(15) .. vmcnt(8) for its eight loads; with requests under a condition
         // it waited for all of them.)
-        const auto request = [&](v4i (&xa)[4], v4i (&xb)[4]) {
+        const auto request = [&](int d) {
+            v4i (&xa)[4] = ra[d];
+            v4i (&xb)[4] = rb[d];
             const int k = ic * F16_BK + pk;
             const uint32_t kb = static_cast<uint32_t>(k) * 2u;
             const bool live = it < my_tiles && k < p.K;
+            if (ANY) { left[d] = p.K - k; da[d] = 0; db[d] = 0; }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int ar = m0 + prow + 32 * i, br = n0 + prow + 32 * i;
                 const uint32_t at = (live && ar < p.M) ? static_cast<uint32_t>(ar) * a_rs_bytes + kb : OUTSIDE;
                 const uint32_t bt = (live && br < p.N) ? static_cast<uint32_t>(br) * b_rs_bytes + kb : OUTSIDE;
-                xa[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, at, 0, 0));
-                xb[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, bt, 0, 0));
+                if (ANY) {
+                    const uint32_t ao = at + a_odd, bo = bt + b_odd;        // (OUTSIDE stays outside)
+                    da[d] |= (ao >> 1 & 1) << i;
+                    db[d] |= (bo >> 1 & 1) << i;
+                    xa[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, ao & ~3u, 0, 0));
+                    xb[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, bo & ~3u, 0, 0));
+                    ea[d][i] = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rsrc_a, (ao & ~3u) + 16u, 0, 0));
+                    eb[d][i] = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rsrc_b, (bo & ~3u) + 16u, 0, 0));
+                } else {
+                    xa[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, at, 0, 0));
+                    xb[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, bt, 0, 0));
+                }
             }
             if (++ic == chunks) {
                 ic = 0;
@@ -1853,7 +1877,19 @@ __global__ __launch_bounds__(512, 2) void gemm_f16_pc_kernel(const GemmParams p,
             }
         };
 #pragma unroll
-        for (int d = 0; d < F16P_AHEAD; ++d) { request(ra[d], rb[d]); __builtin_amdgcn_sched_barrier(0); }   // (in this order)
+        for (int d = 0; d < F16P_AHEAD; ++d) { request(d); __builtin_amdgcn_sched_barrier(0); }   // (in this order)
+        // the eight halves of a piece out of its five words, zeros past K
+        const auto piece = [&](const v4i& w, int e, uint32_t odd, int inside) {
+            if (!ANY) return w;
+            v4i v;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const uint32_t hi = static_cast<uint32_t>(c < 3 ? w[c < 3 ? c + 1 : 0] : e);
+                const uint32_t x = __builtin_amdgcn_alignbit(hi, static_cast<uint32_t>(w[c]), odd * 16);
+                v[c] = static_cast<int>(inside > 2 * c + 1 ? x : inside > 2 * c ? x & 0xffffu : 0u);
+            }
+            return v;
+        };
         // The register sets take turns by name: the loop body is written out F16P_AHEAD times, and runs whole -- the
         // stages past the last one move zeros, and the other waves pass their barriers (a way out of the middle of
         // the body joins the loop's back edge in the compiled code, and the wait at the loop's head then allows
@@ -1865,10 +1901,10 @@ __global__ __launch_bounds__(512, 2) void gemm_f16_pc_kernel(const GemmParams p,
                 uint8_t* half = lds[g & 1];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    *reinterpret_cast<v4i*>(half + put + i * 32 * F16_PITCH) = ra[d][i];
-                    *reinterpret_cast<v4i*>(half + BM * F16_PITCH + put + i * 32 * F16_PITCH) = rb[d][i];
+                    *reinterpret_cast<v4i*>(half + put + i * 32 * F16_PITCH) = piece(ra[d][i], ea[d][i], da[d] >> i & 1, left[d]);
+                    *reinterpret_cast<v4i*>(half + BM * F16_PITCH + put + i * 32 * F16_PITCH) = piece(rb[d][i], eb[d][i], db[d] >> i & 1, left[d]);
                 }
-                request(ra[d], rb[d]);
+                request(d);
                 __syncthreads();
             }
         }
@@ -2625,17 +2661,19 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
     }
     else {
         if (split || p.np2 * p.np3 != 1 || p.a_ks != 1 || p.b_ks != 1) { set_error("%s: no F16 instance for this addressing", what); return RC_BAD_ARGS; }
-        // the streaming form where every load is sixteen aligned bytes and 32-bit offsets reach everything
+        // the streaming form wherever 32-bit offsets reach everything
         const bool aligned8 = p.K % 8 == 0 && p.a_rs % 8 == 0 && p.b_rs % 8 == 0 &&
                               ((reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.B)) & 15) == 0;
         const bool in_reach = ((p.M - 1) * p.a_rs + p.K) * 2 < (1LL << 31) && ((p.N - 1) * p.b_rs + p.K) * 2 < (1LL << 31) &&
                               p.c_ni == 1 && p.M * p.c_mi * 4 < (1LL << 31) && p.c_mi < (1 << 22);
-        if (aligned8 && in_reach) {
+        if (in_reach) {
             const int64_t resident = 2LL * device_cu_count() / 8 * 8;      // two work-groups per CU (LDS: 72 KB each)
             const int64_t wgs = std::max<int64_t>(8, std::min<int64_t>((total + 7) / 8 * 8, resident));
             const dim3 pgrid(static_cast<unsigned>(wgs));
-            if (p.stream_c) hipLaunchKernelGGL((gemm_f16_pc_kernel<true>), pgrid, dim3(512), 0, stream, p, static_cast<int>(total));
-            else hipLaunchKernelGGL((gemm_f16_pc_kernel<false>), pgrid, dim3(512), 0, stream, p, static_cast<int>(total));
+#define PPML_F16PC(STREAM_, ANY_) hipLaunchKernelGGL((gemm_f16_pc_kernel<STREAM_, ANY_>), pgrid, dim3(512), 0, stream, p, static_cast<int>(total))
+            if (aligned8) { if (p.stream_c) PPML_F16PC(true, false); else PPML_F16PC(false, false); }
+            else          { if (p.stream_c) PPML_F16PC(true, true);  else PPML_F16PC(false, true); }
+#undef PPML_F16PC
         }
         else if (p.stream_c) hipLaunchKernelGGL((gemm_f16_kernel<true>), grid, block, 0, stream, p);
         else hipLaunchKernelGGL((gemm_f16_kernel<false>), grid, block, 0, stream, p);

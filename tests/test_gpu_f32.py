@@ -1173,3 +1173,22 @@ def test_linear_layers_with_few_output_features_take_narrow_tiles_with_the_same_
     bd, biasd = _dev(b), _dev(bias)
     assert ops._lib().mul_mat_hip(p(ad), p(bd), p(out), M, K, N, p(biasd), None) == 0
     assert torch.equal(out.view(torch.int32), got.view(torch.int32)) and (buf[:256] == 3.5).all() and (buf[256 + M * N:] == 3.5).all()
+
+
+@pytest.mark.parametrize("M,K,N,bias,at_a,at_b", [(130, 63, 129, True, 0, 0), (257, 65, 40, False, 1, 0), (40, 7, 9, True, 0, 1), (300, 129, 131, True, 1, 1),
+                                                  (70, 198, 33, False, 3, 2), (70000, 27, 12, True, 1, 1), (3, 1, 2, False, 1, 0)])
+def test_mul_mat_f16_rows_that_start_on_any_half(ops, oracle, M, K, N, bias, at_a, at_b):
+    """Any K at any address of a half: what lies around and between the rows (here NaN) has no part in the result."""
+    rng = np.random.default_rng(M + K + N)
+    a = rng.integers(-8, 9, size=(M, K)).astype(np.float16)       # sums of integers below 2^24: exact in any order
+    b = rng.integers(-8, 9, size=(N, K)).astype(np.float16)
+    bv = rng.integers(-4, 5, size=N).astype(np.float32) if bias else None
+
+    def among_nans(x, at):
+        flat = torch.full((x.size + at + 8,), float("nan"), dtype=torch.float16, device="cuda")
+        view = flat[at:at + x.size].view(x.shape)
+        view.copy_(_dev(x))
+        return view
+
+    got = ops.mul_mat_f16(among_nans(a, at_a), among_nans(b, at_b), None if bv is None else _dev(bv)).cpu().numpy()
+    assert (got == oracle.mul_mat_f16(a, b, bv)).all()
