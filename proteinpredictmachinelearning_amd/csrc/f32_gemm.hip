@@ -2575,7 +2575,12 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
                             p.M * p.c_mi * 4 < (1LL << 31) && p.c_mi < (1 << 22) && p.a_rs < (1 << 22) && p.b_rs < (1 << 22);
         // few tiles under a long K (a LinearLayer's weight gradient) go in K slices, whatever their width
         if (k_fast && !fixed_ws && try_pc_slices_done<LOAD_K_CONTIG>(p, stream, what, slices_rc)) return slices_rc;
-        if (k_fast && p.K > 3 * BK && (p.N <= 32 || p.M <= 32)) {
+        // (a narrow side of a single plane too, while 64 x 64 tiles leave CUs idle: half of such a tile is empty, but two chunks
+        // a barrier make its chain shorter.  us, 128 x 32 / 64 x 64: 51 x 256 -> 8  9.4 / 6.6, 10609 x 256 -> 12
+        // 9.8 / 7.2, 16384 x 376 -> 32  13.1 / 9.8; two tiles per CU, 26368 x 256 -> 8  9.9 / 10.1)
+        const int64_t tiles64 = static_cast<int64_t>((p.M + 63) / 64) * ((p.N + 63) / 64);
+        const bool pc64 = k_fast && p.K > 3 * BK && p.np2 * p.np3 == 1 && tiles64 <= (p.M > 32 && p.N > 32 ? 2 : 1) * device_cu_count();
+        if (k_fast && !pc64 && p.K > 3 * BK && (p.N <= 32 || p.M <= 32)) {
             // one narrow side: tiles of 128 x 32 along the other (gemm_bf16x3_pc_narrow_kernel)
             const bool side_n = p.N <= 32;
             const int64_t tiles_long = side_n ? p.tiles_m : p.tiles_n;
@@ -2591,8 +2596,8 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
 #undef PPML_KNARROW_K4
 #undef PPML_KNARROW
         }
-        else if (k_fast && p.K > 3 * BK && p.np2 * p.np3 == 1 && p.M > 32 && p.N > 32 && (static_cast<int64_t>((p.M + 63) / 64) * ((p.N + 63) / 64) <= 2 * device_cu_count())) {
-            const dim3 g64(static_cast<unsigned>((p.M + 63) / 64 * ((p.N + 63) / 64)));
+        else if (pc64) {
+            const dim3 g64(static_cast<unsigned>(tiles64));
 #define PPML_KPC64(STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_pc64_kernel<STREAM_, K4_>), g64, dim3(512), 0, stream, p)
             if (p.K % 4 == 0) { if (p.stream_c) PPML_KPC64(true, true); else PPML_KPC64(false, true); }
             else              { if (p.stream_c) PPML_KPC64(true, false); else PPML_KPC64(false, false); }

@@ -39,3 +39,16 @@ def test_small_linear(ops, M, N, K):
         hot = ops.mul_mat(a, b, bias)
         assert torch.equal(hot.isinf(), (a.double() @ b.double().t()).isinf())
         assert torch.equal(hot[:(M - 1) // 64 * 64, :(N - 1) // 64 * 64], got[:(M - 1) // 64 * 64, :(N - 1) // 64 * 64])
+
+
+@pytest.mark.parametrize("M,N", [(1, 1), (51, 8), (63, 32), (16384, 12), (7, 2601), (32, 16384)])
+@pytest.mark.parametrize("K", [49, 64, 101, 256])
+def test_small_linear_with_a_narrow_side(ops, M, N, K):
+    """Up to 32 rows or columns, one 64 x 64 tile per CU at most: the bits of the form with tiles of 128 x 32, which takes
+    the same rows as part of more of them."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    rows, cols = (40000, N) if N <= 32 else (M, 40000)
+    a, b = torch.randn(rows, K, device="cuda", generator=g), torch.randn(cols, K, device="cuda", generator=g)
+    bias = torch.randn(cols, device="cuda", generator=g)
+    got = ops.mul_mat(a[:M].contiguous(), b[:N].contiguous(), bias[:N].contiguous())
+    assert torch.equal(got, ops.mul_mat(a, b, bias)[:M, :N])
