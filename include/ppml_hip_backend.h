@@ -81,7 +81,10 @@ void ppml_hip_backend_set_fuse_attention_chain(ppml_hip_backend *b, int on);
  *     softmax kernel's way in; same bits.
  *   permutes_into_out_prod (default 1): an OP_OUT_PROD whose operands are both {1,0,2,3} permutations nobody else
  *     reads (src/modules/Attention.cpp:277-281) contracts the unpermuted tensors over their innermost dimension;
- *     same bits, two copies less. */
+ *     same bits, two copies less.
+ *   With these two and scale_into_out_prod on, the whole attention chain above of planes of up to 128 rows (heads of up
+ *     to 32, 32 planes or more, the default arithmetic) runs as one launch where nobody else reads an intermediate: the
+ *     bits of the launches it stands for. */
 void ppml_hip_backend_set_fuse_add_into_soft_max(ppml_hip_backend *b, int on);
 void ppml_hip_backend_set_fuse_permutes_into_out_prod(ppml_hip_backend *b, int on);
 /*   permutes_into_mul_mat (default 1): an F32 OP_MUL_MAT without bias whose operands are both matrix transpositions
