@@ -310,13 +310,16 @@ def main() -> int:
             if rest["skip"]:
                 return
             # pipe: "fp32" = fp32 MFMA; "bf16x3" = binary32 operands split three ways, six bf16 MFMA
-            # products per binary32 product (TFLOPS counts binary32 products, the fraction bf16 ones)
+            # products per binary32 product (TFLOPS counts binary32 products, the fraction bf16 ones); "f16x2" =
+            # large contractions, operands in two scaled halves, three f16 MFMA products per binary32 product
             fn_, ns = make()
             w_, e_ = time_op(fn_, ns, steps, warm)
             extra[name] = {"us": round(e_ * 1e6, 2), "TFLOPS": round(flops / e_ / 1e12, 2),
                            "GBps": round(nbytes / e_ / 1e9, 1), "hbm_frac": round(nbytes / e_ / 1e9 / HBM_PEAK_GBS, 4)}
             if pipe == "bf16x3":
                 extra[name]["bf16_mfma_frac"] = round(6.0 * flops / e_ / 1e12 / BF16_MFMA_PEAK_TFLOPS, 4)
+            elif pipe == "f16x2":
+                extra[name]["f16_mfma_frac"] = round(3.0 * flops / e_ / 1e12 / BF16_MFMA_PEAK_TFLOPS, 4)
             elif pipe == "f16":                         # halves straight to the matrix pipe (same published peak as bf16)
                 extra[name]["f16_mfma_frac"] = round(flops / e_ / 1e12 / BF16_MFMA_PEAK_TFLOPS, 4)
             else:
@@ -483,14 +486,14 @@ def main() -> int:
                             2.0 * rows_sample * 12288 * 256, "TFLOPS",
                             f"{rows_sample} of the 12288 output rows x all 12288 columns x K = 256 (1/16 of the workload)")
         steps, warm = 50, 10
-        f32_case(opm, (2 * 256 * 12288 + 12288 * 12288) * 4, 2.0 * 12288 * 12288 * 256, "opm_dense_12288x256x12288", pipe="bf16x3",
+        f32_case(opm, (2 * 256 * 12288 + 12288 * 12288) * 4, 2.0 * 12288 * 12288 * 256, "opm_dense_12288x256x12288", pipe="f16x2",
                  cpu=opm_cpu)
 
         def dense():
             a = torch.randn(4096, 4096, device=dev, generator=gen)
             b = torch.randn(4096, 4096, device=dev, generator=gen)
             return (lambda i: ops.mul_mat(a, b)), 1
-        f32_case(dense, 3 * 4096 * 4096 * 4, 2.0 * 4096 ** 3, "mul_mat_f32_4096x4096x4096", pipe="bf16x3")
+        f32_case(dense, 3 * 4096 * 4096 * 4, 2.0 * 4096 ** 3, "mul_mat_f32_4096x4096x4096", pipe="f16x2")
 
         # the same two contractions on the fp32 matrix pipe (the library's other arithmetic for binary32 operands)
         ops.set_f32_arithmetic("fp32")
@@ -512,7 +515,7 @@ def main() -> int:
             return (lambda i: ops.outer_prod_mean_back(grad, left, right, Dc, Lc, Nc, 1)), 1
         steps, warm = 20, 5
         f32_case(opm_back, (2 * 12288 * 12288 + 4 * 12288 * 256) * 4, 4.0 * 12288 * 12288 * 256,
-                 "opm_backward_D32_L384_N256", pipe="bf16x3")
+                 "opm_backward_D32_L384_N256", pipe="f16x2")
 
         def weight_grad():
             # dW = X^T dY of the headline projection's f32 twin (src/core/ComputeGraph.cpp:708-773): 256 x 768 outputs,
@@ -524,7 +527,7 @@ def main() -> int:
             return (lambda i: ops.mul_mat_tn(xs[i], dys[i])), ns
         steps, warm = 50, 10
         f32_case(weight_grad, (26368 * 256 + 26368 * 768 + 256 * 768) * 4, 2.0 * 26368 * 256 * 768,
-                 "linear_weight_gradient_26368x256_768", pipe="bf16x3")
+                 "linear_weight_gradient_26368x256_768", pipe="f16x2")
 
         def f16_linear():
             # the headline projection with both operands in halves (F16 x F16 -> F32, src/backend/CPUKernels.cpp:646-672)
