@@ -639,12 +639,14 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     //     split of the other operand weighs more: 464 x 12651 x 392 (49) 42 / 43, 564 x 26377 x 197 (64) 51 / 52;
     //   * otherwise, from more than a tile per CU on (2601 x 512 -> 1024, 168 tiles, 22.4 / 33.4, 10609 x 448 -> 288, 249 tiles, 22.5
     //     / 25.0, 10609 x 328 -> 420, 332 tiles, 28.9 / 26.8): 10609 x 176 -> 532 (15) 20 / 21, 26368 x 256 -> 256 (26) 25 / 21, 26368 x 512 -> 1024 (206) 189 / 101.
+    //     a tile of few stages has less to hide the split ahead behind: 20000 x 197 -> 400 (23) 31.5 / 35.7, 9040 x 221 -> 832 (25)
+    //     25.8 / 28.1, 12000 x 223 -> 800 (32) 32.7 / 34.2, 26368 x 223 -> 512 (45) 47.1 / 39.2; 9040 x 333 -> 600 (27) 34.4 / 29.7.
     // A K below 128 stays with the form that splits in the tile loop at any size (the bits of a contraction that is cut
     // out of a larger one then do not depend on the size).
     if (p.a_lm > 0) { if (load < 22) return -1; }
     else if (compound) { if (load < 30) return -1; }
     else if (sliced) { if (load < 42 || (p.M < 700 && load < 66) || p.K < 128) return -1; }
-    else if (p.K < 128 || tiles128 <= cus || static_cast<double>(p.M) * p.N * p.K < 20.0 * 128 * 128 * 16 * cus) return -1;      // (without the padding: 30001 x 131 -> 260 25.8 / 29.7)
+    else if (p.K < 128 || tiles128 <= cus || static_cast<double>(p.M) * p.N * p.K < (p.K < 256 ? 40.0 : 20.0) * 128 * 128 * 16 * cus) return -1;      // (without the padding: 30001 x 131 -> 260 25.8 / 29.7)
     // Tiles of 128 x 256 by one work-group per CU, or of 128 x 128 by two, which store while the other contracts but read A
     // twice as often: where 256 columns would be half empty, where the wide tiles' last round leaves more than half of the CUs idle (26368 x 256 -> 768: 51.4
     // / 48.8 us; 32768 x 512 -> 1024, whole rounds, 110 / 118), and for compound rows that are not whole lines, whose stores
