@@ -52,7 +52,7 @@ const char *ppml_hip_last_error(void);
 /* ---- f32 GEMM ------------------------------------------------------------------------------ */
 /* Which matrix pipe multiplies binary32 operands in the f32 contractions below: 0 (default) = the bf16 pipe
  * through an exact three-way split of every operand (binary32-grade results, about 1.5 times the speed; large
- * contractions on the f16 pipe through two scaled halves, closer still and faster),
+ * contractions on the f16 pipe through two scaled halves, faster still, see mul_mat_hip),
  * 1 = the fp32 pipe (v_mfma_f32_32x32x2_f32, k ascending two at a time).  The environment variable
  * PPML_HIP_F32_ARITH=fp32 selects 1 before the first call.  Returns the previous setting; other values of
  * `mode` only query.  The setting belongs to the calling thread (threads that want different arithmetic do
@@ -63,8 +63,11 @@ int ppml_hip_set_f32_arithmetic(int mode);
  * C[m*N+n] = (bias ? bias[n] : 0) + sum_k A[m*K+k] * B[n*K+k].  bias may be NULL.
  * Arithmetic of this and the other f32 contractions below: each binary32 operand is the exact sum of
  * three bf16 numbers; six of the nine partial products (all but 2^-23 of |a||b|) are formed exactly on
- * the bf16 matrix pipe and summed in binary32.  (Large contractions: two halves per operand under a power of two per
- * row, three exact products on the f16 pipe, an error half as large.)  Two kinds of operand fall outside what three bf16 parts
+ * the bf16 matrix pipe and summed in binary32.  Large contractions: two halves per operand under a power of two per
+ * row, three exact products on the f16 pipe; all but 2^-21 of |a||b| at worst (operands of one constant each), with
+ * half the exact split's error on random operands.  Outputs to which a row's elements far below its largest one (2^-14 of
+ * it and less) might matter beyond that -- the large ones meet zeros -- are found and computed again by the exact split, at a
+ * third of its speed where they are all of that kind.  Two kinds of operand fall outside what three bf16 parts
  * carry: a non-finite one, and one with bits below 2^-133, bf16's smallest step (subnormal operands and the
  * smallest normal ones).  The kernels notice both while they split the operands and redo the outputs of the
  * affected tile in plain binary32 arithmetic, one product at a time with k ascending (the reference's own

@@ -30,16 +30,6 @@ struct ChainParams {
     int pitch;           // floats per row of scores in LDS
 };
 
-// eight elements as a fragment's three parts
-__device__ __forceinline__ void split8(const v4f (&x)[2], v8bf (&out)[3], SplitGuard& guard) {
-    uint2 lo[3], hi[3];
-    split4(x[0], lo, guard);
-    split4(x[1], hi, guard);
-#pragma unroll
-    for (int s = 0; s < 3; ++s)
-        out[s] = __builtin_bit_cast(v8bf, v4i{static_cast<int>(lo[s].x), static_cast<int>(lo[s].y), static_cast<int>(hi[s].x), static_cast<int>(hi[s].y)});
-}
-
 // VEC: rows of whole 16-byte pieces (L a multiple of four), four elements per lane; otherwise PIECES single ones
 template <bool VEC, int PIECES, bool HAS_BIAS>
 __global__ __launch_bounds__(512, 4) void attention_chain_kernel(const ChainParams p) {

@@ -135,6 +135,16 @@ __device__ __forceinline__ void split4(const v4f& v, uint2 (&out)[3], SplitGuard
 #endif
 }
 
+// eight elements as a fragment's three parts
+__device__ __forceinline__ void split8(const v4f (&x)[2], v8bf (&out)[3], SplitGuard& guard) {
+    uint2 lo[3], hi[3];
+    split4(x[0], lo, guard);
+    split4(x[1], hi, guard);
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+        out[s] = __builtin_bit_cast(v8bf, v4i{static_cast<int>(lo[s].x), static_cast<int>(lo[s].y), static_cast<int>(hi[s].x), static_cast<int>(hi[s].y)});
+}
+
 // op over all 64 lanes, with the partners of a butterfly over lane ^ 32, 16, 8, 4, 2, 1 -- and so its bits, for a commutative
 // op.  No step goes through LDS: the halves and the rows of sixteen lanes change places by v_permlane32_swap / 16_swap (both
 // operands the value: one comes back as the even halves or rows twice over, the other as the odd ones), within a row the

@@ -1,15 +1,25 @@
 // Large binary32 contractions on the f16 matrix pipe.
 //
-// A binary32 number times a power of two that brings the largest element of its row near 2^12 .. 2^15 is, to within 2^-24
-// of itself, the sum of two halves: h = f16(x), l = f16(x - h), eleven significant bits each with the sign of l for one
-// more.  Three products -- h h, h l, l h -- are kept (l l lies below 2^-24 of |a||b|); the matrix pipe forms each exactly
-// and adds it into a binary32 accumulator, and the powers of two leave again by ldexp, exactly.  Against the exact split into three
-// bf16 parts with its six products (gemm_bf16x3_kernel) that is half the matrix work, a third less LDS traffic and less
-// than half the vector work (two v_fma_mixlo/hi per element); and, with half as many additions into the accumulator, half
-// the error.  What it asks for is the scale: a half has five bits of exponent.  One power of two per ROW of either operand
-// and K slice -- not per operand, whose rows may differ by anything -- keeps every element above 2^-17 of its row's largest
-// whole, and smaller ones to 2^-40 of that largest: an error of 2^-40 max_k|a| sum_k|b| at most, far below the binary32
-// rounding of the sum unless the row's largest elements meet only zeros.
+// A binary32 number times a power of two that brings the largest element of its row near 2^12 .. 2^15 is the sum of two
+// halves, h = f16(x), l = f16(x - h), to within 2^-23 of itself.  Three products -- h h, h l, l h -- are kept (l l lies below
+// 2^-22 of |a||b|); the matrix pipe forms each exactly and adds it into a binary32 accumulator, and the powers of two leave
+// again by ldexp, exactly.  Together: 2^-21 of |a||b| at worst, for operands of one constant each; random ones measure half the error
+// of the exact split into three bf16 parts with its six products (gemm_bf16x3_kernel), whose sums take twice as many
+// additions.  Against that form it is half the matrix work, a third less LDS traffic and less than half the vector work (two
+// v_fma_mixlo/hi per element).
+//
+// What it asks for is the scale: a half has five bits of exponent.  One power of two per ROW of either operand and K slice -- not
+// per operand, whose rows may differ by anything -- carries what lies within 2^-14 (A) or 2^-16 (B) of its row's largest
+// element.  A smaller one, below 2^-2 once scaled, is kept to a fixed 2^-25 instead of a share of itself, which is as good as lost where the
+// row's large elements meet zeros (an outlier against a zero weight, a spike of a gradient against a token that a mask made
+// zero).  So those elements are counted, n per row of A and c per row of B: what they cost an output is at most (n + c) 2^-10 in scaled
+// units (the partner lies below 2^15).  An output that is not 2^21 times that -- so that it could lose more than the 2^-21 above
+// -- is computed again, with the tile of 32 x 32 that it lies in, by the exact split (redo_tiles).  The test is against the output itself, or
+// against what its sum was halfway through K: neither is larger than sum |a||b|, so no output gets past it by luck.  Of
+// normal operands one lane in 2^11 fails with one of the two, next to none with both, and the test costs a minimum over the
+// accumulators: 384 residues x 32 features x 256 sequences 292 -> 295 us forward, 512 -> 519 backward, 103 residues 78.6 -> 84.6
+// backward, 26368 x 256 -> 768 52.2 -> 53.  Operands of wide range throughout are contracted twice: 12288 x 256 x 12288 with
+// spikes of 10^9 in one column or log-normal with sigma 3 1.5 ms (0.47 by the exact split alone), 26368 x 256 -> 768 0.29.
 //
 // B (the smaller operand as a rule: a weight, an alignment's projection) is split ahead by split_f16x2_kernel, which sees a
 // whole row of the slice and knows its maximum.  A is split in the tile loop by the loading waves, whose scale
@@ -17,9 +27,8 @@
 // and leaves a factor by which the contracting waves multiply what they hold (a branch that is taken once in a row's life
 // as a rule).
 //
-// What no power of two can bring into range -- infinities, NaN, rows whose largest element lies below 2^-111 -- is noticed
-// with the maxima (v_maximum3_f32 passes NaN on), and the outputs concerned are redone in plain binary32 arithmetic, one
-// product at a time (plain_dot), as everywhere in this library.
+// Infinities and NaN are noticed with the maxima (v_maximum3_f32 passes NaN on), and the outputs concerned are redone in plain
+// binary32 arithmetic, one product at a time (plain_dot), as everywhere in this library.
 #include "gemm.hpp"
 #include "split.hpp"
 
@@ -36,15 +45,22 @@ constexpr int HX_HALF = 576, HX_FRAG = 2 * HX_HALF, HX_STEP = 4 * HX_FRAG + 32, 
 constexpr int HX_BUFS = 3;                         // stages in LDS: one being written, one contracted, one peeked into
 constexpr int HX_AHEAD = 3;                        // stages a loading wave has in flight
 constexpr int HX_EXPS = 4;                         // items whose row exponents are kept (see lds_exp)
-constexpr int HX_BAD = 0x10000;                    // exponent of a row that the split cannot carry
+constexpr int HX_BAD = 511;                        // exponent of a row that holds an infinity or a NaN (others: -115 .. 127) ...
+constexpr int HX_ANY_BAD = 300;                    // ... and what no sum of two others reaches
+constexpr float HX_SMALL = 0.25f;                  // scaled elements below this keep 2^-25, those above it 2^-23 of themselves
+constexpr float HX_LOST = 2048.0f;                 // 2^21 times the 2^-10 that such an element may cost an output
+constexpr float HX_ZEROS = -1e9f;                  // small elements of a row of zeros: it costs nothing, whatever its partner
+constexpr uint32_t HX_PLAIN = 0xffffffffu;         // of a wave's note on an item: all of it, one product at a time
 constexpr uint32_t HX_FIRST_SCALE = (127u + 126u) << 23;      // before a row's first nonzero element: 2^126
 constexpr int HX_KC = 0, HX_RC = 1, HX_KRUN = 2, HX_RRUN = 3; // how A lies: contiguous in k / in its rows; compound indices with runs along k / the rows
 constexpr int HX_PARTIAL = 0, HX_DENSE = 1, HX_COMPOUND = 2;  // where the sums go: the slices' workspace, a dense C, a compound C
 
 struct F16x2Job {
     const uint8_t* wb;        // B's fragments: [stage][part][16-k step][tile of 32 columns][1 KB]
-    const int* eb;            // [slice][nb_pad]: exponent of B's column in the slice, HX_BAD where the split cannot carry it
+    const uint32_t* eb;       // [slice][nb_pad]: of B's column in the slice, the exponent (ten bits, signed) and its small elements (22 bits, all set: zeros)
     float* partial;           // [slice][ma_pad][nb_pad]
+    uint64_t* notes;          // [work-group][contracting wave][most_items]: item and, a bit each, its tiles of 32 x 32 to redo
+    int most_items;           // items of a work-group at most
     int nb_pad, ma_pad;
     int chunks, slice_chunks; // stages in all and per slice: even numbers
     int slices, items;
@@ -61,6 +77,26 @@ __device__ __forceinline__ float max4(float m, const v4f& x) {
 #endif
 }
 
+// the smallest magnitude (a NaN: the row is a bad one, whatever comes of it)
+__device__ __forceinline__ float min4(float m, const v4f& x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    m = __builtin_elementwise_minimum(__builtin_elementwise_minimum(m, __builtin_fabsf(x[0])), __builtin_fabsf(x[1]));
+    return __builtin_elementwise_minimum(__builtin_elementwise_minimum(m, __builtin_fabsf(x[2])), __builtin_fabsf(x[3]));
+#else
+    return m + x[0];
+#endif
+}
+
+// how many of four elements are small ones under this scale (a power of two from 2^-115 to 2^127): not zero, below 2^-2 of it
+__device__ __forceinline__ int count_small4(const v4f& x, float scale) {
+    const float limit = ldexpf(HX_SMALL, 127 - static_cast<int>(__float_as_uint(scale) >> 23));
+    const uint32_t below = (__float_as_uint(limit) << 1) - 1;       // (zeros wrap round to the largest number)
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) n += (__float_as_uint(x[c]) << 1) - 1 < below ? 1 : 0;
+    return n;
+}
+
 // ------------------------------------------------------------------------------------------------------------
 // B ahead of the contraction.  A work-group takes 32 rows of B (columns of the product) and one slice of K: maxima, scale,
 // parts.  A round covers 256 k; a slice of up to eight rounds stays in registers between the two passes.
@@ -68,7 +104,7 @@ constexpr int HX_SPLIT_ROUNDS = 8;
 struct F16x2Split {
     const float* src;
     uint8_t* dst;
-    int* exps;
+    uint32_t* exps;
     int rows, rows_pad, K, chunks, slice_chunks;
     int64_t rs, ks;
     int64_t span;             // elements from src to behind the last one: below 2^29, any 32 rows' offsets too
@@ -77,7 +113,9 @@ struct F16x2Split {
 template <bool KS1>
 __global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) {
     __shared__ uint32_t lds_max[32][33];
+    __shared__ int lds_small[32];
     const int tid = threadIdx.x;
+    if (tid < 32) lds_small[tid] = 0;
     // (row of the 32, octet of k within a round): lanes along k or along the rows, as the operand lies
     const int row = KS1 ? tid >> 5 : tid & 31, oct = KS1 ? tid & 31 : tid >> 5;
     const int r = blockIdx.x * 32 + row;
@@ -130,15 +168,16 @@ __global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) 
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 32; ++i) { const uint32_t o = lds_max[row][i]; top = o > top ? o : top; }
-    // the largest element goes to 2^14 .. 2^15; an all-zero row needs no scale
+    // the largest element goes to 2^14 .. 2^15, or as near as 2^127 brings it; an all-zero row needs no scale
     const int e = static_cast<int>(top >> 23) & 0xff;
-    const bool bad = top >= 0x7f800000u || (e < 14 && top != 0);
-    const int scale_exp = top == 0 || bad ? 127 : 268 - e;          // biased exponent of the scale
+    const bool bad = top >= 0x7f800000u;
+    const int scale_exp = top == 0 || bad ? 127 : e >= 14 ? 268 - e : 254;          // biased exponent of the scale
     const float scale = __uint_as_float(static_cast<uint32_t>(scale_exp) << 23);
-    if (oct == 0) jb.exps[static_cast<int64_t>(blockIdx.y) * jb.rows_pad + r] = bad ? HX_BAD : scale_exp - 127;
+    int small = 0;
     const auto put = [&](int i, const v4f (&v)[2]) {
         const int kb = k_begin + i * 256 + oct * 8;
         if (kb >= k_end) return;
+        if (min4(min4(__builtin_inff(), v[0]), v[1]) * scale < HX_SMALL) small += count_small4(v[0], scale) + count_small4(v[1], scale);
         uint2 lo[2], hi[2];
         split4_f16(v[0], scale, lo);
         split4_f16(v[1], scale, hi);
@@ -160,40 +199,33 @@ __global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) 
             put(i + 1, b);
         }
     }
+    if (small != 0) atomicAdd(&lds_small[row], small);
+    __syncthreads();
+    if (oct == 0) {
+        const uint32_t n = static_cast<uint32_t>(lds_small[row]);
+        jb.exps[static_cast<int64_t>(blockIdx.y) * jb.rows_pad + r] =
+            (static_cast<uint32_t>(bad ? HX_BAD : scale_exp - 127) & 1023u) | (top == 0 ? 0x3fffffu : n < 0x3ffffeu ? n : 0x3ffffeu) << 10;
+    }
 }
 
-// ------------------------------------------------------------------------------------------------------------
-// The contraction.  One work-group of eight waves per CU walks a list of items (128 x 128 TJ tiles, times the slices of K).
-// Waves 4 .. 7 load A three stages ahead, find the rows' maxima, scale, split and write the stage to LDS; they run on into
-// the next item while waves 0 .. 3 store the finished one.  A contracting wave takes all 128 rows and 32 TJ columns: B's
-// fragments belong to it alone and come straight from memory (L2), two stages ahead; A's come from LDS one step ahead of
-// their six MFMAs.  Barrier i + 1 says "stages up to i + 1 are in LDS" and "stage i - 1 has been read".
-template <int AMODE, bool GEN, int TJ, int OUT, bool STREAM>
-__global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const GemmParams p, const F16x2Job jb) {
-    constexpr bool KLOAD = AMODE == HX_KC || AMODE == HX_KRUN;
-    constexpr bool RUNS = AMODE == HX_KRUN || AMODE == HX_RRUN;
-    constexpr int NR = KLOAD ? 4 : 1;                  // rows of A a loading lane has a share of
-    __shared__ __attribute__((aligned(16))) uint8_t lds_a[HX_BUFS * HX_STAGE];
-    __shared__ __attribute__((aligned(16))) float lds_factor[HX_BUFS][HX_M];
-    __shared__ __attribute__((aligned(16))) int lds_mark[HX_BUFS][4];
-    // exponents of the rows' scales, per item: written with an item's last stage, read behind it, by when the loading waves
-    // are at most two stages (two items, were an item one stage) further
-    __shared__ __attribute__((aligned(16))) int lds_exp[HX_EXPS][HX_M];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tiles = p.tiles_m * p.tiles_n;
-
-    // this work-group's items: first, first + step, ...; an XCD's are consecutive ones
-    const int xcd = blockIdx.x & 7, step = gridDim.x >> 3;
-    const int lo = static_cast<int>(static_cast<int64_t>(jb.items) * xcd / 8);
-    const int hi = static_cast<int>(static_cast<int64_t>(jb.items) * (xcd + 1) / 8);
-    const int first = lo + static_cast<int>(blockIdx.x >> 3);
-    const int my_items = first < hi ? (hi - first + step - 1) / step : 0;
-    if (my_items == 0) return;                          // (the whole work-group: no barrier is left behind)
+// A work-group's items: first, first + step, ...; an XCD's are consecutive ones
+template <int TJ>
+struct Items {
     struct Item { int m0, n0, slice, c_begin, nch; };
-    const auto item_at = [&](int i) {
+    const GemmParams& p;
+    const F16x2Job& jb;
+    int first, step, mine;
+    __device__ __forceinline__ Items(const GemmParams& p_, const F16x2Job& jb_) : p(p_), jb(jb_) {
+        const int xcd = blockIdx.x & 7;
+        step = gridDim.x >> 3;
+        const int lo = static_cast<int>(static_cast<int64_t>(jb.items) * xcd / 8);
+        const int hi = static_cast<int>(static_cast<int64_t>(jb.items) * (xcd + 1) / 8);
+        first = lo + static_cast<int>(blockIdx.x >> 3);
+        mine = first < hi ? (hi - first + step - 1) / step : 0;
+    }
+    __device__ __forceinline__ Item at(int i) const {
         Item it;
+        const int tiles = p.tiles_m * p.tiles_n;
         int t = first + i * step;
         it.slice = t / tiles;
         t -= it.slice * tiles;
@@ -206,7 +238,128 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
         it.c_begin = it.slice * jb.slice_chunks;
         it.nch = jb.chunks - it.c_begin < jb.slice_chunks ? jb.chunks - it.c_begin : jb.slice_chunks;
         return it;
+    }
+};
+
+// ------------------------------------------------------------------------------------------------------------
+// Outputs that the scaled parts did not carry, again, by the exact split into three bf16 parts and over the k of a slice: tiles
+// of 32 x 32 from (m0, n0) and from (m0 + 32, n0) on, a bit of `which` each; by one wave, straight from memory.
+template <int OUT, int AHEAD>
+__device__ __forceinline__ void redo_tiles(const GemmParams& p, const F16x2Job& jb, int m0, int n0, int slice, uint32_t which, int lane) {
+    const int k0 = slice * jb.slice_chunks * HX_K;
+    const int k1 = OUT == HX_PARTIAL && k0 + jb.slice_chunks * HX_K < p.K ? k0 + jb.slice_chunks * HX_K : p.K;
+    const bool runs = p.a_lm > 0;
+    const int j = lane & 31, hh = lane >> 5;
+    // both operands by 32-bit byte offsets, as in the tile loop (outside: zero)
+    const int64_t b_span = (static_cast<int64_t>(p.N - 1) * p.b_rs + static_cast<int64_t>(p.K - 1) * p.b_ks + 1) * 4;
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A), 0, static_cast<int>(jb.a_span), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.B), 0, static_cast<int>(b_span), 0x00020000);
+    const uint32_t a_step = static_cast<uint32_t>(runs ? p.a_ki : p.a_ks) * 4u, b_step = static_cast<uint32_t>(p.b_ks) * 4u;
+    const uint32_t carry = runs ? static_cast<uint32_t>(p.a_ko - p.a_lk * p.a_ki) * 4u : 0;      // from behind a run to the next one's start
+    uint32_t a_at[2], b_at;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int m = m0 + 32 * u + j;
+        const int64_t el = runs ? static_cast<int64_t>(m / p.a_lm) * p.a_mo + static_cast<int64_t>(m % p.a_lm) * p.a_mi : static_cast<int64_t>(m) * p.a_rs;
+        a_at[u] = m < p.M ? static_cast<uint32_t>(el) * 4u + 8 * hh * a_step : OUTSIDE;
+    }
+    b_at = n0 + j < p.N ? static_cast<uint32_t>((n0 + j) * p.b_rs) * 4u + 8 * hh * b_step : OUTSIDE;
+    // eight consecutive k from byte offset `at` on, of which `left` are there; from the `turn`-th on they lie in the next run
+    const auto load8 = [](const __amdgpu_buffer_rsrc_t r, uint32_t at, uint32_t step, bool whole, int left, int turn, uint32_t carry_, v4f (&x)[2]) {
+        if (step == 4u && whole) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) x[h] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, at + 16u * h, 0, 0));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                x[i >> 2][i & 3] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, i < left ? at + i * step + (i < turn ? 0u : carry_) : OUTSIDE, 0, 0));
+        }
     };
+    const auto load = [&](int k, v4f (&xa)[2][2], v4f (&xb)[2]) {
+        const int kd = runs ? k / p.a_lk : 0, kr = runs ? k - kd * p.a_lk : k;
+        const uint32_t off = runs ? static_cast<uint32_t>(kd * p.a_ko + kr * p.a_ki) * 4u : static_cast<uint32_t>(k) * a_step;
+        const int turn = runs ? p.a_lk - kr : 16;       // (a run is at least a stage long)
+        const bool in = k + 16 <= k1, whole = in && turn >= 16;
+        const int left = k1 - k - 8 * hh;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) load8(ra, a_at[u] + off, a_step, whole, left, turn - 8 * hh, carry, xa[u]);
+        load8(rb, b_at + static_cast<uint32_t>(k) * b_step, b_step, in, left, 8, 0u, xb);
+    };
+    v16f acc[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[u][r] = 0.0f;
+    SplitGuard guard;
+    v4f xa[AHEAD][2][2], xb[AHEAD][2];                  // steps of 16 k in flight (behind k1: zeros)
+#pragma unroll
+    for (int d = 0; d < AHEAD; ++d) load(k0 + 16 * d, xa[d], xb[d]);
+#pragma unroll 1
+    for (int k = k0; k < k1; k += 16 * AHEAD) {
+#pragma unroll
+        for (int d = 0; d < AHEAD; ++d) {
+            v8bf fa[2][3], fb[3];
+            split8(xa[d][0], fa[0], guard);
+            split8(xa[d][1], fa[1], guard);
+            split8(xb[d], fb, guard);
+            if (k + 16 * AHEAD < k1) load(k + 16 * (AHEAD + d), xa[d], xb[d]);
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[u][SPLIT_TERMS[q][0]], fb[SPLIT_TERMS[q][1]], acc[u], 0, 0, 0);
+        }
+    }
+    const bool fired = __builtin_amdgcn_ballot_w64(guard.fired()) != 0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        if ((which >> u & 1) == 0) continue;
+        if (OUT != HX_PARTIAL && fired) {               // bits below the exact split's own range
+            plain_tile(p, p.A, p.B, p.C, m0 + 32 * u, n0, 32, 32, lane, 64);
+            continue;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = m0 + 32 * u + mfma32_row(r, lane), n = n0 + j;
+            if (m >= p.M || n >= p.N) continue;
+            float v = fired ? __builtin_nanf("") : acc[u][r];       // (NaN: reduce_slices_kernel redoes it)
+            if (OUT == HX_PARTIAL) {
+                jb.partial[(static_cast<size_t>(slice) * jb.ma_pad + m) * jb.nb_pad + n] = v;
+            } else {
+                if (p.bias) v += p.bias[n];
+                p.C[static_cast<int64_t>(m / p.c_lm) * p.c_mo + static_cast<int64_t>(m % p.c_lm) * p.c_mi +
+                    static_cast<int64_t>(n / p.c_ln) * p.c_no + static_cast<int64_t>(n % p.c_ln) * p.c_ni] = v * p.alpha;
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// The contraction.  One work-group of eight waves per CU walks a list of items (128 x 128 TJ tiles, times the slices of K).
+// Waves 4 .. 7 load A three stages ahead, find the rows' maxima, scale, split and write the stage to LDS; they run on into
+// the next item while waves 0 .. 3 store the finished one.  A contracting wave takes all 128 rows and 32 TJ columns: B's
+// fragments belong to it alone and come straight from memory (L2), two stages ahead; A's come from LDS one step ahead of
+// their six MFMAs.  Barrier i + 1 says "stages up to i + 1 are in LDS" and "stage i - 1 has been read".
+template <int AMODE, bool GEN, int TJ, int OUT, bool STREAM>
+__device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job& jb, int (&lds_noted)[4]) {
+    constexpr bool KLOAD = AMODE == HX_KC || AMODE == HX_KRUN;
+    constexpr bool RUNS = AMODE == HX_KRUN || AMODE == HX_RRUN;
+    constexpr int NR = KLOAD ? 4 : 1;                  // rows of A a loading lane has a share of
+    __shared__ __attribute__((aligned(16))) uint8_t lds_a[HX_BUFS * HX_STAGE];
+    __shared__ __attribute__((aligned(16))) float lds_factor[HX_BUFS][HX_M];
+    __shared__ __attribute__((aligned(16))) int lds_mark[HX_BUFS][4];
+    // exponents of the rows' scales, per item: written with an item's last stage, read behind it, by when the loading waves
+    // are at most two stages (two items, were an item one stage) further
+    __shared__ __attribute__((aligned(16))) int lds_exp[HX_EXPS][HX_M];
+    __shared__ __attribute__((aligned(16))) float lds_small[HX_EXPS][HX_M];      // their small elements, HX_ZEROS for a row of zeros ...
+    __shared__ __attribute__((aligned(16))) float lds_most[HX_EXPS][4];          // ... and the most of them in a row, per loading wave
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    const Items<TJ> items(p, jb);
+    const int my_items = items.mine;
+    const auto item_at = [&](int i) { return items.at(i); };
+    if (my_items == 0) return;                          // (the whole work-group: no barrier is left behind)
     int total = 0;                                      // stages of this work-group
     for (int i = 0; i < my_items; ++i) total += item_at(i).nch;
     const int padded = (total + HX_AHEAD - 1) / HX_AHEAD * HX_AHEAD;
@@ -225,7 +378,7 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
         const int u0 = KLOAD ? (lane & 7) * 4 : (lane >> 5) * 16;
         const uint32_t k_step = static_cast<uint32_t>(RUNS ? p.a_ki : p.a_ks) * 4u;        // bytes from k to k + 1
         uint32_t roff[NR];
-        Item load_item = item_at(0);
+        typename Items<TJ>::Item load_item = item_at(0);
         int li = 0, lc = 0, kd = 0, kr = 0;
         const auto open = [&]() {
 #pragma unroll
@@ -304,14 +457,15 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
 
         float scale[NR];
         uint32_t seen[NR];                              // OR of the maxima's bits; the sign bit: infinite or NaN
+        int small[NR];                                  // this lane's share of the row's small elements
         int pi = 0, pc = 0, p_nch = load_item.nch, buf = 0;
         // splits the next stage into LDS
         const auto place = [&](const v4f (&x)[4]) {
             if (pc == 0) {
 #pragma unroll
-                for (int i = 0; i < NR; ++i) { scale[i] = __uint_as_float(HX_FIRST_SCALE); seen[i] = 0; }
+                for (int i = 0; i < NR; ++i) { scale[i] = __uint_as_float(HX_FIRST_SCALE); seen[i] = 0; small[i] = 0; }
             }
-            uint32_t top[NR];
+            uint32_t top[NR], before[NR];
             bool over = false;
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
@@ -327,6 +481,7 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
                     meet(__shfl_xor(b, 32, 64));
                 }
                 top[i] = b;
+                before[i] = seen[i];
                 seen[i] |= b;
                 over |= !(__uint_as_float(b) * scale[i] < 32768.0f);
             }
@@ -344,6 +499,8 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
                             const int f = now - was + 127;
                             factor = f > 0 ? __uint_as_float(static_cast<uint32_t>(f) << 23) : 0.0f;
                             scale[i] = __uint_as_float(static_cast<uint32_t>(now) << 23);
+                            // (what the sums hold may leave binary32's range on this way: less than a small element's share)
+                            if (before[i] != 0 && u0 == 0) ++small[i];
                         }
                     }
                     if (u0 == 0) lds_factor[buf][w * 32 + 8 * i + r0] = factor;
@@ -351,6 +508,18 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
                 mark = 1;
             }
             if (lane == 0) lds_mark[buf][w] = mark;
+            // (zeros pass this test too: an ordinary stage of nonzero elements pays for a minimum, one with zeros or small ones for the count)
+            bool few = false;
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                float m = min4(__builtin_inff(), x[i]);
+                if (!KLOAD) m = min4(min4(min4(m, x[1]), x[2]), x[3]);
+                few |= m * scale[i] < HX_SMALL;
+            }
+            if (__builtin_amdgcn_ballot_w64(few) != 0) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) small[i % NR] += count_small4(x[i], scale[i % NR]);
+            }
             uint8_t* const stage = lds_a + buf * HX_STAGE + w * HX_FRAG;
             if (KLOAD) {
                 uint8_t* const dst = stage + (u0 >> 4) * HX_STEP + ((u0 >> 3) & 1) * HX_HALF + ((u0 >> 2) & 1) * 8 + r0 * 16;
@@ -373,14 +542,25 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
                 }
             }
             if (++pc == p_nch) {
-                if (pi < my_items && u0 == 0) {
+                if (pi < my_items) {
+                    int most = 0;
 #pragma unroll
                     for (int i = 0; i < NR; ++i) {
-                        const uint32_t s = __float_as_uint(scale[i]);
-                        const bool untouched = s == HX_FIRST_SCALE;         // a row of zeros, or of elements below 2^-111
-                        const bool bad = (seen[i] & 0x80000000u) != 0 || (untouched && seen[i] != 0);
-                        lds_exp[pi & (HX_EXPS - 1)][w * 32 + 8 * i + r0] = bad ? HX_BAD : untouched ? 0 : static_cast<int>(s >> 23) - 127;
+                        int n = small[i];               // (the lanes of the row, as with the maxima)
+                        if (KLOAD) {
+                            n += __builtin_amdgcn_mov_dpp(n, 0xB1, 0xf, 0xf, true);
+                            n += __builtin_amdgcn_mov_dpp(n, 0x4E, 0xf, 0xf, true);
+                            n += __builtin_amdgcn_mov_dpp(n, 0x141, 0xf, 0xf, true);
+                        } else {
+                            n += __shfl_xor(n, 32, 64);
+                        }
+                        most = n > most ? n : most;
+                        if (u0 != 0) continue;
+                        lds_exp[pi & (HX_EXPS - 1)][w * 32 + 8 * i + r0] = (seen[i] & 0x80000000u) != 0 ? HX_BAD : seen[i] == 0 ? 0 : static_cast<int>(__float_as_uint(scale[i]) >> 23) - 127;
+                        lds_small[pi & (HX_EXPS - 1)][w * 32 + 8 * i + r0] = seen[i] == 0 ? HX_ZEROS : static_cast<float>(n);
                     }
+                    const float m = wave_max(static_cast<float>(most));
+                    if (lane == 0) lds_most[pi & (HX_EXPS - 1)][w] = m;
                 }
                 pc = 0;
                 if (++pi < my_items) p_nch = item_at(pi).nch;
@@ -407,7 +587,7 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
     const int j = lane & 31, hh = lane >> 5;
     const int wn = wave * 32 * TJ;
     v8h fb[2][TJ][2][2];                                // [stage parity][tile column][16-k step][part]
-    Item b_item = item_at(0);
+    typename Items<TJ>::Item b_item = item_at(0);
     int bi = 0, bc = 0;
     const size_t b_unit = static_cast<size_t>(jb.nb_pad) * 32;
     // the fragments of the next stage of the sequence (behind the last item: of that item's first stages again)
@@ -436,20 +616,37 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
     v4i mark = *reinterpret_cast<const v4i*>(lds_mark[0]);
     v16f acc[4][TJ];
     int g = 0;
-    for (int i = 0; i < my_items; ++i) {
-        const Item it = item_at(i);
-        int eb[TJ];
+    uint64_t* const notes = jb.notes + static_cast<size_t>(blockIdx.x * 4 + wave) * jb.most_items;
+    int noted = 0;                                      // items with outputs to redo
+    // the smallest of this lane's sums
+    const auto least = [&]() {
+        float m = __builtin_inff();
 #pragma unroll
-        for (int tj = 0; tj < TJ; ++tj) eb[tj] = jb.eb[static_cast<size_t>(it.slice) * jb.nb_pad + it.n0 + wn + tj * 32 + j];
+        for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < TJ; ++tj)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) m = __builtin_elementwise_minimum(m, __builtin_fabsf(acc[ti][tj][r]));
+        return m;
+    };
+    for (int i = 0; i < my_items; ++i) {
+        const typename Items<TJ>::Item it = item_at(i);
+        uint32_t of_b[TJ];
+#pragma unroll
+        for (int tj = 0; tj < TJ; ++tj) of_b[tj] = jb.eb[static_cast<size_t>(it.slice) * jb.nb_pad + it.n0 + wn + tj * 32 + j];
 #pragma unroll
         for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
             for (int tj = 0; tj < TJ; ++tj)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[ti][tj][r] = 0.0f;
+        // this lane's smallest sum halfway through K: no sum of |a||b| is smaller than that of a part of it, so a lane that passes the
+        // test below with either need not be looked at
+        float halfway = 0.0f;
         const auto chunk = [&](v8h (&f)[TJ][2][2], int k0, bool fresh) {
             if (!fresh && __builtin_amdgcn_readfirstlane(mark[0] | mark[1] | mark[2] | mark[3]) != 0) {
                 // some rows' scales have moved: what their sums hold so far moves with them
+                halfway = 0.0f;
 #pragma unroll
                 for (int ti = 0; ti < 4; ++ti) {
                     if (__builtin_amdgcn_readfirstlane(mark[ti]) == 0) continue;
@@ -501,20 +698,58 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
             if (g < total) __syncthreads();             // stage g - 1 has been read; stage g + 1 is in LDS
         };
         for (int c = 0; c < it.nch; c += 2) {
+            if (c == it.nch / 4 * 2 && c != 0) halfway = least();
             chunk(fb[0], (it.c_begin + c) * HX_K, c == 0);
             chunk(fb[1], (it.c_begin + c + 1) * HX_K, false);
         }
 
         // ---- the scales leave, the sums go out
         const int (&ea)[HX_M] = lds_exp[i & (HX_EXPS - 1)];
-        int worst = ea[lane] > ea[lane + 64] ? ea[lane] : ea[lane + 64];
+        int eb[TJ], worst = ea[lane] > ea[lane + 64] ? ea[lane] : ea[lane + 64];
+        float cb[TJ], bound = 0.0f;
 #pragma unroll
-        for (int tj = 0; tj < TJ; ++tj) worst = eb[tj] > worst ? eb[tj] : worst;
-        const bool any_bad = __builtin_amdgcn_ballot_w64(worst >= HX_BAD / 2) != 0;
+        for (int tj = 0; tj < TJ; ++tj) {
+            eb[tj] = static_cast<int>(of_b[tj] << 22) >> 22;
+            worst = eb[tj] > worst ? eb[tj] : worst;
+            cb[tj] = of_b[tj] >> 10 == 0x3fffffu ? HX_ZEROS : static_cast<float>(of_b[tj] >> 10);
+            bound = fmaxf(bound, cb[tj]);
+        }
+        const bool any_bad = __builtin_amdgcn_ballot_w64(worst >= HX_ANY_BAD) != 0;
         if (OUT != HX_PARTIAL && any_bad) {
-            // operands of this wave's columns that the split could not carry: all of them again, the reference's way
-            plain_tile(p, p.A, p.B, p.C, it.m0, it.n0 + wn, HX_M, 32 * TJ, lane, 64);
+            // infinities or NaN in this wave's tile: all of it again, the reference's way
+            if (lane == 0) notes[noted] = static_cast<uint64_t>(i) << 32 | HX_PLAIN;
+            ++noted;
             continue;
+        }
+        // outputs that the small elements of their rows may have cost more than the products' own error (see above): by the most of
+        // them in a row first, which all but a few tiles pass, then row by row; the tiles of 32 x 32 that fail are noted
+        const v4f most = *reinterpret_cast<const v4f*>(lds_most[i & (HX_EXPS - 1)]);
+        bound = HX_LOST * (bound + fmaxf(fmaxf(most[0], most[1]), fmaxf(most[2], most[3])));
+        if (__builtin_amdgcn_ballot_w64(!(halfway >= bound)) != 0) {
+            const bool open = !(halfway >= bound) && !(least() >= bound);
+            if (__builtin_amdgcn_ballot_w64(open) != 0) {
+                const float (&na)[HX_M] = lds_small[i & (HX_EXPS - 1)];
+                uint32_t which = 0;
+#pragma unroll
+                for (int ti = 0; ti < 4; ++ti) {
+                    uint64_t lost[TJ] = {};
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const v4f n4 = *reinterpret_cast<const v4f*>(&na[ti * 32 + 8 * q + 4 * hh]);
+#pragma unroll
+                        for (int tj = 0; tj < TJ; ++tj)
+#pragma unroll
+                            for (int c = 0; c < 4; ++c)             // (a NaN comes from a row that is a bad one)
+                                lost[tj] |= __builtin_amdgcn_ballot_w64(__builtin_fabsf(acc[ti][tj][4 * q + c]) < HX_LOST * (n4[c] + cb[tj]));
+                    }
+#pragma unroll
+                    for (int tj = 0; tj < TJ; ++tj) which |= (lost[tj] & __builtin_amdgcn_ballot_w64(open)) != 0 ? 1u << (ti * TJ + tj) : 0u;
+                }
+                if (which != 0) {
+                    if (lane == 0) notes[noted] = static_cast<uint64_t>(i) << 32 | which;
+                    ++noted;
+                }
+            }
         }
         if (OUT == HX_PARTIAL && any_bad) {             // NaN: reduce_slices_kernel redoes those
 #pragma unroll
@@ -523,7 +758,7 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
                 for (int r = 0; r < 16; ++r)
 #pragma unroll
                     for (int tj = 0; tj < TJ; ++tj)
-                        if (ea[ti * 32 + 8 * (r >> 2) + 4 * hh + (r & 3)] + eb[tj] >= HX_BAD / 2) acc[ti][tj][r] = __builtin_nanf("");
+                        if (ea[ti * 32 + 8 * (r >> 2) + 4 * hh + (r & 3)] + eb[tj] >= HX_ANY_BAD) acc[ti][tj][r] = __builtin_nanf("");
         }
         // (one tile row at a time: with all sixty-four exponents read ahead the kernel spills)
         const auto unscale = [&](int ti) {
@@ -577,6 +812,48 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
         }
     }
     for (; g < padded; ++g) __syncthreads();
+    if (lane == 0) lds_noted[wave] = noted;
+}
+
+template <int AMODE, bool GEN, int TJ, int OUT, bool STREAM>
+__global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const GemmParams p, const F16x2Job jb) {
+    __shared__ int lds_noted[4];
+    if (threadIdx.x < 4) lds_noted[threadIdx.x] = 0;    // (a work-group without items leaves them so)
+    f16x2_items<AMODE, GEN, TJ, OUT, STREAM>(p, jb, lds_noted);
+    // What the items left to redo, by all eight waves.  Behind the last item, where nothing else is held in registers (among the items the
+    // two-to-a-CU form spilled its fragments), and with the parameters read again, which the items then need not hold either.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (the notes, and the stores of the outputs concerned, have landed)
+    __syncthreads();
+    int counts[4], any = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) { counts[w] = __builtin_amdgcn_readfirstlane(lds_noted[w]); any |= counts[w]; }
+    if (any == 0) return;
+    typedef const __attribute__((address_space(4))) GemmParams* KernargPtr;
+    KernargPtr again = (KernargPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(again));
+    const GemmParams pr = *(const GemmParams*)again;
+    const Items<TJ> items(pr, jb);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int unit = 0;
+#pragma unroll 1
+    for (int w = 0; w < 4; ++w) {
+        const int count = w == 0 ? counts[0] : w == 1 ? counts[1] : w == 2 ? counts[2] : counts[3];
+#pragma unroll 1
+        for (int u = 0; u < count * 2 * TJ; ++u) {      // (64 rows x 32 columns each)
+            if ((unit++ & 7) != wave) continue;
+            const uint64_t note = jb.notes[static_cast<size_t>(blockIdx.x * 4 + w) * jb.most_items + u / (2 * TJ)];
+            const auto it = items.at(__builtin_amdgcn_readfirstlane(static_cast<int>(note >> 32)));
+            const uint32_t which = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(note));
+            const int ti = u / TJ % 2 * 2, tj = u % TJ;
+            const int m0 = it.m0 + ti * 32, n0 = it.n0 + (w * TJ + tj) * 32;
+            if (OUT != HX_PARTIAL && which == HX_PLAIN) {
+                plain_tile(pr, pr.A, pr.B, pr.C, m0, n0, 64, 32, lane, 64);
+                continue;
+            }
+            const uint32_t these = (which >> (ti * TJ + tj) & 1) | (which >> ((ti + 1) * TJ + tj) & 1) << 1;
+            if (these != 0) redo_tiles<OUT, TJ>(pr, jb, m0, n0, it.slice, these, lane);
+        }
+    }
 }
 
 }  // namespace
@@ -679,7 +956,10 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     const bool partial = slices > 1 || p.a_lm > 0 || p.c_ni != 1;     // (no direct instances for a compound A)
     const size_t part_bytes = partial ? static_cast<size_t>(slices) * ma_pad * nb_pad * 4 : 0;
     if (static_cast<size_t>(ma_pad) * nb_pad * 4 >= (1ull << 31) && partial) return -1;
-    const size_t need = b_bytes + e_bytes + part_bytes;
+    const int wgs = std::min<int64_t>((tiles * slices + 7) / 8 * 8, tj == 1 ? 2 * cus : cus);
+    const int most_items = static_cast<int>(((tiles * slices + 7) / 8 + wgs / 8 - 1) / (wgs / 8));
+    const size_t n_bytes = (static_cast<size_t>(wgs) * 4 * most_items * 8 + 255) / 256 * 256;
+    const size_t need = b_bytes + e_bytes + n_bytes + part_bytes;
     uint8_t* ws = fixed_ws;
     Workspace held;
     if (fixed_ws) {
@@ -691,9 +971,11 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     }
     F16x2Job jb{};
     jb.wb = ws;
-    int* const exps = reinterpret_cast<int*>(ws + b_bytes);
+    uint32_t* const exps = reinterpret_cast<uint32_t*>(ws + b_bytes);
     jb.eb = exps;
-    jb.partial = reinterpret_cast<float*>(ws + b_bytes + e_bytes);
+    jb.notes = reinterpret_cast<uint64_t*>(ws + b_bytes + e_bytes);
+    jb.most_items = most_items;
+    jb.partial = reinterpret_cast<float*>(ws + b_bytes + e_bytes + n_bytes);
     jb.nb_pad = nb_pad; jb.ma_pad = ma_pad;
     jb.chunks = chunks; jb.slice_chunks = slice_chunks; jb.slices = slices;
     jb.items = static_cast<int>(tiles) * slices;
@@ -704,7 +986,6 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     else             hipLaunchKernelGGL((split_f16x2_kernel<false>), sgrid, dim3(1024), 0, stream, sp);
     int rc = check_launch(what);
     if (rc == RC_OK) {
-        const int wgs = std::min<int64_t>((jb.items + 7) / 8 * 8, tj == 1 ? 2 * cus : cus);
         const int out = partial ? HX_PARTIAL : compound ? HX_COMPOUND : HX_DENSE;
         const bool stream_c = p.stream_c && !partial;
 #define PPML_HX(A_, G_, T_, O_, S_) hipLaunchKernelGGL((gemm_f16x2_kernel<A_, G_, T_, O_, S_>), dim3(wgs), dim3(512), 0, stream, p, jb)

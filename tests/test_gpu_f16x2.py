@@ -3,9 +3,11 @@ k with whole and ragged pieces, contiguous in its rows, runs of the outer-produc
 that are not), both tile widths, every kind of output, and what the scales have to follow: rows that differ by 2^80, rows
 that grow along k, rows of zeros, and rows that no scale can bring into range.
 
-The bound: a product of two parts each is within 3 * 2^-24 of |a||b| (two splits, the dropped product), a sum of K terms in
-binary32 within K * 2^-24 of sum |a||b|: (K + 4) * 2^-24 together, for every output by itself.  An element far below the
-largest of its row (2^-17 of it) is kept to 2^-40 of that largest, which these operands never come near."""
+The bound of the first tests: a product of two parts each is within 2^-21 of |a||b| (two splits of 2^-23, the dropped product of
+2^-22), a sum of K terms in binary32 within K / 16 * 2^-24 of sum |a||b|, sixteen products at a time: below (K + 4) * 2^-24
+together from K = 72 on, for every output by itself.  It grows with K, where the errors of random operands average out: the tests
+after them hold bounds that do not, on operands with ranges within a row (an element below 2^-14 of its row's largest is kept
+to 2^-37 of that largest; the outputs to which that matters are computed again) and on parts that are left out."""
 import numpy as np
 import pytest
 import torch
@@ -107,3 +109,80 @@ def test_operands_no_scale_brings_into_range(ops, M, K, N):
     for m in (7, 300, 600):
         far[m // 128 * 128:m // 128 * 128 + 128] = False
     assert torch.equal(got[far][:, 128:], clean[far][:, 128:])
+
+
+def _narrow(got, a, b, scale=1.0):
+    """|got - scale a b^T| within 2^-20 of scale sum |a||b| (the products' 2^-21, as much again for small elements), whatever K is: the
+    binary32 sums of these operands, which change sign, stay far below that"""
+    want, size = scale * (a @ b.t()), scale * (a.abs() @ b.abs().t())
+    bad = ~((got.double() - want).abs() <= 2.0 ** -20 * size + 1e-45)
+    assert not bool(bad.any()), (int(bad.sum()), float(((got.double() - want).abs() / size)[bad].max()))
+
+
+def _spikes(g, a, b, size, where):
+    """Columns of k where one operand is enormous and the other zero: one, one in every 32, a tenth of them"""
+    K = a.shape[1]
+    ks = {"one": [K // 3], "stages": list(range(5, K, 32)), "tenth": list(range(3, K, 10))}[where]
+    a, b = a.clone(), b.clone()
+    a[:, ks] = size * torch.randn(a.shape[0], len(ks), device="cuda", generator=g)
+    b[:, ks] = 0
+    return a, b
+
+
+# Rows whose large elements meet zeros, in either operand, through every way A may lie and every kind of output
+@pytest.mark.parametrize("where", ["one", "stages", "tenth"])
+@pytest.mark.parametrize("size", [1e5, 1e7, 1e9, 1e12, 1e30])
+def test_large_elements_that_meet_zeros(ops, size, where):
+    g = torch.Generator(device="cuda").manual_seed(int(np.log10(size)) * 3 + len(where))
+    for M, K, N in ((20011, 136, 1004), (26368, 256, 200), (9001, 403, 390)):
+        a, b = (torch.randn(n, K, device="cuda", generator=g) for n in (M, N))
+        for first in (True, False):
+            x, y = _spikes(g, a, b, size, where) if first else _spikes(g, b, a, size, where)[::-1]
+            got = ops.mul_mat(x, y)
+            _narrow(got, x.double(), y.double())
+            assert torch.equal(got.view(torch.int32), ops.mul_mat_tn(x.t().contiguous(), y.t().contiguous()).view(torch.int32))
+    for M, K, N in ((768, 26368, 256), (900, 10609, 321)):      # slices
+        a, b = (torch.randn(n, K, device="cuda", generator=g) for n in (M, N))
+        for first in (True, False):
+            x, y = _spikes(g, a, b, size, where) if first else _spikes(g, b, a, size, where)[::-1]
+            _narrow(ops.mul_mat_tn(x.t().contiguous(), y.t().contiguous(), 0.5), x.double(), y.double(), 0.5)
+    for D, L, N in ((32, 96, 256), (32, 103, 130)):             # outer-product-mean and its gradients
+        left, right = (torch.randn(D * L, N, device="cuda", generator=g) for _ in range(2))
+        x, y = _spikes(g, left, right, size, where)
+        out = ops.outer_product_mean(x.reshape(-1), y.reshape(-1), D, L, N, 1)
+        _narrow(out.reshape(D, D, L, L).permute(0, 2, 1, 3).reshape(D * L, D * L), x.double(), y.double(), 1.0 / N)
+        grad = torch.randn(D * L, D * L, device="cuda", generator=g)
+        # enormous gradients of residues whose projection is zero, on the right for one gradient, on the left for the other
+        gr_l, right0 = _spikes(g, grad, right.t().contiguous(), size, where)
+        gr_r, left0 = _spikes(g, grad.t().contiguous(), left.t().contiguous(), size, where)
+        for full, l, r in ((gr_l, left, right0.t().contiguous()), (gr_r.t().contiguous(), left0.t().contiguous(), right)):
+            g4 = full.reshape(D, L, D, L).permute(0, 2, 1, 3).contiguous()
+            dl, dr = ops.outer_prod_mean_back(g4.reshape(-1), l.reshape(-1), r.reshape(-1), D, L, N, 1)
+            if full is gr_l:
+                _narrow(dl.reshape(D * L, N), full.double(), r.double().t().contiguous(), 1.0 / N)
+            else:
+                _narrow(dr.reshape(D * L, N), full.double().t().contiguous(), l.double().t().contiguous(), 1.0 / N)
+
+
+def test_large_elements_in_a_few_rows_and_rows_that_grow(ops):
+    """A spike in single rows, rows whose later elements are larger by 2^100 and meet zeros (what the sums held by then leaves
+    binary32's range), rows and columns of zeros between them, a bias, and rows far below the smallest normal number"""
+    g = torch.Generator(device="cuda").manual_seed(11)
+    M, K, N = 20011, 136, 1004
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g)
+    b[:, 70:] = 0
+    a[5, 100] = 1e20
+    a[300:310, 71] = -3e8
+    for k, e in ((0, -90), (33, -50), (66, 0), (100, 60), (130, 120)):
+        a[700:720, k:] = torch.randn(20, K - k, device="cuda", generator=g) * 2.0 ** e
+    a[1000:1003] = 0
+    a[2000:2010] *= 2.0 ** -122
+    b[17] = 0
+    b[40:44, 3] = 1e15
+    a[:, 3] *= (torch.arange(M, device="cuda") % 2).float()
+    bias = torch.randn(N, device="cuda", generator=g)
+    _narrow(ops.mul_mat(a, b), a.double(), b.double())
+    got = ops.mul_mat(a, b, bias).double()
+    want, size = a.double() @ b.double().t() + bias.double(), a.double().abs() @ b.double().abs().t() + bias.double().abs()
+    assert bool(((got - want).abs() <= 2.0 ** -20 * size).all())
+    assert not bool(ops.mul_mat(a, b)[1000:1003].any()) and not bool(ops.mul_mat(a, b)[:, 17].any())
