@@ -211,13 +211,17 @@ int mul_mat_tn_hip(const float *A, const float *Bm, float *O, int M, int K, int 
                    ppml_hip_stream_t stream);
 
 /* mul_mat_tn_hip for callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses
- * that forbid hipMalloc): the same contraction with the same kernels and the same bits, but the workspace the
- * large cases need (the bf16 planes of both operands, 6 bytes per padded operand element, plus the partial sums
- * of K slices) is a static 64 MiB device array of the library instead of a pool allocation.  It has no
- * counterpart in the reference.  The call allocates and frees nothing and records no statistics.  A contraction
- * whose workspace exceeds 64 MiB is refused with status 1 and a message that names both sizes (for two square
+ * that forbid hipMalloc): the same contraction with the same kernels and the same bits, but the workspace that
+ * some cases need (two halves: 4 bytes per padded element of the smaller operand; bf16 planes of both operands: 6
+ * bytes per padded element; both plus the partial sums of K slices; K slices alone: their partial sums) is a static
+ * 64 MiB device array of the library instead of a pool allocation.  It has no
+ * counterpart in the reference.  The call allocates and frees nothing and records no statistics.  A contraction of at
+ * least 512 work-groups of 256 x 128 outputs, or of K slices with 2^20 outputs or more, whose bf16 planes exceed 64 MiB
+ * is refused with status 1 and a message that names both sizes (for two square
  * operands without K slices that is (M_pad + N_pad) * K_pad * 6 bytes, M padded to 256, N to 128, K to 16:
- * e.g. 12288 x 256 x 12288 takes 36 MiB); contractions that need no workspace run whatever their size.  The
+ * e.g. 12288 x 256 x 12288 takes 36 MiB); any other runs, in a form without workspace where the one that
+ * mul_mat_tn_hip takes does not fit into the array (more than 16 Mi elements in the smaller operand, 16 Mi partial sums): the
+ * bits are then those of the exact split.  The
  * array's address on a device is looked up by ppml_hip_init(device) -- or by the first call on a device that
  * was never initialised, so call ppml_hip_init first where even that lookup is unwelcome.  All calls on one GPU
  * share that GPU's array: calls that overlap in time on one GPU (two streams, two threads) race; order them. */

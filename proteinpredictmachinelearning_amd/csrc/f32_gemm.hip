@@ -2217,9 +2217,6 @@ int f32_arithmetic() {
     return t_f32_arithmetic;
 }
 
-// `fixed_ws` / `fixed_cap`: a workspace the caller brings (the static array of the entry point that allocates
-// nothing).  With one, the pool is never touched: a contraction that wants more workspace than `fixed_cap`
-// is refused, one that wants none runs as it always does.
 // gemm_bf16x3_half_split_kernel for a single-plane contraction whose tall operand A has compound indices; -1 when the
 // contraction is not of that kind (the caller goes on to the other forms).  p.tiles_m / p.tiles_n / p.stream_c are set.
 int try_half_split(const GemmParams& p, hipStream_t stream, const char* what) {
@@ -2277,7 +2274,7 @@ int try_half_split(const GemmParams& p, hipStream_t stream, const char* what) {
 // gemm_bf16x3_pc_slices_kernel for a single dense plane with few output tiles under a long K; -1 when the contraction
 // is not of that kind or no workspace is to be had (the caller goes on to the unsliced forms).
 template <int MODE>
-int try_pc_slices(const GemmParams& p, hipStream_t stream, const char* what) {
+int try_pc_slices(const GemmParams& p, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap) {
     const int chunks = (p.K + BK - 1) / BK;
     const int groups = p.tiles_m * p.tiles_n;
     // (two launches: about 10 us before the first chunk.  us over K for one to nine tiles, unsliced: 256 12, 400 16.5,
@@ -2291,7 +2288,7 @@ int try_pc_slices(const GemmParams& p, hipStream_t stream, const char* what) {
     slices = (chunks + slice_chunks - 1) / slice_chunks;
     const int ma_pad = p.tiles_m * BM, nb_pad = p.tiles_n * BN;
     const size_t part_bytes = static_cast<size_t>(slices) * ma_pad * nb_pad * 4;
-    const Workspace held = workspace_take(part_bytes, stream);
+    const Workspace held = workspace_take(part_bytes, stream, fixed_ws, fixed_cap);
     uint8_t* ws = held.ptr;
     if (!ws) return -1;
     float* partial = reinterpret_cast<float*>(ws);
@@ -2314,8 +2311,8 @@ int try_pc_slices(const GemmParams& p, hipStream_t stream, const char* what) {
 }
 
 template <int MODE>
-bool try_pc_slices_done(const GemmParams& p, hipStream_t stream, const char* what, int& rc) {
-    rc = try_pc_slices<MODE>(p, stream, what);
+bool try_pc_slices_done(const GemmParams& p, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap, int& rc) {
+    rc = try_pc_slices<MODE>(p, stream, what, fixed_ws, fixed_cap);
     return rc >= 0;
 }
 
@@ -2373,6 +2370,9 @@ int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what
     return check_launch(what);
 }
 
+// `fixed_ws` / `fixed_cap`: a workspace the caller brings (the static array of the entry point that allocates
+// nothing).  With one, the pool is never touched: a contraction whose bf16 planes would be larger than `fixed_cap`
+// is refused, any other runs, in the form that it takes without one where that fits.
 int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fixed_ws = nullptr, size_t fixed_cap = 0) {
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
@@ -2409,8 +2409,9 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
     }
     const bool planes_fit = slices > 1 ? planes_groups * slices >= PLANES_MIN_GROUPS / 2 && static_cast<int64_t>(p.M) * p.N >= (1 << 20)
                                        : p.tiles_m >= PLANES_MIN_TILES && p.tiles_n >= PLANES_MIN_TILES && planes_groups >= PLANES_MIN_GROUPS;
-    if (!fp32_pipe && !fixed_ws) {
-        const int rc = try_f16x2(p, stream, what, nullptr, 0);
+    // (a caller's own workspace that the bf16 planes do not fit is refused below, whatever this form would take)
+    if (!fp32_pipe && !(fixed_ws && planes_fit)) {
+        const int rc = try_f16x2(p, stream, what, fixed_ws, fixed_cap);
         if (rc >= 0) return rc;
     }
     if (!fp32_pipe && !fixed_ws && p.a_lm > 0) {
@@ -2544,8 +2545,8 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
                 return check_launch(what);
             }
         }
-        if (!fixed_ws) {
-            const int rc = try_pc_slices<LOAD_ROW_CONTIG>(p, stream, what);
+        {
+            const int rc = try_pc_slices<LOAD_ROW_CONTIG>(p, stream, what, fixed_ws, fixed_cap);
             if (rc >= 0) return rc;
         }
         if (p.K > 3 * BK && (p.N <= 32) != (p.M <= 32)) {
@@ -2575,7 +2576,7 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
                             ((p.M - 1) * p.a_rs + p.K) * 4 < (1LL << 31) && ((p.N - 1) * p.b_rs + p.K) * 4 < (1LL << 31) &&
                             p.M * p.c_mi * 4 < (1LL << 31) && p.c_mi < (1 << 22) && p.a_rs < (1 << 22) && p.b_rs < (1 << 22);
         // few tiles under a long K (a LinearLayer's weight gradient) go in K slices, whatever their width
-        if (k_fast && !fixed_ws && try_pc_slices_done<LOAD_K_CONTIG>(p, stream, what, slices_rc)) return slices_rc;
+        if (k_fast && try_pc_slices_done<LOAD_K_CONTIG>(p, stream, what, fixed_ws, fixed_cap, slices_rc)) return slices_rc;
         // (a narrow side of a single plane too, while 64 x 64 tiles leave CUs idle: half of such a tile is empty, but two chunks
         // a barrier make its chain shorter.  us, 128 x 32 / 64 x 64: 51 x 256 -> 8  9.4 / 6.6, 10609 x 256 -> 12
         // 9.8 / 7.2, 16384 x 376 -> 32  13.1 / 9.8; two tiles per CU, 26368 x 256 -> 8  9.9 / 10.1)

@@ -30,6 +30,15 @@ struct GemmParams {
     int64_t a_mo, a_mi, a_ko, a_ki;
 };
 
+// Workspace of a contraction: the pool's, or out of the array that the caller brings (`fixed`, of `cap` bytes: the pool is then
+// never touched); null where there is none.  Given back by workspace_give either way.
+inline Workspace workspace_take(size_t bytes, hipStream_t stream, uint8_t* fixed, size_t cap) {
+    if (!fixed) return workspace_take(bytes, stream);
+    Workspace ws;
+    ws.ptr = bytes <= cap ? fixed : nullptr;
+    return ws;
+}
+
 // gemm_f16x2.hip: a large single-plane contraction in two f16 parts; -1 when the contraction is not of the kind that form is
 // for or no workspace is to be had.  `fixed_ws` / `fixed_cap`: a workspace the caller brings.
 int try_f16x2(const GemmParams& p, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap);

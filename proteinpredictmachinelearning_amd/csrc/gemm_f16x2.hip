@@ -960,15 +960,9 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     const int most_items = static_cast<int>(((tiles * slices + 7) / 8 + wgs / 8 - 1) / (wgs / 8));
     const size_t n_bytes = (static_cast<size_t>(wgs) * 4 * most_items * 8 + 255) / 256 * 256;
     const size_t need = b_bytes + e_bytes + n_bytes + part_bytes;
-    uint8_t* ws = fixed_ws;
-    Workspace held;
-    if (fixed_ws) {
-        if (need > fixed_cap) return -1;
-    } else {
-        held = workspace_take(need, stream);
-        ws = held.ptr;
-        if (!ws) return -1;
-    }
+    const Workspace held = workspace_take(need, stream, fixed_ws, fixed_cap);
+    uint8_t* const ws = held.ptr;
+    if (!ws) return -1;
     F16x2Job jb{};
     jb.wb = ws;
     uint32_t* const exps = reinterpret_cast<uint32_t*>(ws + b_bytes);
@@ -1012,7 +1006,7 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
         rc = check_launch(what);
     }
     if (rc == RC_OK && partial) rc = launch_reduce_slices(p, stream, what, jb.partial, slices, ma_pad, nb_pad);
-    if (!fixed_ws) workspace_give(held, stream);
+    workspace_give(held, stream);
     return rc;
 }
 

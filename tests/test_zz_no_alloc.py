@@ -18,14 +18,16 @@ def _call(fn, a, b, out, M, K, N, alpha):
     return fn(C.c_void_p(a.data_ptr()), C.c_void_p(b.data_ptr()), C.c_void_p(out.data_ptr()), M, K, N, alpha, stream)
 
 
-def test_no_alloc_entry_point_matches_the_allocating_one_on_calls_in_a_row():
+# (then those too small for planes ahead: in two halves, tall and in K slices, and K slices of the exact split)
+@pytest.mark.parametrize("more", [[], [(26368, 256, 768), (26368, 256, 256), (768, 26368, 256), (64, 8192, 64), (321, 4100, 100)]])
+def test_no_alloc_entry_point_matches_the_allocating_one_on_calls_in_a_row(more):
     from proteinpredictmachinelearning_amd import cabi, ops
 
     lib = ops._lib()                                    # loads the library and runs ppml_hip_init on the device
     g = torch.Generator(device="cuda").manual_seed(77)
     # (M, K, N): a large one whose planes take 36 of the 64 MiB; a smaller one that still splits ahead; one that
     # is cut into K slices (planes + partial sums, 61.5 MiB); one small enough to need no workspace at all
-    shapes = [(12288, 256, 12288), (4100, 77, 3900), (1024, 2048, 1030), (300, 64, 200)]
+    shapes = [(12288, 256, 12288), (4100, 77, 3900), (1024, 2048, 1030), (300, 64, 200)] + more
     cases = []
     for M, K, N in shapes:
         a = torch.randn(K, M, device="cuda", generator=g) * 0.1
