@@ -62,8 +62,9 @@ void ppml_hip_backend_set_q8_1_activations(ppml_hip_backend *b, int on);
  * tensors are never written.  0 (default): every node is executed as it stands. */
 void ppml_hip_backend_set_fuse_attention_bridges(ppml_hip_backend *b, int on);
 /* Folding of element-wise nodes into the contraction beside them.  The rule is the reference's own for eliminating
- * an intermediate (exactly one reader in the graph, include/ppml/ComputeGraph.h:73-87), plus "not marked OUTPUT";
- * a folded tensor is never written.
+ * an intermediate (exactly one reader in the graph, include/ppml/ComputeGraph.h:73-87), plus "not marked OUTPUT" and
+ * "its sources stand until the node runs that then reads them" (an allocator may hand their memory on as soon as the
+ * folded node would have run: to a node in between, or to that node itself); a folded tensor is never written.
  *   relu_into_q8 (default 1): an OP_UNARY/RELU read only -- directly or through whole OP_VIEW / OP_RESHAPE nodes --
  *     by the activation side of a quantized OP_MUL_MAT is applied by that matmul's quantizer
  *     (src/modules/Attention.cpp:1097-1104); same bits as the two nodes run one after the other.

@@ -163,7 +163,8 @@ public:
 
     // Fusion of the element-wise nodes into the contraction beside them.  The legality rule is the reference's own
     // for eliminating an intermediate (include/ppml/ComputeGraph.h:73-87): the tensor has exactly one reader in the
-    // graph handed to graph_compute; here it must also not be marked TENSOR_FLAG_OUTPUT.  A fused-away tensor is
+    // graph handed to graph_compute; here it must also not be marked TENSOR_FLAG_OUTPUT, and no node may write the memory of
+    // its sources before the node that then reads them has run.  A fused-away tensor is
     // never written.  Both are ON by default and give the same bits as the nodes run one by one:
     //   relu   -- an OP_UNARY/RELU node read only (directly or through whole OP_VIEW / OP_RESHAPE nodes) by the
     //             activation side of a quantized OP_MUL_MAT is not executed; the matmul's quantizer applies it

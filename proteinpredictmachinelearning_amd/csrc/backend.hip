@@ -729,10 +729,11 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         fuse_add_into_soft_max_ || fuse_permutes_into_out_prod_ || fuse_permutes_into_mul_mat_) {
         std::unordered_map<const Tensor*, int> uses, position;
         std::unordered_map<const Tensor*, Tensor*> single_user;
-        int pos = 0;
+        std::vector<const Tensor*> order;               // the nodes by their positions
         for (Tensor* n : *graph) {
             if (!n) continue;
-            position[n] = pos++;
+            position[n] = static_cast<int>(order.size());
+            order.push_back(n);
             bool view_counted = false;
             for (Tensor* s : n->src) if (s) { ++uses[s]; single_user[s] = n; view_counted = view_counted || s == n->view_src; }
             if (n->view_src && !view_counted) { ++uses[n->view_src]; single_user[n->view_src] = n; }
@@ -751,35 +752,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
             return t->op_params[0] == 1 && t->op_params[1] == 0 && t->op_params[2] == 2 && t->op_params[3] == 3 &&
                    t->src[0] && t->src[0]->type == TENSOR_TYPE_F32 && t->src[0]->ndim == 4 && !t->view_src;
         };
-
-        // (1) the layout bridges around fused attention nodes (ComputeGraphHelper.cpp:456-458, 483): a permutation
-        // {1,0,2,3} that feeds only the attention node, or is the only reader of its result, is not executed; the
-        // attention kernel reads / writes that layout itself.  All three inputs fuse together or not at all.
-        if (fuse_attention_bridges_) {
-            for (Tensor* n : *graph) {
-                if (!n || n->op != OP_FLASH_ATTN_EXT || !node_supported(n)) continue;
-                Plan b;
-                b.bridges_in = true;
-                for (int s = 0; s < 3; ++s) {
-                    const Tensor* pq = n->src[s];
-                    b.bridges_in = b.bridges_in && is_bridge(pq) && uses[pq] == 1 && before(pq, n);
-                }
-                // a tensor that feeds two of the three slots (self-attention on one projection) has uses == 2: not fused
-                Tensor* user = uses[n] == 1 ? single_user[n] : nullptr;
-                if (user && is_bridge(user) && user->src[0] == n && before(n, user)) b.bridge_out = user;
-                if (!b.bridges_in && !b.bridge_out) continue;
-                plans[n] = b;
-                if (b.bridges_in) for (int s = 0; s < 3; ++s) skipped.insert(n->src[s]);
-                if (b.bridge_out) skipped.insert(b.bridge_out);
-            }
-        }
-
-        // (2) the reference's default attention chain (src/modules/Attention.cpp:264-281) as one launch: the fused attention
-        // where the caller asked for it, otherwise (with the three passes below on, whose launches it replaces) the one that has
-        // the bits of the nodes, for planes of up to 128 rows.  Fewer than 32 planes stay three launches, as they were.
-        const int arithmetic_here = f32_arithmetic_ >= 0 ? f32_arithmetic_ : ppml_hip_set_f32_arithmetic(-1);
-        const bool chain_bits = !fuse_attention_chain_ && fuse_scale_into_out_prod_ && fuse_add_into_soft_max_ &&
-                                fuse_permutes_into_out_prod_ && arithmetic_here != 1;
+        // A node that stands for others reads their sources when it runs, not when they would have.  An allocator may have given
+        // the memory of a source whose last reader was folded away to a node in between, or to the node itself.
         // a tensor's memory as far as it is settled before the graph runs (what is not gets memory of its own)
         struct Range { uintptr_t lo = 0, hi = 0; };
         const auto memory_of = [](const Tensor* t) {
@@ -794,9 +768,79 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
             return m;
         };
         const auto meet = [&](const Tensor* a, const Tensor* b) {
+            if (!a || !b) return false;
             const Range x = memory_of(a), y = memory_of(b);
             return x.lo < y.hi && y.lo < x.hi;
         };
+        // m runs and writes memory of t's (the outputs of a node: as in the allocation below)
+        const auto overwrites = [&](const Tensor* m, const Tensor* t) {
+            if (m->op == OP_NONE || m->op == OP_VIEW || m->op == OP_RESHAPE || skipped.count(m)) return false;
+            if (m->op == OP_FLASH_ATTN_BACK)
+                return (m->op_params[5] != 0 && meet(m, t)) || meet(m->src[7], t) || meet(m->src[8], t) || meet(m->src[9], t);
+            const bool two_outputs = m->op == OP_TRI_MUL_BACK || m->op == OP_OUTER_PROD_MEAN_BACK;
+            const auto plan = plans.find(m);
+            return meet(m, t) || ((two_outputs || m->op == OP_FLASH_ATTN_EXT) && meet(m->src[4], t)) || (two_outputs && meet(m->src[3], t)) ||
+                   (plan != plans.end() && meet(plan->second.bridge_out, t));
+        };
+        // what `from` reads of t can be read by `n` instead (nodes folded away in between are in `skipped` already)
+        const auto stands_until = [&](const Tensor* from, const Tensor* n, const Tensor* t) {
+            if (!t) return true;
+            for (int i = position[from] + 1, end = position[n]; i < end; ++i)
+                if (overwrites(order[i], t)) return false;
+            return !meet(n, t);
+        };
+        // takes nodes out of the graph if `legal` then holds
+        const auto fold = [&](std::initializer_list<const Tensor*> nodes, const auto& legal) {
+            std::vector<const Tensor*> added;
+            for (const Tensor* t : nodes) if (t && skipped.insert(t).second) added.push_back(t);
+            if (legal()) return true;
+            for (const Tensor* t : added) skipped.erase(t);
+            return false;
+        };
+
+        // (1) the layout bridges around fused attention nodes (ComputeGraphHelper.cpp:456-458, 483): a permutation
+        // {1,0,2,3} that feeds only the attention node, or is the only reader of its result, is not executed; the
+        // attention kernel reads / writes that layout itself.  All three inputs fuse together or not at all.
+        if (fuse_attention_bridges_) {
+            for (Tensor* n : *graph) {
+                if (!n || n->op != OP_FLASH_ATTN_EXT || !node_supported(n)) continue;
+                Plan b;
+                b.bridges_in = true;
+                for (int s = 0; s < 3; ++s) {
+                    const Tensor* pq = n->src[s];
+                    b.bridges_in = b.bridges_in && is_bridge(pq) && uses[pq] == 1 && before(pq, n);
+                }
+                b.bridges_in = b.bridges_in && fold({n->src[0], n->src[1], n->src[2]}, [&] {
+                    for (int s = 0; s < 3; ++s)
+                        if (!stands_until(n->src[s], n, n->src[s]->src[0]) || meet(n->src[4], n->src[s]->src[0])) return false;
+                    return true;
+                });
+                // a tensor that feeds two of the three slots (self-attention on one projection) has uses == 2: not fused
+                Tensor* user = uses[n] == 1 ? single_user[n] : nullptr;
+                if (user && is_bridge(user) && user->src[0] == n && before(n, user)) {
+                    // the attention node then writes the permutation's memory: nobody reads or writes that until the permutation would have
+                    b.bridge_out = user;
+                    for (int i = position[n], end = position[user]; i < end && b.bridge_out; ++i) {
+                        const Tensor* m = order[i];
+                        if (m != n && overwrites(m, user)) b.bridge_out = nullptr;
+                        for (int s = 0; s < 10 && b.bridge_out; ++s) {
+                            const bool permuted = m == n && b.bridges_in && s < 3;
+                            if (!skipped.count(m) && meet(permuted ? m->src[s]->src[0] : m->src[s], user)) b.bridge_out = nullptr;
+                        }
+                    }
+                }
+                if (!b.bridges_in && !b.bridge_out) continue;
+                plans[n] = b;
+                if (b.bridge_out) skipped.insert(b.bridge_out);
+            }
+        }
+
+        // (2) the reference's default attention chain (src/modules/Attention.cpp:264-281) as one launch: the fused attention
+        // where the caller asked for it, otherwise (with the three passes below on, whose launches it replaces) the one that has
+        // the bits of the nodes, for planes of up to 128 rows.  Fewer than 32 planes stay three launches, as they were.
+        const int arithmetic_here = f32_arithmetic_ >= 0 ? f32_arithmetic_ : ppml_hip_set_f32_arithmetic(-1);
+        const bool chain_bits = !fuse_attention_chain_ && fuse_scale_into_out_prod_ && fuse_add_into_soft_max_ &&
+                                fuse_permutes_into_out_prod_ && arithmetic_here != 1;
         if (fuse_attention_chain_ || chain_bits) {
             for (Tensor* n : *graph) {
                 if (!n || n->op != OP_OUT_PROD || n->type != TENSOR_TYPE_F32 || n->ndim != 4) continue;
@@ -837,29 +881,17 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                     for (const Tensor* t : {static_cast<const Tensor*>(scores), static_cast<const Tensor*>(x), static_cast<const Tensor*>(added),
                                             static_cast<const Tensor*>(attn), static_cast<const Tensor*>(attn_t), static_cast<const Tensor*>(v_t)})
                         if (t) free = free && node_supported(t) && !t->data && !t->buffer;
-                    // Q, K and the bias are read when the last node runs: nothing in between may write there, nor that node itself
-                    for (const Tensor* r : {static_cast<const Tensor*>(q), static_cast<const Tensor*>(k), static_cast<const Tensor*>(v), static_cast<const Tensor*>(bias)})
-                        if (r) free = free && !meet(n, r);
-                    for (Tensor* m : *graph) {
-                        if (!free) break;
-                        if (m == x || m == added || m == attn || m == attn_t || m == v_t || !before(scores, m) || !before(m, n)) continue;
-                        if (m->op == OP_NONE || m->op == OP_VIEW || m->op == OP_RESHAPE) continue;
-                        free = (m->op == OP_MUL_MAT || m->op == OP_OUT_PROD || m->op == OP_PERMUTE || m->op == OP_TRANSPOSE || m->op == OP_ADD ||
-                                m->op == OP_SCALE || m->op == OP_UNARY || m->op == OP_SOFT_MAX) &&
-                               !meet(m, q) && !meet(m, k) && !(bias && meet(m, bias));
-                    }
                     if (!free) continue;
                 }
+                if (!fold({attn_t, v_t, attn, added, x, scores}, [&] {
+                        return stands_until(scores, n, k) && stands_until(scores, n, q) && stands_until(added, n, bias) && stands_until(v_t, n, v);
+                    })) continue;
                 Plan c;
                 c.chain = true;
                 c.chain_bits = chain_bits;
                 c.q = q; c.k = k; c.v = v; c.bias = bias;
                 c.scale = x->param_f32(0);
                 plans[n] = c;
-                for (const Tensor* t : {static_cast<const Tensor*>(attn_t), static_cast<const Tensor*>(v_t),
-                                        static_cast<const Tensor*>(attn), static_cast<const Tensor*>(added),
-                                        static_cast<const Tensor*>(x), static_cast<const Tensor*>(scores)})
-                    if (t) skipped.insert(t);
             }
         }
 
@@ -883,10 +915,10 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 }
                 if (!t || t->op != OP_UNARY || t->op_params[0] != UNARY_OP_RELU || !private_to(t, reader)) continue;
                 if (!t->src[0] || t->src[0]->type != TENSOR_TYPE_F32 || t->src[0]->numel() != t->numel()) continue;
+                if (!fold({t}, [&] { return stands_until(t, n, t->src[0]); })) continue;
                 Plan& r = plans[n];
                 r.relu_slot = slot;
                 r.relu = t;
-                skipped.insert(t);
             }
         }
 
@@ -896,8 +928,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 if (!n || n->op != OP_SCALE || skipped.count(n) || !node_supported(n)) continue;
                 Tensor* p = n->src[0];
                 if (!p || p->op != OP_OUT_PROD || !node_supported(p) || !private_to(p, n) || p->numel() != n->numel()) continue;
+                if (!fold({p}, [&] { return stands_until(p, n, p->src[0]) && stands_until(p, n, p->src[1]); })) continue;
                 plans[n].out_prod = p;
-                skipped.insert(p);
             }
         }
 
@@ -912,8 +944,14 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 const int64_t row = n->dims[0];
                 if (!full || !bias || full->type != TENSOR_TYPE_F32 || bias->type != TENSOR_TYPE_F32 || full->numel() != x->numel() ||
                     row <= 0 || bias->numel() <= 0 || bias->numel() % row != 0 || (x->numel() / row) % (bias->numel() / row) != 0) continue;
+                // (the row that a wave writes is the one that it holds: in place on the first operand's memory is fine)
+                const Range mine = memory_of(n), first = memory_of(full);
+                const bool in_place = mine.lo == first.lo && mine.hi == first.hi;
+                if (!fold({x}, [&] {
+                        for (int i = position[x] + 1, end = position[n]; i < end; ++i) if (overwrites(order[i], full)) return false;
+                        return (in_place || !meet(n, full)) && stands_until(x, n, bias);
+                    })) continue;
                 plans[n].added = x;
-                skipped.insert(x);
             }
         }
 
@@ -928,9 +966,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 Tensor* p1 = n->src[1];
                 if (p0 == p1 || !is_bridge(p0) || !is_bridge(p1) || !private_to(p0, n) || !private_to(p1, n)) continue;
                 if (p0->src[0]->numel() != p0->numel() || p1->src[0]->numel() != p1->numel()) continue;
+                if (!fold({p0, p1}, [&] { return stands_until(p0, n, p0->src[0]) && stands_until(p1, n, p1->src[0]); })) continue;
                 plans[n].transposed = true;
-                skipped.insert(p0);
-                skipped.insert(p1);
             }
         }
 
@@ -950,9 +987,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 Tensor* p0 = n->src[0];
                 Tensor* p1 = n->src[1];
                 if (p0 == p1 || !is_mat_t(p0) || !is_mat_t(p1) || !private_to(p0, n) || !private_to(p1, n)) continue;
+                if (!fold({p0, p1}, [&] { return stands_until(p0, n, p0->src[0]) && stands_until(p1, n, p1->src[0]); })) continue;
                 plans[n].transposed = true;
-                skipped.insert(p0);
-                skipped.insert(p1);
             }
         }
         nodes_fused_away_ = skipped.size();
