@@ -379,10 +379,8 @@ int launch_flash(AttnParams p, hipStream_t stream) {
     const int stages = (l32 + T::CH - 1) / T::CH;
     p.stage_rows = (l32 / 32 + stages - 1) / stages * 32;
     const size_t lds = static_cast<size_t>(p.stage_rows / 32) * (T::KT_BYTES + T::VT_BYTES);
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(T::lds_bytes));
-    if (attr != hipSuccess) {
-        (void)hipGetLastError();
+    static LdsLimit limit;
+    if (!limit.reserve(reinterpret_cast<const void*>(kernel), T::lds_bytes)) {
         set_error("flash_attn_forward_hip: cannot reserve %zu bytes of LDS", T::lds_bytes);
         return RC_LAUNCH;
     }

@@ -924,10 +924,8 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_fused_kernel(const
 template <int NW, bool BIAS, int DB, bool CAUSAL>
 int launch_fused(const AttnBackParams& p, hipStream_t stream) {
     using F = FusedBack<NW>;
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_attn_back_fused_kernel<NW, BIAS, DB, CAUSAL>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(F::LDS));
-    if (attr != hipSuccess) {
-        (void)hipGetLastError();
+    static LdsLimit limit;
+    if (!limit.reserve(reinterpret_cast<const void*>(&flash_attn_back_fused_kernel<NW, BIAS, DB, CAUSAL>), F::LDS)) {
         set_error("flash_attn_backward_hip: cannot reserve the LDS of the one-pass kernel");
         return RC_LAUNCH;
     }
@@ -943,11 +941,9 @@ int launch_rows(AttnBackParams p, hipStream_t stream) {
     const int l32 = (p.L + 31) / 32 * 32;
     p.stage_rows = l32 < T::CH_ROWS ? l32 : T::CH_ROWS;
     const size_t lds = static_cast<size_t>(p.stage_rows / 32) * (2 * T::ROW_BYTES + T::COL_BYTES);
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_attn_back_rows_kernel<DP, NW, TWIN, BIAS, LATE>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       (T::CH_ROWS / 32) * (2 * T::ROW_BYTES + T::COL_BYTES));
-    if (attr != hipSuccess) {
-        (void)hipGetLastError();
+    static LdsLimit limit;
+    if (!limit.reserve(reinterpret_cast<const void*>(&flash_attn_back_rows_kernel<DP, NW, TWIN, BIAS, LATE>),
+                       (T::CH_ROWS / 32) * (2 * T::ROW_BYTES + T::COL_BYTES))) {
         set_error("flash_attn_backward_hip: cannot reserve the LDS of the rows kernel");
         return RC_LAUNCH;
     }
@@ -980,11 +976,9 @@ int launch_back(AttnBackParams p, hipStream_t stream) {
         p.stage_rows = l32 < T::CH_COLS ? l32 : T::CH_COLS;
         const size_t lds = static_cast<size_t>(p.stage_rows / 32) * (2 * T::ROW_BYTES + 2 * T::COL_BYTES) +
                            static_cast<size_t>(p.stage_rows) * 2 * sizeof(float);
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_attn_back_cols_kernel<DP, NW>),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                           (T::CH_COLS / 32) * (2 * T::ROW_BYTES + 2 * T::COL_BYTES) + T::CH_COLS * 8);
-        if (attr != hipSuccess) {
-            (void)hipGetLastError();
+        static LdsLimit limit;
+        if (!limit.reserve(reinterpret_cast<const void*>(&flash_attn_back_cols_kernel<DP, NW>),
+                           (T::CH_COLS / 32) * (2 * T::ROW_BYTES + 2 * T::COL_BYTES) + T::CH_COLS * 8)) {
             set_error("flash_attn_backward_hip: cannot reserve the LDS of the columns kernel");
             return RC_LAUNCH;
         }

@@ -279,10 +279,8 @@ int launch_chain(const ChainParams& p, hipStream_t stream) {
         const int k = tiles_ * 6144, s = tiles_ * 32 * pitch * 4;
         return chunks_ * 3072 + (k > s ? k : s);
     };
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       bytes(CHAIN_ROWS / 16, CHAIN_ROWS / 32, CHAIN_ROWS + 4));
-    if (attr != hipSuccess) {
-        (void)hipGetLastError();
+    static LdsLimit limit;
+    if (!limit.reserve(reinterpret_cast<const void*>(kernel), bytes(CHAIN_ROWS / 16, CHAIN_ROWS / 32, CHAIN_ROWS + 4))) {
         set_error("attention_chain: cannot reserve its LDS");
         return RC_LAUNCH;
     }

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <cstdarg>
@@ -49,6 +50,26 @@ Workspace workspace_take(size_t bytes, hipStream_t stream);
 void workspace_give(const Workspace& ws, hipStream_t stream);
 int noalloc_scratch_setup(uint8_t** out);   // address of the no-allocation entry point's static workspace on the current device
 int device_cu_count();
+// The dynamic LDS that a kernel may be launched with: a limit of the kernel on a device, set by the first launch there.  One
+// object per kernel, static where it is launched.
+class LdsLimit {
+public:
+    bool reserve(const void* kernel, size_t bytes) {
+        int dev = -1;
+        if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); dev = -1; }
+        const uint64_t bit = dev >= 0 && dev < 64 ? 1ull << dev : 0;
+        if ((set_.load(std::memory_order_acquire) & bit) != 0) return true;
+        if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        set_.fetch_or(bit, std::memory_order_release);
+        return true;
+    }
+
+private:
+    std::atomic<uint64_t> set_{0};                      // a bit per device
+};
 // The default attention's nodes in one launch (attention_chain.hip): Q, K, V, O [planes][d][L], bias [planes][L][L] or null
 bool attention_chain_fits(int64_t planes, int64_t L, int64_t d);
 int attention_chain(const float* Q, const float* K, const float* V, const float* bias, float* O, int64_t planes, int L, int d, float scale,

@@ -1257,20 +1257,10 @@ int launch_q8_linear_ws(const void* W, const float* X, float* C, int M, int N, i
         dump = &q8_linear_ws64_kernel<NW, TPW, NBLK, WL, true, Q81, CSPLIT>;
     }
     if (lds > 64 * 1024) {
-        // (once per instance; where the launcher chooses between two forms of the kernel, once per form)
-        static hipError_t attr_fast[2] = {hipErrorNotReady, hipErrorNotReady}, attr_dump[2] = {hipErrorNotReady, hipErrorNotReady};
-        static std::mutex attr_lock;
-        {
-            std::lock_guard<std::mutex> hold(attr_lock);
-            if (attr_fast[early] == hipErrorNotReady) {
-                attr_fast[early] = hipFuncSetAttribute(reinterpret_cast<const void*>(fast), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-                attr_dump[early] = hipFuncSetAttribute(reinterpret_cast<const void*>(dump), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-            }
-        }
-        if (attr_fast[early] != hipSuccess || attr_dump[early] != hipSuccess) {
-            (void)hipGetLastError();
+        // (where the launcher chooses between two forms of the kernel, a limit for each)
+        static LdsLimit limit_fast[2], limit_dump[2];
+        if (!limit_fast[early].reserve(reinterpret_cast<const void*>(fast), lds) || !limit_dump[early].reserve(reinterpret_cast<const void*>(dump), lds))
             return -1;                                  // fall back to the general kernel
-        }
     }
     if (xq_dump || sums_dump)
         hipLaunchKernelGGL(dump, grid, block, lds, stream, static_cast<const uint8_t*>(W), X, C, M, N, ntiles, npart, relu,

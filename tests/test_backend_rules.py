@@ -3,9 +3,12 @@
 The table restates what the reference's CUDA backend answers for the three ops of this path
 (src/backend/CUDABackend.cpp:121-163 OP_MUL_MAT, OP_OUT_PROD; 410-416 OP_OUTER_PROD_MEAN).
 """
+import os
+
 import pytest
 
 from proteinpredictmachinelearning_amd import backend as B
+from proteinpredictmachinelearning_amd import cabi
 
 
 def _mm(t0, t1, out=B.F32, bias=None, k0=64, k1=64):
@@ -148,3 +151,12 @@ def test_supports_op_fused_attention_backward():
         assert B.supports_op(B.Tensor((10, 10, 2, 1), B.F32, B.OP_FLASH_ATTN_BACK, [q])) == want, d
     assert not B.supports_op(B.Tensor((10, 10, 2, 1), B.F32, B.OP_FLASH_ATTN_BACK, []))
     assert not B.supports_op(B.Tensor((10, 10, 2, 1), B.F32, B.OP_FLASH_ATTN_BACK, [B.Tensor((32, 10, 2, 1), B.F16)]))
+
+
+def test_the_lds_limit_of_a_kernel_is_set_for_every_device():
+    """hipFuncSetAttribute acts on the current device.  One class sets the limit, once per kernel and device (LdsLimit); a
+    launcher that remembers its own call would leave the limit unset on every device but the first."""
+    csrc = os.path.join(os.path.dirname(cabi.__file__), "csrc")
+    users = [f for f in sorted(os.listdir(csrc)) if f.endswith((".hip", ".hpp"))
+             and "hipFuncSetAttribute" in open(os.path.join(csrc, f)).read()]
+    assert users == ["common.hpp"]
