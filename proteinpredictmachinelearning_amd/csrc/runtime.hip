@@ -218,7 +218,7 @@ Workspace workspace_take(size_t bytes, hipStream_t stream) {
     // (a replay then reads and writes memory that is not theirs -- an illegal access on the device).  The caller takes
     // the form of its operation that needs no workspace; mul_mat_tn_noalloc_hip brings the forms that do to recorded code.
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (stream != nullptr && stream != hipStreamPerThread && hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
+    if (stream != nullptr && hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
         (void)hipGetLastError();
         capturing = hipStreamCaptureStatusActive;        // (cannot tell: treat it as the careful case)
     }

@@ -186,3 +186,40 @@ def test_large_elements_in_a_few_rows_and_rows_that_grow(ops):
     want, size = a.double() @ b.double().t() + bias.double(), a.double().abs() @ b.double().abs().t() + bias.double().abs()
     assert bool(((got - want).abs() <= 2.0 ** -20 * size).all())
     assert not bool(ops.mul_mat(a, b)[1000:1003].any()) and not bool(ops.mul_mat(a, b)[:, 17].any())
+
+
+@pytest.mark.parametrize("per_thread", [False, True])
+def test_recorded_calls_take_no_workspace(ops, per_thread):
+    """Contractions that take a workspace, recorded into a graph from a stream of the caller's and from the per-thread default
+    stream: an allocation made meanwhile would be gone by the time the graph runs.  Replayed with other work in between, on other
+    operands each time; the bits are those of the forms without workspace, the result the eager one's."""
+    import ctypes as C
+
+    from proteinpredictmachinelearning_amd import cabi
+
+    lib = cabi.load()                                   # (its handle finds the runtime that it is bound to, too)
+    ops._lib()
+    own = torch.cuda.Stream()
+    stream = C.c_void_p(2 if per_thread else own.cuda_stream)         # 2: hipStreamPerThread
+    g = torch.Generator(device="cuda").manual_seed(8)
+    cases = [(torch.randn(M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g), torch.empty(M, N, device="cuda"))
+             for M, K, N in ((26368, 256, 200), (64, 8192, 64))]
+    torch.cuda.synchronize()
+    graph, exe = C.c_void_p(), C.c_void_p()
+    assert lib.hipStreamBeginCapture(stream, 2) == 0
+    for a, b, c in cases:
+        cabi.check("mul_mat_hip", lib.mul_mat_hip(a.data_ptr(), b.data_ptr(), c.data_ptr(), a.shape[0], a.shape[1], b.shape[0], None, stream))
+    assert lib.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert lib.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+    for _ in range(3):
+        for a, b, c in cases:
+            a.normal_(generator=g)
+            c.fill_(float("nan"))
+        torch.cuda.synchronize()
+        assert lib.hipGraphLaunch(exe, stream) == 0
+        torch.cuda.synchronize()
+        for a, b, c in cases:
+            _within(c, a.double(), b.double())
+            eager = ops.mul_mat(a, b).double()
+            assert bool(((c.double() - eager).abs() <= 2.0 ** -19 * (a.double().abs() @ b.double().abs().t())).all())
+    assert lib.hipGraphExecDestroy(exe) == 0 and lib.hipGraphDestroy(graph) == 0
