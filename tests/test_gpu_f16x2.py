@@ -188,6 +188,33 @@ def test_large_elements_in_a_few_rows_and_rows_that_grow(ops):
     assert not bool(ops.mul_mat(a, b)[1000:1003].any()) and not bool(ops.mul_mat(a, b)[:, 17].any())
 
 
+# One constant in all elements: the errors of the parts add up instead of averaging out
+def test_constants_with_the_largest_rounding(ops):
+    x, y = 1 + 2.0 ** -11 - 2.0 ** -23, 1 + 2.0 ** -10 - 2.0 ** -11 + 3 * 2.0 ** -23
+    a, b = torch.full((20011, 128), x, device="cuda"), torch.full((1004, 128), y, device="cuda")
+    want = 128 * float(np.float32(x)) * float(np.float32(y))
+    # the parts' 2^-21, and eight binary32 additions of sixteen products
+    assert bool(((ops.mul_mat(a, b).double() - want).abs() <= (2.0 ** -21 + 8 * 2.0 ** -24) * want).all())
+
+
+# A bound that does not grow with K, which operands without their low halves (or a product that is left out) fail
+@pytest.mark.parametrize("M,K,N", [(20011, 136, 1004), (768, 26368, 256), (900, 10609, 321), (1024, 4100, 1030)])
+def test_the_low_halves_are_there(ops, M, K, N):
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    a, b = (torch.randn(n, K, device="cuda", generator=g) for n in (M, N))
+    a64, b64 = a.double(), b.double()
+    want = a64 @ b64.t()
+    spread = ((a64 * a64) @ (b64 * b64).t()).sqrt()
+
+    def rms(c):
+        return float((((c - want) / spread) ** 2).mean().sqrt())
+
+    assert rms(ops.mul_mat(a, b).double()) <= 2.0 ** -19
+    assert rms(ops.mul_mat_tn(a.t().contiguous(), b.t().contiguous()).double()) <= 2.0 ** -19
+    for part_a, part_b in ((a.half(), b.half()), (a.half(), b), (a, b.half())):      # (each 2^-13 or more)
+        assert rms(part_a.double() @ part_b.double().t()) > 2.0 ** -15
+
+
 @pytest.mark.parametrize("per_thread", [False, True])
 def test_recorded_calls_take_no_workspace(ops, per_thread):
     """Contractions that take a workspace, recorded into a graph from a stream of the caller's and from the per-thread default
