@@ -17,9 +17,10 @@
 // -- is computed again, with the tile of 32 x 32 that it lies in, by the exact split (redo_tiles).  The test is against the output itself, or
 // against what its sum was halfway through K: neither is larger than sum |a||b|, so no output gets past it by luck.  Of
 // normal operands one lane in 2^11 fails with one of the two, next to none with both, and the test costs a minimum over the
-// accumulators: 384 residues x 32 features x 256 sequences 292 -> 295 us forward, 512 -> 519 backward, 103 residues 78.6 -> 84.6
-// backward, 26368 x 256 -> 768 52.2 -> 53.  Operands of wide range throughout are contracted twice: 12288 x 256 x 12288 with
-// spikes of 10^9 in one column or log-normal with sigma 3 1.5 ms (0.47 by the exact split alone), 26368 x 256 -> 768 0.29.
+// accumulators.  With the counting, us without / with: 384 residues x 32 features x 256 sequences 294 / 301 forward, 518 / 525
+// backward, 103 residues 41.9 / 42.3 and 79.3 / 83.1, 26368 x 256 -> 768 53.0 / 54.4, its weight gradient 57.5 / 58.3.  Operands of wide
+// range throughout are contracted twice: 12288 x 256 x 12288 with spikes of 10^9 in one column or log-normal with sigma 3
+// 1.5 ms (0.47 by the exact split alone), 26368 x 256 -> 768 0.29.
 //
 // B (the smaller operand as a rule: a weight, an alignment's projection) is split ahead by split_f16x2_kernel, which sees a
 // whole row of the slice and knows its maximum.  A is split in the tile loop by the loading waves, whose scale
@@ -618,15 +619,13 @@ __device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job&
     int g = 0;
     uint64_t* const notes = jb.notes + static_cast<size_t>(blockIdx.x * 4 + wave) * jb.most_items;
     int noted = 0;                                      // items with outputs to redo
-    // the smallest of this lane's sums
-    const auto least = [&]() {
+    // the smallest of this lane's sums in a tile row
+    const auto least = [&](int ti) {
         float m = __builtin_inff();
 #pragma unroll
-        for (int ti = 0; ti < 4; ++ti)
+        for (int tj = 0; tj < TJ; ++tj)
 #pragma unroll
-            for (int tj = 0; tj < TJ; ++tj)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) m = __builtin_elementwise_minimum(m, __builtin_fabsf(acc[ti][tj][r]));
+            for (int r = 0; r < 16; ++r) m = __builtin_elementwise_minimum(m, __builtin_fabsf(acc[ti][tj][r]));
         return m;
     };
     for (int i = 0; i < my_items; ++i) {
@@ -698,7 +697,12 @@ __device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job&
             if (g < total) __syncthreads();             // stage g - 1 has been read; stage g + 1 is in LDS
         };
         for (int c = 0; c < it.nch; c += 2) {
-            if (c == it.nch / 4 * 2 && c != 0) halfway = least();
+            if (c == it.nch / 4 * 2 && c != 0) {
+                halfway = __builtin_inff();
+#pragma unroll
+                for (int ti = 0; ti < 4; ++ti)          // (tile rows past the matrix hold zeros)
+                    if (it.m0 + ti * 32 < p.M) halfway = __builtin_elementwise_minimum(halfway, least(ti));
+            }
             chunk(fb[0], (it.c_begin + c) * HX_K, c == 0);
             chunk(fb[1], (it.c_begin + c + 1) * HX_K, false);
         }
@@ -726,29 +730,28 @@ __device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job&
         const v4f most = *reinterpret_cast<const v4f*>(lds_most[i & (HX_EXPS - 1)]);
         bound = HX_LOST * (bound + fmaxf(fmaxf(most[0], most[1]), fmaxf(most[2], most[3])));
         if (__builtin_amdgcn_ballot_w64(!(halfway >= bound)) != 0) {
-            const bool open = !(halfway >= bound) && !(least() >= bound);
-            if (__builtin_amdgcn_ballot_w64(open) != 0) {
-                const float (&na)[HX_M] = lds_small[i & (HX_EXPS - 1)];
-                uint32_t which = 0;
+            const float (&na)[HX_M] = lds_small[i & (HX_EXPS - 1)];
+            uint32_t which = 0;
 #pragma unroll
-                for (int ti = 0; ti < 4; ++ti) {
-                    uint64_t lost[TJ] = {};
+            for (int ti = 0; ti < 4; ++ti) {
+                const uint64_t open = __builtin_amdgcn_ballot_w64(!(halfway >= bound) && !(least(ti) >= bound));
+                if (it.m0 + ti * 32 >= p.M || open == 0) continue;
+                uint64_t lost[TJ] = {};
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const v4f n4 = *reinterpret_cast<const v4f*>(&na[ti * 32 + 8 * q + 4 * hh]);
+                for (int q = 0; q < 4; ++q) {
+                    const v4f n4 = *reinterpret_cast<const v4f*>(&na[ti * 32 + 8 * q + 4 * hh]);
 #pragma unroll
-                        for (int tj = 0; tj < TJ; ++tj)
+                    for (int tj = 0; tj < TJ; ++tj)
 #pragma unroll
-                            for (int c = 0; c < 4; ++c)             // (a NaN comes from a row that is a bad one)
-                                lost[tj] |= __builtin_amdgcn_ballot_w64(__builtin_fabsf(acc[ti][tj][4 * q + c]) < HX_LOST * (n4[c] + cb[tj]));
-                    }
-#pragma unroll
-                    for (int tj = 0; tj < TJ; ++tj) which |= (lost[tj] & __builtin_amdgcn_ballot_w64(open)) != 0 ? 1u << (ti * TJ + tj) : 0u;
+                        for (int c = 0; c < 4; ++c)     // (a NaN comes from a row that is a bad one)
+                            lost[tj] |= __builtin_amdgcn_ballot_w64(__builtin_fabsf(acc[ti][tj][4 * q + c]) < HX_LOST * (n4[c] + cb[tj]));
                 }
-                if (which != 0) {
-                    if (lane == 0) notes[noted] = static_cast<uint64_t>(i) << 32 | which;
-                    ++noted;
-                }
+#pragma unroll
+                for (int tj = 0; tj < TJ; ++tj) which |= (lost[tj] & open) != 0 ? 1u << (ti * TJ + tj) : 0u;
+            }
+            if (which != 0) {
+                if (lane == 0) notes[noted] = static_cast<uint64_t>(i) << 32 | which;
+                ++noted;
             }
         }
         if (OUT == HX_PARTIAL && any_bad) {             // NaN: reduce_slices_kernel redoes those

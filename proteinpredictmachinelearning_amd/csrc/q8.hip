@@ -1945,8 +1945,10 @@ int try_q8_tiled(const void* W, int wtype, const float* X, float* C, int M, int 
     // (us, general / this one): three blocks below 512 features, 26368 x 96 -> 128  8.9 / 9.5 (from there on 10.7 / 7.8 at
     // 5000 x 96 -> 768); up to eight blocks of up to 128 features, where the quantized copy of the activations is most of
     // the traffic, 26368 x 160 -> 128  10.6 / 11.6, 26368 x 192 -> 64  9.1 / 11.1; middling widths of many tokens, whose
-    // last round of tiles is thin, 26368 x 480 -> 320  32.1 / 34.3 (2601 x 480 -> 768  21.3 / 12.2, 10609 x 288 -> 320
-    // 14.6 / 11.8, 26368 x 480 -> 128  23.8 / 20.5 for the others).  Beyond 31 blocks odd numbers stay with the general one.
+    // last round of tiles is thin, 26368 x 480 -> 320  32.5 / 34.1 (2601 x 480 -> 768  21.3 / 12.2, 10609 x 288 -> 320
+    // 14.6 / 11.8, 26368 x 480 -> 128  23.8 / 20.5 for the others).  That last line, over 17000 to 32768 tokens, 160 to 736
+    // features and 5 to 15 blocks (100 shapes): the general kernel takes 0.77 to 1.11 of the tiled one's time, 0.96 in the
+    // middle, least at few features (17000 x 224 -> 160  10.3 / 13.4), most at many (17000 x 480 -> 736  40.1 / 36.1).  Beyond 31 blocks odd numbers stay with the general one.
     if (nblk % 2 != 0 && nblk > 31) return -1;
     if (wtype == PPML_WTYPE_Q8_0M) {
         if (nblk == 3 && M < 512) return -1;
