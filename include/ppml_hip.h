@@ -73,13 +73,16 @@ int ppml_hip_set_f32_arithmetic(int mode);
  * affected tile in plain binary32 arithmetic, one product at a time with k ascending (the reference's own
  * loop): +-inf, NaN and the bits down to 2^-149 come out as the reference's.  The fused attention kernels
  * (flash_attn_*_hip) split without that check; ppml_hip_set_f32_arithmetic(1) selects the fp32 pipe, which
- * carries every operand, for all of them.  Contractions of at
+ * carries every operand, for all of them.  Contractions in
+ * two halves (single planes of K >= 128 with more than a tile of 128 x 128 outputs per CU, a compound output or a long K
+ * under few tiles, where they pay: 4 bytes per element of the smaller operand), contractions of at
  * least 512 work-groups of 256 x 128 outputs (6 bytes per operand element) and contractions of few output
  * tiles under a long K (the partial sums of their K slices) use a workspace from a stream-ordered pool of
  * the library's; a stream keeps one such buffer between calls (the per-thread default stream allocates and
  * releases per call).  A stream under capture gets no workspace -- an allocation made while a graph is recorded
  * is gone before the graph runs -- and its calls take the forms that need none; mul_mat_tn_noalloc_hip brings the
- * sliced forms to recorded code. */
+ * others to recorded code.  Two halves, K slices and one sum over all of K round differently: from K = 128 on the bits of
+ * an output depend on how many rows and columns are computed with it and on whether the call was recorded. */
 int mul_mat_hip(const float *A, const float *B, float *C, int M, int K, int N,
                 const float *bias, ppml_hip_stream_t stream);
 

@@ -84,8 +84,9 @@ void ppml_hip_backend_set_fuse_attention_chain(ppml_hip_backend *b, int on);
  *     reads (src/modules/Attention.cpp:277-281) contracts the unpermuted tensors over their innermost dimension;
  *     same bits, two copies less.
  *   With these two and scale_into_out_prod on, the whole attention chain above of planes of up to 128 rows (heads of up
- *     to 32, 32 planes or more, the default arithmetic) runs as one launch where nobody else reads an intermediate: the
- *     bits of the launches it stands for. */
+ *     to 32, 32 planes or more, the default arithmetic) runs as one launch where nobody else reads an intermediate and none of
+ *     them has memory bound to it (a scheduler with an allocator of its own binds them all: three launches there, which
+ *     write the memory of the logits and of the probabilities): the bits of the launches it stands for. */
 void ppml_hip_backend_set_fuse_add_into_soft_max(ppml_hip_backend *b, int on);
 void ppml_hip_backend_set_fuse_permutes_into_out_prod(ppml_hip_backend *b, int on);
 /*   permutes_into_mul_mat (default 1): an F32 OP_MUL_MAT without bias whose operands are both matrix transpositions

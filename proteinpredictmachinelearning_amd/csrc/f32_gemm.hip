@@ -11,7 +11,7 @@
 // split (gemm_bf16x3_kernel, and gemm_planes_kernel for large problems, which splits ahead of the
 // matrix work): products to within 2^-23 of |a||b|, sums in binary32, sixteen k per accumulation step,
 // starting from bias[n] (or 0); alpha multiplies the finished sum.  Large contractions go in two halves per
-// operand under a power of two per row instead (gemm_f16x2.hip), with half the products and a smaller error.  Half operands go to the f16 matrix
+// operand under a power of two per row instead (gemm_f16x2.hip), with half the products.  Half operands go to the f16 matrix
 // pipe unchanged (gemm_f16_kernel).  The clamped contraction of the triangle multiplication, whose
 // result depends on how infinities propagate, stays on the fp32 pipe (gemm_f32_kernel:
 // v_mfma_f32_32x32x2_f32, k ascending two at a time).
