@@ -134,7 +134,7 @@ def _spikes(g, a, b, size, where):
 @pytest.mark.parametrize("size", [1e5, 1e7, 1e9, 1e12, 1e30])
 def test_large_elements_that_meet_zeros(ops, size, where):
     g = torch.Generator(device="cuda").manual_seed(int(np.log10(size)) * 3 + len(where))
-    for M, K, N in ((20011, 136, 1004), (26368, 256, 200), (9001, 403, 390)):
+    for M, K, N in ((20011, 136, 1004), (26368, 256, 200), (9001, 403, 390), (22000, 165, 768)):      # (the last: streaming stores)
         a, b = (torch.randn(n, K, device="cuda", generator=g) for n in (M, N))
         for first in (True, False):
             x, y = _spikes(g, a, b, size, where) if first else _spikes(g, b, a, size, where)[::-1]
@@ -146,7 +146,7 @@ def test_large_elements_that_meet_zeros(ops, size, where):
         for first in (True, False):
             x, y = _spikes(g, a, b, size, where) if first else _spikes(g, b, a, size, where)[::-1]
             _narrow(ops.mul_mat_tn(x.t().contiguous(), y.t().contiguous(), 0.5), x.double(), y.double(), 0.5)
-    for D, L, N in ((32, 96, 256), (32, 103, 130)):             # outer-product-mean and its gradients
+    for D, L, N in ((32, 96, 256), (32, 103, 130), (32, 192, 72)):        # outer-product-mean and its gradients (the last: streaming stores)
         left, right = (torch.randn(D * L, N, device="cuda", generator=g) for _ in range(2))
         x, y = _spikes(g, left, right, size, where)
         out = ops.outer_product_mean(x.reshape(-1), y.reshape(-1), D, L, N, 1)
