@@ -65,7 +65,8 @@ int ppml_hip_set_f32_arithmetic(int mode);
  * three bf16 numbers; six of the nine partial products (all but 2^-23 of |a||b|) are formed exactly on
  * the bf16 matrix pipe and summed in binary32.  Large contractions: two halves per operand under a power of two per
  * row, three exact products on the f16 pipe; all but 2^-21 of |a||b| at worst (operands of one constant each), with
- * half the exact split's error on random operands.  Outputs to which a row's elements far below its largest one (2^-14 of
+ * half the exact split's error on random operands, and exact products where one operand has at most 11 significant
+ * bits and the other 23.  Outputs to which a row's elements far below its largest one (2^-14 of
  * it and less) might matter beyond that -- the large ones meet zeros -- are found and computed again by the exact split, at a
  * third of its speed where they are all of that kind.  Two kinds of operand fall outside what three bf16 parts
  * carry: a non-finite one, and one with bits below 2^-133, bf16's smallest step (subnormal operands and the

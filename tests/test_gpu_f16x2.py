@@ -197,6 +197,22 @@ def test_constants_with_the_largest_rounding(ops):
     assert bool(((ops.mul_mat(a, b).double() - want).abs() <= (2.0 ** -21 + 8 * 2.0 ** -24) * want).all())
 
 
+# Products that binary32 holds (24 bits together) and that the three kept ones carry: 11 bits against up to 23, either way round
+@pytest.mark.parametrize("wide_first", [True, False])
+@pytest.mark.parametrize("wide,narrow", [(13, 11), (23, 1)])
+def test_exact_products_stay_exact(ops, wide, narrow, wide_first):
+    g = torch.Generator(device="cuda").manual_seed(3)
+
+    def whole(bits, *shape):
+        x = torch.randint(2 ** (bits - 1), 2 ** bits, shape, device="cuda", generator=g).float()
+        return x * (torch.randint(0, 2, shape, device="cuda", generator=g) * 2 - 1) * torch.exp2(torch.randint(0, 4, shape, device="cuda", generator=g).float())
+
+    a = torch.zeros(20011, 136, device="cuda")
+    a[torch.arange(20011), torch.randint(0, 136, (20011,), device="cuda", generator=g)] = whole(wide if wide_first else narrow, 20011)   # one a row: no sum to round
+    b = whole(narrow if wide_first else wide, 1004, 136)
+    assert torch.equal(ops.mul_mat(a, b).double(), a.double() @ b.double().t())
+
+
 # A bound that does not grow with K, which operands without their low halves (or a product that is left out) fail
 @pytest.mark.parametrize("M,K,N", [(20011, 136, 1004), (768, 26368, 256), (900, 10609, 321), (1024, 4100, 1030)])
 def test_the_low_halves_are_there(ops, M, K, N):
