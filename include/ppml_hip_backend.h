@@ -92,7 +92,10 @@ void ppml_hip_backend_set_fuse_permutes_into_out_prod(ppml_hip_backend *b, int o
 /*   permutes_into_mul_mat (default 1): an F32 OP_MUL_MAT without bias whose operands are both matrix transpositions
  *     nobody else reads -- the weight gradient of a LinearLayer, mul_mat(mat_transpose(grad), mat_transpose(x)),
  *     src/core/ComputeGraph.cpp:733-738 -- contracts the untransposed matrices over their rows; same bits, and the
- *     copies of the activations and of their gradient are not made. */
+ *     copies of the activations and of their gradient are not made.  The transposition of the second operand alone (the weight's, in
+ *     front of the input's gradient) is folded too, same bits, where its memory is nobody's.  An OP_REPEAT_BACK behind a weight gradient
+ *     folded like this, of the same gradient down to its first dimension (the bias gradient), is left beside it: its sum is the
+ *     contraction's pass over the gradient, in another order than the node's own. */
 void ppml_hip_backend_set_fuse_permutes_into_mul_mat(ppml_hip_backend *b, int on);
 /* how many nodes the last graph_compute folded into a neighbour and did not execute */
 int ppml_hip_backend_nodes_fused_away(const ppml_hip_backend *b);

@@ -192,7 +192,9 @@ public:
     // (src/core/ComputeGraph.cpp:733-738): an F32 OP_MUL_MAT without bias both of whose operands are matrix
     // transpositions nobody else reads contracts the untransposed matrices over their rows (mul_mat_tn_hip); the two
     // copies -- of the activations and of their gradient, the largest tensors of the backward pass -- are not made.
-    // ON by default; same bits as the nodes run one by one.
+    // ON by default; same bits as the nodes run one by one.  So is the weight's transposition in front of the input's gradient,
+    // mul_mat(grad, mat_transpose(w)), where no memory is bound to it; and the bias gradient, the OP_REPEAT_BACK of the same
+    // gradient behind it, is summed on the weight gradient's way through it (a sum of T terms in another order).
     void set_fuse_permutes_into_mul_mat(bool v) { fuse_permutes_into_mul_mat_ = v; }
     bool fuse_permutes_into_mul_mat() const { return fuse_permutes_into_mul_mat_; }
     // Off by default.  On: the reference's default attention chain (src/modules/Attention.cpp:264-281)
@@ -259,6 +261,8 @@ private:
     bool out_prod_scaled_ = false;
     bool out_prod_transposed_ = false;                   // the out_prod being dispatched reads the sources of two fused-away permutations
     bool mul_mat_transposed_ = false;                    // the same for the mul_mat being dispatched
+    Tensor* bias_grad_ = nullptr;                        // ... and, transposed, leaves the sums over its first operand's rows there
+    bool mul_mat_rows_b_ = false;                        // the mul_mat being dispatched reads its second operand untransposed
     const Tensor* soft_max_bias_ = nullptr;              // second operand of a fused-away OP_ADD in front of the softmax being dispatched
     std::string error_;
     std::vector<std::unique_ptr<Buffer>> owned_;         // node outputs allocated here, packed weights

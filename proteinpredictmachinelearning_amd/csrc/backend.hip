@@ -350,12 +350,24 @@ Status HipBackend::kernel_mul_mat(Tensor* node) {
         if (s0->type != TENSOR_TYPE_F32 || s1->type != TENSOR_TYPE_F32 || node->type != TENSOR_TYPE_F32 || node->src[2] ||
             s0->dims[0] != M || s1->dims[0] != N || s1->dims[1] != K || s0->numel() != M * K || s1->numel() != N * K)
             return fail(Status::ABORTED, "mul_mat: the folded transpositions do not fit the node");
-        const int rc = mul_mat_tn_hip(static_cast<const float*>(s0->data), static_cast<const float*>(s1->data), static_cast<float*>(node->data),
-                                      static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), 1.0f, nullptr);
+        const int rc = bias_grad_ ? mul_mat_tn_sums(static_cast<const float*>(s0->data), static_cast<const float*>(s1->data), static_cast<float*>(node->data),
+                                                    static_cast<float*>(bias_grad_->data), static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), nullptr)
+                                  : mul_mat_tn_hip(static_cast<const float*>(s0->data), static_cast<const float*>(s1->data), static_cast<float*>(node->data),
+                                                   static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), 1.0f, nullptr);
         if (rc != 0) return fail(status_of_rc(rc), std::string("mul_mat: ") + ppml_hip_last_error());
         return Status::SUCCESS;
     }
     const int64_t M = node->dims[1], N = node->dims[0], K = s0->dims[0];
+    if (mul_mat_rows_b_) {
+        // s1 is the source of the folded transposition: K rows of N elements
+        if (s0->type != TENSOR_TYPE_F32 || s1->type != TENSOR_TYPE_F32 || node->type != TENSOR_TYPE_F32 || node->src[2] ||
+            s1->dims[0] != N || s1->dims[1] != K || s0->numel() != M * K || s1->numel() != N * K)
+            return fail(Status::ABORTED, "mul_mat: the folded transposition does not fit the node");
+        const int rc = mul_mat_nn(static_cast<const float*>(s0->data), static_cast<const float*>(s1->data), static_cast<float*>(node->data),
+                                  static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), nullptr);
+        if (rc != 0) return fail(status_of_rc(rc), std::string("mul_mat: ") + ppml_hip_last_error());
+        return Status::SUCCESS;
+    }
     if (s1->dims[0] != K) return fail(Status::NOT_SUPPORTED, "mul_mat: inner dimensions differ");
     if (s0->numel() != M * K || s1->numel() != N * K)
         return fail(Status::NOT_SUPPORTED, "mul_mat: source shapes do not match the node's [N, M]");
@@ -716,6 +728,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         Tensor* relu = nullptr;
         Tensor* out_prod = nullptr;         // OP_SCALE node that runs as the (skipped) out_prod it reads, scaled
         Tensor* added = nullptr;            // OP_SOFT_MAX node that adds the second operand of this (skipped) OP_ADD on its way in
+        Tensor* bias_grad = nullptr;        // transposed OP_MUL_MAT that leaves this (skipped) OP_REPEAT_BACK's result beside its own
+        bool rows_b = false;                // OP_MUL_MAT that reads the source of its second operand's (skipped) transposition
         bool transposed = false;            // OP_OUT_PROD / OP_MUL_MAT that reads the sources of its two (skipped) {1,0,2,3} permutations
         bool chain = false;                 // out_prod(attn_t, V_t) that runs as the whole attention chain ...
         bool chain_bits = false;            // ... with the bits of its nodes (attention_chain)
@@ -972,8 +986,9 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         }
 
         // (7) the two matrix transpositions in front of a LinearLayer's weight gradient,
-        // mul_mat(mat_transpose(grad), mat_transpose(x)) (src/core/ComputeGraph.cpp:733-738; mat_transpose is a
-        // permutation copy of dims[0] and dims[1], src/core/ComputeGraphHelper.cpp:375-382)
+        // mul_mat(mat_transpose(grad), mat_transpose(x)), and the one in front of its input's gradient
+        // (src/core/ComputeGraph.cpp:733-738; mat_transpose is a permutation copy of dims[0] and dims[1],
+        // src/core/ComputeGraphHelper.cpp:375-382)
         if (fuse_permutes_into_mul_mat_) {
             const auto is_mat_t = [](const Tensor* t) {
                 if (!t || (t->op != OP_PERMUTE && t->op != OP_TRANSPOSE) || t->ndim < 2 || t->type != TENSOR_TYPE_F32 || t->view_src) return false;
@@ -986,9 +1001,45 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 if (!n || n->op != OP_MUL_MAT || n->type != TENSOR_TYPE_F32 || n->src[2] || skipped.count(n) || !node_supported(n)) continue;
                 Tensor* p0 = n->src[0];
                 Tensor* p1 = n->src[1];
-                if (p0 == p1 || !is_mat_t(p0) || !is_mat_t(p1) || !private_to(p0, n) || !private_to(p1, n)) continue;
+                if (p0 == p1 || !is_mat_t(p1) || !private_to(p1, n)) continue;
+                if (!is_mat_t(p0) || !private_to(p0, n)) {
+                    // the weight's alone, in front of the input's gradient, mul_mat(grad, mat_transpose(w)): where the kernels that
+                    // take the weight as it lies are those that its copy would have gone to, and the copy's memory is nobody's
+                    if (!p0 || p0->type != TENSOR_TYPE_F32 || arithmetic_here == 1 || p1->data || p1->buffer || !node_supported(p1)) continue;
+                    const int64_t M = n->dims[1], K = p0->dims[0], N = n->dims[0];
+                    if (p1->dims[0] != K || p1->dims[1] != N || p0->numel() != M * K || n->numel() != M * N || !mul_mat_nn_fits(M, K, N)) continue;
+                    if (!fold({p1}, [&] { return stands_until(p1, n, p1->src[0]); })) continue;
+                    plans[n].rows_b = true;
+                    continue;
+                }
                 if (!fold({p0, p1}, [&] { return stands_until(p0, n, p0->src[0]) && stands_until(p1, n, p1->src[0]); })) continue;
                 plans[n].transposed = true;
+            }
+        }
+        // (8) a LinearLayer's bias gradient behind its weight gradient (src/core/ComputeGraph.cpp:738, 742): the sums over the
+        // rows that the contraction reads, left beside it.  The sum then runs before its place, so nothing between the two may
+        // read or write its memory, or write the gradient's.
+        if (fuse_permutes_into_mul_mat_) {
+            for (Tensor* n : *graph) {
+                if (!n || n->op != OP_MUL_MAT || skipped.count(n)) continue;
+                const auto planned = plans.find(n);
+                if (planned == plans.end() || !planned->second.transposed) continue;
+                const Tensor* g = n->src[0]->src[0];
+                const Tensor* x = n->src[1]->src[0];
+                for (int at = position[n] + 1; at < static_cast<int>(order.size()); ++at) {
+                    const Tensor* r = order[at];
+                    if (r->op != OP_REPEAT_BACK || r->src[0] != g || skipped.count(r) || !node_supported(r)) continue;
+                    if (r->view_src || r->dims[0] != g->dims[0] || r->numel() != g->dims[0] || g->numel() != g->dims[0] * g->dims[1]) continue;
+                    bool free = !meet(r, n) && !meet(r, g) && !meet(r, x) && !meet(n, g);
+                    for (int i = position[n] + 1; i < at && free; ++i) {
+                        free = !overwrites(order[i], r) && !overwrites(order[i], g);
+                        for (int s = 0; s < 10 && free; ++s) free = !meet(order[i]->src[s], r);
+                    }
+                    if (!free) continue;
+                    skipped.insert(r);
+                    planned->second.bias_grad = const_cast<Tensor*>(r);
+                    break;
+                }
             }
         }
         nodes_fused_away_ = skipped.size();
@@ -1003,6 +1054,7 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
 
     HostShadows shadows;                                // restored and freed on every way out of this function
     host_shadows_made_ = 0;
+    const auto position_of = [&](const Tensor* t) { return std::find(graph->begin(), graph->end(), t) - graph->begin(); };
     int index = -1;
     for (Tensor* node : *graph) {
         ++index;
@@ -1025,6 +1077,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         out_prod_scaled_ = false;
         out_prod_transposed_ = false;
         mul_mat_transposed_ = false;
+        mul_mat_rows_b_ = false;
+        bias_grad_ = nullptr;
         soft_max_bias_ = nullptr;
         const auto plan = plans.find(node);
         if (plan != plans.end()) {
@@ -1069,8 +1123,13 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
             if (pl.transposed) {
                 rewired.src[0] = node->src[0]->src[0];
                 rewired.src[1] = node->src[1]->src[0];
+                bias_grad_ = pl.bias_grad;
                 if (node->op == OP_MUL_MAT) mul_mat_transposed_ = true;
                 else out_prod_transposed_ = true;
+            }
+            if (pl.rows_b) {
+                rewired.src[1] = node->src[1]->src[0];
+                mul_mat_rows_b_ = true;
             }
             if (pl.chain) {
                 // src/core/ComputeGraphHelper.cpp:450-484: Q, K, V, bias in src 0..3; scale, causal, eps, Br, Bc
@@ -1102,6 +1161,7 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         Tensor* outputs[5] = {attn_back && node->op_params[5] == 0 ? nullptr : storage,
                               node->op == OP_FLASH_ATTN_EXT || two_outputs ? node->src[4] : nullptr,
                               two_outputs ? node->src[3] : nullptr, nullptr, nullptr};
+        if (bias_grad_) outputs[1] = bias_grad_;
         if (attn_back) { outputs[1] = node->src[7]; outputs[2] = node->src[8]; outputs[3] = node->src[9]; }
         for (Tensor* out : outputs) {
             if (!out || skip_alloc_ || out->data) continue;
@@ -1121,6 +1181,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
 
         if (!(attn_back && node->op_params[5] == 0) && !device_pointer_ok(exec))
             return fail(Status::NOT_SUPPORTED, "node " + std::to_string(index) + ": output is not device memory inside its buffer");
+        if (bias_grad_ && !device_pointer_ok(bias_grad_))
+            return fail(Status::NOT_SUPPORTED, "node " + std::to_string(position_of(bias_grad_)) + ": output is not device memory inside its buffer");
         for (int j = 0; j < 10; ++j) {
             if (exec->src[j] && !device_pointer_ok(exec->src[j]))
                 return fail(Status::NOT_SUPPORTED, "node " + std::to_string(index) + ": src" + std::to_string(j) +
@@ -1134,6 +1196,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         out_prod_scaled_ = false;
         out_prod_transposed_ = false;
         mul_mat_transposed_ = false;
+        mul_mat_rows_b_ = false;
+        bias_grad_ = nullptr;
         soft_max_bias_ = nullptr;
         if (st != Status::SUCCESS) return st;
         const hipError_t e = hipGetLastError();

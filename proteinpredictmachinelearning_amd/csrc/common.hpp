@@ -70,6 +70,12 @@ public:
 private:
     std::atomic<uint64_t> set_{0};                      // a bit per device
 };
+// C[M][N] = A[M][K] B[K][N] (f32_gemm.hip): a contraction over the rows of a matrix that mul_mat would have transposed first
+bool mul_mat_nn_fits(int64_t M, int64_t K, int64_t N);
+int mul_mat_nn(const float* A, const float* B, float* C, int M, int K, int N, hipStream_t stream);
+// O[M][Nc] = sum over k of A[k][M] Bm[k][Nc] (mul_mat_tn_hip) and sums[M] = the sums over k of A[k][M] (repeat_back_hip): a linear layer's
+// weight and bias gradients, in one pass over the gradient where the contraction goes in K slices
+int mul_mat_tn_sums(const float* A, const float* Bm, float* O, float* sums, int M, int K, int Nc, hipStream_t stream);
 // The default attention's nodes in one launch (attention_chain.hip): Q, K, V, O [planes][d][L], bias [planes][L][L] or null
 bool attention_chain_fits(int64_t planes, int64_t L, int64_t d);
 int attention_chain(const float* Q, const float* K, const float* V, const float* bias, float* O, int64_t planes, int L, int d, float scale,

@@ -809,7 +809,9 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_kernel(const GemmParams p)
 constexpr int PC64_AHEAD = 4;                     // stages of 32 k in flight
 constexpr int PC64_PLANE = 64 * SPLIT_PITCH;      // one of the three planes of 64 rows x 16 k
 constexpr int PC64_OPERAND = 2 * 3 * PC64_PLANE;  // [16 k][plane][row]
-template <bool STREAM_C, bool K4>
+// BMODE LOAD_ROW_CONTIG: B(n, k) = B[k * b_ks + n], a weight as it lies under a contraction over its rows (the gradient of a linear
+// layer's input): a thread then loads one column of the tile and eight k of the stage, and writes what the other form writes.
+template <bool STREAM_C, bool K4, int BMODE = LOAD_K_CONTIG>
 __global__ __launch_bounds__(512) void gemm_bf16x3_pc64_kernel(const GemmParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t lds_ab[2][2 * PC64_OPERAND];
     const int tid = threadIdx.x;
@@ -823,7 +825,8 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc64_kernel(const GemmParams 
     int fired = 0;
     if (wave >= 4) {
         const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A), 0, static_cast<int>(((p.M - 1) * p.a_rs + p.K) * 4), 0x00020000);
-        const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.B), 0, static_cast<int>(((p.N - 1) * p.b_rs + p.K) * 4), 0x00020000);
+        const int64_t b_plane = BMODE == LOAD_K_CONTIG ? (p.N - 1) * p.b_rs + p.K : p.K * p.b_ks;
+        const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.B), 0, static_cast<int>(b_plane * 4), 0x00020000);
         // a thread: row (tid % 256) / 4 of either tile, four k of each chunk of the stage
         const int ptid = tid & 255, row = ptid >> 2, kq = (ptid & 3) * 4;
         const uint32_t a_at = m0 + row < p.M ? static_cast<uint32_t>(m0 + row) * static_cast<uint32_t>(p.a_rs) * 4u : OUTSIDE;
@@ -840,10 +843,23 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc64_kernel(const GemmParams 
                 }
             }
         };
+        // (k behind K: behind the end of the plane)
+        const int brow = ptid & 63, bk = ptid >> 6;     // column of the tile, octet of k
+        const uint32_t b_col = n0 + brow < p.N ? static_cast<uint32_t>(n0 + brow) * 4u : OUTSIDE;
+        const auto load_rows = [&](int stage, v4f (&x)[2]) {
+            const uint32_t kb = static_cast<uint32_t>(stage * 32 + __builtin_amdgcn_readfirstlane(bk) * 8), step = static_cast<uint32_t>(p.b_ks) * 4u;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) x[c >> 2][c & 3] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_b, b_col + (kb + c) * step, 0, 0));
+        };
+        const auto load_both = [&](int stage, v4f (&a)[2], v4f (&b)[2]) {
+            load(rsrc_a, a_at, stage, a);
+            if (BMODE == LOAD_K_CONTIG) load(rsrc_b, b_at, stage, b);
+            else load_rows(stage, b);
+        };
         v4f xa[PC64_AHEAD][2], xb[PC64_AHEAD][2];
 #pragma unroll
         for (int d = 0; d < PC64_AHEAD; ++d)
-            if (d < stages) { load(rsrc_a, a_at, d, xa[d]); load(rsrc_b, b_at, d, xb[d]); }
+            if (d < stages) load_both(d, xa[d], xb[d]);
         SplitGuard guard;
         for (int g = 0; g < stages; g += PC64_AHEAD) {
 #pragma unroll
@@ -851,18 +867,24 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc64_kernel(const GemmParams 
                 const int s = g + d;
                 if (s >= stages) break;                 // uniform
                 uint8_t* const dst = lds_ab[s & 1] + row * SPLIT_PITCH + kq * 2;
+                uint8_t* const dst_b = lds_ab[s & 1] + PC64_OPERAND + brow * SPLIT_PITCH + (bk >> 1) * 3 * PC64_PLANE + (bk & 1) * 16;
+                uint2 b[2][3];
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    uint2 a[3], b[3];
+                    uint2 a[3];
                     split4(xa[d][c], a, guard);
-                    split4(xb[d][c], b, guard);
+                    split4(xb[d][c], b[c], guard);
 #pragma unroll
                     for (int q = 0; q < 3; ++q) {
                         *reinterpret_cast<uint2*>(dst + (c * 3 + q) * PC64_PLANE) = a[q];
-                        *reinterpret_cast<uint2*>(dst + PC64_OPERAND + (c * 3 + q) * PC64_PLANE) = b[q];
+                        if (BMODE == LOAD_K_CONTIG) *reinterpret_cast<uint2*>(dst + PC64_OPERAND + (c * 3 + q) * PC64_PLANE) = b[c][q];
                     }
                 }
-                if (s + PC64_AHEAD < stages) { load(rsrc_a, a_at, s + PC64_AHEAD, xa[d]); load(rsrc_b, b_at, s + PC64_AHEAD, xb[d]); }
+                if (BMODE == LOAD_ROW_CONTIG) {
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) *reinterpret_cast<uint4*>(dst_b + q * PC64_PLANE) = uint4{b[0][q].x, b[0][q].y, b[1][q].x, b[1][q].y};
+                }
+                if (s + PC64_AHEAD < stages) load_both(s + PC64_AHEAD, xa[d], xb[d]);
                 __syncthreads();
             }
         }
@@ -939,10 +961,11 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_pair_kernel(const GemmPara
 // order, applies bias, factor and the output's addressing.  A slice whose split could not carry an operand leaves NaN
 // for its whole tile, and reduce_slices_kernel computes every output whose sum is NaN the reference's way (no flags to
 // clear ahead: one launch less).
-template <int MODE, bool K4>
+template <int MODE, bool K4, int BMODE = MODE>
 __global__ __launch_bounds__(512) void gemm_bf16x3_pc_slices_kernel(const GemmParams p, int chunks, int slice_chunks, float* __restrict__ partial,
-                                                                    int ma_pad, int nb_pad) {
+                                                                    int ma_pad, int nb_pad, float* __restrict__ row_sums) {
     static_assert(MODE == LOAD_ROW_CONTIG || MODE == LOAD_K_CONTIG, "buffer addressing");
+    static_assert(BMODE == LOAD_ROW_CONTIG || BMODE == LOAD_K_CONTIG, "buffer addressing");
     constexpr int STAGE = 3 * SPLIT_PLANE;
     __shared__ __attribute__((aligned(16))) uint8_t lds_ab[2][2 * STAGE];
 
@@ -961,7 +984,7 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_slices_kernel(const GemmPa
     const int nch = c_end - c_begin;
 
     const int64_t a_plane = MODE == LOAD_K_CONTIG ? (p.M - 1) * p.a_rs + p.K : p.K * p.a_ks;
-    const int64_t b_plane = MODE == LOAD_K_CONTIG ? (p.N - 1) * p.b_rs + p.K : p.K * p.b_ks;
+    const int64_t b_plane = BMODE == LOAD_K_CONTIG ? (p.N - 1) * p.b_rs + p.K : p.K * p.b_ks;
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A), 0, static_cast<int>(a_plane * 4), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.B), 0, static_cast<int>(b_plane * 4), 0x00020000);
 
@@ -971,32 +994,37 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_slices_kernel(const GemmPa
     if (producer) {
         v4f ra[PC_AHEAD][2], rb[PC_AHEAD][2];
         const auto load_both = [&](int c, v4f (&xa)[2], v4f (&xb)[2]) {
-            if (MODE == LOAD_K_CONTIG) {
-                load_kcontig_buffer<K4>(rsrc_a, static_cast<uint32_t>(p.a_rs) * 4u, m0, p.M, c * BK, p.K, ptid, xa);
-                load_kcontig_buffer<K4>(rsrc_b, static_cast<uint32_t>(p.b_rs) * 4u, n0, p.N, c * BK, p.K, ptid, xb);
-            } else {
-                load_rows8_buffer(rsrc_a, static_cast<uint32_t>(p.a_ks) * 4u, m0, p.M, c * BK, ptid, xa);
-                load_rows8_buffer(rsrc_b, static_cast<uint32_t>(p.b_ks) * 4u, n0, p.N, c * BK, ptid, xb);
-            }
+            if (MODE == LOAD_K_CONTIG) load_kcontig_buffer<K4>(rsrc_a, static_cast<uint32_t>(p.a_rs) * 4u, m0, p.M, c * BK, p.K, ptid, xa);
+            else load_rows8_buffer(rsrc_a, static_cast<uint32_t>(p.a_ks) * 4u, m0, p.M, c * BK, ptid, xa);
+            if (BMODE == LOAD_K_CONTIG) load_kcontig_buffer<K4>(rsrc_b, static_cast<uint32_t>(p.b_rs) * 4u, n0, p.N, c * BK, p.K, ptid, xb);
+            else load_rows8_buffer(rsrc_b, static_cast<uint32_t>(p.b_ks) * 4u, n0, p.N, c * BK, ptid, xb);
         };
 #pragma unroll
         for (int d = 0; d < PC_AHEAD; ++d)
             if (d < nch) load_both(c_begin + d, ra[d], rb[d]);
         SplitGuard guard;
+        float sum[2] = {0.0f, 0.0f};                    // this thread's share of its row's sum, where that is asked for
+        const bool sums = MODE == LOAD_ROW_CONTIG && row_sums && n0 == 0;
         for (int cg = 0; cg < nch; cg += PC_AHEAD) {
 #pragma unroll
             for (int d = 0; d < PC_AHEAD; ++d) {
                 const int c = cg + d;
                 if (c >= nch) break;                    // uniform
                 uint8_t* half = lds_ab[c & 1];
+                if (sums) {
+                    const v4f x = ra[d][0] + ra[d][1];
+                    sum[d & 1] += (x[0] + x[1]) + (x[2] + x[3]);
+                }
                 split_store<MODE>(half, ptid, ra[d], guard);
-                split_store<MODE>(half + STAGE, ptid, rb[d], guard);
+                split_store<BMODE>(half + STAGE, ptid, rb[d], guard);
                 if (c + PC_AHEAD < nch) load_both(c_begin + c + PC_AHEAD, ra[d], rb[d]);
                 __syncthreads();
             }
         }
         __syncthreads();
         fired = guard.fired() ? 1 : 0;
+        // (its octet of a chunk's k is one of two: partial sums [slice][octet][row])
+        if (sums) row_sums[static_cast<size_t>(slice * 2 + (ptid >> 7)) * ma_pad + m0 + (ptid & 127)] = sum[0] + sum[1];
     } else {
 #pragma unroll
     for (int ti = 0; ti < 2; ++ti)
@@ -2139,11 +2167,36 @@ __global__ __launch_bounds__(256, 2) void gemm_planes_kernel(const GemmParams p,
 }
 
 // C = alpha * (bias + sum over the K slices, in slice order) with the contraction's own output addressing
-template <bool SPLIT_C>
+template <bool SPLIT_C, bool SUMS = false>
 __global__ __launch_bounds__(256) void reduce_slices_kernel(const GemmParams p, const float* __restrict__ partial,
                                                             int slices, int ma_pad, int nb_pad,
-                                                            const int* __restrict__ fired_a, const int* __restrict__ fired_b) {
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+                                                            const int* __restrict__ fired_a, const int* __restrict__ fired_b,
+                                                            const RowSumParts rs, int sum_blocks) {
+    // the row sums' work-groups first: theirs is the longer chain
+    if (SUMS && static_cast<int>(blockIdx.x) < sum_blocks) {
+        const int r = blockIdx.x * 256 + threadIdx.x;
+        if (r >= rs.rows) return;
+        const float* at = rs.partial + r;
+        // sixteen sums of every sixteenth part, which also shortens the chain of roundings: 12949 rows x 68, 256 parts, 2.7e-7
+        // of the result in one sum, 1.0e-7 this way (the separate kernel: 1.2e-7)
+        float acc[16];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) acc[c] = 0.0f;
+        for (int i = 0; i < rs.parts; i += 16) {
+            float x[16];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) x[c] = i + c < rs.parts ? at[static_cast<size_t>(i + c) * rs.pad] : 0.0f;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) acc[c] += x[c];
+        }
+#pragma unroll
+        for (int d = 8; d >= 1; d >>= 1)
+#pragma unroll
+            for (int c = 0; c < d; ++c) acc[c] += acc[c + d];
+        rs.out[r] = acc[0];
+        return;
+    }
+    const int64_t idx = static_cast<int64_t>(SUMS ? blockIdx.x - sum_blocks : blockIdx.x) * 256 + threadIdx.x;
     const int nq = (p.N + 3) / 4;
     const int m = static_cast<int>(idx / nq);
     const int n4 = static_cast<int>(idx - static_cast<int64_t>(m) * nq) * 4;
@@ -2255,7 +2308,7 @@ int try_half_split(const GemmParams& p, hipStream_t stream, const char* what) {
     if (rc == RC_OK) {
         const int64_t threads = static_cast<int64_t>(p.M) * ((p.N + 3) / 4);
         hipLaunchKernelGGL((reduce_slices_kernel<false>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, p, partial, slices,
-                           ma_pad, nb_pad, fired_a, fired_b);
+                           ma_pad, nb_pad, fired_a, fired_b, RowSumParts{}, 0);
         rc = check_launch(what);
     }
     workspace_give(held, stream);
@@ -2264,8 +2317,8 @@ int try_half_split(const GemmParams& p, hipStream_t stream, const char* what) {
 
 // gemm_bf16x3_pc_slices_kernel for a single dense plane with few output tiles under a long K; -1 when the contraction
 // is not of that kind or no workspace is to be had (the caller goes on to the unsliced forms).
-template <int MODE>
-int try_pc_slices(const GemmParams& p, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap) {
+template <int MODE, int BMODE = MODE>
+int try_pc_slices(const GemmParams& p, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap, bool* sums_done = nullptr) {
     const int chunks = (p.K + BK - 1) / BK;
     const int groups = p.tiles_m * p.tiles_n;
     // (two launches: about 10 us before the first chunk.  us over K for one to nine tiles, unsliced: 256 12, 400 16.5,
@@ -2279,25 +2332,25 @@ int try_pc_slices(const GemmParams& p, hipStream_t stream, const char* what, uin
     slices = (chunks + slice_chunks - 1) / slice_chunks;
     const int ma_pad = p.tiles_m * BM, nb_pad = p.tiles_n * BN;
     const size_t part_bytes = static_cast<size_t>(slices) * ma_pad * nb_pad * 4;
-    const Workspace held = workspace_take(part_bytes, stream, fixed_ws, fixed_cap);
+    const bool sums = MODE == LOAD_ROW_CONTIG && sums_done && p.row_sums;
+    const size_t sum_bytes = sums ? static_cast<size_t>(slices) * 2 * ma_pad * 4 : 0;
+    const Workspace held = workspace_take(part_bytes + sum_bytes, stream, fixed_ws, fixed_cap);
     uint8_t* ws = held.ptr;
     if (!ws) return -1;
     float* partial = reinterpret_cast<float*>(ws);
+    float* const sum_partial = sums ? reinterpret_cast<float*>(ws + part_bytes) : nullptr;
     GemmParams q = p;
     q.np2 = slices;                                      // the tile numbering walks the slices as planes
     const dim3 grid(static_cast<unsigned>(groups * slices)), block(512);
     if (MODE == LOAD_K_CONTIG && p.K % 4 != 0)
-        hipLaunchKernelGGL((gemm_bf16x3_pc_slices_kernel<MODE, false>), grid, block, 0, stream, q, chunks, slice_chunks, partial, ma_pad, nb_pad);
+        hipLaunchKernelGGL((gemm_bf16x3_pc_slices_kernel<MODE, false, BMODE>), grid, block, 0, stream, q, chunks, slice_chunks, partial, ma_pad, nb_pad, sum_partial);
     else
-        hipLaunchKernelGGL((gemm_bf16x3_pc_slices_kernel<MODE, true>), grid, block, 0, stream, q, chunks, slice_chunks, partial, ma_pad, nb_pad);
+        hipLaunchKernelGGL((gemm_bf16x3_pc_slices_kernel<MODE, true, BMODE>), grid, block, 0, stream, q, chunks, slice_chunks, partial, ma_pad, nb_pad, sum_partial);
     int rc = check_launch(what);
-    if (rc == RC_OK) {
-        const int64_t threads = static_cast<int64_t>(p.M) * ((p.N + 3) / 4);
-        hipLaunchKernelGGL((reduce_slices_kernel<false>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, p, partial, slices,
-                           ma_pad, nb_pad, static_cast<const int*>(nullptr), static_cast<const int*>(nullptr));
-        rc = check_launch(what);
-    }
+    if (rc == RC_OK)
+        rc = launch_reduce_slices(p, stream, what, partial, slices, ma_pad, nb_pad, RowSumParts{sum_partial, p.row_sums, p.M, slices * 2, ma_pad});
     workspace_give(held, stream);
+    if (sums) *sums_done = true;
     return rc;
 }
 
@@ -2364,7 +2417,8 @@ int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what
 // `fixed_ws` / `fixed_cap`: a workspace the caller brings (the static array of the entry point that allocates
 // nothing).  With one, the pool is never touched: a contraction whose bf16 planes would be larger than `fixed_cap`
 // is refused, any other runs, in the form that it takes without one where that fits.
-int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fixed_ws = nullptr, size_t fixed_cap = 0) {
+// sums_done: set where p.row_sums has been seen to.
+int launch_gemm_sums(GemmParams p, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap, bool& sums_done) {
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
     p.stream_c = streams_output(p);
@@ -2402,7 +2456,7 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
                                        : p.tiles_m >= PLANES_MIN_TILES && p.tiles_n >= PLANES_MIN_TILES && planes_groups >= PLANES_MIN_GROUPS;
     // (a caller's own workspace that the bf16 planes do not fit is refused below, whatever this form would take)
     if (!fp32_pipe && !(fixed_ws && planes_fit)) {
-        const int rc = try_f16x2(p, stream, what, fixed_ws, fixed_cap);
+        const int rc = try_f16x2(p, stream, what, fixed_ws, fixed_cap, sums_done);
         if (rc >= 0) return rc;
     }
     if (!fp32_pipe && !fixed_ws && p.a_lm > 0) {
@@ -2426,7 +2480,7 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
                 set_error("%s: this contraction needs %zu bytes of workspace, the static one holds %zu", what, ws_bytes, fixed_cap);
                 return RC_BAD_ARGS;
             }
-            const int rc = try_f16x2(p, stream, what, fixed_ws, fixed_cap);
+            const int rc = try_f16x2(p, stream, what, fixed_ws, fixed_cap, sums_done);
             if (rc >= 0) return rc;
             ws = fixed_ws;
         } else {
@@ -2460,8 +2514,8 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
             if (rc == RC_OK && partial) {
                 const int64_t threads = static_cast<int64_t>(p.M) * ((p.N + 3) / 4);
                 const dim3 rgrid(static_cast<unsigned>((threads + 255) / 256));
-                if (split) hipLaunchKernelGGL((reduce_slices_kernel<true>), rgrid, block, 0, stream, p, partial, slices, ma_pad, nb_pad, fired_a, fired_b);
-                else       hipLaunchKernelGGL((reduce_slices_kernel<false>), rgrid, block, 0, stream, p, partial, slices, ma_pad, nb_pad, fired_a, fired_b);
+                if (split) hipLaunchKernelGGL((reduce_slices_kernel<true>), rgrid, block, 0, stream, p, partial, slices, ma_pad, nb_pad, fired_a, fired_b, RowSumParts{}, 0);
+                else       hipLaunchKernelGGL((reduce_slices_kernel<false>), rgrid, block, 0, stream, p, partial, slices, ma_pad, nb_pad, fired_a, fired_b, RowSumParts{}, 0);
                 rc = check_launch(what);
             }
             if (!fixed_ws) workspace_give(held, stream);
@@ -2537,7 +2591,7 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
             }
         }
         {
-            const int rc = try_pc_slices<LOAD_ROW_CONTIG>(p, stream, what, fixed_ws, fixed_cap);
+            const int rc = try_pc_slices<LOAD_ROW_CONTIG>(p, stream, what, fixed_ws, fixed_cap, &sums_done);
             if (rc >= 0) return rc;
         }
         if (p.K > 3 * BK && (p.N <= 32) != (p.M <= 32)) {
@@ -2632,6 +2686,19 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
         else if (p.a_ks == 1 && p.b_rs == 1 && p.a_lm == 0 && !split && p.c_ni == 1 && p.K > BK &&
                  ((p.M - 1) * p.a_rs + p.K) * 4 < (1LL << 31) && p.K * p.b_ks * 4 < (1LL << 31) && p.M * p.c_mi * 4 < (1LL << 31) &&
                  p.c_mi < (1 << 22) && p.a_rs < (1 << 22) && p.b_ks < (1 << 24)) {
+            {
+                const int rc = try_pc_slices<LOAD_K_CONTIG, LOAD_ROW_CONTIG>(p, stream, what, fixed_ws, fixed_cap);
+                if (rc >= 0) return rc;
+            }
+            // (a single plane whose 64 x 64 tiles are few, by the rule above)
+            if (p.np2 * p.np3 == 1 && p.K > 3 * BK && tiles64 <= (p.M > 32 && p.N > 32 ? 2 : 1) * device_cu_count()) {
+                const dim3 g64(static_cast<unsigned>(tiles64));
+#define PPML_MPC64(STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_pc64_kernel<STREAM_, K4_, LOAD_ROW_CONTIG>), g64, dim3(512), 0, stream, p)
+                if (p.K % 4 == 0) { if (p.stream_c) PPML_MPC64(true, true); else PPML_MPC64(false, true); }
+                else              { if (p.stream_c) PPML_MPC64(true, false); else PPML_MPC64(false, false); }
+#undef PPML_MPC64
+                return check_launch(what);
+            }
 #define PPML_MIXED(STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_pc_kernel<LOAD_K_CONTIG, STREAM_, K4_, LOAD_ROW_CONTIG>), grid, dim3(512), 0, stream, p)
             if (p.K % 4 == 0) { if (p.stream_c) PPML_MIXED(true, true); else PPML_MIXED(false, true); }
             else              { if (p.stream_c) PPML_MIXED(true, false); else PPML_MIXED(false, false); }
@@ -2682,6 +2749,11 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, uint8_t* fix
     return check_launch(what);
 }
 
+int launch_gemm(const GemmParams& p, hipStream_t stream, const char* what, uint8_t* fixed_ws = nullptr, size_t fixed_cap = 0) {
+    bool sums_done = false;
+    return launch_gemm_sums(p, stream, what, fixed_ws, fixed_cap, sums_done);
+}
+
 }  // namespace
 
 // How many K slices make `groups` output tiles come out even over the CUs (a CU's rate does not depend on how many
@@ -2700,10 +2772,14 @@ int even_slices(int groups, int chunks, int most_slices, int least_chunks) {
     return slices;
 }
 
-int launch_reduce_slices(const GemmParams& p, hipStream_t stream, const char* what, const float* partial, int slices, int ma_pad, int nb_pad) {
+int launch_reduce_slices(const GemmParams& p, hipStream_t stream, const char* what, const float* partial, int slices, int ma_pad, int nb_pad,
+                         const RowSumParts& sums) {
     const int64_t threads = static_cast<int64_t>(p.M) * ((p.N + 3) / 4);
-    hipLaunchKernelGGL((reduce_slices_kernel<false>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, p, partial, slices,
-                       ma_pad, nb_pad, static_cast<const int*>(nullptr), static_cast<const int*>(nullptr));
+    const int sum_blocks = sums.partial ? (sums.rows + 255) / 256 : 0;
+    const dim3 grid(static_cast<unsigned>((threads + 255) / 256 + sum_blocks));
+    const int* const none = nullptr;
+    if (sum_blocks) hipLaunchKernelGGL((reduce_slices_kernel<false, true>), grid, dim3(256), 0, stream, p, partial, slices, ma_pad, nb_pad, none, none, sums, sum_blocks);
+    else            hipLaunchKernelGGL((reduce_slices_kernel<false>), grid, dim3(256), 0, stream, p, partial, slices, ma_pad, nb_pad, none, none, sums, 0);
     return check_launch(what);
 }
 
@@ -2741,6 +2817,28 @@ extern "C" int mul_mat_hip(const float* A, const float* B, float* C, int M, int 
     return launch_gemm(p, static_cast<hipStream_t>(stream), "mul_mat_hip");
 }
 
+namespace ppmlhip {
+// Where the form below takes the kernels that the transposed copy would lead to: operands within 32-bit offsets, a weight
+// that is not a narrow side of many tiles (those have a kernel for operands that are contiguous in k only).
+bool mul_mat_nn_fits(int64_t M, int64_t K, int64_t N) {
+    if (M <= 0 || K <= 3 * BK || N <= 0 || M * K >= (1LL << 29) || K * N >= (1LL << 28) || M * N >= (1LL << 29) || K >= (1 << 20) || N >= (1 << 20)) return false;
+    return M > 32 && (N > 32 || (M + 63) / 64 <= device_cu_count());
+}
+
+// C[M][N] = A[M][K] B[K][N]: mul_mat_hip with B's transposition folded into the loads: same products in the same order, same bits.  The copy
+// is a launch of 2.8 to 5.9 us, whatever the size, in front of a contraction of 4.4 to 43: the linear layer's forward and backward of
+// 527 x 478 -> 60 39.2 -> 36.7 us, 1058 x 480 -> 27 41.6 -> 38.
+int mul_mat_nn(const float* A, const float* B, float* C, int M, int K, int N, hipStream_t stream) {
+    StatsScope stat("hip/mul_mat", M, K, N, stream);
+    GemmParams p = plain_params();
+    p.A = A; p.B = B; p.C = C;
+    p.M = M; p.N = N; p.K = K;
+    p.a_rs = K; p.a_ks = 1; p.b_rs = 1; p.b_ks = N;
+    p.c_mi = N; p.c_ni = 1;
+    return launch_gemm(p, stream, "mul_mat_hip");
+}
+}  // namespace ppmlhip
+
 extern "C" int mul_mat_f16_hip(const void* A16, const void* B16, float* C, int M, int K, int N,
                                const float* bias, ppml_hip_stream_t stream) {
     if (!A16 || !B16 || !C || M <= 0 || K <= 0 || N <= 0) { set_error("mul_mat_f16_hip: bad arguments (M=%d K=%d N=%d)", M, K, N); return RC_BAD_ARGS; }
@@ -2765,6 +2863,26 @@ extern "C" int mul_mat_tn_hip(const float* A, const float* Bm, float* O, int M, 
     p.c_mi = Nc; p.c_ni = 1;
     p.alpha = alpha;
     return launch_gemm(p, static_cast<hipStream_t>(stream), "mul_mat_tn_hip");
+}
+
+// The sum as a kernel of its own reads the whole gradient again, and adds its runs in another launch: 16.9 + 4.7 us at 26368 x 256 -> 768,
+// 4.0 + 2.8 at 5763 x 72 -> 52.  Beside the contraction it is an addition per element that a loading wave holds anyway, and a
+// few more work-groups in the kernel that adds the slices.  Forward and backward, this and the weight's transposition folded (mul_mat_nn): 26368 x 256
+// -> 768 180 -> 154 us, 22373 x 368 -> 224 109 -> 95, 5763 x 72 -> 52 32.4 -> 23.5, 1058 x 480 -> 27 41.6 -> 35.5.
+int ppmlhip::mul_mat_tn_sums(const float* A, const float* Bm, float* O, float* sums, int M, int K, int Nc, hipStream_t stream) {
+    bool sums_done = false;
+    {
+        StatsScope stat("hip/mul_mat-tn", M, K, Nc, stream);
+        GemmParams p = plain_params();
+        p.A = A; p.B = Bm; p.C = O;
+        p.M = M; p.N = Nc; p.K = K;
+        p.a_rs = 1; p.a_ks = M; p.b_rs = 1; p.b_ks = Nc;
+        p.c_mi = Nc; p.c_ni = 1;
+        p.row_sums = sums;
+        const int rc = launch_gemm_sums(p, stream, "mul_mat_tn_hip", nullptr, 0, sums_done);
+        if (rc != RC_OK) return rc;
+    }
+    return sums_done ? RC_OK : repeat_back_hip(A, sums, M, K, 1, 1, M, 1, 1, 1, 1, K, 1, 1, stream);
 }
 
 // ---- the entry point that allocates nothing -------------------------------------------------------------

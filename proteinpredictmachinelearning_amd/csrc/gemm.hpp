@@ -28,6 +28,16 @@ struct GemmParams {
     // LOAD_SPLIT_A: both indices of A are compound, A(m,k) = A[(m/a_lm)*a_mo + (m%a_lm)*a_mi + (k/a_lk)*a_ko + (k%a_lk)*a_ki]
     int a_lm, a_lk;
     int64_t a_mo, a_mi, a_ko, a_ki;
+    // the sums over k of A's rows, which the forms with K slices leave beside the product (a linear layer's bias gradient, whose
+    // terms its weight gradient reads anyway); null where nobody wants them, and again once they are taken care of
+    float* row_sums;
+};
+
+// What reduce_slices_kernel adds up besides: partial[part][pad] of `rows` sums, parts in their order
+struct RowSumParts {
+    const float* partial;
+    float* out;
+    int rows, parts, pad;
 };
 
 // Workspace of a contraction: the pool's, or out of the array that the caller brings (`fixed`, of `cap` bytes: the pool is then
@@ -41,9 +51,11 @@ inline Workspace workspace_take(size_t bytes, hipStream_t stream, uint8_t* fixed
 
 // gemm_f16x2.hip: a large single-plane contraction in two f16 parts; -1 when the contraction is not of the kind that form is
 // for or no workspace is to be had.  `fixed_ws` / `fixed_cap`: a workspace the caller brings.
-int try_f16x2(const GemmParams& p, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap);
+// sums_done: set where p.row_sums has been seen to.
+int try_f16x2(const GemmParams& p, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap, bool& sums_done);
 // f32_gemm.hip: C = alpha * (bias + sum over the slices of partial[slice][ma_pad][nb_pad]), NaN sums redone the reference's way
-int launch_reduce_slices(const GemmParams& p, hipStream_t stream, const char* what, const float* partial, int slices, int ma_pad, int nb_pad);
+int launch_reduce_slices(const GemmParams& p, hipStream_t stream, const char* what, const float* partial, int slices, int ma_pad, int nb_pad,
+                         const RowSumParts& sums);
 // How many K slices make `groups` output tiles come out even over the CUs (f32_gemm.hip)
 int even_slices(int groups, int chunks, int most_slices, int least_chunks);
 

@@ -66,6 +66,7 @@ struct F16x2Job {
     int chunks, slice_chunks; // stages in all and per slice: even numbers
     int slices, items;
     uint32_t a_span;          // bytes of A from its base to behind its last element
+    float* a_sums;            // [slice][ma_pad]: the sums over k of A's rows, or null
 };
 
 // the largest magnitude, NaN if there is one
@@ -86,6 +87,11 @@ __device__ __forceinline__ float min4(float m, const v4f& x) {
 #else
     return m + x[0];
 #endif
+}
+
+__device__ __forceinline__ float sum8(const v4f (&x)[2]) {
+    const v4f s = x[0] + x[1];
+    return (s[0] + s[1]) + (s[2] + s[3]);
 }
 
 // how many of four elements are small ones under this scale (a power of two from 2^-115 to 2^127): not zero, below 2^-2 of it
@@ -109,6 +115,7 @@ struct F16x2Split {
     int rows, rows_pad, K, chunks, slice_chunks;
     int64_t rs, ks;
     int64_t span;             // elements from src to behind the last one: below 2^29, any 32 rows' offsets too
+    float* sums;              // [slice][rows_pad]: the rows' sums, or null
 };
 
 template <bool KS1>
@@ -147,7 +154,9 @@ __global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) 
     const bool kept = rounds <= HX_SPLIT_ROUNDS;
     v4f held[HX_SPLIT_ROUNDS][2];
     uint32_t top = 0;
+    float sum = 0.0f;
     const auto see = [&](const v4f (&v)[2]) {
+        if (jb.sums) sum += sum8(v);
         const uint32_t b = __float_as_uint(max4(max4(0.0f, v[0]), v[1]));
         top = b > top ? b : top;
     };
@@ -169,6 +178,17 @@ __global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) 
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 32; ++i) { const uint32_t o = lds_max[row][i]; top = o > top ? o : top; }
+    if (jb.sums) {                                      // (the maxima's places, once they have been read)
+        __syncthreads();
+        lds_max[row][oct] = __float_as_uint(sum);
+        __syncthreads();
+        if (oct == 0) {
+            float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int i = 0; i < 32; ++i) s[i & 3] += __uint_as_float(lds_max[row][i]);
+            jb.sums[static_cast<int64_t>(blockIdx.y) * jb.rows_pad + r] = (s[0] + s[1]) + (s[2] + s[3]);
+        }
+    }
     // the largest element goes to 2^14 .. 2^15, or as near as 2^127 brings it; an all-zero row needs no scale
     const int e = static_cast<int>(top >> 23) & 0xff;
     const bool bad = top >= 0x7f800000u;
@@ -459,13 +479,16 @@ __device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job&
         float scale[NR];
         uint32_t seen[NR];                              // OR of the maxima's bits; the sign bit: infinite or NaN
         int small[NR];                                  // this lane's share of the row's small elements
+        float sum = 0.0f;                               // ... and, where they are asked for, of its sum (HX_RC)
         int pi = 0, pc = 0, p_nch = load_item.nch, buf = 0;
         // splits the next stage into LDS
         const auto place = [&](const v4f (&x)[4]) {
             if (pc == 0) {
 #pragma unroll
                 for (int i = 0; i < NR; ++i) { scale[i] = __uint_as_float(HX_FIRST_SCALE); seen[i] = 0; small[i] = 0; }
+                sum = 0.0f;
             }
+            if (AMODE == HX_RC && OUT == HX_PARTIAL && jb.a_sums) sum += sum8({x[0], x[1]}) + sum8({x[2], x[3]});
             uint32_t top[NR], before[NR];
             bool over = false;
 #pragma unroll
@@ -562,6 +585,12 @@ __device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job&
                     }
                     const float m = wave_max(static_cast<float>(most));
                     if (lane == 0) lds_most[pi & (HX_EXPS - 1)][w] = m;
+                    if (AMODE == HX_RC && OUT == HX_PARTIAL && jb.a_sums) {
+                        sum += __shfl_xor(sum, 32, 64);
+                        const typename Items<TJ>::Item it = item_at(pi);
+                        // (the tiles of one column of tiles see every row of A once)
+                        if (it.n0 == 0 && lane < 32) jb.a_sums[static_cast<size_t>(it.slice) * jb.ma_pad + it.m0 + w * 32 + r0] = sum;
+                    }
                 }
                 pc = 0;
                 if (++pi < my_items) p_nch = item_at(pi).nch;
@@ -861,7 +890,7 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
 
 }  // namespace
 
-int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap) {
+int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap, bool& sums_done) {
     GemmParams p = p0;
     if (p.np2 * p.np3 != 1 || p.clamp || p.f16_in) return -1;
     if (p.K < 64 || p.N <= 32) return -1;
@@ -872,7 +901,9 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     const int64_t load = tiles128 * ((p.K + 15) / 16) / cus;
     // few tiles under a long K (a LinearLayer's weight gradient): slices of K, and the smaller operand is split ahead
     const bool sliced = !compound && p.a_lm == 0 && tiles128 * 2 <= cus;
+    bool swapped = false;
     if (sliced && p.M < p.N && !p.bias) {
+        swapped = true;
         std::swap(p.A, p.B);
         std::swap(p.M, p.N);
         std::swap(p.a_rs, p.b_rs);
@@ -962,7 +993,11 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     const int wgs = std::min<int64_t>((tiles * slices + 7) / 8 * 8, tj == 1 ? 2 * cus : cus);
     const int most_items = static_cast<int>(((tiles * slices + 7) / 8 + wgs / 8 - 1) / (wgs / 8));
     const size_t n_bytes = (static_cast<size_t>(wgs) * 4 * most_items * 8 + 255) / 256 * 256;
-    const size_t need = b_bytes + e_bytes + n_bytes + part_bytes;
+    // row sums: of the operand split ahead, or of the other one by its loading waves
+    const bool sums = p.row_sums && partial && (swapped || amode == HX_RC);
+    const int sum_pad = swapped ? nb_pad : ma_pad;
+    const size_t sum_bytes = sums ? static_cast<size_t>(slices) * sum_pad * 4 : 0;
+    const size_t need = b_bytes + e_bytes + n_bytes + part_bytes + sum_bytes;
     const Workspace held = workspace_take(need, stream, fixed_ws, fixed_cap);
     uint8_t* const ws = held.ptr;
     if (!ws) return -1;
@@ -977,7 +1012,9 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     jb.chunks = chunks; jb.slice_chunks = slice_chunks; jb.slices = slices;
     jb.items = static_cast<int>(tiles) * slices;
     jb.a_span = static_cast<uint32_t>(span * 4);
-    const F16x2Split sp{p.B, ws, exps, p.N, nb_pad, p.K, chunks, slice_chunks, p.b_rs, p.b_ks, b_span};
+    float* const sum_partial = sums ? reinterpret_cast<float*>(ws + b_bytes + e_bytes + n_bytes + part_bytes) : nullptr;
+    jb.a_sums = swapped ? nullptr : sum_partial;
+    const F16x2Split sp{p.B, ws, exps, p.N, nb_pad, p.K, chunks, slice_chunks, p.b_rs, p.b_ks, b_span, swapped ? sum_partial : nullptr};
     const dim3 sgrid(nb_pad / 32, slices);
     if (p.b_ks == 1) hipLaunchKernelGGL((split_f16x2_kernel<true>), sgrid, dim3(1024), 0, stream, sp);
     else             hipLaunchKernelGGL((split_f16x2_kernel<false>), sgrid, dim3(1024), 0, stream, sp);
@@ -1008,8 +1045,10 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
 #undef PPML_HX
         rc = check_launch(what);
     }
-    if (rc == RC_OK && partial) rc = launch_reduce_slices(p, stream, what, jb.partial, slices, ma_pad, nb_pad);
+    if (rc == RC_OK && partial)
+        rc = launch_reduce_slices(p, stream, what, jb.partial, slices, ma_pad, nb_pad, RowSumParts{sum_partial, p.row_sums, swapped ? p.N : p.M, slices, sum_pad});
     workspace_give(held, stream);
+    sums_done = sums;
     return rc;
 }
 

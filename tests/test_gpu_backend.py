@@ -532,6 +532,106 @@ def test_weight_gradient_reads_the_untransposed_matrices(be, T, K, N):
     assert np.array_equal(be.download(xt).reshape(K, T), X.T)
 
 
+# tokens, features in and out: the two-halves form with whole and ragged k, K slices of the exact split (one k short of a chunk, odd
+# numbers), tiles of 64 x 64, of 128 x 128 (more than two of 64 per CU), few output features, fewer tokens than a tile, a K below the fold
+@pytest.mark.parametrize("T,K,N", [(26368, 256, 256), (9040, 600, 333), (1058, 480, 395), (701, 64, 397), (408, 256, 256), (51, 33, 49),
+                                   (22373, 368, 100), (10609, 21, 128), (26368, 24, 64), (2601, 132, 50), (97, 40, 48)])
+def test_input_gradient_reads_the_weight_as_it_lies(be, T, K, N):
+    """dX = mul_mat(grad, mat_transpose(w)) (src/core/ComputeGraph.cpp:735): the copy of the weight is not made when nobody else
+    reads it, and the result has the bits of the two nodes run one by one."""
+    rng = np.random.default_rng(T + N)
+    W = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    G = rng.standard_normal((T, N)).astype(np.float32)
+    results = {}
+    for fused in (True, False):
+        be.set_fuse_permutes_into_mul_mat(fused)
+        try:
+            w, g = _leaf(be, W), _leaf(be, G)
+            wt = B.Tensor((N, K), B.F32, B.OP_PERMUTE, [w]); wt.set_param(0, 1).set_param(1, 0)
+            dX = B.Tensor((K, T), B.F32, B.OP_MUL_MAT, [g, wt])
+            assert be.graph_compute([wt, dX]) == B.SUCCESS, be.last_error
+            # (a narrow side of many tiles and a K of three chunks at most keep the copy)
+            assert be.nodes_fused_away == (1 if fused and N > 48 and (K > 32 or T <= 64 * 256) else 0)
+            results[fused] = be.download(dX).reshape(T, K)
+        finally:
+            be.set_fuse_permutes_into_mul_mat(True)
+    assert np.array_equal(results[True].view(np.int32), results[False].view(np.int32))
+    want = G.astype(np.float64) @ W.astype(np.float64)
+    bound = (np.abs(G.astype(np.float64)) @ np.abs(W.astype(np.float64))) * (N + 2) * 2.0 ** -24
+    assert np.all(np.abs(results[True] - want) <= bound)
+
+
+# the two-halves form with the gradient for either operand, K slices of the exact split (odd numbers, a narrow side, a row in the second
+# tile), and contractions without slices, where the sum is a kernel of its own
+@pytest.mark.parametrize("T,K,N", [(26368, 256, 768), (26368, 768, 256), (22373, 368, 224), (1058, 480, 27), (5763, 72, 52), (2601, 21, 130),
+                                   (300, 40, 24), (97, 64, 256)])
+def test_bias_gradient_beside_the_weight_gradient(be, T, K, N):
+    """dW = mul_mat(mat_transpose(grad), mat_transpose(x)) and dbias = repeat_back(grad) (src/core/ComputeGraph.cpp:738, 742) in one
+    pass over the gradient: the weight gradient's bits are those of the node alone, the sums are within the rounding of a sum of T terms.  A node
+    between the two that reads the sum's memory, or writes the gradient's, keeps them apart."""
+    rng = np.random.default_rng(T + K)
+    X = rng.standard_normal((T, K)).astype(np.float32)
+    G = (rng.standard_normal((T, N)) + 0.25).astype(np.float32)
+    want = G.astype(np.float64).sum(axis=0)
+    # (runs of at most 600 terms one after the other, their sums added in 256 parts at most)
+    bound = np.abs(G.astype(np.float64)).sum(axis=0) * 860 * 2.0 ** -24
+
+    def build(between=None):
+        x, g = _leaf(be, X), _leaf(be, G)
+        gt = B.Tensor((T, N), B.F32, B.OP_PERMUTE, [g]); gt.set_param(0, 1).set_param(1, 0)
+        xt = B.Tensor((T, K), B.F32, B.OP_PERMUTE, [x]); xt.set_param(0, 1).set_param(1, 0)
+        dW = B.Tensor((K, N), B.F32, B.OP_MUL_MAT, [gt, xt])
+        db = B.Tensor((N,), B.F32, B.OP_REPEAT_BACK, [g])
+        return g, [gt, xt, dW] + ([between(g, db)] if between else []) + [db], dW, db
+
+    g, nodes, dW, db = build()
+    assert be.graph_compute(nodes[:3]) == B.SUCCESS, be.last_error
+    alone = be.download(dW).reshape(N, K)
+    g, nodes, dW, db = build()
+    assert be.graph_compute(nodes) == B.SUCCESS, be.last_error
+    assert be.nodes_fused_away == 3
+    assert np.array_equal(be.download(dW).reshape(N, K).view(np.int32), alone.view(np.int32))
+    assert np.all(np.abs(be.download(db).reshape(N) - want) <= bound)
+    # an infinity and a NaN of the gradient reach their columns' sums and no other
+    G2 = G.copy()
+    G2[T // 2, 0], G2[T - 1, N - 1] = np.inf, np.nan
+    keep, G = G, G2
+    g, nodes, dW, db = build()
+    assert be.graph_compute(nodes) == B.SUCCESS, be.last_error
+    got = be.download(db).reshape(N)
+    assert got[0] == np.inf and np.isnan(got[N - 1]) and np.all(np.abs(got[1:-1] - want[1:-1]) <= bound[1:-1])
+    G = keep
+    # the sum's memory read before its place in the graph: what the reader sees is what stood there
+    import torch
+    home = torch.full((N,), 7.0, device="cuda")
+
+    def reader(g, db):
+        db.bind(home.data_ptr())
+        old = B.Tensor((N,), B.F32).bind(home.data_ptr())
+        reader.node = B.Tensor((N,), B.F32, B.OP_SCALE, [old]).set_param(0, 2.0)
+        return reader.node
+
+    g, nodes, dW, db = build(reader)
+    assert be.graph_compute(nodes) == B.SUCCESS, be.last_error
+    assert be.nodes_fused_away == 2
+    assert np.all(be.download(reader.node) == 14.0)
+    assert np.all(np.abs(home.cpu().numpy() - want) <= bound)
+
+    # the gradient's memory written before the sum's place: the sum is of what was written
+    def writer(g, db):
+        return B.Tensor((N, T), B.F32, B.OP_SCALE, [g]).set_param(0, 2.0).bind(writer.home.data_ptr())
+
+    writer.home = torch.from_numpy(G).cuda()
+    x, gl = _leaf(be, X), B.Tensor((N, T), B.F32).bind(writer.home.data_ptr())
+    gt = B.Tensor((T, N), B.F32, B.OP_PERMUTE, [gl]); gt.set_param(0, 1).set_param(1, 0)
+    xt = B.Tensor((T, K), B.F32, B.OP_PERMUTE, [x]); xt.set_param(0, 1).set_param(1, 0)
+    dW = B.Tensor((K, N), B.F32, B.OP_MUL_MAT, [gt, xt])
+    db = B.Tensor((N,), B.F32, B.OP_REPEAT_BACK, [gl])
+    assert be.graph_compute([gt, xt, dW, writer(gl, db), db]) == B.SUCCESS, be.last_error
+    assert be.nodes_fused_away == 2
+    assert np.all(np.abs(be.download(db).reshape(N) - 2 * want) <= 2 * bound)
+
+
 def test_f32_arithmetic_is_a_field_of_the_backend(be, oracle):
     # two backends with different pipes do not disturb each other or the calling thread's own setting
     import torch
