@@ -1250,17 +1250,29 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc_narrow_kernel(const GemmPa
 // end behind the last one, so every element takes its own load, whose offset is picked between the two runs' bases.
 // The K loop is cut into slices (tile numbering: the slice is the plane; one slice is allowed): raw sums go to
 // partial[slice][m][n] for reduce_slices_kernel, which adds them in slice order, applies bias, factor and the output's
-// addressing, and computes the rows and columns flagged here (fired_a, one per 32 rows) or by the small operand's split
-// (fired_b) the reference's way.
+// addressing, and computes what is NaN the reference's way: 32 rows whose split could not carry an element of the tall operand
+// leave NaN, and so does every column of the small one that its own split marked with a NaN for a first part.
 constexpr int HS_KRUN = 0, HS_RRUN = 1;
 constexpr int HS_AHEAD = 2;
+constexpr int HS_STAGE = 3 * SPLIT_PLANE;
+struct HalfSplitJob {
+    const uint8_t* wb;        // the small operand's planes
+    float* partial;
+    int nb_pad, ma_pad, chunks, slice_chunks;
+    uint32_t a_span_bytes;
+};
+struct HalfSplitLds {
+    __attribute__((aligned(16))) uint8_t a[2][HS_STAGE];
+    int again;                                          // a bit per 32 rows of the tile: the split could not carry an element
+};
 template <int AMODE, bool GEN>
-__global__ __launch_bounds__(512, 2) void gemm_bf16x3_half_split_kernel(const GemmParams p, const uint8_t* __restrict__ wb, int nb_pad, int chunks,
-                                                                        int slice_chunks, float* __restrict__ partial, int ma_pad,
-                                                                        int* __restrict__ fired_a, uint32_t a_span_bytes) {
-    constexpr int STAGE = 3 * SPLIT_PLANE;
+__device__ __forceinline__ void half_split_tile(const GemmParams& p, const HalfSplitJob& jb, HalfSplitLds& lds, int group) {
     constexpr int SMODE = AMODE == HS_KRUN ? LOAD_K_CONTIG : LOAD_ROW_CONTIG;     // the thread-to-element mapping of the split
-    __shared__ __attribute__((aligned(16))) uint8_t lds_a[2][STAGE];
+    uint8_t (&lds_a)[2][HS_STAGE] = lds.a;
+    const uint8_t* __restrict__ const wb = jb.wb;
+    float* __restrict__ const partial = jb.partial;
+    const int nb_pad = jb.nb_pad, ma_pad = jb.ma_pad, chunks = jb.chunks, slice_chunks = jb.slice_chunks;
+    const uint32_t a_span_bytes = jb.a_span_bytes;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1270,13 +1282,14 @@ __global__ __launch_bounds__(512, 2) void gemm_bf16x3_half_split_kernel(const Ge
     const int wn = (wave & 3) * 32;
 
     int slice, m0, n0;
-    tile_of_group(p, slice, m0, n0);
+    tile_of_group(p, slice, m0, n0, group);
     const int c_begin = slice * slice_chunks;
     const int c_end = c_begin + slice_chunks < chunks ? c_begin + slice_chunks : chunks;
     const int nch = c_end - c_begin;
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A), 0, static_cast<int>(a_span_bytes), 0x00020000);
 
     // (barriers: nch + 1 in either loop, as in gemm_bf16x3_pc_kernel)
+    if (tid == 0) lds.again = 0;
     if (producer) {
         // byte offsets of this lane's rows (and, HS_KRUN, of its four k within a chunk); 2^31 for rows past the matrix
         uint32_t roff[2];
@@ -1351,10 +1364,11 @@ __global__ __launch_bounds__(512, 2) void gemm_bf16x3_half_split_kernel(const Ge
             }
         }
         __syncthreads();
-        if (guard.fired()) {                            // (every writer writes the same value)
-            if (AMODE == HS_KRUN) { fired_a[(m0 + (ptid >> 2)) >> 5] = 1; fired_a[(m0 + (ptid >> 2) + 64) >> 5] = 1; }
-            else fired_a[(m0 + (ptid & 127)) >> 5] = 1;
+        if (guard.fired()) {
+            const int r = AMODE == HS_KRUN ? ptid >> 2 : ptid & 127;
+            atomicOr(&lds.again, AMODE == HS_KRUN ? 5 << (r >> 5) : 1 << (r >> 5));       // (HS_KRUN: rows r and r + 64)
         }
+        __syncthreads();
         return;
     }
 
@@ -1397,12 +1411,34 @@ __global__ __launch_bounds__(512, 2) void gemm_bf16x3_half_split_kernel(const Ge
         }
     }
 
-    // raw sums of this slice: the padded workspace takes every row and column of the tile
+    // raw sums of this slice (NaN for 32 rows to be computed again): the padded workspace takes every row and column of the tile
+    __syncthreads();
+    const int again = lds.again;
+    const float nan = __builtin_nanf("");
     float* dst = partial + (static_cast<size_t>(slice) * ma_pad + m0 + 4 * hh) * nb_pad + n0 + wn + j;
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) dst[static_cast<size_t>(ti * 32 + 8 * (r >> 2) + (r & 3)) * nb_pad] = acc[ti][r];
+        for (int r = 0; r < 16; ++r) dst[static_cast<size_t>(ti * 32 + 8 * (r >> 2) + (r & 3)) * nb_pad] = (again >> ti & 1) != 0 ? nan : acc[ti][r];
+}
+
+template <int AMODE, bool GEN>
+__global__ __launch_bounds__(512, 2) void gemm_bf16x3_half_split_kernel(const GemmParams p, const HalfSplitJob jb) {
+    __shared__ HalfSplitLds lds;
+    half_split_tile<AMODE, GEN>(p, jb, lds, static_cast<int>(blockIdx.x));
+}
+
+// Both gradients of an outer-product-mean, which read the same tensor one along its columns and one along its rows, in one
+// launch: either by itself leaves two thirds of the CUs without a work-group while its chain of chunks runs.  Each tile is what
+// the launch for it alone computes: same bits.  212 residues x 8 features x 118 sequences, forward and both gradients: 66.6 -> 40.6 us, of
+// which clearing the flags that the NaN marks stand for now was 7, and a second split ahead and sum of slices 8.
+template <bool GEN>
+__global__ __launch_bounds__(512, 2) void gemm_bf16x3_half_split_pair_kernel(const GemmParams pa, const HalfSplitJob ja, const GemmParams pb, const HalfSplitJob jb,
+                                                                             int groups_a) {
+    __shared__ HalfSplitLds lds;
+    const int group = static_cast<int>(blockIdx.x);
+    if (group < groups_a) half_split_tile<HS_KRUN, GEN>(pa, ja, lds, group);
+    else half_split_tile<HS_RRUN, GEN>(pb, jb, lds, group - groups_a);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1993,12 +2029,12 @@ struct SplitJob {
     int64_t rs, ks;                                   // element (row, k) at src[row * rs + k * ks] ...
     int lm, lk;                                       // ... or, with lm > 0, at the compound address of LOAD_SPLIT_A
     int64_t mo, mi, ko, ki;
-    int* fired;                                       // [rows_pad / 32]: set where a SplitGuard fired for that tile of 32 rows
+    int* fired;                                       // [rows_pad / 32]: set where a SplitGuard fired for that tile of 32 rows; or null:
+                                                      // NaN in the first part of the octets concerned
 };
 
 template <bool KS1, bool COMPOUND>
-__global__ __launch_bounds__(256) void split_operand_kernel(const SplitJob jb) {
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+__device__ __forceinline__ void split_octet(const SplitJob& jb, int64_t idx) {
     const int kq = static_cast<int>(idx & 1);
     const int64_t rc = idx >> 1;
     const int row = static_cast<int>(rc % jb.rows_pad);
@@ -2041,12 +2077,25 @@ __global__ __launch_bounds__(256) void split_operand_kernel(const SplitJob jb) {
     SplitGuard guard;
     split4(v[0], lo, guard);
     split4(v[1], hi, guard);
+    if (guard.fired()) {                                // (rare; every writer of a flag writes the same value)
+        if (jb.fired) jb.fired[row >> 5] = 1;
+        else lo[0] = hi[0] = uint2{0x7fc07fc0u, 0x7fc07fc0u};
+    }
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
         uint8_t* dst = jb.dst + ((static_cast<int64_t>(s) * jb.chunks + c) * jb.rows_pad + (row & ~31)) * 32 + kq * 512 + (row & 31) * 16;
         *reinterpret_cast<uint4*>(dst) = uint4{lo[s].x, lo[s].y, hi[s].x, hi[s].y};
     }
-    if (guard.fired()) jb.fired[row >> 5] = 1;          // (rare; every writer writes the same value)
+}
+
+template <bool KS1, bool COMPOUND>
+__global__ __launch_bounds__(256) void split_operand_kernel(const SplitJob jb) {
+    split_octet<KS1, COMPOUND>(jb, static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x);
+}
+
+// two operands of the same sizes, contiguous in their rows
+__global__ __launch_bounds__(256) void split_operand_pair_kernel(const SplitJob ja, const SplitJob jb) {
+    split_octet<false, false>(blockIdx.y == 0 ? ja : jb, static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x);
 }
 
 __global__ __launch_bounds__(256) void clear_flags_kernel(int* __restrict__ flags, int n) {
@@ -2167,36 +2216,9 @@ __global__ __launch_bounds__(256, 2) void gemm_planes_kernel(const GemmParams p,
 }
 
 // C = alpha * (bias + sum over the K slices, in slice order) with the contraction's own output addressing
-template <bool SPLIT_C, bool SUMS = false>
-__global__ __launch_bounds__(256) void reduce_slices_kernel(const GemmParams p, const float* __restrict__ partial,
-                                                            int slices, int ma_pad, int nb_pad,
-                                                            const int* __restrict__ fired_a, const int* __restrict__ fired_b,
-                                                            const RowSumParts rs, int sum_blocks) {
-    // the row sums' work-groups first: theirs is the longer chain
-    if (SUMS && static_cast<int>(blockIdx.x) < sum_blocks) {
-        const int r = blockIdx.x * 256 + threadIdx.x;
-        if (r >= rs.rows) return;
-        const float* at = rs.partial + r;
-        // sixteen sums of every sixteenth part, which also shortens the chain of roundings: 12949 rows x 68, 256 parts, 2.7e-7
-        // of the result in one sum, 1.0e-7 this way (the separate kernel: 1.2e-7)
-        float acc[16];
-#pragma unroll
-        for (int c = 0; c < 16; ++c) acc[c] = 0.0f;
-        for (int i = 0; i < rs.parts; i += 16) {
-            float x[16];
-#pragma unroll
-            for (int c = 0; c < 16; ++c) x[c] = i + c < rs.parts ? at[static_cast<size_t>(i + c) * rs.pad] : 0.0f;
-#pragma unroll
-            for (int c = 0; c < 16; ++c) acc[c] += x[c];
-        }
-#pragma unroll
-        for (int d = 8; d >= 1; d >>= 1)
-#pragma unroll
-            for (int c = 0; c < d; ++c) acc[c] += acc[c + d];
-        rs.out[r] = acc[0];
-        return;
-    }
-    const int64_t idx = static_cast<int64_t>(SUMS ? blockIdx.x - sum_blocks : blockIdx.x) * 256 + threadIdx.x;
+template <bool SPLIT_C>
+__device__ __forceinline__ void reduce_quad(const GemmParams& p, const float* __restrict__ partial, int slices, int ma_pad, int nb_pad,
+                                            const int* __restrict__ fired_a, const int* __restrict__ fired_b, int64_t idx) {
     const int nq = (p.N + 3) / 4;
     const int m = static_cast<int>(idx / nq);
     const int n4 = static_cast<int>(idx - static_cast<int64_t>(m) * nq) * 4;
@@ -2239,6 +2261,46 @@ __global__ __launch_bounds__(256) void reduce_slices_kernel(const GemmParams p, 
     }
 }
 
+template <bool SPLIT_C, bool SUMS = false>
+__global__ __launch_bounds__(256) void reduce_slices_kernel(const GemmParams p, const float* __restrict__ partial,
+                                                            int slices, int ma_pad, int nb_pad,
+                                                            const int* __restrict__ fired_a, const int* __restrict__ fired_b,
+                                                            const RowSumParts rs, int sum_blocks) {
+    // the row sums' work-groups first: theirs is the longer chain
+    if (SUMS && static_cast<int>(blockIdx.x) < sum_blocks) {
+        const int r = blockIdx.x * 256 + threadIdx.x;
+        if (r >= rs.rows) return;
+        const float* at = rs.partial + r;
+        // sixteen sums of every sixteenth part, which also shortens the chain of roundings: 12949 rows x 68, 256 parts, 2.7e-7
+        // of the result in one sum, 1.0e-7 this way (the separate kernel: 1.2e-7)
+        float acc[16];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) acc[c] = 0.0f;
+        for (int i = 0; i < rs.parts; i += 16) {
+            float x[16];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) x[c] = i + c < rs.parts ? at[static_cast<size_t>(i + c) * rs.pad] : 0.0f;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) acc[c] += x[c];
+        }
+#pragma unroll
+        for (int d = 8; d >= 1; d >>= 1)
+#pragma unroll
+            for (int c = 0; c < d; ++c) acc[c] += acc[c + d];
+        rs.out[r] = acc[0];
+        return;
+    }
+    reduce_quad<SPLIT_C>(p, partial, slices, ma_pad, nb_pad, fired_a, fired_b, static_cast<int64_t>(SUMS ? blockIdx.x - sum_blocks : blockIdx.x) * 256 + threadIdx.x);
+}
+
+// two dense outputs of the same sizes and slices
+__global__ __launch_bounds__(256) void reduce_slices_pair_kernel(const GemmParams pa, const float* __restrict__ partial_a, const GemmParams pb,
+                                                                 const float* __restrict__ partial_b, int slices, int ma_pad, int nb_pad) {
+    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (blockIdx.y == 0) reduce_quad<false>(pa, partial_a, slices, ma_pad, nb_pad, nullptr, nullptr, idx);
+    else reduce_quad<false>(pb, partial_b, slices, ma_pad, nb_pad, nullptr, nullptr, idx);
+}
+
 int launch_split(const SplitJob& jb, hipStream_t stream) {
     const int64_t threads = static_cast<int64_t>(jb.chunks) * jb.rows_pad * 2;
     const dim3 grid(static_cast<unsigned>((threads + 255) / 256)), block(256);
@@ -2261,56 +2323,90 @@ int f32_arithmetic() {
     return t_f32_arithmetic;
 }
 
-// gemm_bf16x3_half_split_kernel for a single-plane contraction whose tall operand A has compound indices; -1 when the
-// contraction is not of that kind (the caller goes on to the other forms).  p.tiles_m / p.tiles_n / p.stream_c are set.
-int try_half_split(const GemmParams& p, hipStream_t stream, const char* what) {
-    if (p.a_lm <= 0 || p.np2 * p.np3 != 1 || p.clamp || p.f16_in || !(p.c_lm >= p.M && p.c_ln >= p.N)) return -1;
-    if (p.a_lk < BK || p.K % p.a_lk != 0 || p.tiles_n > 16 || p.tiles_m < 3) return -1;
-    const bool gen = p.a_lk % BK != 0;                  // runs that are not whole chunks (that form: a span of at most 2^30 bytes)
-    const int amode = p.a_ki == 1 ? HS_KRUN : p.a_mi == 1 ? HS_RRUN : -1;
-    if (amode < 0) return -1;
+// gemm_bf16x3_half_split_kernel for a single-plane contraction whose tall operand A has compound indices, or the pair of two of the
+// same sizes; -1 when the contraction is not of that kind (the caller goes on to the other forms).  p.tiles_m / p.tiles_n / p.stream_c
+// are set.
+struct HalfSplitPlan {
+    int amode;
+    bool gen;
+    int64_t a_span;
+    int chunks, slices, slice_chunks, groups, ma_pad, nb_pad;
+    size_t b_bytes, part_bytes;
+    size_t bytes() const { return b_bytes + part_bytes; }
+    HalfSplitJob job(uint8_t* ws) const { return {ws, reinterpret_cast<float*>(ws + b_bytes), nb_pad, ma_pad, chunks, slice_chunks, static_cast<uint32_t>(a_span * 4)}; }
+    SplitJob split(const GemmParams& p, uint8_t* ws) const { return {p.B, ws, p.N, nb_pad, p.K, chunks, p.b_rs, p.b_ks, 0, 0, 0, 0, 0, 0, nullptr}; }
+};
+
+bool plan_half_split(const GemmParams& p, HalfSplitPlan& pl) {
+    if (p.a_lm <= 0 || p.np2 * p.np3 != 1 || p.clamp || p.f16_in || !(p.c_lm >= p.M && p.c_ln >= p.N)) return false;
+    if (p.a_lk < BK || p.K % p.a_lk != 0 || p.tiles_n > 16 || p.tiles_m < 3) return false;
+    pl.gen = p.a_lk % BK != 0;                          // runs that are not whole chunks (that form: a span of at most 2^30 bytes)
+    pl.amode = p.a_ki == 1 ? HS_KRUN : p.a_mi == 1 ? HS_RRUN : -1;
+    if (pl.amode < 0) return false;
     // 32-bit byte offsets: the tall operand's span and the dense output below 2 GiB
-    const int64_t a_span = static_cast<int64_t>((p.M - 1) / p.a_lm) * p.a_mo + static_cast<int64_t>(p.a_lm - 1) * p.a_mi +
-                           static_cast<int64_t>((p.K - 1) / p.a_lk) * p.a_ko + static_cast<int64_t>(p.a_lk - 1) * p.a_ki + 1;
-    if (p.a_mo < 0 || p.a_mi < 0 || p.a_ko < 0 || p.a_ki < 0 || a_span * 4 >= (1LL << 31) || (gen && a_span * 4 > (1LL << 30))) return -1;
-    const int chunks = (p.K + BK - 1) / BK;
-    const int groups = p.tiles_m * p.tiles_n;
-    int slices = even_slices(groups, chunks, 16, PLANES_MIN_SLICE_CHUNKS);
-    const int slice_chunks = (chunks + slices - 1) / slices;
-    slices = (chunks + slice_chunks - 1) / slice_chunks;
-    const int ma_pad = p.tiles_m * BM, nb_pad = p.tiles_n * BN;
-    const size_t b_bytes = static_cast<size_t>(3) * chunks * nb_pad * 32;
-    const size_t part_bytes = static_cast<size_t>(slices) * ma_pad * nb_pad * 4;
-    const int n_flags = ma_pad / 32 + nb_pad / 32;
-    const size_t flag_bytes = (static_cast<size_t>(n_flags) * 4 + 255) / 256 * 256;
-    const Workspace held = workspace_take(b_bytes + part_bytes + flag_bytes, stream);
+    pl.a_span = static_cast<int64_t>((p.M - 1) / p.a_lm) * p.a_mo + static_cast<int64_t>(p.a_lm - 1) * p.a_mi +
+                static_cast<int64_t>((p.K - 1) / p.a_lk) * p.a_ko + static_cast<int64_t>(p.a_lk - 1) * p.a_ki + 1;
+    if (p.a_mo < 0 || p.a_mi < 0 || p.a_ko < 0 || p.a_ki < 0 || pl.a_span * 4 >= (1LL << 31) || (pl.gen && pl.a_span * 4 > (1LL << 30))) return false;
+    pl.chunks = (p.K + BK - 1) / BK;
+    pl.groups = p.tiles_m * p.tiles_n;
+    pl.slices = even_slices(pl.groups, pl.chunks, 16, PLANES_MIN_SLICE_CHUNKS);
+    pl.slice_chunks = (pl.chunks + pl.slices - 1) / pl.slices;
+    pl.slices = (pl.chunks + pl.slice_chunks - 1) / pl.slice_chunks;
+    pl.ma_pad = p.tiles_m * BM;
+    pl.nb_pad = p.tiles_n * BN;
+    pl.b_bytes = static_cast<size_t>(3) * pl.chunks * pl.nb_pad * 32;
+    pl.part_bytes = static_cast<size_t>(pl.slices) * pl.ma_pad * pl.nb_pad * 4;
+    return true;
+}
+
+int try_half_split(const GemmParams& p, hipStream_t stream, const char* what) {
+    HalfSplitPlan pl;
+    if (!plan_half_split(p, pl)) return -1;
+    const Workspace held = workspace_take(pl.bytes(), stream);
     uint8_t* ws = held.ptr;
     if (!ws) return -1;
-    float* partial = reinterpret_cast<float*>(ws + b_bytes);
-    int* fired_a = reinterpret_cast<int*>(ws + b_bytes + part_bytes);
-    int* fired_b = fired_a + ma_pad / 32;
+    const HalfSplitJob jb = pl.job(ws);
     GemmParams q = p;
-    q.np2 = slices;                                      // the tile numbering walks the slices as planes
-    const dim3 grid(static_cast<unsigned>(groups * slices)), block(512);
-    hipLaunchKernelGGL(clear_flags_kernel, dim3((n_flags + 255) / 256), dim3(256), 0, stream, fired_a, n_flags);
-    int rc = check_launch(what);
-    const SplitJob jb{p.B, ws, p.N, nb_pad, p.K, chunks, p.b_rs, p.b_ks, 0, 0, 0, 0, 0, 0, fired_b};
-    if (rc == RC_OK) rc = launch_split(jb, stream);
+    q.np2 = pl.slices;                                   // the tile numbering walks the slices as planes
+    const dim3 grid(static_cast<unsigned>(pl.groups * pl.slices)), block(512);
+    int rc = launch_split(pl.split(p, ws), stream);
     if (rc == RC_OK) {
-        const uint32_t span_bytes = static_cast<uint32_t>(a_span * 4);
-#define PPML_HS(AMODE_, GEN_) hipLaunchKernelGGL((gemm_bf16x3_half_split_kernel<AMODE_, GEN_>), grid, block, 0, stream, q, ws, nb_pad, chunks, slice_chunks, \
-                                                 partial, ma_pad, fired_a, span_bytes)
-        if (amode == HS_KRUN) { if (gen) PPML_HS(HS_KRUN, true); else PPML_HS(HS_KRUN, false); }
-        else                  { if (gen) PPML_HS(HS_RRUN, true); else PPML_HS(HS_RRUN, false); }
+#define PPML_HS(AMODE_, GEN_) hipLaunchKernelGGL((gemm_bf16x3_half_split_kernel<AMODE_, GEN_>), grid, block, 0, stream, q, jb)
+        if (pl.amode == HS_KRUN) { if (pl.gen) PPML_HS(HS_KRUN, true); else PPML_HS(HS_KRUN, false); }
+        else                     { if (pl.gen) PPML_HS(HS_RRUN, true); else PPML_HS(HS_RRUN, false); }
 #undef PPML_HS
         rc = check_launch(what);
     }
+    if (rc == RC_OK) rc = launch_reduce_slices(p, stream, what, jb.partial, pl.slices, pl.ma_pad, pl.nb_pad, RowSumParts{});
+    workspace_give(held, stream);
+    return rc;
+}
+
+// Both gradients of an outer-product-mean, sizes and strides alike but for the run's direction.
+int try_half_split_pair(const GemmParams& a, const GemmParams& b, hipStream_t stream, const char* what) {
+    HalfSplitPlan pa, pb;
+    if (!plan_half_split(a, pa) || !plan_half_split(b, pb)) return -1;
+    if (pa.amode != HS_KRUN || pb.amode != HS_RRUN || pa.gen != pb.gen || a.M != b.M || a.N != b.N || a.K != b.K || pa.slices != pb.slices) return -1;
+    if (a.b_ks == 1 || b.b_ks == 1) return -1;           // (split_operand_pair_kernel)
+    const size_t need_a = (pa.bytes() + 255) / 256 * 256;
+    const Workspace held = workspace_take(need_a + pb.bytes(), stream);
+    uint8_t* ws = held.ptr;
+    if (!ws) return -1;
+    StatsScope stat("hip/outer_prod_mean_back_pair", a.M, a.K, a.N, stream);
+    const HalfSplitJob ja = pa.job(ws), jb = pb.job(ws + need_a);
+    GemmParams qa = a, qb = b;
+    qa.np2 = qb.np2 = pa.slices;
+    const int64_t split_threads = static_cast<int64_t>(pa.chunks) * pa.nb_pad * 2;
+    hipLaunchKernelGGL(split_operand_pair_kernel, dim3(static_cast<unsigned>((split_threads + 255) / 256), 2), dim3(256), 0, stream, pa.split(a, ws), pb.split(b, ws + need_a));
+    int rc = check_launch(what);
     if (rc == RC_OK) {
-        const int64_t threads = static_cast<int64_t>(p.M) * ((p.N + 3) / 4);
-        hipLaunchKernelGGL((reduce_slices_kernel<false>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, p, partial, slices,
-                           ma_pad, nb_pad, fired_a, fired_b, RowSumParts{}, 0);
+        const int groups = pa.groups * pa.slices;
+        const dim3 grid(static_cast<unsigned>(2 * groups)), block(512);
+        if (pa.gen) hipLaunchKernelGGL((gemm_bf16x3_half_split_pair_kernel<true>), grid, block, 0, stream, qa, ja, qb, jb, groups);
+        else        hipLaunchKernelGGL((gemm_bf16x3_half_split_pair_kernel<false>), grid, block, 0, stream, qa, ja, qb, jb, groups);
         rc = check_launch(what);
     }
+    if (rc == RC_OK) rc = launch_reduce_slices_pair(a, b, stream, what, ja.partial, jb.partial, pa.slices, pa.ma_pad, pa.nb_pad);
     workspace_give(held, stream);
     return rc;
 }
@@ -2754,6 +2850,21 @@ int launch_gemm(const GemmParams& p, hipStream_t stream, const char* what, uint8
     return launch_gemm_sums(p, stream, what, fixed_ws, fixed_cap, sums_done);
 }
 
+// Two contractions of an outer-product-mean's backward in shared launches, by the form that launch_gemm would give to either; -1 when
+// that is none that has a pair.
+int launch_gemm_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what) {
+    if (f32_arithmetic() == 1) return -1;
+    for (GemmParams* p : {&a, &b}) {
+        p->tiles_m = (p->M + BM - 1) / BM;
+        p->tiles_n = (p->N + BN - 1) / BN;
+        p->stream_c = streams_output(*p);
+    }
+    bool wanted = false;
+    const int rc = try_f16x2_pair(a, b, stream, what, wanted);
+    if (rc >= 0 || wanted) return rc;
+    return try_half_split_pair(a, b, stream, what);
+}
+
 }  // namespace
 
 // How many K slices make `groups` output tiles come out even over the CUs (a CU's rate does not depend on how many
@@ -2780,6 +2891,13 @@ int launch_reduce_slices(const GemmParams& p, hipStream_t stream, const char* wh
     const int* const none = nullptr;
     if (sum_blocks) hipLaunchKernelGGL((reduce_slices_kernel<false, true>), grid, dim3(256), 0, stream, p, partial, slices, ma_pad, nb_pad, none, none, sums, sum_blocks);
     else            hipLaunchKernelGGL((reduce_slices_kernel<false>), grid, dim3(256), 0, stream, p, partial, slices, ma_pad, nb_pad, none, none, sums, 0);
+    return check_launch(what);
+}
+
+int launch_reduce_slices_pair(const GemmParams& a, const GemmParams& b, hipStream_t stream, const char* what, const float* partial_a, const float* partial_b,
+                              int slices, int ma_pad, int nb_pad) {
+    const int64_t threads = static_cast<int64_t>(a.M) * ((a.N + 3) / 4);
+    hipLaunchKernelGGL(reduce_slices_pair_kernel, dim3(static_cast<unsigned>((threads + 255) / 256), 2), dim3(256), 0, stream, a, partial_a, b, partial_b, slices, ma_pad, nb_pad);
     return check_launch(what);
 }
 
@@ -3154,8 +3272,7 @@ extern "C" int outer_prod_mean_back_hip(const float* grad, const float* left, co
     // grad[d1][d2][i][j][b]; gleft[(d1,i)][n] = inv_N * sum_{(d2,j)} grad * right[(d2,j)][n],
     //                        gright[(d2,j)][n] = inv_N * sum_{(d1,i)} grad * left[(d1,i)][n]:
     // two contractions whose first operand has a compound row index and a compound contraction index.
-    const auto launch = [&](const float* other, float* out, int64_t mo, int64_t mi, int64_t ko, int64_t ki) {
-        StatsScope stat("hip/outer_prod_mean_back", D * L, D * L, N, static_cast<hipStream_t>(stream));
+    const auto params = [&](const float* other, float* out, int64_t mo, int64_t mi, int64_t ko, int64_t ki) {
         GemmParams p = plain_params();
         p.A = grad; p.B = other; p.C = out;
         p.M = static_cast<int>(D * L); p.N = static_cast<int>(N); p.K = static_cast<int>(D * L);
@@ -3166,10 +3283,27 @@ extern "C" int outer_prod_mean_back_hip(const float* grad, const float* left, co
         p.np2 = static_cast<int>(B);
         p.a_p2 = 1; p.b_p2 = 1; p.c_p2 = 1;
         p.alpha = inv_N;
+        return p;
+    };
+    const GemmParams pl = params(right, gleft, D * L * L, L, L * L, 1);          // m = (d1,i), k = (d2,j)
+    const GemmParams pr = params(left, gright, L * L, 1, D * L * L, L);          // m = (d2,j), k = (d1,i)
+    const auto launch = [&](const GemmParams& p) {
+        StatsScope stat("hip/outer_prod_mean_back", D * L, D * L, N, static_cast<hipStream_t>(stream));
         return launch_gemm(p, static_cast<hipStream_t>(stream), "outer_prod_mean_back_hip");
     };
+    // Both in one launch of each kind, where no output lies on an operand or on the other (the two in turn otherwise: the second
+    // then reads what the first has written).
+    if (gleft && gright && B == 1) {
+        const int64_t n = D * L * N, g = D * L * D * L;
+        const auto apart = [](const float* x, int64_t nx, const float* y, int64_t ny) { return x + nx <= y || y + ny <= x; };
+        if (apart(gleft, n, grad, g) && apart(gright, n, grad, g) && apart(gleft, n, left, n) && apart(gleft, n, right, n) && apart(gright, n, left, n) &&
+            apart(gright, n, right, n) && apart(gleft, n, gright, n)) {
+            const int rc = launch_gemm_pair(pl, pr, static_cast<hipStream_t>(stream), "outer_prod_mean_back_hip");
+            if (rc >= 0) return rc;
+        }
+    }
     int rc = RC_OK;
-    if (gleft)  rc = launch(right, gleft, D * L * L, L, L * L, 1);          // m = (d1,i), k = (d2,j)
-    if (rc == RC_OK && gright) rc = launch(left, gright, L * L, 1, D * L * L, L);   // m = (d2,j), k = (d1,i)
+    if (gleft) rc = launch(pl);
+    if (rc == RC_OK && gright) rc = launch(pr);
     return rc;
 }

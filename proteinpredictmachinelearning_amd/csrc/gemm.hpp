@@ -56,6 +56,11 @@ int try_f16x2(const GemmParams& p, hipStream_t stream, const char* what, uint8_t
 // f32_gemm.hip: C = alpha * (bias + sum over the slices of partial[slice][ma_pad][nb_pad]), NaN sums redone the reference's way
 int launch_reduce_slices(const GemmParams& p, hipStream_t stream, const char* what, const float* partial, int slices, int ma_pad, int nb_pad,
                          const RowSumParts& sums);
+int launch_reduce_slices_pair(const GemmParams& a, const GemmParams& b, hipStream_t stream, const char* what, const float* partial_a, const float* partial_b,
+                              int slices, int ma_pad, int nb_pad);
+// gemm_f16x2.hip: both gradients of an outer-product-mean, in shared launches; -1 as above, `wanted` where either by itself would take
+// that form all the same
+int try_f16x2_pair(const GemmParams& a, const GemmParams& b, hipStream_t stream, const char* what, bool& wanted);
 // How many K slices make `groups` output tiles come out even over the CUs (f32_gemm.hip)
 int even_slices(int groups, int chunks, int most_slices, int least_chunks);
 

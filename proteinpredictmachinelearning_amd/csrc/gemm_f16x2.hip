@@ -65,6 +65,7 @@ struct F16x2Job {
     int nb_pad, ma_pad;
     int chunks, slice_chunks; // stages in all and per slice: even numbers
     int slices, items;
+    int wgs;                  // work-groups of this contraction: a multiple of eight
     uint32_t a_span;          // bytes of A from its base to behind its last element
     float* a_sums;            // [slice][ma_pad]: the sums over k of A's rows, or null
 };
@@ -119,7 +120,7 @@ struct F16x2Split {
 };
 
 template <bool KS1>
-__global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) {
+__device__ __forceinline__ void split_f16x2(const F16x2Split& jb) {
     __shared__ uint32_t lds_max[32][33];
     __shared__ int lds_small[32];
     const int tid = threadIdx.x;
@@ -229,6 +230,11 @@ __global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) 
     }
 }
 
+template <bool KS1>
+__global__ __launch_bounds__(1024) void split_f16x2_kernel(const F16x2Split jb) { split_f16x2<KS1>(jb); }
+// two operands of the same sizes, contiguous in their rows
+__global__ __launch_bounds__(1024) void split_f16x2_pair_kernel(const F16x2Split ja, const F16x2Split jb) { split_f16x2<false>(blockIdx.z == 0 ? ja : jb); }
+
 // A work-group's items: first, first + step, ...; an XCD's are consecutive ones
 template <int TJ>
 struct Items {
@@ -236,12 +242,12 @@ struct Items {
     const GemmParams& p;
     const F16x2Job& jb;
     int first, step, mine;
-    __device__ __forceinline__ Items(const GemmParams& p_, const F16x2Job& jb_) : p(p_), jb(jb_) {
-        const int xcd = blockIdx.x & 7;
-        step = gridDim.x >> 3;
+    __device__ __forceinline__ Items(const GemmParams& p_, const F16x2Job& jb_, int block) : p(p_), jb(jb_) {
+        const int xcd = block & 7;
+        step = jb.wgs >> 3;
         const int lo = static_cast<int>(static_cast<int64_t>(jb.items) * xcd / 8);
         const int hi = static_cast<int>(static_cast<int64_t>(jb.items) * (xcd + 1) / 8);
-        first = lo + static_cast<int>(blockIdx.x >> 3);
+        first = lo + (block >> 3);
         mine = first < hi ? (hi - first + step - 1) / step : 0;
     }
     __device__ __forceinline__ Item at(int i) const {
@@ -360,24 +366,34 @@ __device__ __forceinline__ void redo_tiles(const GemmParams& p, const F16x2Job& 
 // the next item while waves 0 .. 3 store the finished one.  A contracting wave takes all 128 rows and 32 TJ columns: B's
 // fragments belong to it alone and come straight from memory (L2), two stages ahead; A's come from LDS one step ahead of
 // their six MFMAs.  Barrier i + 1 says "stages up to i + 1 are in LDS" and "stage i - 1 has been read".
+struct F16x2Lds {
+    __attribute__((aligned(16))) uint8_t a[HX_BUFS * HX_STAGE];
+    __attribute__((aligned(16))) float factor[HX_BUFS][HX_M];
+    __attribute__((aligned(16))) int mark[HX_BUFS][4];
+    // exponents of the rows' scales, per item: written with an item's last stage, read behind it, by when the loading waves
+    // are at most two stages (two items, were an item one stage) further
+    __attribute__((aligned(16))) int exp[HX_EXPS][HX_M];
+    __attribute__((aligned(16))) float small[HX_EXPS][HX_M];      // their small elements, HX_ZEROS for a row of zeros ...
+    __attribute__((aligned(16))) float most[HX_EXPS][4];          // ... and the most of them in a row, per loading wave
+    int noted[4];
+};
 template <int AMODE, bool GEN, int TJ, int OUT, bool STREAM>
-__device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job& jb, int (&lds_noted)[4]) {
+__device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job& jb, F16x2Lds& lds, int block) {
     constexpr bool KLOAD = AMODE == HX_KC || AMODE == HX_KRUN;
     constexpr bool RUNS = AMODE == HX_KRUN || AMODE == HX_RRUN;
     constexpr int NR = KLOAD ? 4 : 1;                  // rows of A a loading lane has a share of
-    __shared__ __attribute__((aligned(16))) uint8_t lds_a[HX_BUFS * HX_STAGE];
-    __shared__ __attribute__((aligned(16))) float lds_factor[HX_BUFS][HX_M];
-    __shared__ __attribute__((aligned(16))) int lds_mark[HX_BUFS][4];
-    // exponents of the rows' scales, per item: written with an item's last stage, read behind it, by when the loading waves
-    // are at most two stages (two items, were an item one stage) further
-    __shared__ __attribute__((aligned(16))) int lds_exp[HX_EXPS][HX_M];
-    __shared__ __attribute__((aligned(16))) float lds_small[HX_EXPS][HX_M];      // their small elements, HX_ZEROS for a row of zeros ...
-    __shared__ __attribute__((aligned(16))) float lds_most[HX_EXPS][4];          // ... and the most of them in a row, per loading wave
+    uint8_t (&lds_a)[HX_BUFS * HX_STAGE] = lds.a;
+    float (&lds_factor)[HX_BUFS][HX_M] = lds.factor;
+    int (&lds_mark)[HX_BUFS][4] = lds.mark;
+    int (&lds_exp)[HX_EXPS][HX_M] = lds.exp;
+    float (&lds_small)[HX_EXPS][HX_M] = lds.small;
+    float (&lds_most)[HX_EXPS][4] = lds.most;
+    int (&lds_noted)[4] = lds.noted;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    const Items<TJ> items(p, jb);
+    const Items<TJ> items(p, jb, block);
     const int my_items = items.mine;
     const auto item_at = [&](int i) { return items.at(i); };
     if (my_items == 0) return;                          // (the whole work-group: no barrier is left behind)
@@ -646,7 +662,7 @@ __device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job&
     v4i mark = *reinterpret_cast<const v4i*>(lds_mark[0]);
     v16f acc[4][TJ];
     int g = 0;
-    uint64_t* const notes = jb.notes + static_cast<size_t>(blockIdx.x * 4 + wave) * jb.most_items;
+    uint64_t* const notes = jb.notes + static_cast<size_t>(block * 4 + wave) * jb.most_items;
     int noted = 0;                                      // items with outputs to redo
     // the smallest of this lane's sums in a tile row
     const auto least = [&](int ti) {
@@ -847,24 +863,25 @@ __device__ __forceinline__ void f16x2_items(const GemmParams& p, const F16x2Job&
     if (lane == 0) lds_noted[wave] = noted;
 }
 
+// (kernarg_at: where the parameters lie in the kernel's arguments)
 template <int AMODE, bool GEN, int TJ, int OUT, bool STREAM>
-__global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const GemmParams p, const F16x2Job jb) {
-    __shared__ int lds_noted[4];
-    if (threadIdx.x < 4) lds_noted[threadIdx.x] = 0;    // (a work-group without items leaves them so)
-    f16x2_items<AMODE, GEN, TJ, OUT, STREAM>(p, jb, lds_noted);
+__device__ __forceinline__ void f16x2_contract(const GemmParams& p, const F16x2Job& jb, F16x2Lds& lds, int block, size_t kernarg_at) {
+    if (threadIdx.x < 4) lds.noted[threadIdx.x] = 0;    // (a work-group without items leaves them so)
+    f16x2_items<AMODE, GEN, TJ, OUT, STREAM>(p, jb, lds, block);
     // What the items left to redo, by all eight waves.  Behind the last item, where nothing else is held in registers (among the items the
     // two-to-a-CU form spilled its fragments), and with the parameters read again, which the items then need not hold either.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (the notes, and the stores of the outputs concerned, have landed)
     __syncthreads();
     int counts[4], any = 0;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) { counts[w] = __builtin_amdgcn_readfirstlane(lds_noted[w]); any |= counts[w]; }
+    for (int w = 0; w < 4; ++w) { counts[w] = __builtin_amdgcn_readfirstlane(lds.noted[w]); any |= counts[w]; }
     if (any == 0) return;
     typedef const __attribute__((address_space(4))) GemmParams* KernargPtr;
-    KernargPtr again = (KernargPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    typedef const __attribute__((address_space(4))) uint8_t* KernargBytes;
+    KernargPtr again = (KernargPtr)((KernargBytes)__builtin_amdgcn_kernarg_segment_ptr() + kernarg_at);
     asm volatile("" : "+s"(again));
     const GemmParams pr = *(const GemmParams*)again;
-    const Items<TJ> items(pr, jb);
+    const Items<TJ> items(pr, jb, block);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int unit = 0;
 #pragma unroll 1
@@ -873,7 +890,7 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
 #pragma unroll 1
         for (int u = 0; u < count * 2 * TJ; ++u) {      // (64 rows x 32 columns each)
             if ((unit++ & 7) != wave) continue;
-            const uint64_t note = jb.notes[static_cast<size_t>(blockIdx.x * 4 + w) * jb.most_items + u / (2 * TJ)];
+            const uint64_t note = jb.notes[static_cast<size_t>(block * 4 + w) * jb.most_items + u / (2 * TJ)];
             const auto it = items.at(__builtin_amdgcn_readfirstlane(static_cast<int>(note >> 32)));
             const uint32_t which = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(note));
             const int ti = u / TJ % 2 * 2, tj = u % TJ;
@@ -888,12 +905,55 @@ __global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const 
     }
 }
 
-}  // namespace
+template <int AMODE, bool GEN, int TJ, int OUT, bool STREAM>
+__global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_kernel(const GemmParams p, const F16x2Job jb) {
+    __shared__ F16x2Lds lds;
+    f16x2_contract<AMODE, GEN, TJ, OUT, STREAM>(p, jb, lds, static_cast<int>(blockIdx.x), 0);
+}
 
-int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap, bool& sums_done) {
-    GemmParams p = p0;
-    if (p.np2 * p.np3 != 1 || p.clamp || p.f16_in) return -1;
-    if (p.K < 64 || p.N <= 32) return -1;
+// Both gradients of an outer-product-mean in one launch, each by half of the work-groups: the same tiles, and bits, as in two, without the
+// second's start, and with the splits ahead and the sums of the slices in one launch each too.  Forward and both gradients, in two / this way, us:
+// 103 residues x 32 features x 256 sequences 124 / 109, 384 residues 853 / 841.
+struct F16x2Pair { GemmParams pa, pb; F16x2Job ja, jb; };
+template <bool GEN, int TJ>
+__global__ __launch_bounds__(512, TJ == 1 ? 4 : 2) void gemm_f16x2_pair_kernel(const F16x2Pair pair) {
+    __shared__ F16x2Lds lds;
+    const int block = static_cast<int>(blockIdx.x);
+    if (block < pair.ja.wgs) f16x2_contract<HX_KRUN, GEN, TJ, HX_PARTIAL, false>(pair.pa, pair.ja, lds, block, offsetof(F16x2Pair, pa));
+    else f16x2_contract<HX_RRUN, GEN, TJ, HX_PARTIAL, false>(pair.pb, pair.jb, lds, block - pair.ja.wgs, offsetof(F16x2Pair, pb));
+}
+
+// How one contraction goes: what try_f16x2 settles before it has memory
+struct F16x2Plan {
+    GemmParams p;
+    F16x2Job jb;
+    int amode, tj, out, sum_pad;
+    bool gen, partial, swapped, sums, compound;
+    int64_t b_span;
+    size_t b_bytes, e_bytes, n_bytes, part_bytes, sum_bytes;
+    size_t bytes() const { return b_bytes + e_bytes + n_bytes + part_bytes + sum_bytes; }
+    float* sum_partial(uint8_t* ws) const { return sums ? reinterpret_cast<float*>(ws + b_bytes + e_bytes + n_bytes + part_bytes) : nullptr; }
+    F16x2Job job(uint8_t* ws) const {
+        F16x2Job j = jb;
+        j.wb = ws;
+        j.eb = reinterpret_cast<uint32_t*>(ws + b_bytes);
+        j.notes = reinterpret_cast<uint64_t*>(ws + b_bytes + e_bytes);
+        j.partial = reinterpret_cast<float*>(ws + b_bytes + e_bytes + n_bytes);
+        j.a_sums = swapped ? nullptr : sum_partial(ws);
+        return j;
+    }
+    F16x2Split split(uint8_t* ws) const {
+        return {p.B, ws, reinterpret_cast<uint32_t*>(ws + b_bytes), p.N, jb.nb_pad, p.K, jb.chunks, jb.slice_chunks, p.b_rs, p.b_ks, b_span, swapped ? sum_partial(ws) : nullptr};
+    }
+    dim3 split_grid(int operands = 1) const { return dim3(jb.nb_pad / 32, jb.slices, operands); }
+};
+
+// cu_share: the part of the CUs this contraction is to have (a half where two go side by side)
+bool plan_f16x2(const GemmParams& p0, F16x2Plan& pl, int cu_share = 1) {
+    GemmParams& p = pl.p;
+    p = p0;
+    if (p.np2 * p.np3 != 1 || p.clamp || p.f16_in) return false;
+    if (p.K < 64 || p.N <= 32) return false;
     const bool compound = !(p.c_lm >= p.M && p.c_ln >= p.N);
     const int cus = device_cu_count() / 8 * 8;
     // matrix work: 16-k steps of 128 x 128 tiles per CU
@@ -910,36 +970,36 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
         std::swap(p.a_ks, p.b_ks);
         std::swap(p.c_mi, p.c_ni);
     }
-    if (p.M < 128) return -1;
+    if (p.M < 128) return false;
     // how A lies, and 32-bit byte offsets into it
     int amode;
     bool gen = false;
     int64_t span;
     if (p.a_lm > 0) {
-        if (p.a_lk < HX_K || p.K % p.a_lk != 0 || p.a_mo < 0 || p.a_mi < 0 || p.a_ko < 0 || p.a_ki < 0) return -1;
+        if (p.a_lk < HX_K || p.K % p.a_lk != 0 || p.a_mo < 0 || p.a_mi < 0 || p.a_ko < 0 || p.a_ki < 0) return false;
         amode = p.a_ki == 1 ? HX_KRUN : p.a_mi == 1 ? HX_RRUN : -1;
         gen = p.a_lk % HX_K != 0;
         span = static_cast<int64_t>((p.M - 1) / p.a_lm) * p.a_mo + static_cast<int64_t>(std::min(p.a_lm, p.M) - 1) * p.a_mi +
                static_cast<int64_t>((p.K - 1) / p.a_lk) * p.a_ko + static_cast<int64_t>(p.a_lk - 1) * p.a_ki + 1;
-        if (gen && span * 4 > (1LL << 30)) return -1;
+        if (gen && span * 4 > (1LL << 30)) return false;
     } else if (p.a_ks == 1) {
         amode = HX_KC;
         gen = p.K % 4 != 0;
         span = static_cast<int64_t>(p.M - 1) * p.a_rs + p.K;
-        if (p.a_rs < p.K) return -1;
+        if (p.a_rs < p.K) return false;
     } else if (p.a_rs == 1) {
         amode = HX_RC;
         span = static_cast<int64_t>(p.K) * p.a_ks;
-        if (p.a_ks < p.M || (span + 128 * p.a_ks) * 4 >= (1LL << 31)) return -1;
+        if (p.a_ks < p.M || (span + 128 * p.a_ks) * 4 >= (1LL << 31)) return false;
     } else {
-        return -1;
+        return false;
     }
-    if (amode < 0 || span * 4 >= (1LL << 31) - 65536) return -1;
+    if (amode < 0 || span * 4 >= (1LL << 31) - 65536) return false;
     // B by 32-bit byte offsets as well
     const int64_t b_span = static_cast<int64_t>(p.N - 1) * p.b_rs + static_cast<int64_t>(p.K - 1) * p.b_ks + 1;
-    if (p.b_rs <= 0 || p.b_ks <= 0 || b_span * 4 >= (1LL << 31) || (static_cast<int64_t>(p.K) + 64) * p.b_ks * 4 + 32 * p.b_rs * 4 >= (1LL << 31)) return -1;
+    if (p.b_rs <= 0 || p.b_ks <= 0 || b_span * 4 >= (1LL << 31) || (static_cast<int64_t>(p.K) + 64) * p.b_ks * 4 + 32 * p.b_rs * 4 >= (1LL << 31)) return false;
     // the output (slices: any strides)
-    if (compound ? p.c_span == 0 : (p.c_ni != 1 && !sliced) || static_cast<int64_t>(p.M + HX_M) * p.c_mi * 4 >= (1LL << 31)) return -1;
+    if (compound ? p.c_span == 0 : (p.c_ni != 1 && !sliced) || static_cast<int64_t>(p.M + HX_M) * p.c_mi * 4 >= (1LL << 31)) return false;
 
     // Where the lines lie (us, the other forms / this one; `load` in steps).  The split ahead and a deeper pipeline cost 5 us
     // before the first tile, so the contraction has to be worth it:
@@ -954,10 +1014,10 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     //     25.8 / 28.1, 12000 x 223 -> 800 (32) 32.7 / 34.2, 26368 x 223 -> 512 (45) 47.1 / 39.2; 9040 x 333 -> 600 (27) 34.4 / 29.7.
     // A K below 128 stays with the form that splits in the tile loop at any size (the bits of a contraction that is cut
     // out of a larger one then do not depend on the size).
-    if (p.a_lm > 0) { if (load < 22) return -1; }
-    else if (compound) { if (load < 30) return -1; }
-    else if (sliced) { if (load < 42 || (p.M < 700 && load < 66) || p.K < 128) return -1; }
-    else if (p.K < 128 || tiles128 <= cus || static_cast<double>(p.M) * p.N * p.K < (p.K < 256 ? 40.0 : 20.0) * 128 * 128 * 16 * cus) return -1;      // (without the padding: 30001 x 131 -> 260 25.8 / 29.7)
+    if (p.a_lm > 0) { if (load < 22) return false; }
+    else if (compound) { if (load < 30) return false; }
+    else if (sliced) { if (load < 42 || (p.M < 700 && load < 66) || p.K < 128) return false; }
+    else if (p.K < 128 || tiles128 <= cus || static_cast<double>(p.M) * p.N * p.K < (p.K < 256 ? 40.0 : 20.0) * 128 * 128 * 16 * cus) return false;      // (without the padding: 30001 x 131 -> 260 25.8 / 29.7)
     // Tiles of 128 x 256 by one work-group per CU, or of 128 x 128 by two, which store while the other contracts but read A
     // twice as often: where 256 columns would be half empty, where the wide tiles' last round leaves more than half of the CUs idle (26368 x 256 -> 768: 51.4
     // / 48.8 us; 32768 x 512 -> 1024, whole rounds, 110 / 118), and for compound rows that are not whole lines, whose stores
@@ -981,7 +1041,7 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     if (!compound && tiles * 4 < 3 * cus) {
         slices = even_slices(static_cast<int>(tiles), chunks / 2, 128, 4);      // (whole pairs of stages, at least 256 k)
     }
-    if (tiles > (1 << 24) || tiles * slices < 32 || (compound && p.c_ni <= 0)) return -1;
+    if (tiles > (1 << 24) || tiles * slices < 32 || (compound && p.c_ni <= 0)) return false;
     const int slice_chunks = (chunks / 2 + slices - 1) / slices * 2;
     slices = (chunks + slice_chunks - 1) / slice_chunks;
     const int ma_pad = p.tiles_m * HX_M, nb_pad = p.tiles_n * nt;
@@ -989,39 +1049,48 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
     const size_t e_bytes = (static_cast<size_t>(slices) * nb_pad * 4 + 255) / 256 * 256;
     const bool partial = slices > 1 || p.a_lm > 0 || p.c_ni != 1;     // (no direct instances for a compound A)
     const size_t part_bytes = partial ? static_cast<size_t>(slices) * ma_pad * nb_pad * 4 : 0;
-    if (static_cast<size_t>(ma_pad) * nb_pad * 4 >= (1ull << 31) && partial) return -1;
-    const int wgs = std::min<int64_t>((tiles * slices + 7) / 8 * 8, tj == 1 ? 2 * cus : cus);
+    if (static_cast<size_t>(ma_pad) * nb_pad * 4 >= (1ull << 31) && partial) return false;
+    const int wgs = std::min<int64_t>((tiles * slices + 7) / 8 * 8, (tj == 1 ? 2 * cus : cus) / cu_share / 8 * 8);
     const int most_items = static_cast<int>(((tiles * slices + 7) / 8 + wgs / 8 - 1) / (wgs / 8));
-    const size_t n_bytes = (static_cast<size_t>(wgs) * 4 * most_items * 8 + 255) / 256 * 256;
+    pl.b_bytes = b_bytes;
+    pl.e_bytes = e_bytes;
+    pl.n_bytes = (static_cast<size_t>(wgs) * 4 * most_items * 8 + 255) / 256 * 256;
+    pl.part_bytes = part_bytes;
     // row sums: of the operand split ahead, or of the other one by its loading waves
-    const bool sums = p.row_sums && partial && (swapped || amode == HX_RC);
-    const int sum_pad = swapped ? nb_pad : ma_pad;
-    const size_t sum_bytes = sums ? static_cast<size_t>(slices) * sum_pad * 4 : 0;
-    const size_t need = b_bytes + e_bytes + n_bytes + part_bytes + sum_bytes;
-    const Workspace held = workspace_take(need, stream, fixed_ws, fixed_cap);
-    uint8_t* const ws = held.ptr;
-    if (!ws) return -1;
-    F16x2Job jb{};
-    jb.wb = ws;
-    uint32_t* const exps = reinterpret_cast<uint32_t*>(ws + b_bytes);
-    jb.eb = exps;
-    jb.notes = reinterpret_cast<uint64_t*>(ws + b_bytes + e_bytes);
+    pl.sums = p.row_sums && partial && (swapped || amode == HX_RC);
+    pl.sum_pad = swapped ? nb_pad : ma_pad;
+    pl.sum_bytes = pl.sums ? static_cast<size_t>(slices) * pl.sum_pad * 4 : 0;
+    pl.amode = amode; pl.tj = tj; pl.gen = gen; pl.partial = partial; pl.swapped = swapped; pl.compound = compound; pl.b_span = b_span;
+    pl.out = partial ? HX_PARTIAL : compound ? HX_COMPOUND : HX_DENSE;
+    F16x2Job& jb = pl.jb;
+    jb = F16x2Job{};
     jb.most_items = most_items;
-    jb.partial = reinterpret_cast<float*>(ws + b_bytes + e_bytes + n_bytes);
     jb.nb_pad = nb_pad; jb.ma_pad = ma_pad;
     jb.chunks = chunks; jb.slice_chunks = slice_chunks; jb.slices = slices;
     jb.items = static_cast<int>(tiles) * slices;
+    jb.wgs = wgs;
     jb.a_span = static_cast<uint32_t>(span * 4);
-    float* const sum_partial = sums ? reinterpret_cast<float*>(ws + b_bytes + e_bytes + n_bytes + part_bytes) : nullptr;
-    jb.a_sums = swapped ? nullptr : sum_partial;
-    const F16x2Split sp{p.B, ws, exps, p.N, nb_pad, p.K, chunks, slice_chunks, p.b_rs, p.b_ks, b_span, swapped ? sum_partial : nullptr};
-    const dim3 sgrid(nb_pad / 32, slices);
-    if (p.b_ks == 1) hipLaunchKernelGGL((split_f16x2_kernel<true>), sgrid, dim3(1024), 0, stream, sp);
-    else             hipLaunchKernelGGL((split_f16x2_kernel<false>), sgrid, dim3(1024), 0, stream, sp);
+    return true;
+}
+
+}  // namespace
+
+int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap, bool& sums_done) {
+    F16x2Plan pl;
+    if (!plan_f16x2(p0, pl)) return -1;
+    const Workspace held = workspace_take(pl.bytes(), stream, fixed_ws, fixed_cap);
+    uint8_t* const ws = held.ptr;
+    if (!ws) return -1;
+    const GemmParams& p = pl.p;
+    const F16x2Job jb = pl.job(ws);
+    const int amode = pl.amode, tj = pl.tj, out = pl.out, wgs = jb.wgs;
+    const bool gen = pl.gen;
+    const F16x2Split sp = pl.split(ws);
+    if (p.b_ks == 1) hipLaunchKernelGGL((split_f16x2_kernel<true>), pl.split_grid(), dim3(1024), 0, stream, sp);
+    else             hipLaunchKernelGGL((split_f16x2_kernel<false>), pl.split_grid(), dim3(1024), 0, stream, sp);
     int rc = check_launch(what);
     if (rc == RC_OK) {
-        const int out = partial ? HX_PARTIAL : compound ? HX_COMPOUND : HX_DENSE;
-        const bool stream_c = p.stream_c && !partial;
+        const bool stream_c = p.stream_c && !pl.partial;
 #define PPML_HX(A_, G_, T_, O_, S_) hipLaunchKernelGGL((gemm_f16x2_kernel<A_, G_, T_, O_, S_>), dim3(wgs), dim3(512), 0, stream, p, jb)
 #define PPML_HX_T(A_, G_, O_, S_) do { if (tj == 1) PPML_HX(A_, G_, 1, O_, S_); else PPML_HX(A_, G_, 2, O_, S_); } while (0)
 #define PPML_HX_O(A_, G_)                                                                                         \
@@ -1045,10 +1114,38 @@ int try_f16x2(const GemmParams& p0, hipStream_t stream, const char* what, uint8_
 #undef PPML_HX
         rc = check_launch(what);
     }
-    if (rc == RC_OK && partial)
-        rc = launch_reduce_slices(p, stream, what, jb.partial, slices, ma_pad, nb_pad, RowSumParts{sum_partial, p.row_sums, swapped ? p.N : p.M, slices, sum_pad});
+    if (rc == RC_OK && pl.partial)
+        rc = launch_reduce_slices(p, stream, what, jb.partial, jb.slices, jb.ma_pad, jb.nb_pad,
+                                  RowSumParts{pl.sum_partial(ws), p.row_sums, pl.swapped ? p.N : p.M, jb.slices, pl.sum_pad});
     workspace_give(held, stream);
-    sums_done = sums;
+    sums_done = pl.sums;
+    return rc;
+}
+
+int try_f16x2_pair(const GemmParams& a, const GemmParams& b, hipStream_t stream, const char* what, bool& wanted) {
+    F16x2Plan pa, pb;
+    const bool fa = plan_f16x2(a, pa, 2), fb = plan_f16x2(b, pb, 2);
+    wanted = fa || fb;
+    if (!fa || !fb || pa.amode != HX_KRUN || pb.amode != HX_RRUN || pa.gen != pb.gen || pa.tj != pb.tj || !pa.partial || !pb.partial) return -1;
+    if (a.M != b.M || a.N != b.N || a.K != b.K || pa.jb.slices != pb.jb.slices || a.b_ks == 1 || b.b_ks == 1) return -1;
+    const size_t need_a = (pa.bytes() + 255) / 256 * 256;
+    const Workspace held = workspace_take(need_a + pb.bytes(), stream);
+    uint8_t* const ws = held.ptr;
+    if (!ws) return -1;
+    StatsScope stat("hip/outer_prod_mean_back_pair", a.M, a.K, a.N, stream);
+    const F16x2Pair pair{pa.p, pb.p, pa.job(ws), pb.job(ws + need_a)};
+    hipLaunchKernelGGL(split_f16x2_pair_kernel, pa.split_grid(2), dim3(1024), 0, stream, pa.split(ws), pb.split(ws + need_a));
+    int rc = check_launch(what);
+    if (rc == RC_OK) {
+        const dim3 grid(pair.ja.wgs + pair.jb.wgs);
+#define PPML_HX_PAIR(G_, T_) hipLaunchKernelGGL((gemm_f16x2_pair_kernel<G_, T_>), grid, dim3(512), 0, stream, pair)
+        if (pa.tj == 1) { if (pa.gen) PPML_HX_PAIR(true, 1); else PPML_HX_PAIR(false, 1); }
+        else            { if (pa.gen) PPML_HX_PAIR(true, 2); else PPML_HX_PAIR(false, 2); }
+#undef PPML_HX_PAIR
+        rc = check_launch(what);
+    }
+    if (rc == RC_OK) rc = launch_reduce_slices_pair(pa.p, pb.p, stream, what, pair.ja.partial, pair.jb.partial, pair.ja.slices, pair.ja.ma_pad, pair.ja.nb_pad);
+    workspace_give(held, stream);
     return rc;
 }
 

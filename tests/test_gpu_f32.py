@@ -890,6 +890,28 @@ def test_outer_prod_mean_back(ops, oracle, D, L, N, Bt):
         assert none is None and np.array_equal(gr.cpu().numpy(), wr)
 
 
+# the exact split in the tile loop (runs of whole chunks, of any length; one column tile and two), two halves (either run; tiles of 128 and
+# of 256 columns), and a size whose two contractions stay launches of their own
+@pytest.mark.parametrize("D,L,N", [(8, 48, 64), (8, 103, 200), (8, 212, 118), (32, 128, 100), (32, 111, 128), (32, 96, 256), (32, 103, 256), (8, 24, 33)])
+def test_outer_prod_mean_back_both_gradients_have_the_bits_of_one_at_a_time(ops, D, L, N):
+    torch.manual_seed(D + L + N)
+    n = D * L * N
+    left, right, grad = (torch.randn(s, device="cuda") for s in (n, n, D * D * L * L))
+    grad[5] = float("inf")
+    right[11 * N + 3] = float("nan")
+    gl, gr = ops.outer_prod_mean_back(grad, left, right, D, L, N, 1)
+    one_l, _ = ops.outer_prod_mean_back(grad, left, right, D, L, N, 1, want_right=False)
+    _, one_r = ops.outer_prod_mean_back(grad, left, right, D, L, N, 1, want_left=False)
+    assert torch.equal(gl.view(torch.int32), one_l.view(torch.int32)) and torch.equal(gr.view(torch.int32), one_r.view(torch.int32))
+    # a gradient on the memory of an operand that the other one reads: in turn, so the second is of what the first has written
+    here = left.clone()
+    out = torch.empty(n, device="cuda")
+    lib = ops._lib()
+    assert lib.outer_prod_mean_back_hip(grad.data_ptr(), here.data_ptr(), right.data_ptr(), here.data_ptr(), out.data_ptr(), D, L, N, 1, 1.0 / N, ops._stream()) == 0
+    _, after = ops.outer_prod_mean_back(grad, gl, right, D, L, N, 1, want_left=False)
+    assert torch.equal(here.view(torch.int32), gl.view(torch.int32)) and torch.equal(out.view(torch.int32), after.view(torch.int32))
+
+
 @pytest.mark.parametrize("planes,K,ne00,ne10", [(824, 256, 256, 32), (412, 103, 103, 32), (7, 70, 300, 5), (3, 200, 33, 32), (50, 64, 128, 16),
                                                 (5, 90, 20, 200), (2, 1000, 129, 31)])
 def test_out_prod_with_a_narrow_side_takes_narrow_tiles_with_the_same_bits(ops, planes, K, ne00, ne10):
