@@ -67,7 +67,10 @@ void ppml_hip_backend_set_fuse_attention_bridges(ppml_hip_backend *b, int on);
  * folded node would have run: to a node in between, or to that node itself); a folded tensor is never written.
  *   relu_into_q8 (default 1): an OP_UNARY/RELU read only -- directly or through whole OP_VIEW / OP_RESHAPE nodes --
  *     by the activation side of a quantized OP_MUL_MAT is applied by that matmul's quantizer
- *     (src/modules/Attention.cpp:1097-1104); same bits as the two nodes run one after the other.
+ *     (src/modules/Attention.cpp:1097-1104); same bits as the two nodes run one after the other.  Where the ReLU's own
+ *     source is another quantized OP_MUL_MAT nobody else reads and no memory is bound to -- K -> H -> K features, K of 64,
+ *     128, 192 or 256, H of 2 K or 4 K, weights both packed or both Q8_0R, default activations -- both run in one launch, same bits, and
+ *     the hidden tensor is not written.
  *   scale_into_out_prod (default 1): an OP_SCALE whose source is an OP_OUT_PROD nobody else reads runs as one
  *     scaled contraction (src/modules/Attention.cpp:264-270); same bits.
  *   attention_chain (default 0): out_prod(K,Q) -> scale -> [add bias] -> softmax -> permute / permute(V) ->
@@ -97,7 +100,7 @@ void ppml_hip_backend_set_fuse_permutes_into_out_prod(ppml_hip_backend *b, int o
  *     folded like this, of the same gradient down to its first dimension (the bias gradient), is left beside it: its sum is the
  *     contraction's pass over the gradient, in another order than the node's own. */
 void ppml_hip_backend_set_fuse_permutes_into_mul_mat(ppml_hip_backend *b, int on);
-/* how many nodes the last graph_compute folded into a neighbour and did not execute */
+/* how many nodes the last graph_compute folded into a neighbour and did not execute (two linears in one launch both count as executed) */
 int ppml_hip_backend_nodes_fused_away(const ppml_hip_backend *b);
 /* Matrix pipe of this backend's f32 contractions for the length of each graph_compute: 0 = bf16 pipe through
  * the exact three-way split, 1 = fp32 pipe, anything else = the calling thread's ppml_hip_set_f32_arithmetic

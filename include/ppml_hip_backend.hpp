@@ -168,7 +168,8 @@ public:
     // never written.  Both are ON by default and give the same bits as the nodes run one by one:
     //   relu   -- an OP_UNARY/RELU node read only (directly or through whole OP_VIEW / OP_RESHAPE nodes) by the
     //             activation side of a quantized OP_MUL_MAT is not executed; the matmul's quantizer applies it
-    //             (src/modules/Attention.cpp:1097-1104: linear1 -> relu -> linear2 of the pair feed-forward);
+    //             (src/modules/Attention.cpp:1097-1104: linear1 -> relu -> linear2 of the pair feed-forward); a linear1 nobody
+    //             else reads, without memory of its own, then goes in linear2's launch, and its result is not written;
     //   scale  -- an OP_SCALE whose source is an OP_OUT_PROD nobody else reads runs as one scaled contraction
     //             (src/modules/Attention.cpp:264-270: the attention logits and their 1/sqrt(D)).
     void set_fuse_relu_into_q8(bool v) { fuse_relu_into_q8_ = v; }
@@ -257,6 +258,7 @@ private:
     int attn_layout_ = 0;                                // layout bits of the attention node being dispatched
     bool attn_nodes_ = false;                            // ... which stands for the default chain, with its nodes' bits
     bool relu_in_quantizer_ = false;                     // the matmul being dispatched applies a fused-away ReLU
+    bool feed_forward_ = false;                          // ... and stands for the matmul in front of that ReLU too (its weight in src[2])
     float out_prod_alpha_ = 1.0f;                        // scale of a fused-away OP_SCALE behind the out_prod being dispatched
     bool out_prod_scaled_ = false;
     bool out_prod_transposed_ = false;                   // the out_prod being dispatched reads the sources of two fused-away permutations

@@ -332,6 +332,10 @@ private:
     std::vector<Tensor*> borrowed_;
 };
 
+static int q8_wtype(const Tensor* w) {
+    return w->type == TENSOR_TYPE_Q8_1 ? PPML_WTYPE_Q8_1 : w->type == TENSOR_TYPE_Q8_0R ? PPML_WTYPE_Q8_0R : w->type == TENSOR_TYPE_Q8_0M ? PPML_WTYPE_Q8_0M : PPML_WTYPE_Q8_0;
+}
+
 static Status status_of_rc(int rc) {
     if (rc == 0) return Status::SUCCESS;
     if (rc == 3) return Status::ALLOC_FAILED;
@@ -343,6 +347,14 @@ Status HipBackend::kernel_mul_mat(Tensor* node) {
     Tensor* s0 = node->src[0];
     Tensor* s1 = node->src[1];
     if (!s0 || !s1) return fail(Status::NOT_SUPPORTED, "mul_mat: missing source");
+    if (feed_forward_) {
+        // s0 the activations, s1 the second linear's weight, src[2] the first one's
+        const Tensor* w1 = node->src[2];
+        const int rc = q8_feed_forward(w1->data, s1->data, static_cast<const float*>(s0->data), static_cast<float*>(node->data), static_cast<int>(node->dims[1]),
+                                       static_cast<int>(node->dims[0]), static_cast<int>(s1->dims[0]), q8_wtype(s1), nullptr);
+        if (rc != 0) return fail(status_of_rc(rc), std::string("mul_mat: ") + ppml_hip_last_error());
+        return Status::SUCCESS;
+    }
     if (mul_mat_transposed_) {
         // s0, s1 are the sources of the two folded transpositions: [M, K] and [N, K] in the reference's order of
         // dimensions, i.e. K rows of M and of N elements; the node is [N, M]
@@ -383,9 +395,7 @@ Status HipBackend::kernel_mul_mat(Tensor* node) {
         Tensor* a = q0 ? s1 : s0;
         if (!w->quant_shape_valid() || a->type != TENSOR_TYPE_F32 || node->type != TENSOR_TYPE_F32 || K % 32 != 0)
             return fail(Status::NOT_SUPPORTED, "mul_mat: unsupported quantized combination");
-        const int wtype = w->type == TENSOR_TYPE_Q8_1 ? PPML_WTYPE_Q8_1
-                        : w->type == TENSOR_TYPE_Q8_0R ? PPML_WTYPE_Q8_0R
-                        : w->type == TENSOR_TYPE_Q8_0M ? PPML_WTYPE_Q8_0M : PPML_WTYPE_Q8_0;
+        const int wtype = q8_wtype(w);
         // weight rows are the out features: with the weight in src0 they index the node's dims[1]
         const int64_t Mq = q0 ? M : N, Nq = q0 ? N : M;
         const int c_trans = q0 ? 0 : 1;
@@ -726,6 +736,7 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         Tensor* bridge_out = nullptr;       // ... and this trailing one, whose storage the node writes
         int relu_slot = -1;                 // quantized mul_mat: activation slot whose chain ends in a skipped ReLU
         Tensor* relu = nullptr;
+        Tensor* first = nullptr;            // ... and this quantized mul_mat in front of the ReLU goes in the same launch
         Tensor* out_prod = nullptr;         // OP_SCALE node that runs as the (skipped) out_prod it reads, scaled
         Tensor* added = nullptr;            // OP_SOFT_MAX node that adds the second operand of this (skipped) OP_ADD on its way in
         Tensor* bias_grad = nullptr;        // transposed OP_MUL_MAT that leaves this (skipped) OP_REPEAT_BACK's result beside its own
@@ -1043,6 +1054,32 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
             }
         }
         nodes_fused_away_ = skipped.size();
+
+        // (9) the linear in front of a folded ReLU (src/modules/Attention.cpp:1097-1104) in the launch of the one behind it, where
+        // nobody looks at the hidden tensor between them and its memory is nobody's.  (Both run: neither counts as folded away.)
+        if (fuse_relu_into_q8_ && !q8_1_activations_) {
+            for (Tensor* n : *graph) {
+                const auto planned = plans.find(n);
+                if (!n || planned == plans.end() || !planned->second.relu || planned->second.relu_slot != 0 || n->src[2]) continue;
+                const Tensor* reader = planned->second.relu;
+                Tensor* t = reader->src[0];
+                for (int guard = 0; guard < 16 && t && (t->op == OP_VIEW || t->op == OP_RESHAPE); ++guard) {
+                    Tensor* from = t->view_src ? t->view_src : t->src[0];
+                    if (!from || (t->flag & TENSOR_FLAG_OUTPUT) || uses[t] != 1 || t->view_offs != 0 || t->data || from->numel() != t->numel() ||
+                        !before(t, reader)) { t = nullptr; break; }
+                    reader = t;
+                    t = from;
+                }
+                if (!t || t->op != OP_MUL_MAT || !private_to(t, reader) || t->data || t->buffer || !node_supported(t) || t->src[2] || plans.count(t)) continue;
+                const Tensor *x = t->src[0], *w1 = t->src[1], *w2 = n->src[1];
+                if (!x || !w1 || !w2 || x->type != TENSOR_TYPE_F32 || !is_quantized_type(w1->type) || !is_quantized_type(w2->type)) continue;
+                const int64_t N = n->dims[1], K = n->dims[0], H = t->dims[0];
+                if (t->dims[1] != N || x->dims[0] != K || x->numel() != N * K || w1->dims[0] != K || w1->numel() != K * H || w2->dims[0] != H ||
+                    w2->numel() != K * H || n->numel() != N * K || t->numel() != N * H || !q8_feed_forward_fits(N, K, H, q8_wtype(w1), q8_wtype(w2))) continue;
+                if (!fold({t}, [&] { return stands_until(t, n, x) && stands_until(t, n, w1); })) continue;
+                planned->second.first = t;
+            }
+        }
     }
 
     // the arithmetic this backend's f32 contractions were configured with, for the length of this call
@@ -1079,6 +1116,7 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         mul_mat_transposed_ = false;
         mul_mat_rows_b_ = false;
         bias_grad_ = nullptr;
+        feed_forward_ = false;
         soft_max_bias_ = nullptr;
         const auto plan = plans.find(node);
         if (plan != plans.end()) {
@@ -1093,7 +1131,12 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 storage = pl.bridge_out;
                 attn_layout_ |= 2;
             }
-            if (pl.relu) {
+            if (pl.first) {
+                resolve_views(pl.first);                // binds its own sources if they are views
+                rewired.src[0] = pl.first->src[0];
+                rewired.src[2] = pl.first->src[1];      // (covered and checked with the other sources below)
+                feed_forward_ = true;
+            } else if (pl.relu) {
                 resolve_views(pl.relu);                 // binds the ReLU's own source if it is a view
                 Tensor* in = pl.relu->src[0];
                 if (!skip_alloc_) shadows.cover(in);
@@ -1198,6 +1241,7 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
         mul_mat_transposed_ = false;
         mul_mat_rows_b_ = false;
         bias_grad_ = nullptr;
+        feed_forward_ = false;
         soft_max_bias_ = nullptr;
         if (st != Status::SUCCESS) return st;
         const hipError_t e = hipGetLastError();

@@ -80,6 +80,9 @@ int mul_mat_tn_sums(const float* A, const float* Bm, float* O, float* sums, int 
 bool attention_chain_fits(int64_t planes, int64_t L, int64_t d);
 int attention_chain(const float* Q, const float* K, const float* V, const float* bias, float* O, int64_t planes, int L, int d, float scale,
                     hipStream_t stream);
+// Y = Q8 linear(W2, ReLU(Q8 linear(W1, X))), N tokens, K -> H -> K features, in one launch (q8.hip); wtype of either weight
+bool q8_feed_forward_fits(int64_t N, int64_t K, int64_t H, int wtype1, int wtype2);
+int q8_feed_forward(const void* W1, const void* W2, const float* X, float* Y, int N, int K, int H, int wtype, hipStream_t stream);
 void set_q8_path(int path);              // what ppml_hip_q8_last_path() reports for the calling thread
 
 typedef int   v4i  __attribute__((ext_vector_type(4)));

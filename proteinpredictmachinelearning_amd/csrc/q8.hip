@@ -336,11 +336,8 @@ __device__ __forceinline__ uint16_t load_wd(const WGeom& g, int ct, int b, int l
 }
 
 template <int WT>
-__global__ __launch_bounds__(64) void q8_weight_pack_kernel(const uint8_t* __restrict__ W,
-                                                            uint8_t* __restrict__ out, int M, int nblk,
-                                                            int mct_pad) {
-    const int frag = blockIdx.x;                       // ct * nblk + b
-    const int ct = frag / nblk, b = frag - ct * nblk;
+__device__ __forceinline__ void pack_fragment(const uint8_t* __restrict__ W, uint8_t* __restrict__ out, int M, int nblk, int mct_pad, int frag) {
+    const int ct = frag / nblk, b = frag - ct * nblk;  // frag: ct * nblk + b
     const int lane = threadIdx.x;
     const WGeom g{W, M, nblk, mct_pad};
     const bool live = ct * 32 + (lane & 31) < M;
@@ -352,6 +349,20 @@ __global__ __launch_bounds__(64) void q8_weight_pack_kernel(const uint8_t* __res
         uint16_t* dplane = reinterpret_cast<uint16_t*>(out + static_cast<int64_t>(mct_pad) * nblk * 1024);
         dplane[static_cast<int64_t>(frag) * 32 + lane] = d;
     }
+}
+template <int WT>
+__global__ __launch_bounds__(64) void q8_weight_pack_kernel(const uint8_t* __restrict__ W,
+                                                            uint8_t* __restrict__ out, int M, int nblk,
+                                                            int mct_pad) {
+    pack_fragment<WT>(W, out, M, nblk, mct_pad, static_cast<int>(blockIdx.x));
+}
+// two weights, of M1 x nblk1 and M2 x nblk2 blocks
+template <int WT>
+__global__ __launch_bounds__(64) void q8_weight_pack_pair_kernel(const uint8_t* __restrict__ Wa, uint8_t* __restrict__ out_a, int Ma, int nblk_a,
+                                                                 const uint8_t* __restrict__ Wb, uint8_t* __restrict__ out_b, int Mb, int nblk_b) {
+    const int frag = static_cast<int>(blockIdx.x), in_a = packed_tiles(Ma) * nblk_a;
+    if (frag < in_a) pack_fragment<WT>(Wa, out_a, Ma, nblk_a, packed_tiles(Ma), frag);
+    else pack_fragment<WT>(Wb, out_b, Mb, nblk_b, packed_tiles(Mb), frag - in_a);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1630,6 +1641,231 @@ int try_q8_linear_ll(const void* W, const float* X, float* C, int M, int N, int 
     return -1;
 }
 
+// ------------------------------------------------------------------------------------------
+// Two linears with a ReLU between them, K -> H -> K features (the feed-forward of the pair and alignment tracks), in one launch:
+// the hidden tensor -- four times the activations, written and read again by two kernels of 8 to 12 us each, chains of load,
+// quantize, contract and store -- stays in LDS as the quantized blocks that the second contraction reads.
+//
+// A work-group of eight waves takes 32 tokens; two of them share a CU (128 registers), at different stages.
+//   * The tokens' activations are requested at once, the first weight fragments behind them, and quantized into LDS.
+//   * Hidden tiles of 32 features are dealt to the waves.  The weight is the A operand here: a lane then holds sixteen features
+//     of ONE token, its neighbour 32 lanes on the other sixteen, and the block's maximum is fifteen maxima and one exchange; the
+//     same two halves trade places to bring the quants into the order of an operand fragment (two v_permlane32_swap).
+//   * After a barrier each wave contracts one tile of 32 output features over the hidden blocks, activations first (a lane
+//     is a feature: rows leave as whole lines).  With four such tiles or fewer a wave settles and stores sixteen of the 32 tokens:
+//     the matrix pipe repeats itself, which it has the time for, the vector pipe does not.
+// Weight fragments come from L2, a tile (or eight blocks) ahead, from packed weights or -- sixteen consecutive quants of a row as
+// they are -- from Q8_0R planes, which then need no packing launch.  Blocks ascend per output and every settlement is the same
+// fma as everywhere else: same bits.
+//
+// What bounds it: up to some 8000 tokens one work-group's chain; beyond, the vector pipe (settlements 0.5 of its time, quantization the
+// rest) and, from 256 KB of weights on, their way out of L2 for every 32 tokens.  us, two kernels / this one, packed weights: 128 -> 512
+// 1600 tokens 8.5 / 7.7, 10609 20.2 / 11.5, 25600 30.9 / 19.9; 64 -> 256, 10609 11.4 / 5.6; 192 -> 768, 361 19.3 / 11.7, 10609 36 / 18.6;
+// 256 -> 1024, 10609 39 / 26, 25600 75 / 49; 192 -> 384, 1600 8.6 / 7.9, 10609 28 / 11.2.  No size between 361 and 25600 tokens was slower.
+// ------------------------------------------------------------------------------------------
+
+// ReLU and quantization of the 32 hidden features a lane and its neighbour 32 lanes on hold of one token: registers as
+// the MFMA leaves them (mfma32_row).  The arithmetic of quantize_block_lane<false, true>.
+__device__ __forceinline__ uint16_t quantize_hidden(const float (&x)[16], v4i& frag) {
+    float top = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) top = fmaxf(top, x[r]);               // fmaxf drops NaN like std::fmax
+    const float amax = fold32(top, top, [](float a, float b) {
+        const uint32_t p = __float_as_uint(a) & 0x7fffffffu, q = __float_as_uint(b) & 0x7fffffffu;
+        return __uint_as_float(p > q ? p : q);
+    });
+    float d = div_by_127(amax), inv;
+    const bool zero = amax == 0.0f;
+    const bool fast = __builtin_amdgcn_ballot_w64(!(zero || rcp_normal_ok(d))) == 0;
+    if (__builtin_expect(fast, 1)) {
+        inv = rcp_normal(d);
+    } else {
+        d = amax / 127.0f;
+        inv = 1.0f / d;
+    }
+    if (zero) inv = 0.0f;
+    uint32_t w[4];
+    if (fast) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            unsigned q[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float u = x[4 * g + c] * inv + 0x1.fffffep-2f;
+                asm("v_cvt_u32_f32 %0, %1" : "=v"(q[c]) : "v"(u));
+            }
+            w[g] = pack4(static_cast<int>(q[0]), static_cast<int>(q[1]), static_cast<int>(q[2]), static_cast<int>(q[3]));
+        }
+    } else {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            int q[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                q[c] = round_half_away_to_int(x[4 * g + c] * inv);
+                q[c] = q[c] > 127 ? 127 : (q[c] < 0 ? 0 : q[c]);
+            }
+            w[g] = pack4(q[0], q[1], q[2], q[3]);
+        }
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+    // features 8 g + 4 hh .. + 3 -> 16 hh .. 16 hh + 15
+    const auto s02 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false), s13 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+    frag = v4i{static_cast<int>(s02[0]), static_cast<int>(s02[1]), static_cast<int>(s13[0]), static_cast<int>(s13[1])};
+#endif
+    return __half_as_ushort(__float2half_rn(d));
+}
+
+constexpr int FF_TOK = 32, FF_WAVES = 8;
+// Fragments and scales of a weight of NBLK blocks by TILES whole tiles of 32 rows: a place that is the same for the wave and an
+// offset per lane, so that a load is one instruction on a scalar base (as load_wq and load_wd give them, 4 x 16 blocks took 36 registers more)
+template <int WT, int NBLK, int TILES>
+struct FfWeight {
+    static constexpr size_t SCALES = static_cast<size_t>(WT == PPML_WTYPE_Q8_0M ? (TILES + 1) & ~1 : TILES) * NBLK * 1024;
+    const uint8_t* W;
+    uint32_t q_lane, d_lane;
+    __device__ __forceinline__ FfWeight(const uint8_t* w, int lane) : W(w) {
+        const uint32_t j = lane & 31, hh = lane >> 5;
+        q_lane = WT == PPML_WTYPE_Q8_0M ? static_cast<uint32_t>(lane) * 16u : j * (NBLK * 32u) + hh * 16u;
+        d_lane = WT == PPML_WTYPE_Q8_0M ? j * 2u : j * (NBLK * 2u);
+    }
+    __device__ __forceinline__ v4i quants(int ct, int b) const {
+        typedef int v4i_u __attribute__((ext_vector_type(4), aligned(4)));
+        return *reinterpret_cast<const v4i_u*>(W + (WT == PPML_WTYPE_Q8_0M ? (ct * NBLK + b) * 1024 : ct * (32 * NBLK * 32) + b * 32) + q_lane);
+    }
+    __device__ __forceinline__ uint16_t scale(int ct, int b) const {
+        return *reinterpret_cast<const uint16_t*>(W + SCALES + (WT == PPML_WTYPE_Q8_0M ? (ct * NBLK + b) * 64 : ct * (32 * NBLK * 2) + b * 2) + d_lane);
+    }
+};
+// NB1: blocks of K; NB2: blocks of H, i.e. hidden tiles
+template <int NB1, int NB2, int WT>
+__global__ __launch_bounds__(FF_WAVES * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void q8_feed_forward_kernel(
+    const uint8_t* __restrict__ W1, const uint8_t* __restrict__ W2, const float* __restrict__ X, float* __restrict__ Y, int N) {
+    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+    constexpr int K = NB1 * QK;
+    constexpr int NUNITS = (FF_TOK / 8) * (NB1 / 2), UPW = (NUNITS + FF_WAVES - 1) / FF_WAVES;
+    constexpr bool HALVES = 2 * NB1 <= FF_WAVES;       // two waves to a tile of output features, sixteen tokens each
+    constexpr int RV = HALVES ? 8 : 16;
+    constexpr int RING = NB2 % 8 == 0 ? 8 : 4;
+    __shared__ __attribute__((aligned(16))) v4i lds_x[NB1 * 64], lds_h[NB2 * 64];       // [block][k half][token][16 quants]
+    __shared__ __attribute__((aligned(8))) uint2 lds_dx[NB1 * 32 + 1], lds_dh[NB2 * 32 + 1];     // [block][token] {fp16 scale, 0, 0, 0}, zeros at the end
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 31, hh = lane >> 5;
+    const int tok0 = xcd_contiguous_index(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) * FF_TOK;
+    const int grp = lane >> 2, c4 = lane & 3;
+    const int urow = grp & 7, ublk = grp >> 3;
+
+    v4f xv[UPW][2];
+#pragma unroll
+    for (int s = 0; s < UPW; ++s) {
+        int u = wave + s * FF_WAVES;
+        u = u < NUNITS ? u : NUNITS - 1;               // surplus slots repeat the last unit
+        int t = tok0 + (u & 3) * 8 + urow;
+        t = t < N ? t : N - 1;                         // rows past the end repeat the last row; never stored
+        const float* src = X + static_cast<int64_t>(t) * K + ((u >> 2) * 2 + ublk) * QK + c4 * 8;
+        xv[s][0] = *reinterpret_cast<const v4f_u*>(src);
+        xv[s][1] = *reinterpret_cast<const v4f_u*>(src + 4);
+    }
+    const FfWeight<WT, NB1, NB2> w1(W1, lane);
+    const FfWeight<WT, NB2, NB1> w2(W2, lane);
+    // a weight scale as an operand: in the lower lanes only (the product is one k long)
+    const auto scale_op = [&](uint16_t d) { return __builtin_bit_cast(v4h, uint2{hh ? 0u : d, 0u}); };
+    v4i wq[NB1];
+    uint16_t wd[NB1];
+    if (wave < NB2) {
+#pragma unroll
+        for (int b = 0; b < NB1; ++b) { wq[b] = w1.quants(wave, b); wd[b] = w1.scale(wave, b); }
+    }
+#pragma unroll
+    for (int s = 0; s < UPW; ++s) {
+        const int u = wave + s * FF_WAVES;
+        if (u >= NUNITS) break;                        // wave-uniform
+        const int row = (u & 3) * 8 + urow, bl = (u >> 2) * 2 + ublk;
+        const BlockQuant bq = quantize_block_lane<false, false>(xv[s][0], xv[s][1]);
+        *(reinterpret_cast<uint2*>(lds_x) + ((bl * 64 + (c4 >> 1) * 32 + row) * 2 + (c4 & 1))) = uint2{bq.q_lo, bq.q_hi};
+        if (c4 == 0) lds_dx[bl * 32 + row] = uint2{bq.d_bits, 0u};
+    }
+    if (tid == 0) lds_dx[NB1 * 32] = lds_dh[NB2 * 32] = uint2{0u, 0u};
+    __syncthreads();
+
+    const v16i zero_i = {};
+    const v16f zero_f = {};
+    // ---- hidden tiles
+#pragma unroll 1
+    for (int ct = wave; ct < NB2; ct += FF_WAVES) {
+        float acc[16];
+#pragma unroll
+        for (int b = 0; b < NB1; ++b) {
+            if (!opaque_one()) continue;                // a basic block per step, as in q8_linear_ll_body: the matrix work of all of them would be kept alive
+            const v4i xq = lds_x[b * 64 + lane];
+            const uint2 dx = lds_dx[hh ? NB1 * 32 : b * 32 + j];
+            v16i s = __builtin_amdgcn_mfma_i32_32x32x32_i8(wq[b], xq, zero_i, 0, 0, 0);
+            v16f scl = __builtin_amdgcn_mfma_f32_32x32x8f16(scale_op(wd[b]), __builtin_bit_cast(v4h, dx), zero_f, 0, 0, 0);
+            asm volatile("" : "+v"(s), "+v"(scl));
+            __builtin_amdgcn_sched_barrier(0);
+            if ((b % 4 == 3 || b == NB1 - 1) && ct + FF_WAVES < NB2) {
+#pragma unroll
+                for (int i = b & ~3; i <= b; ++i) { wq[i] = w1.quants(ct + FF_WAVES, i); wd[i] = w1.scale(ct + FF_WAVES, i); }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[r] = __builtin_fmaf(static_cast<float>(s[r]), scl[r], b == 0 ? 0.0f : acc[r]);
+        }
+        v4i frag;
+        const uint16_t d = quantize_hidden(acc, frag);
+        lds_h[ct * 64 + lane] = frag;
+        if (hh == 0) lds_dh[ct * 32 + j] = uint2{d, 0u};
+    }
+    // ---- output tiles
+    const int ot = HALVES ? wave % NB1 : wave, part = HALVES ? wave / NB1 : 0;
+    const bool mine = HALVES ? wave < 2 * NB1 : wave < NB1;
+    v4i vq[RING];
+    uint16_t vd[RING];
+    if (mine) {
+#pragma unroll
+        for (int b = 0; b < RING; ++b) { vq[b] = w2.quants(ot, b); vd[b] = w2.scale(ot, b); }
+    }
+    __syncthreads();
+    if (!mine) return;
+    float acc[RV];
+#pragma unroll
+    for (int r = 0; r < RV; ++r) acc[r] = 0.0f;
+    const auto contract = [&](auto which) {
+        constexpr int R0 = decltype(which)::value;
+        int blocks = NB2;                               // (opaque: with two rounds the loop is taken apart otherwise, and spills)
+        asm volatile("" : "+s"(blocks));
+#pragma unroll 1
+        for (int b0 = 0; b0 < blocks; b0 += RING) {
+#pragma unroll
+            for (int i = 0; i < RING; ++i) {
+                if (!opaque_one()) continue;
+                const int b = b0 + i;
+                const v4i hq = lds_h[b * 64 + lane];
+                const uint2 dh = lds_dh[hh ? NB2 * 32 : b * 32 + j];
+                v16i s = __builtin_amdgcn_mfma_i32_32x32x32_i8(hq, vq[i], zero_i, 0, 0, 0);
+                v16f scl = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, dh), scale_op(vd[i]), zero_f, 0, 0, 0);
+                asm volatile("" : "+v"(s), "+v"(scl));
+                __builtin_amdgcn_sched_barrier(0);
+                if (i % 4 == 3 && b + RING < blocks) {
+#pragma unroll
+                    for (int c = i - 3; c <= i; ++c) { vq[c] = w2.quants(ot, b0 + c + RING); vd[c] = w2.scale(ot, b0 + c + RING); }
+                }
+#pragma unroll
+                for (int r = 0; r < RV; ++r) acc[r] = __builtin_fmaf(static_cast<float>(s[R0 + r]), scl[R0 + r], acc[r]);
+            }
+        }
+        float* const out = Y + ot * 32 + j;
+#pragma unroll
+        for (int r = 0; r < RV; ++r) {
+            const int tok = tok0 + mfma32_row(R0 + r, lane);
+            if (tok < N) __builtin_nontemporal_store(acc[r], out + static_cast<int64_t>(tok) * K);
+        }
+    };
+    if (HALVES && part == 1) contract(std::integral_constant<int, 16 - RV>{});
+    else contract(std::integral_constant<int, 0>{});
+}
+
 template <int WT>
 int dispatch_q8_linear(const void* W, const float* X, float* C, int M, int N, int nblk, int c_trans,
                        int relu, void* xq_dump, int32_t* sums_dump, hipStream_t stream) {
@@ -2128,6 +2364,53 @@ extern "C" int mul_mat_q8_ex_hip(const void* W, const float* X, float* C, int M,
         default: set_error("mul_mat_q8_hip: unsupported wtype %d", wtype); return RC_WTYPE;
     }
 }
+
+// K -> H -> K features with a ReLU between, both weights packed or both Q8_0R: q8_feed_forward_kernel's instances
+namespace ppmlhip {
+bool q8_feed_forward_fits(int64_t N, int64_t K, int64_t H, int wtype1, int wtype2) {
+    if (wtype1 != wtype2 || (wtype1 != PPML_WTYPE_Q8_0M && wtype1 != PPML_WTYPE_Q8_0R)) return false;
+    if (N < 1 || N > (1 << 24)) return false;
+    return (K == 64 || K == 128 || K == 192 || K == 256) && (H == 2 * K || H == 4 * K);
+}
+
+int q8_feed_forward(const void* W1, const void* W2, const float* X, float* Y, int N, int K, int H, int wtype, hipStream_t stream) {
+    StatsScope stat("hip/q8-feed-forward", H, K, N, stream);
+    set_q8_path(PPML_Q8_PATH_LOW_LATENCY);
+    const dim3 grid((N + FF_TOK - 1) / FF_TOK), block(FF_WAVES * 64);
+    // Q8_0R planes are read in place or packed first, both in one launch (2.5 us).  A fragment of such a weight is 32 pieces one
+    // row apart: rows of 512 bytes or 1 KB put them in the same sets of the vector cache, whose lines are fetched again then.  us, in place / packed
+    // weights, without the packing: 128 -> 512, 361 tokens 11.5 / 7.9, 10609 18.6 / 11.6; 256 -> 1024, 10609 44.6 / 26.5;
+    // 128 -> 256, 10609 9.7 / 7.6, 25600 18.2 / 12.8; 192 -> 768, 361 13.6 / 11.8, 10609 22.4 / 18.9; 192 -> 384 8.8 / 7.8, 12.2 / 11.5.
+    Workspace held;
+    if (wtype == PPML_WTYPE_Q8_0R && (H == 512 || H == 1024 || (K == 128 && N >= 14000))) {
+        const size_t bytes1 = (q8_weight_packed_bytes_hip(H, K) + 255) / 256 * 256;
+        held = workspace_take(bytes1 + q8_weight_packed_bytes_hip(K, H), stream);
+        if (held.ptr) {
+            const int frags = packed_tiles(H) * (K / QK) + packed_tiles(K) * (H / QK);
+            hipLaunchKernelGGL(q8_weight_pack_pair_kernel<PPML_WTYPE_Q8_0R>, dim3(frags), dim3(64), 0, stream, static_cast<const uint8_t*>(W1), held.ptr, H, K / QK,
+                               static_cast<const uint8_t*>(W2), held.ptr + bytes1, K, H / QK);
+            const int rc = check_launch("q8_weight_pack_pair_kernel");
+            if (rc != RC_OK) { workspace_give(held, stream); return rc; }
+            W1 = held.ptr;
+            W2 = held.ptr + bytes1;
+            wtype = PPML_WTYPE_Q8_0M;
+        }
+    }
+    const uint8_t* const w1 = static_cast<const uint8_t*>(W1);
+    const uint8_t* const w2 = static_cast<const uint8_t*>(W2);
+    int rc = RC_BAD_ARGS;
+#define PPML_FF(NB1, NB2)                                                                                              \
+    if (K == NB1 * QK && H == NB2 * QK) {                                                                              \
+        if (wtype == PPML_WTYPE_Q8_0M) hipLaunchKernelGGL((q8_feed_forward_kernel<NB1, NB2, PPML_WTYPE_Q8_0M>), grid, block, 0, stream, w1, w2, X, Y, N); \
+        else hipLaunchKernelGGL((q8_feed_forward_kernel<NB1, NB2, PPML_WTYPE_Q8_0R>), grid, block, 0, stream, w1, w2, X, Y, N); \
+        rc = check_launch("q8_feed_forward_kernel");                                                                   \
+    }
+    PPML_FF(2, 4) PPML_FF(2, 8) PPML_FF(4, 8) PPML_FF(4, 16) PPML_FF(6, 12) PPML_FF(6, 24) PPML_FF(8, 16) PPML_FF(8, 32)
+#undef PPML_FF
+    if (held.ptr) workspace_give(held, stream);
+    return rc;
+}
+}  // namespace ppmlhip
 
 // What mul_mat_q8_cuda would report in *path_out for this call (src/cuda/MulMatQ8Kernel.cu:493-496): 1 (its
 // MMQ kernels) when PPML_MMQ is not 0 and the token count reaches PPML_MMQ_MIN_N (default 16) or the weight is

@@ -728,6 +728,65 @@ def test_pair_feed_forward_graph_fused_and_node_by_node(be, oracle, layout, L):
     assert np.array_equal(results[0], results[1])
 
 
+# every instance; one token, one short of a work-group's 32, one more, a ragged many; planes read in place and packed on the way
+@pytest.mark.parametrize("layout", ["Q8_0R", "packed"])
+@pytest.mark.parametrize("D,H", [(64, 128), (64, 256), (128, 256), (128, 512), (192, 384), (192, 768), (256, 512), (256, 1024)])
+def test_feed_forward_in_one_launch_has_the_bits_of_its_nodes(be, oracle, layout, D, H):
+    """Both linears and the ReLU between them in one launch (the hidden tensor in LDS), and node by node: the same bits, with ordinary
+    values, with tokens whose hidden features are zero, subnormal, infinite or NaN, and with scales that overflow a half."""
+    import torch
+    rng = np.random.default_rng(D + H)
+    w1 = (rng.standard_normal((H, D)) * 0.05).astype(np.float32)
+    w2 = (rng.standard_normal((D, H)) * 0.05).astype(np.float32)
+    w1t, w1q = _q8_leaf(be, oracle, w1, layout)
+    w2t, w2q = _q8_leaf(be, oracle, w2, layout)
+    for tok in (1, 31, 33, 1009) + ((14001,) if (D, H) == (128, 256) else ()):
+        x = rng.standard_normal((tok, D)).astype(np.float32)
+        for t, scale in ((3, 0.0), (5, 1e-38), (7, 1e30), (11, -1.0), (30, 3e7)):
+            if t < tok:
+                x[t] = np.abs(x[t]) * np.float32(scale)
+        if tok > 20:
+            x[13, 5], x[17, 9] = np.inf, np.nan
+
+        def run(hidden_home=None):
+            xl = _leaf(be, x)
+            h = B.Tensor((H, tok), B.F32, B.OP_MUL_MAT, [xl, w1t])
+            if hidden_home is not None:
+                h.bind(hidden_home.data_ptr())
+            r = B.Tensor((H, tok), B.F32, B.OP_UNARY, [h]).set_param(0, B.UNARY_OP_RELU)
+            y = B.Tensor((D, tok), B.F32, B.OP_MUL_MAT, [r, w2t])
+            assert be.graph_compute([h, r, y]) == B.SUCCESS, be.last_error
+            return be.download(y).reshape(tok, D), h
+
+        got, h = run()
+        with pytest.raises(RuntimeError):                # the hidden tensor has no memory: the one launch is what ran
+            be.download(h)
+        be.set_fuse_relu_into_q8(False)
+        try:
+            want, h = run()
+            hidden = be.download(h).reshape(tok, H)
+        finally:
+            be.set_fuse_relu_into_q8(True)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), tok
+        if tok == 33:
+            finite = np.isfinite(x).all(axis=1)
+            ref = oracle.mul_mat_q8(w2q, oracle.relu(oracle.mul_mat_q8(w1q, x[finite], wtype=0, c_trans=1, fma=1)), wtype=0, c_trans=1, fma=1)
+            ok = np.isfinite(ref).all(axis=1)
+            assert np.array_equal(got[finite][ok].view(np.uint32), ref[ok].view(np.uint32))
+        # memory of the hidden tensor's own: it is written
+        home = torch.zeros(tok * H, device="cuda")
+        again, h = run(home)
+        assert np.array_equal(home.cpu().numpy().reshape(tok, H).view(np.uint32), hidden.view(np.uint32))
+        assert np.array_equal(again.view(np.uint32), want.view(np.uint32))
+    # the other rule for the activations has no such launch
+    be.set_q8_1_activations(True)
+    try:
+        got, h = run()
+        be.download(h)
+    finally:
+        be.set_q8_1_activations(False)
+
+
 def test_relu_is_not_folded_when_somebody_else_needs_it(be, oracle):
     D, H, L = 64, 96, 9
     rng = np.random.default_rng(77)
