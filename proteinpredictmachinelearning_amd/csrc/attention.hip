@@ -35,10 +35,20 @@ namespace {
 
 typedef float v2f __attribute__((ext_vector_type(2)));
 
-template <int DP, int NW> struct AttnTiling {
+// Loads go through buffer resources, which return zero for an offset that is outside: under conditions of the lane they were waited
+// for one after the other, and a row's end under its own.  With a stage's loads all in flight at once, and short rows of narrow heads in
+// one stage of up to 128 keys: 412 planes of 103 with bias 15.1 -> 13.4 us (8 features 13.1 -> 11.5), of 160 20.4 -> 19.6 (64 features 53.0 ->
+// 50.3), 824 of 256 81.8 -> 79.0; without bias 824 of 103 22.7 -> 21.6, of 52 11.5 in both.
+constexpr uint32_t OUTSIDE = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const float* base, int64_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, static_cast<int>(bytes), 0x00020000);
+}
+
+template <int DP, int NW, bool PF> struct AttnTiling {
     // keys staged in LDS at a time: 36 KB per four-wave work-group (four of them share a CU and its
-    // 160 KB; 128 keys would leave room for three, measured 64.7 against 61.2 us at the MSA shape)
-    static constexpr int CH = DP <= 32 ? (NW == 4 ? 96 : 128) : (NW == 4 ? 64 : 128);
+    // 160 KB; 128 keys would leave room for three, measured 64.7 against 61.2 us at the MSA shape).  The form of short
+    // rows has the registers for three anyway, and with 128 its rows are one stage.
+    static constexpr int CH = DP <= 32 ? (NW == 4 && !PF ? 96 : 128) : (NW == 4 ? 64 : 128);
     static constexpr int NC = DP / 16;                // 16-feature chunks of the score contraction
     // a 32-key tile of K in LDS: one 1 KB MFMA operand fragment per (chunk, bf16 part), [half][key][8 bf16]
     static constexpr int KT_BYTES = NC * 3 * 1024;
@@ -47,6 +57,8 @@ template <int DP, int NW> struct AttnTiling {
     static constexpr int VT_BYTES = (DP / 32) * 2 * 3 * 1024;
     static constexpr size_t lds_bytes = static_cast<size_t>(CH / 32) * (KT_BYTES + VT_BYTES);
 };
+
+constexpr int MASKED = 0, PLAIN = 1, HEAD = 2;          // kinds of tiles (see where they are told apart)
 
 struct AttnParams {
     const float* Q; const float* K; const float* V; const float* bias;
@@ -69,9 +81,9 @@ __device__ __forceinline__ float lane_xor32(float x) {
 // the instance for short sequences uses it: there a work-group is a chain of memory latencies and the
 // machine is far from full anyway.
 template <int DP, int NW, bool PF>
-// (the instance for long sequences is held to 128 registers: four waves per SIMD)
-__global__ __launch_bounds__(NW * 64, (DP <= 32 && !PF) ? 4 : 1) void flash_attn_forward_kernel(const AttnParams p) {
-    using T = AttnTiling<DP, NW>;
+// (the instance for long sequences is held to 128 registers: four waves per SIMD; the other one of narrow heads to three)
+__global__ __launch_bounds__(NW * 64, DP <= 32 ? (PF ? 3 : 4) : 1) void flash_attn_forward_kernel(const AttnParams p) {
+    using T = AttnTiling<DP, NW, PF>;
     constexpr int NC = T::NC, KT_BYTES = T::KT_BYTES, VT_BYTES = T::VT_BYTES;
     constexpr int NB = DP / 32;                       // 32-row blocks of the transposed output
     extern __shared__ __attribute__((aligned(16))) float attn_lds[];
@@ -93,31 +105,38 @@ __global__ __launch_bounds__(NW * 64, (DP <= 32 && !PF) ? 4 : 1) void flash_attn
     // ---- this lane's slice of its query row, times scale * log2(e), as the B operand of the score MFMAs:
     // chunk c holds features 16 c + 8 half .. + 7 (zero past d / past L), split into three bf16 parts
     v8bf qb[NC][3];
+    const auto load4 = [](const __amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0)); };
+    const auto load1 = [](const __amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0)); };
+    if (wave_active) {
+        // the wave's rows, or the whole plane where a row is a feature
+        const int64_t q_bytes = p.in_ld ? static_cast<int64_t>(L) * d * 4 : (L - q0 < 32 ? L - q0 : 32) * d * 4;
+        const __amdgpu_buffer_rsrc_t rq = buffer_of(p.Q + plane_off + (p.in_ld ? 0 : static_cast<int64_t>(q0) * d), q_bytes < 0x7fffffff ? q_bytes : 0x7fffffff);
+        v4f xq[NC][2];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        const int e0 = 16 * c + 8 * half;
-        v4f x0 = {0.0f, 0.0f, 0.0f, 0.0f}, x1 = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (p.in_ld) {
-            // [d][L]: one element per feature row, lanes along the queries (whole 128-byte runs)
+        for (int c = 0; c < NC; ++c) {
+            const int e0 = 16 * c + 8 * half;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (q < L && e0 + i < d) x0[i] = p.Q[plane_off + static_cast<int64_t>(e0 + i) * L + q];
-                if (q < L && e0 + 4 + i < d) x1[i] = p.Q[plane_off + static_cast<int64_t>(e0 + 4 + i) * L + q];
+            for (int h = 0; h < 2; ++h) {
+                if (p.in_ld) {
+                    // [d][L]: one element per feature row, lanes along the queries (whole 128-byte runs)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        xq[c][h][i] = load1(rq, q < L && e0 + 4 * h + i < d ? static_cast<uint32_t>((e0 + 4 * h + i) * L + q) * 4u : OUTSIDE);
+                } else {
+                    xq[c][h] = load4(rq, q < L && e0 + 4 * h < d ? static_cast<uint32_t>(j * d + e0 + 4 * h) * 4u : OUTSIDE);
+                }
             }
-        } else {
-            const float* qrow = p.Q + plane_off + static_cast<int64_t>(q) * d;
-            if (q < L && e0 < d) x0 = *reinterpret_cast<const v4f*>(qrow + e0);
-            if (q < L && e0 + 4 < d) x1 = *reinterpret_cast<const v4f*>(qrow + e0 + 4);
         }
-        x0 *= sc2;
-        x1 *= sc2;
-        uint2 lo[3], hi[3];
-        split4(x0, lo);
-        split4(x1, hi);
 #pragma unroll
-        for (int part = 0; part < 3; ++part)
-            qb[c][part] = __builtin_bit_cast(v8bf, v4i{static_cast<int>(lo[part].x), static_cast<int>(lo[part].y),
-                                                      static_cast<int>(hi[part].x), static_cast<int>(hi[part].y)});
+        for (int c = 0; c < NC; ++c) {
+            uint2 lo[3], hi[3];
+            split4(xq[c][0] * sc2, lo);
+            split4(xq[c][1] * sc2, hi);
+#pragma unroll
+            for (int part = 0; part < 3; ++part)
+                qb[c][part] = __builtin_bit_cast(v8bf, v4i{static_cast<int>(lo[part].x), static_cast<int>(lo[part].y),
+                                                          static_cast<int>(hi[part].x), static_cast<int>(hi[part].y)});
+        }
     }
 
     v16f acc_o[NB];
@@ -131,34 +150,30 @@ __global__ __launch_bounds__(NW * 64, (DP <= 32 && !PF) ? 4 : 1) void flash_attn
     const int head_keys = p.head < row_keys ? p.head : row_keys;
     // keys any query of this wave may see (wave-uniform)
     const int wave_keys = p.causal ? (q0 + 32 < L ? q0 + 32 : L) : L;
-    // lanes past the last query read the last row (never stored)
-    const float* bias_row = p.bias ? p.bias + (static_cast<int64_t>(plane) * L + (q < L ? q : L - 1)) * L : nullptr;
-
-    // Bias of this lane's 16 keys of the tile starting at key0 (zeros past L), into bias_buf.  Rows of a
-    // length that is no multiple of 4 are read with 16-byte loads all the same (4-byte aligned).
+    // Bias of this lane's 16 keys of the tile starting at key0, into bias_buf: sixteen bytes per load, four-byte aligned, without
+    // a test of the row's end -- what lies behind it is masked out with the scores (behind the rows of the wave: zero).
+    const bool has_bias = p.bias != nullptr;
+    const int bias_rows = wave_active ? (L - q0 < 32 ? L - q0 : 32) : 0;
+    const __amdgpu_buffer_rsrc_t rb = buffer_of(has_bias ? p.bias + (static_cast<int64_t>(plane) * L + (wave_active ? q0 : 0)) * L : p.Q,
+                                                has_bias ? static_cast<int64_t>(bias_rows) * L * 4 : 0);
+    const uint32_t bias_at = static_cast<uint32_t>(j * L + 4 * half) * 4u;
     float bias_buf[16];
     auto load_bias = [&](int key0) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int key = key0 + 8 * g + 4 * half;
-            if (key + 3 < L) {
-                const v4f x = *reinterpret_cast<const v4f_u*>(bias_row + key);
-                bias_buf[4 * g] = x[0]; bias_buf[4 * g + 1] = x[1]; bias_buf[4 * g + 2] = x[2]; bias_buf[4 * g + 3] = x[3];
-            } else {
+            const v4f x = load4(rb, bias_at + static_cast<uint32_t>(key0 + 8 * g) * 4u);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) bias_buf[4 * g + i] = key + i < L ? bias_row[key + i] : 0.0f;
-            }
+            for (int i = 0; i < 4; ++i) bias_buf[4 * g + i] = x[i];
         }
     };
-    if (PF && bias_row && wave_active) load_bias(0);
+    if (PF && has_bias && wave_active) load_bias(0);
 
     // One tile of 32 keys for the wave's 32 queries.  Scores live in the base-2 domain (the query slice
     // carries scale * log2(e)), so a probability is one subtraction and one v_exp_f32.
-    auto do_tile = [&](auto plain_t, int kt, int key0) {
-        constexpr bool PLAIN = decltype(plain_t)::value;
+    auto do_tile = [&](auto kind_t, int kt, int key0) {
+        constexpr int KIND = decltype(kind_t)::value;
         // ---- bias of this lane's 16 keys, requested before the matrix work (or a tile ago)
         float bv[16];
-        const bool has_bias = bias_row != nullptr;     // wave-uniform
         if (has_bias) {
             if (!PF) load_bias(key0);
 #pragma unroll
@@ -186,7 +201,7 @@ __global__ __launch_bounds__(NW * 64, (DP <= 32 && !PF) ? 4 : 1) void flash_attn
 #pragma unroll
             for (int r = 0; r < 16; ++r) st[r] = __builtin_fmaf(bv[r], LOG2E, st[r]);
         }
-        if (!PLAIN) {
+        if (KIND == MASKED) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int key = key0 + 8 * (r >> 2) + 4 * half + (r & 3);
@@ -196,6 +211,7 @@ __global__ __launch_bounds__(NW * 64, (DP <= 32 && !PF) ? 4 : 1) void flash_attn
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) m_tile = fmaxf(m_tile, st[r]);
+        if (KIND == HEAD) m_head = fmaxf(m_head, m_tile);
         m_tile = fmaxf(m_tile, lane_xor32(m_tile));
         const float m_new = fmaxf(m_run, m_tile);
         const float alpha = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
@@ -241,7 +257,24 @@ __global__ __launch_bounds__(NW * 64, (DP <= 32 && !PF) ? 4 : 1) void flash_attn
         }
     };
 
+    // A stage of K and V, [L][d]: every load of it is in flight before the first value is used
+    constexpr int NI = (T::CH * (DP / 4) + NW * 64 - 1) / (NW * 64);
     const int stage = p.stage_rows;
+    const auto request = [&](int c0, v4f (&kx)[NI], v4f (&vx)[NI]) {
+        const int ckeys = L - c0 < stage ? L - c0 : stage;
+        const int64_t from = plane_off + static_cast<int64_t>(c0) * d;
+        const __amdgpu_buffer_rsrc_t rk = buffer_of(p.K + from, ckeys * d * 4), rv = buffer_of(p.V + from, ckeys * d * 4);
+        const int pieces = (ckeys + 31) / 32 * 32 * (DP / 4);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            if ((PF || DP > 32) && i * NW * 64 >= pieces) break;      // (the same for the work-group)
+            const int idx = tid + i * NW * 64;
+            const int key = idx / (DP / 4), c = (idx % (DP / 4)) * 4;
+            const uint32_t at = key < ckeys && c < d ? static_cast<uint32_t>(key * d + c) * 4u : OUTSIDE;
+            kx[i] = load4(rk, at);
+            vx[i] = load4(rv, at);
+        }
+    };
     for (int c0 = 0; c0 < L; c0 += stage) {
         // ---- stage keys c0 .. c0+stage-1 of K and V (zeros past L and past d; whole tiles of 32 only)
         __syncthreads();
@@ -292,22 +325,22 @@ __global__ __launch_bounds__(NW * 64, (DP <= 32 && !PF) ? 4 : 1) void flash_attn
                 }
             }
         } else {
-            for (int idx = tid; idx < rows * (DP / 4); idx += NW * 64) {
+            v4f kx[NI], vx[NI];
+            request(c0, kx, vx);
+#pragma unroll
+            for (int it = 0; it < NI; ++it) {
+                if (it * NW * 64 >= rows * (DP / 4)) break;
+                const int idx = tid + it * NW * 64;
                 const int key = idx / (DP / 4), c = (idx % (DP / 4)) * 4;
-                v4f kx = {0.0f, 0.0f, 0.0f, 0.0f}, vx = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (key < ckeys && c < d) {
-                    const int64_t off = plane_off + static_cast<int64_t>(c0 + key) * d + c;
-                    kx = *reinterpret_cast<const v4f*>(p.K + off);
-                    vx = *reinterpret_cast<const v4f*>(p.V + off);
-                }
+                if (key >= rows) break;
                 // features c .. c+3 of one key: eight bytes of each part's fragment
                 uint2 parts[3];
-                split4(kx, parts);
+                split4(kx[it], parts);
                 uint8_t* dst = lds_k + (key >> 5) * KT_BYTES + (c >> 4) * 3072 + ((c >> 3) & 1) * 512 + (key & 31) * 16 + ((c >> 2) & 1) * 8;
 #pragma unroll
                 for (int part = 0; part < 3; ++part) *reinterpret_cast<uint2*>(dst + part * 1024) = parts[part];
                 // V: features c .. c+3 of one key go to four lane slots of the fragments of V^T, two bytes each
-                split4(vx, parts);
+                split4(vx[it], parts);
                 {
                     const int kc = key & 15;
                     const int slot = 4 * (kc >> 3) + (kc & 3);
@@ -331,11 +364,14 @@ __global__ __launch_bounds__(NW * 64, (DP <= 32 && !PF) ? 4 : 1) void flash_attn
             const int key0 = c0 + kt * 32;             // first key of the tile
             if (key0 >= wave_keys) break;              // causal: nothing left for any query of the wave
             // A tile is plain when every query of the wave sees all 32 keys and the tile lies behind the
-            // reference's first block; plain tiles skip the masks and the first-block bookkeeping.
-            const bool plain = key0 + 32 <= L && (!p.causal || key0 + 32 <= q0 + 1) && key0 >= p.head;
-            if (plain) do_tile(std::true_type{}, kt, key0);
-            else do_tile(std::false_type{}, kt, key0);
+            // reference's first block, or inside it: such tiles skip the masks, and behind it the first-block bookkeeping too.
+            // (the form of long rows of narrow heads has no room for a third kind in its 128 registers, and one tile in many in that block)
+            const bool seen = key0 + 32 <= L && (!p.causal || key0 + 32 <= q0 + 1);
+            if (seen && key0 >= p.head) do_tile(std::integral_constant<int, PLAIN>{}, kt, key0);
+            else if ((DP > 32 || PF) && seen && key0 + 32 <= p.head) do_tile(std::integral_constant<int, HEAD>{}, kt, key0);
+            else do_tile(std::integral_constant<int, MASKED>{}, kt, key0);
         }
+        if (PF && T::CH >= 128) break;                  // (that instance's rows are one stage)
     }
     if (!wave_active || q >= L) return;
 
@@ -372,10 +408,10 @@ __global__ __launch_bounds__(NW * 64, (DP <= 32 && !PF) ? 4 : 1) void flash_attn
 
 template <int DP, int NW, bool PF>
 int launch_flash(AttnParams p, hipStream_t stream) {
-    using T = AttnTiling<DP, NW>;
+    using T = AttnTiling<DP, NW, PF>;
     auto kernel = &flash_attn_forward_kernel<DP, NW, PF>;
     const int l32 = (p.L + 31) / 32 * 32;
-    // stages of even size: 103 keys go 64 + 64, not 96 + 32 (412 planes with bias 16.1 -> 15.7 us)
+    // stages of even size: eight waves take 160 keys as 96 + 64, not 128 + 32
     const int stages = (l32 + T::CH - 1) / T::CH;
     p.stage_rows = (l32 / 32 + stages - 1) / stages * 32;
     const size_t lds = static_cast<size_t>(p.stage_rows / 32) * (T::KT_BYTES + T::VT_BYTES);

@@ -397,3 +397,29 @@ def test_backward_reference_golden_vectors(ops):
         ops.synchronize()
         for g, key, shp in zip(got, ("dq", "dk", "dv", "dbias"), (shape, shape, shape, sq)):
             _check_grad(g.cpu().numpy(), f32(c[key], shp), key)
+
+
+# rows that end inside a tile of 32 keys, on one, and one past it; one work-group per plane and several, four waves and eight; every instance
+@pytest.mark.parametrize("L", [3, 33, 50, 64, 103, 131, 161, 257])
+@pytest.mark.parametrize("d", [4, 32, 48])
+@pytest.mark.parametrize("causal", [False, True])
+def test_forward_keeps_to_its_own_rows(ops, L, d, causal):
+    """Bias is read in pieces of sixteen bytes without a test of the row's end: what the next row, or the next plane, begins with must
+    not reach a row's result.  A row of NaN, and a plane of infinities, leave every other row the bits it has without them."""
+    torch.manual_seed(L * d)
+    planes = 3
+    for in_ld in (False, True):
+        shape = (1, planes, d, L) if in_ld else (1, planes, L, d)
+        q, k, v = (torch.randn(shape, device="cuda") for _ in range(3))
+        bias = torch.randn(1, planes, L, L, device="cuda")
+        clean, lse = ops.flash_attn_forward(q, k, v, bias, causal=causal, in_ld=in_ld)
+        bad = bias.clone()
+        r = L // 2
+        bad[0, 0, r] = float("nan")
+        bad[0, 2] = float("-inf")
+        out, lse2 = ops.flash_attn_forward(q, k, v, bad, causal=causal, in_ld=in_ld)
+        keep = torch.ones(planes, L, dtype=torch.bool, device="cuda")
+        keep[0, r] = False
+        keep[2] = False
+        assert torch.equal(out[0][keep].view(torch.int32), clean[0][keep].view(torch.int32))
+        assert torch.equal(lse2[0][keep].view(torch.int32), lse[0][keep].view(torch.int32))
