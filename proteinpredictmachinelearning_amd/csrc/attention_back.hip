@@ -44,114 +44,119 @@ struct AttnBackParams {
 
 __device__ __forceinline__ float lane_xor32(float x) { return __shfl_xor(x, 32, 64); }
 
+// Loads through a buffer resource return zero for an offset that is outside; under conditions of the lane they were waited for one after
+// the other.
+constexpr uint32_t OUTSIDE = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const float* base, int64_t elements) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, elements * 4 < 0x7fffffff ? static_cast<int>(elements * 4) : 0x7fffffff, 0x00020000);
+}
+__device__ __forceinline__ v4f buffer_load4(const __amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0)); }
+__device__ __forceinline__ float buffer_load1(const __amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0)); }
+
 template <int DP> struct BackTiling {
     static constexpr int NC = DP / 16;                // 16-feature chunks of a contraction over the features
     static constexpr int NB = DP / 32;                // 32-feature blocks of a transposed gradient
-    // A 32-row tile of a streamed matrix in LDS, as 1 KB MFMA operand fragments (lane l reads bytes 16 l ..):
-    //   "row" fragments, one per (chunk, part): lane (row, half) holds features 16 c + 8 half .. + 7 of its row;
-    //   "column" fragments of the transpose, one per (feature block, 16-row chunk, part): slot i of lane
-    //   (feature, half) holds row 16 ch + 8 (i / 4) + 4 half + i % 4 -- the order in which the accumulator
-    //   registers 8 ch .. 8 ch + 7 of a 32 x 32 product hold the rows.
-    static constexpr int ROW_BYTES = NC * 3 * 1024;
-    static constexpr int COL_BYTES = NB * 2 * 3 * 1024;
-    static constexpr int CH_ROWS = 64;                // rows staged at a time by the rows kernel (K both ways, V by rows)
-    static constexpr int CH_COLS = 96;                // ... by the columns kernel (Q and dO both ways)
+    // A 32-row tile of a streamed matrix in LDS, as MFMA operand fragments, one per (chunk, part): features 8 half .. + 7 of
+    // the chunk, sixteen bytes per row, the two halves 576 bytes apart (the transposing reads and the staging writes then touch every bank
+    // once).  The same fragments serve the contraction over the tile's rows: ds_read_b64_tr_b16 hands them out transposed
+    // (read_transposed), in the order in which the accumulator registers 8 ch .. 8 ch + 7 of a 32 x 32 product hold the rows.
+    static constexpr int HALF = 576, FRAG = 2 * HALF, CHUNK = 3 * FRAG;
+    static constexpr int TILE = NC * CHUNK;
+    static constexpr int CH_ROWS = 64;                // rows staged at a time by the rows kernel
+    static constexpr int CH_COLS = DP <= 32 ? 96 : 32;     // ... by the columns kernel: two work-groups' share a CU's 160 KB
 };
+
+// eight 16-bit elements of this lane's column, four rows at `at` and four at `at + step`, each piece transposed on the
+// way (a group of sixteen lanes names four rows of sixteen columns, four columns per lane)
+typedef short v4s __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ v8bf read_transposed(const uint8_t* at, int step) {
+    typedef __attribute__((address_space(3))) v4s* lds_v4s;
+    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at));
+    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at + step));
+    return __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+// this lane's place in a tile: its row's half chunk, and what it names of the transposed reads of 32 features
+template <int DP> __device__ __forceinline__ int row_place(int lane) { return (lane & 31) * 16 + (lane >> 5) * BackTiling<DP>::HALF; }
+template <int DP> __device__ __forceinline__ int column_place(int lane) {
+    using T = BackTiling<DP>;
+    const int grp = lane & 15;
+    return ((lane >> 4) & 1) * T::CHUNK + ((grp >> 1) & 1) * T::HALF + (4 * (lane >> 5) + (grp >> 2)) * 16 + (grp & 1) * 8;
+}
 
 __device__ __forceinline__ v8bf pack_parts(const uint2& lo, const uint2& hi) {
     return __builtin_bit_cast(v8bf, v4i{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(hi.x), static_cast<int>(hi.y)});
 }
 
-// This lane's slice of row `row` of a [L][d] matrix times `factor`, as the B operand of a contraction over the
-// features: chunk c holds features 16 c + 8 half .. + 7 (zero past d and past L), split into three bf16 parts.
+// This lane's slice of row `first` + j of a [L][d] matrix, as the B operand of a contraction over the features: chunk c holds features
+// 16 c + 8 half .. + 7 (zero past d and past L).  `first` is the same for the wave and below L.
 template <int DP>
-__device__ __forceinline__ void load_slice_parts(const float* base, int row, int L, int d, int half, float factor,
-                                                 v8bf (&out)[DP / 16][3]) {
+__device__ __forceinline__ void load_slice(const float* base, int first, int j, int L, int d, int half, v4f (&x)[DP / 16][2]) {
+    const int rows = L - first < 32 ? L - first : 32;
+    const __amdgpu_buffer_rsrc_t r = buffer_of(base + static_cast<int64_t>(first) * d, rows * d);
+#pragma unroll
+    for (int c = 0; c < DP / 16; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int e = 16 * c + 8 * half + 4 * h;
+            x[c][h] = buffer_load4(r, j < rows && e < d ? static_cast<uint32_t>(j * d + e) * 4u : OUTSIDE);
+        }
+}
+
+// ... times `factor`, split into three bf16 parts
+template <int DP>
+__device__ __forceinline__ void slice_parts(const v4f (&x)[DP / 16][2], float factor, v8bf (&out)[DP / 16][3]) {
 #pragma unroll
     for (int c = 0; c < DP / 16; ++c) {
-        const int e0 = 16 * c + 8 * half;
-        v4f x0 = {0.0f, 0.0f, 0.0f, 0.0f}, x1 = {0.0f, 0.0f, 0.0f, 0.0f};
-        const float* src = base + static_cast<int64_t>(row) * d;
-        if (row < L && e0 < d) x0 = *reinterpret_cast<const v4f*>(src + e0);
-        if (row < L && e0 + 4 < d) x1 = *reinterpret_cast<const v4f*>(src + e0 + 4);
-        x0 *= factor;
-        x1 *= factor;
         uint2 lo[3], hi[3];
-        split4(x0, lo);
-        split4(x1, hi);
+        split4(x[c][0] * factor, lo);
+        split4(x[c][1] * factor, hi);
 #pragma unroll
         for (int part = 0; part < 3; ++part) out[c][part] = pack_parts(lo[part], hi[part]);
     }
 }
 
-// Writes features c .. c+3 of row `row` of a staged matrix into its fragments: row fragments at lds_row and / or
-// column fragments at lds_col (null = not wanted).
+// Writes features c .. c+3 of row `row` of a staged matrix into its tiles: eight bytes of each part's fragment.
 template <int DP>
-__device__ __forceinline__ void put_fragments(const v4f& x, int row, int c, uint8_t* lds_row, uint8_t* lds_col) {
+__device__ __forceinline__ void put_fragments(const v4f& x, int row, int c, uint8_t* tiles) {
     using T = BackTiling<DP>;
     uint2 parts[3];
     split4(x, parts);
-    if (lds_row) {
-        // eight bytes of each part's fragment
-        uint8_t* dst = lds_row + (row >> 5) * T::ROW_BYTES + (c >> 4) * 3072 + ((c >> 3) & 1) * 512 + (row & 31) * 16 + ((c >> 2) & 1) * 8;
+    uint8_t* dst = tiles + (row >> 5) * T::TILE + (c >> 4) * T::CHUNK + ((c >> 3) & 1) * T::HALF + (row & 31) * 16 + ((c >> 2) & 1) * 8;
 #pragma unroll
-        for (int part = 0; part < 3; ++part) *reinterpret_cast<uint2*>(dst + part * 1024) = parts[part];
-    }
-    if (lds_col) {
-        // the same four features go to four lane slots of the transposed fragments, two bytes each
-        const int kc = row & 15;
-        const int slot = 4 * (kc >> 3) + (kc & 3);
-        uint8_t* dst = lds_col + (row >> 5) * T::COL_BYTES + (((c >> 5) * 2 + ((row >> 4) & 1)) * 3) * 1024 +
-                       (((kc >> 2) & 1) * 32 + (c & 31)) * 16 + slot * 2;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int part = 0; part < 3; ++part) {
-                const uint32_t w = (i < 2 ? parts[part].x : parts[part].y) >> (16 * (i & 1));
-                *reinterpret_cast<uint16_t*>(dst + part * 1024 + i * 16) = static_cast<uint16_t>(w);
-            }
-    }
+    for (int part = 0; part < 3; ++part) *reinterpret_cast<uint2*>(dst + part * T::FRAG) = parts[part];
 }
 
 // Stages rows r0 .. r0+rows-1 (at most MAXROWS) of two [L][d] matrices into LDS as fragments (zeros past `valid`
-// rows and past d); SCALED: the first one's row fragments times a_factor.  Every load of the stage is issued before the first value is used: a work-group waits for
+// rows and past d); SCALED: the first one times a_factor at `a_lds`, and as it is at `a_plain`.  Every load of the stage is issued before the first value is used: a work-group waits for
 // one memory round trip per stage, not one per loop iteration.
 template <int DP, int NT, int MAXROWS, bool SCALED>
-__device__ __forceinline__ void stage_two(const float* a, uint8_t* a_row, uint8_t* a_col, float a_factor,
-                                          const float* b, uint8_t* b_row, uint8_t* b_col,
+__device__ __forceinline__ void stage_two(const float* a, uint8_t* a_lds, uint8_t* a_plain, float a_factor, const float* b, uint8_t* b_lds,
                                           int r0, int rows, int valid, int d, int tid) {
     constexpr int NI = (MAXROWS * (DP / 4) + NT - 1) / NT;
+    const __amdgpu_buffer_rsrc_t ra = buffer_of(a + static_cast<int64_t>(r0) * d, valid * d), rb = buffer_of(b + static_cast<int64_t>(r0) * d, valid * d);
     v4f xa[NI], xb[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int idx = tid + i * NT;
         const int row = idx / (DP / 4), c = (idx % (DP / 4)) * 4;
-        xa[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        xb[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        if (row < valid && c < d) {
-            const int64_t off = static_cast<int64_t>(r0 + row) * d + c;
-            xa[i] = *reinterpret_cast<const v4f*>(a + off);
-            xb[i] = *reinterpret_cast<const v4f*>(b + off);
-        }
+        const uint32_t at = row < valid && c < d ? static_cast<uint32_t>(row * d + c) * 4u : OUTSIDE;
+        xa[i] = buffer_load4(ra, at);
+        xb[i] = buffer_load4(rb, at);
     }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int idx = tid + i * NT;
         const int row = idx / (DP / 4), c = (idx % (DP / 4)) * 4;
         if (row < rows) {
-            if (SCALED) {
-                put_fragments<DP>(xa[i] * a_factor, row, c, a_row, nullptr);
-                put_fragments<DP>(xa[i], row, c, nullptr, a_col);
-            } else {
-                put_fragments<DP>(xa[i], row, c, a_row, a_col);
-            }
-            put_fragments<DP>(xb[i], row, c, b_row, b_col);
+            put_fragments<DP>(SCALED ? xa[i] * a_factor : xa[i], row, c, a_lds);
+            if (SCALED) put_fragments<DP>(xa[i], row, c, a_plain);
+            put_fragments<DP>(xb[i], row, c, b_lds);
         }
     }
 }
 
-// acc(32 x 32) = tile(32 rows x DP, row fragments in LDS, rows = accumulator rows) . slice^T (this lane's column);
-// `frags` points at this lane's 16 bytes of the tile's first fragment.  SWAP: the partial products in the order of the
+// acc(32 x 32) = tile(32 rows x DP in LDS, rows = accumulator rows) . slice^T (this lane's column);
+// `frags` points at this lane's place in the tile (row_place).  SWAP: the partial products in the order of the
 // transposed product (the bits of slice . tile^T)
 template <int DP, bool SWAP = false>
 __device__ __forceinline__ v16f tile_times_slice(const uint8_t* frags, const v8bf (&slice)[DP / 16][3]) {
@@ -160,7 +165,7 @@ __device__ __forceinline__ v16f tile_times_slice(const uint8_t* frags, const v8b
     for (int c = 0; c < DP / 16; ++c) {
         v8bf a[3];
 #pragma unroll
-        for (int part = 0; part < 3; ++part) a[part] = *reinterpret_cast<const v8bf*>(frags + (c * 3 + part) * 1024);
+        for (int part = 0; part < 3; ++part) a[part] = *reinterpret_cast<const v8bf*>(frags + c * BackTiling<DP>::CHUNK + part * BackTiling<DP>::FRAG);
 #pragma unroll
         for (int t = 0; t < 6; ++t) {
             // the first product starts from the constant zero: no registers to clear
@@ -172,7 +177,7 @@ __device__ __forceinline__ v16f tile_times_slice(const uint8_t* frags, const v8b
 }
 
 // out^T(DP features x 32 columns) += tile^T . w, contracting the 32 rows of the tile in the order in which the
-// accumulator registers of `w` hold them; `frags` points at this lane's 16 bytes of the tile's first column fragment.
+// accumulator registers of `w` hold them; `frags` points at this lane's place in the tile (column_place).
 // FROM_ZERO: without what `out` held (the constant zero as the first product's addend: no registers to clear).
 template <int DP, bool FROM_ZERO = false>
 __device__ __forceinline__ void accumulate_transposed(v16f (&out)[DP / 32], const uint8_t* frags, const v16f& w) {
@@ -188,7 +193,7 @@ __device__ __forceinline__ void accumulate_transposed(v16f (&out)[DP / 32], cons
         for (int b = 0; b < DP / 32; ++b) {
             v8bf a[3];
 #pragma unroll
-            for (int part = 0; part < 3; ++part) a[part] = *reinterpret_cast<const v8bf*>(frags + ((b * 2 + ch) * 3 + part) * 1024);
+            for (int part = 0; part < 3; ++part) a[part] = read_transposed(frags + b * 2 * BackTiling<DP>::CHUNK + part * BackTiling<DP>::FRAG + ch * 256, 128);
 #pragma unroll
             for (int t = 0; t < 6; ++t)
                 out[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[SPLIT_TERMS[t][0]], wb[SPLIT_TERMS[t][1]], FROM_ZERO && ch == 0 && t == 0 ? v16f{} : out[b], 0, 0, 0);
@@ -214,31 +219,36 @@ __global__ __launch_bounds__(NW * 64, !TWIN ? 1 : BIAS && LATE ? 2 : 3) void fla
     static_assert(TWIN ? (NB == 1 && NC == 2) : !LATE, "the one-pass kernel's features");
     extern __shared__ __attribute__((aligned(16))) uint8_t back_lds[];
     const int tiles_staged = p.stage_rows / 32;
-    uint8_t* lds_k_row = back_lds;                                  // K by rows: S^T = K . Q^T
-    uint8_t* lds_k_col = lds_k_row + tiles_staged * T::ROW_BYTES;   // K^T: dQ^T += K^T . dS
-    uint8_t* lds_v_row = lds_k_col + tiles_staged * T::COL_BYTES;   // V by rows: (dO V^T)^T = V . dO^T
+    uint8_t* const lds_v = back_lds;                                // V: (dO V^T)^T = V . dO^T
+    uint8_t* const lds_k = lds_v + tiles_staged * T::TILE;          // K: S^T = K . Q^T and, transposed,
+    uint8_t* const lds_kt = TWIN ? lds_k + tiles_staged * T::TILE : lds_k;      // dQ^T += K^T . dS (without the scale)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 31, half = lane >> 5;
+    const int row_at = row_place<DP>(lane), col_at = column_place<DP>(lane);
     const int plane = blockIdx.y, L = p.L, d = p.d;
     const int q0 = (blockIdx.x * NW + wave) * 32, q = q0 + j;
     const bool wave_active = q0 < L;
     const int64_t po = static_cast<int64_t>(plane) * L * d;
 
     v8bf qb[NC][3], dob[NC][3];
-    load_slice_parts<DP>(p.Q + po, q, L, d, half, TWIN ? 1.0f : p.scale * LOG2E, qb);
-    load_slice_parts<DP>(p.dO + po, q, L, d, half, 1.0f, dob);
     // D_i = sum_d dO_id * O_id: this lane's half of the features, then the other half from lane j + 32
-    float D_i = 0.0f, D_c[NC] = {};
-    if (q < L) {
+    float D_i = 0.0f, D_c[NC] = {}, lse = -INFINITY;
+    if (wave_active) {
+        v4f xq[NC][2], xdo[NC][2], xo[NC][2];
+        load_slice<DP>(p.Q + po, q0, j, L, d, half, xq);
+        load_slice<DP>(p.dO + po, q0, j, L, d, half, xdo);
+        load_slice<DP>(p.O + po, q0, j, L, d, half, xo);
+        if (q < L) lse = p.LSE[static_cast<int64_t>(plane) * L + q];
+        slice_parts<DP>(xq, TWIN ? 1.0f : p.scale * LOG2E, qb);
+        slice_parts<DP>(xdo, 1.0f, dob);
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
-            for (int e = 16 * c + 8 * half; e < 16 * c + 8 * half + 8; e += 4) {
-                if (e >= d) continue;
-                const v4f a = *reinterpret_cast<const v4f*>(p.dO + po + static_cast<int64_t>(q) * d + e);
-                const v4f o = *reinterpret_cast<const v4f*>(p.O + po + static_cast<int64_t>(q) * d + e);
+            for (int h = 0; h < 2; ++h) {
+                const v4f a = xdo[c][h], o = xo[c][h];
                 const float quad = a[0] * o[0] + a[1] * o[1] + a[2] * o[2] + a[3] * o[3];
+                if (16 * c + 8 * half + 4 * h >= d) continue;
                 D_i += quad;
                 D_c[c] += quad;
             }
@@ -249,12 +259,15 @@ __global__ __launch_bounds__(NW * 64, !TWIN ? 1 : BIAS && LATE ? 2 : 3) void fla
     } else {
         D_i += lane_xor32(D_i);
     }
-    const float lse = q < L ? p.LSE[static_cast<int64_t>(plane) * L + q] : -INFINITY;
     // a row without any visible key (LSE = -inf) has no gradient: +inf makes every probability exp2(-inf) = 0
     const float lse2 = lse > -INFINITY ? lse * LOG2E : INFINITY;
     const int row_keys = p.causal ? (q + 1 < L ? q + 1 : L) : L;
     const int wave_keys = p.causal ? (q0 + 32 < L ? q0 + 32 : L) : L;
-    const float* bias_row = BIAS && p.bias ? p.bias + (static_cast<int64_t>(plane) * L + (q < L ? q : L - 1)) * L : nullptr;
+    const bool has_bias = BIAS && p.bias;
+    const int wave_rows = !wave_active ? 0 : L - q0 < 32 ? L - q0 : 32;
+    const __amdgpu_buffer_rsrc_t rbias = buffer_of(has_bias && wave_active ? p.bias + (static_cast<int64_t>(plane) * L + q0) * L : p.Q,
+                                                   has_bias ? static_cast<int64_t>(wave_rows) * L : 0);
+    const uint32_t bias_at = static_cast<uint32_t>(j * L + 4 * half) * 4u;
     float* dbias_row = p.dbias ? p.dbias + (static_cast<int64_t>(plane) * L + (q < L ? q : L - 1)) * L : nullptr;
 
     v16f acc_q[NB];
@@ -280,20 +293,16 @@ __global__ __launch_bounds__(NW * 64, !TWIN ? 1 : BIAS && LATE ? 2 : 3) void fla
             }
     };
 
-    // Bias of this lane's 16 keys of the tile that starts at key0 (zeros past L), 16 bytes at a time.
+    // Bias of this lane's 16 keys of the tile that starts at key0, 16 bytes at a time (what lies behind a row's end is masked with
+    // the probabilities).
     float bv[16];
     const auto load_bias = [&](int key0) {
-        if (!BIAS || !bias_row) return;
+        if (!BIAS || !has_bias) return;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int key = key0 + 8 * g + 4 * half;
-            if (key + 3 < L) {
-                const v4f x = *reinterpret_cast<const v4f_u*>(bias_row + key);
-                bv[4 * g] = x[0]; bv[4 * g + 1] = x[1]; bv[4 * g + 2] = x[2]; bv[4 * g + 3] = x[3];
-            } else {
+            const v4f x = buffer_load4(rbias, bias_at + static_cast<uint32_t>(key0 + 8 * g) * 4u);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) bv[4 * g + i] = key + i < L ? bias_row[key + i] : 0.0f;
-            }
+            for (int i = 0; i < 4; ++i) bv[4 * g + i] = x[i];
         }
     };
     if (wave_active) load_bias(0);
@@ -303,20 +312,20 @@ __global__ __launch_bounds__(NW * 64, !TWIN ? 1 : BIAS && LATE ? 2 : 3) void fla
         __syncthreads();
         const int ckeys = L - c0 < stage ? L - c0 : stage;
         const int rows = (ckeys + 31) / 32 * 32;
-        stage_two<DP, NW * 64, T::CH_ROWS, TWIN>(p.K + po, lds_k_row, lds_k_col, p.scale * LOG2E, p.V + po, lds_v_row, nullptr, c0, rows, ckeys, d, tid);
+        stage_two<DP, NW * 64, T::CH_ROWS, TWIN>(p.K + po, lds_k, lds_kt, p.scale * LOG2E, p.V + po, lds_v, c0, rows, ckeys, d, tid);
         __syncthreads();
         if (!wave_active) continue;
         for (int kt = 0; kt < rows / 32; ++kt) {
             const int key0 = c0 + kt * 32;
             // ---- probabilities of this lane's query for its 16 keys of the tile (their bias was requested a
             // tile ago, see below)
-            v16f st = tile_times_slice<DP, TWIN>(lds_k_row + kt * T::ROW_BYTES + lane * 16, qb);
-            v16f dp = tile_times_slice<DP, TWIN>(lds_v_row + kt * T::ROW_BYTES + lane * 16, dob);
+            v16f st = tile_times_slice<DP, TWIN>(lds_k + kt * T::TILE + row_at, qb);
+            v16f dp = tile_times_slice<DP, TWIN>(lds_v + kt * T::TILE + row_at, dob);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int key = key0 + 8 * (r >> 2) + 4 * half + (r & 3);
                 float s2 = st[r];
-                if (BIAS && bias_row) s2 = __builtin_fmaf(bv[r], LOG2E, s2);
+                if (BIAS && has_bias) s2 = __builtin_fmaf(bv[r], LOG2E, s2);
                 // dS (chosen behind the product: 0 * NaN is not 0)
                 st[r] = key < row_keys ? __builtin_amdgcn_exp2f(s2 - lse2) * (dp[r] - D_i) : 0.0f;
             }
@@ -347,11 +356,11 @@ __global__ __launch_bounds__(NW * 64, !TWIN ? 1 : BIAS && LATE ? 2 : 3) void fla
                 }
                 v16f share[NB];
                 if (LATE) acc_q[0] += late;
-                accumulate_transposed<DP, true>(share, lds_k_col + kt * T::COL_BYTES + lane * 16, st);
+                accumulate_transposed<DP, true>(share, lds_kt + kt * T::TILE + col_at, st);
                 if (LATE) late = share[0];
                 else acc_q[0] += share[0];
             } else {
-                accumulate_transposed<DP>(acc_q, lds_k_col + kt * T::COL_BYTES + lane * 16, st);
+                accumulate_transposed<DP>(acc_q, lds_kt + kt * T::TILE + col_at, st);
             }
         }
     }
@@ -363,28 +372,32 @@ __global__ __launch_bounds__(NW * 64, !TWIN ? 1 : BIAS && LATE ? 2 : 3) void fla
 // ------------------------------------------------------------------------------------------------------------
 // dK and dV: a wave owns 32 keys and walks over the queries.
 template <int DP, int NW>
-__global__ __launch_bounds__(NW * 64) void flash_attn_back_cols_kernel(const AttnBackParams p) {
+__global__ __launch_bounds__(NW * 64, 2) void flash_attn_back_cols_kernel(const AttnBackParams p) {
     using T = BackTiling<DP>;
     constexpr int NB = T::NB, NC = T::NC;
     extern __shared__ __attribute__((aligned(16))) uint8_t back_lds[];
     const int tiles_staged = p.stage_rows / 32;
-    uint8_t* lds_q_row = back_lds;                                   // Q by rows: S = Q . K^T
-    uint8_t* lds_q_col = lds_q_row + tiles_staged * T::ROW_BYTES;    // Q^T: dK^T += Q^T . dS
-    uint8_t* lds_do_row = lds_q_col + tiles_staged * T::COL_BYTES;   // dO by rows: dO . V^T
-    uint8_t* lds_do_col = lds_do_row + tiles_staged * T::ROW_BYTES;  // dO^T: dV^T += dO^T . P
-    float* lds_lse = reinterpret_cast<float*>(lds_do_col + tiles_staged * T::COL_BYTES);   // LSE * log2(e) of the staged queries (+inf for dead rows)
+    uint8_t* const lds_q = back_lds;                                 // Q: S = Q . K^T and, transposed, dK^T += Q^T . dS
+    uint8_t* const lds_do = lds_q + tiles_staged * T::TILE;          // dO: dO . V^T and, transposed, dV^T += dO^T . P
+    float* lds_lse = reinterpret_cast<float*>(lds_do + tiles_staged * T::TILE);       // LSE * log2(e) of the staged queries (+inf for dead rows)
     float* lds_D = lds_lse + p.stage_rows;             // D of the staged queries
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 31, half = lane >> 5;
+    const int row_at = row_place<DP>(lane), col_at = column_place<DP>(lane);
     const int plane = blockIdx.y, L = p.L, d = p.d;
     const int k0w = (blockIdx.x * NW + wave) * 32, key = k0w + j;       // this lane's key
     const bool wave_active = k0w < L;
     const int64_t po = static_cast<int64_t>(plane) * L * d;
 
     v8bf kb[NC][3], vb[NC][3];
-    load_slice_parts<DP>(p.K + po, key, L, d, half, p.scale * LOG2E, kb);
-    load_slice_parts<DP>(p.V + po, key, L, d, half, 1.0f, vb);
+    if (wave_active) {
+        v4f xk[NC][2], xv[NC][2];
+        load_slice<DP>(p.K + po, k0w, j, L, d, half, xk);
+        load_slice<DP>(p.V + po, k0w, j, L, d, half, xv);
+        slice_parts<DP>(xk, p.scale * LOG2E, kb);
+        slice_parts<DP>(xv, 1.0f, vb);
+    }
     const float* bias_plane = p.bias ? p.bias + static_cast<int64_t>(plane) * L * L : nullptr;
 
     v16f acc_k[NB], acc_v[NB];
@@ -405,23 +418,20 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_cols_kernel(const Att
         {
             constexpr int NT = NW * 64, NI = (T::CH_COLS * (DP / 4) + NT - 1) / NT;
             static_assert(DP / 4 == 8 || DP / 4 == 16, "eight or sixteen threads per staged row");
+            const int64_t from = po + static_cast<int64_t>(c0) * d;
+            const __amdgpu_buffer_rsrc_t rq = buffer_of(p.Q + from, cq * d), rdo = buffer_of(p.dO + from, cq * d), ro = buffer_of(p.O + from, cq * d),
+                                         rlse = buffer_of(p.LSE + static_cast<int64_t>(plane) * L + c0, cq);
             v4f xq[NI], xdo[NI], xo[NI];
             float lse_in[NI];
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
                 const int idx = tid + i * NT;
                 const int row = idx / (DP / 4), c = (idx % (DP / 4)) * 4;
-                xq[i] = xdo[i] = xo[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-                lse_in[i] = -INFINITY;
-                if (row < cq) {
-                    if (c < d) {
-                        const int64_t off = po + static_cast<int64_t>(c0 + row) * d + c;
-                        xq[i] = *reinterpret_cast<const v4f*>(p.Q + off);
-                        xdo[i] = *reinterpret_cast<const v4f*>(p.dO + off);
-                        xo[i] = *reinterpret_cast<const v4f*>(p.O + off);
-                    }
-                    if (c == 0) lse_in[i] = p.LSE[static_cast<int64_t>(plane) * L + c0 + row];
-                }
+                const uint32_t at = row < cq && c < d ? static_cast<uint32_t>(row * d + c) * 4u : OUTSIDE;
+                xq[i] = buffer_load4(rq, at);
+                xdo[i] = buffer_load4(rdo, at);
+                xo[i] = buffer_load4(ro, at);
+                lse_in[i] = buffer_load1(rlse, static_cast<uint32_t>(row) * 4u);
             }
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
@@ -433,10 +443,10 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_cols_kernel(const Att
                 sum += __shfl_xor(sum, 4, 64);
                 if (DP / 4 == 16) sum += __shfl_xor(sum, 8, 64);
                 if (row < rows) {
-                    put_fragments<DP>(xq[i], row, c, lds_q_row, lds_q_col);
-                    put_fragments<DP>(xdo[i], row, c, lds_do_row, lds_do_col);
+                    put_fragments<DP>(xq[i], row, c, lds_q);
+                    put_fragments<DP>(xdo[i], row, c, lds_do);
                     if (c == 0) {
-                        lds_lse[row] = lse_in[i] > -INFINITY ? lse_in[i] * LOG2E : INFINITY;
+                        lds_lse[row] = row < cq && lse_in[i] > -INFINITY ? lse_in[i] * LOG2E : INFINITY;
                         lds_D[row] = sum;
                     }
                 }
@@ -450,36 +460,54 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_cols_kernel(const Att
             // bias of this lane's key for its 16 queries of the tile, requested before the matrix work
             float bv[16];
             if (bias_plane) {
-                const float* bcol = bias_plane + (key < L ? key : L - 1);
+                // (from the tile's first row on: 32-bit offsets whatever the length; rows and keys past the matrix: zero, and masked below)
+                const __amdgpu_buffer_rsrc_t rbias = buffer_of(bias_plane + static_cast<int64_t>(qbase) * L, static_cast<int64_t>(L - qbase < 32 ? L - qbase : 32) * L);
+                const uint32_t row_bytes = static_cast<uint32_t>(L) * 4u;
+                uint32_t at = key < L ? static_cast<uint32_t>(key) * 4u + 4u * half * row_bytes : OUTSIDE;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int qq = qbase + 8 * (r >> 2) + 4 * half + (r & 3);
-                    bv[r] = bcol[static_cast<int64_t>(qq < L ? qq : L - 1) * L];
+                    bv[r] = buffer_load1(rbias, at);
+                    // (opaque: one offset that moves on, not sixteen at once)
+                    at += (r & 3) == 3 ? 5 * row_bytes : row_bytes;
+                    asm volatile("" : "+v"(at));
                 }
             }
-            // ---- S[query][key] and dO V^T, un-transposed: this lane's key, 16 of the tile's queries
-            v16f st = tile_times_slice<DP>(lds_q_row + qt * T::ROW_BYTES + lane * 16, kb);
-            v16f dp = tile_times_slice<DP>(lds_do_row + qt * T::ROW_BYTES + lane * 16, vb);
-            v16f ds;
+            // ---- S[query][key], un-transposed: this lane's key, 16 of the tile's queries
+            // (heads wider than one block of features: one phase after the other, the held slices and sums leave no registers for two)
+            const auto phase = [] { if (DP > 32) __builtin_amdgcn_sched_barrier(0); };
+            v16f st = tile_times_slice<DP>(lds_q + qt * T::TILE + row_at, kb), dp;
+            phase();
+            if (DP <= 32) dp = tile_times_slice<DP>(lds_do + qt * T::TILE + row_at, vb);
+            const auto seen = [&](int r) {
+                const int qq = qbase + 8 * (r >> 2) + 4 * half + (r & 3);
+                return qq < L && (!p.causal || key <= qq);
+            };
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const v4f lse4 = *reinterpret_cast<const v4f*>(lds_lse + qt * 32 + 8 * g + 4 * half);
-                const v4f D4 = *reinterpret_cast<const v4f*>(lds_D + qt * 32 + 8 * g + 4 * half);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int r = 4 * g + i;
-                    const int qq = qbase + 8 * g + 4 * half + i;
                     float s2 = st[r];
                     if (bias_plane) s2 = __builtin_fmaf(bv[r], LOG2E, s2);
-                    const bool seen = qq < L && (!p.causal || key <= qq);
-                    const float pr = seen ? __builtin_amdgcn_exp2f(s2 - lse4[i]) : 0.0f;
-                    st[r] = pr;                                    // P
-                    ds[r] = pr * (dp[r] - D4[i]);                  // dS
+                    st[r] = seen(r) ? __builtin_amdgcn_exp2f(s2 - lse4[i]) : 0.0f;      // P
                 }
             }
-            // ---- dV^T += dO^T . P,  dK^T += Q^T . dS
-            if (p.dV) accumulate_transposed<DP>(acc_v, lds_do_col + qt * T::COL_BYTES + lane * 16, st);
-            if (p.dK) accumulate_transposed<DP>(acc_k, lds_q_col + qt * T::COL_BYTES + lane * 16, ds);
+            phase();
+            // ---- dV^T += dO^T . P,  dO V^T,  dS = P (dO V^T - D),  dK^T += Q^T . dS
+            if (p.dV) accumulate_transposed<DP>(acc_v, lds_do + qt * T::TILE + col_at, st);
+            phase();
+            if (!p.dK) continue;
+            if (DP > 32) dp = tile_times_slice<DP>(lds_do + qt * T::TILE + row_at, vb);
+            phase();
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const v4f D4 = *reinterpret_cast<const v4f*>(lds_D + qt * 32 + 8 * g + 4 * half);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) st[4 * g + i] *= dp[4 * g + i] - D4[i];
+            }
+            phase();
+            accumulate_transposed<DP>(acc_k, lds_q + qt * T::TILE + col_at, st);
         }
     }
     if (!wave_active || key >= L) return;
@@ -522,8 +550,6 @@ __global__ __launch_bounds__(NW * 64) void flash_attn_back_cols_kernel(const Att
 // With all tiles contracted and P = 0 at masked pairs, one NaN behind a query reached its gradients as 0 * NaN.  With bias,
 // us, contracted / left out / the two kernels: 412 planes of 256 72 / 67 / 152, 412 of 192 54 / 47 / 101, 412 of 257
 // 162 / 101 / 208, 128 of 640 238 / 148 / 260; of 103, where every wave has a diagonal tile, 24.6 / 23.0 / 41.
-typedef short v4s __attribute__((ext_vector_type(4)));
-
 template <int NW> struct FusedBack {
     // Row fragments of 32 rows x 32 features as in BackTiling, but with the halves (features 8 .. 15 of a chunk) 576 bytes
     // apart: the transposing reads and the staging writes then touch every bank once.
@@ -539,15 +565,6 @@ template <int NW> struct FusedBack {
     static constexpr size_t LDS = 2 * STAGE + 2 * NW * static_cast<size_t>(REGION) + NO_KEY;
     static_assert(32 * QP * 4 <= REGION, "the partial tile takes the place of the parts");
 };
-
-// eight 16-bit elements of this lane's column, four rows at `at` and four at `at + step`, each piece transposed on the
-// way (a group of sixteen lanes names four rows of sixteen columns, four columns per lane)
-__device__ __forceinline__ v8bf read_transposed(const uint8_t* at, int step) {
-    typedef __attribute__((address_space(3))) v4s* lds_v4s;
-    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at));
-    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at + step));
-    return __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
 
 // DB: dbias not wanted / ordinary stores / streaming stores (rows of whole 128-byte lines)
 constexpr int DB_NONE = 0, DB_ORDINARY = 1, DB_STREAM = 2;
@@ -937,13 +954,13 @@ int launch_fused(const AttnBackParams& p, hipStream_t stream) {
 template <int DP, bool TWIN, bool BIAS, bool LATE>
 int launch_rows(AttnBackParams p, hipStream_t stream) {
     using T = BackTiling<DP>;
-    constexpr int NW = 4;
+    constexpr int NW = 4, MATRICES = TWIN ? 3 : 2;
     const int l32 = (p.L + 31) / 32 * 32;
     p.stage_rows = l32 < T::CH_ROWS ? l32 : T::CH_ROWS;
-    const size_t lds = static_cast<size_t>(p.stage_rows / 32) * (2 * T::ROW_BYTES + T::COL_BYTES);
+    const size_t lds = static_cast<size_t>(p.stage_rows / 32) * MATRICES * T::TILE;
     static LdsLimit limit;
     if (!limit.reserve(reinterpret_cast<const void*>(&flash_attn_back_rows_kernel<DP, NW, TWIN, BIAS, LATE>),
-                       (T::CH_ROWS / 32) * (2 * T::ROW_BYTES + T::COL_BYTES))) {
+                       (T::CH_ROWS / 32) * MATRICES * T::TILE)) {
         set_error("flash_attn_backward_hip: cannot reserve the LDS of the rows kernel");
         return RC_LAUNCH;
     }
@@ -974,11 +991,11 @@ int launch_back(AttnBackParams p, hipStream_t stream) {
     }
     if (p.dK || p.dV) {
         p.stage_rows = l32 < T::CH_COLS ? l32 : T::CH_COLS;
-        const size_t lds = static_cast<size_t>(p.stage_rows / 32) * (2 * T::ROW_BYTES + 2 * T::COL_BYTES) +
+        const size_t lds = static_cast<size_t>(p.stage_rows / 32) * 2 * T::TILE +
                            static_cast<size_t>(p.stage_rows) * 2 * sizeof(float);
         static LdsLimit limit;
         if (!limit.reserve(reinterpret_cast<const void*>(&flash_attn_back_cols_kernel<DP, NW>),
-                           (T::CH_COLS / 32) * (2 * T::ROW_BYTES + 2 * T::COL_BYTES) + T::CH_COLS * 8)) {
+                           (T::CH_COLS / 32) * 2 * T::TILE + T::CH_COLS * 8)) {
             set_error("flash_attn_backward_hip: cannot reserve the LDS of the columns kernel");
             return RC_LAUNCH;
         }
