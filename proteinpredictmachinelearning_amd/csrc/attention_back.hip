@@ -18,8 +18,11 @@
 //     dK^T += Q^T dS; LSE and D of the tile's queries come from LDS.
 // All five contractions run on the bf16 matrix pipe at binary32 accuracy (exact three-way split of every
 // operand, six partial products per 16 contracted elements; common.hpp): the streamed side lies in LDS as ready
-// MFMA fragments, in two arrangements where it is contracted both ways (over the features for S and dO V^T,
-// over its rows for the gradients), the held side and the freshly computed P / dS are split in registers.
+// MFMA fragments of its rows (for S and dO V^T), which transposing reads also serve as those of its columns (for the gradients), the
+// held side and the freshly computed P / dS are split in registers.
+// Measured, us, forward and all gradients, with a second arrangement of the streamed side in LDS (two-byte writes) and one work-group per
+// CU in the columns kernel / this way: 64 features, bias, 412 planes of 103 122 / 86, of 160 278 / 184, 824 of 256 778 / 584, without 669 /
+// 468; 52 of 52 37.7 / 30.3; 32 features, 40 planes of 384 98 / 88.
 // No atomics and no scratch memory: every output element has one owner, so the results do not depend on
 // scheduling (the reference's CUDA path accumulates dK and dV with atomicAdd).
 #include "common.hpp"
@@ -63,7 +66,9 @@ template <int DP> struct BackTiling {
     static constexpr int HALF = 576, FRAG = 2 * HALF, CHUNK = 3 * FRAG;
     static constexpr int TILE = NC * CHUNK;
     static constexpr int CH_ROWS = 64;                // rows staged at a time by the rows kernel
-    static constexpr int CH_COLS = DP <= 32 ? 96 : 32;     // ... by the columns kernel: two work-groups' share a CU's 160 KB
+    // ... by the columns kernel.  Wide heads: its loads' registers beside the held slices and sums have to leave room for a second wave per
+    // SIMD (64 rows at a time: 45 registers spilled, 412 planes of 103 91 us against 86)
+    static constexpr int CH_COLS = DP <= 32 ? 96 : 32;
 };
 
 // eight 16-bit elements of this lane's column, four rows at `at` and four at `at + step`, each piece transposed on the

@@ -423,3 +423,25 @@ def test_forward_keeps_to_its_own_rows(ops, L, d, causal):
         keep[2] = False
         assert torch.equal(out[0][keep].view(torch.int32), clean[0][keep].view(torch.int32))
         assert torch.equal(lse2[0][keep].view(torch.int32), lse[0][keep].view(torch.int32))
+
+
+@pytest.mark.parametrize("L", [3, 33, 50, 103, 131])
+@pytest.mark.parametrize("d", [4, 32, 48])
+@pytest.mark.parametrize("causal", [False, True])
+def test_backward_keeps_to_its_own_rows(ops, L, d, causal):
+    """The rows kernel reads the bias like the forward: a row of NaN leaves dQ and dbias of every other row the bits they have without it."""
+    torch.manual_seed(L + d)
+    planes = 3
+    q, k, v, do = (torch.randn(1, planes, L, d, device="cuda") for _ in range(4))
+    bias = torch.randn(1, planes, L, L, device="cuda")
+    o, lse = ops.flash_attn_forward(q, k, v, bias, causal=causal)
+    bad = bias.clone()
+    r = L // 2
+    bad[0, 0, r] = float("nan")
+    want = ("dq", "dbias")
+    dq, _, _, db = ops.flash_attn_backward(q, k, v, bias, o, do, lse, causal=causal, want=want)
+    dq2, _, _, db2 = ops.flash_attn_backward(q, k, v, bad, o, do, lse, causal=causal, want=want)
+    keep = torch.ones(planes, L, dtype=torch.bool, device="cuda")
+    keep[0, r] = False
+    assert torch.equal(dq[0][keep].view(torch.int32), dq2[0][keep].view(torch.int32))
+    assert torch.equal(db[0][keep].view(torch.int32), db2[0][keep].view(torch.int32))
