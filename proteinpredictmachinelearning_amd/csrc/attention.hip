@@ -44,7 +44,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const float* base, i
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, static_cast<int>(bytes), 0x00020000);
 }
 
-template <int DP, int NW, bool PF> struct AttnTiling {
+template <int DP, int NW, bool PF, bool IN_LD> struct AttnTiling {
     // keys staged in LDS at a time: 36 KB per four-wave work-group (four of them share a CU and its
     // 160 KB; 128 keys would leave room for three, measured 64.7 against 61.2 us at the MSA shape).  The form of short
     // rows has the registers for three anyway, and with 128 its rows are one stage.
@@ -52,9 +52,13 @@ template <int DP, int NW, bool PF> struct AttnTiling {
     static constexpr int NC = DP / 16;                // 16-feature chunks of the score contraction
     // a 32-key tile of K in LDS: one 1 KB MFMA operand fragment per (chunk, bf16 part), [half][key][8 bf16]
     static constexpr int KT_BYTES = NC * 3 * 1024;
-    // a 32-key tile of V in LDS: fragments of V^T per (32 features, 16 keys, bf16 part); slot i of lane
-    // (feature, half) holds key 16 ch + 8 (i / 4) + 4 half + i % 4 of the tile
-    static constexpr int VT_BYTES = (DP / 32) * 2 * 3 * 1024;
+    // a 32-key tile of V in LDS.  As fragments of V^T per (32 features, 16 keys, bf16 part) where the source rows run along the keys: slot i of
+    // lane (feature, half) holds key 16 ch + 8 (i / 4) + 4 half + i % 4 of the tile.  Otherwise fragments of its rows like K's, the
+    // halves 576 bytes apart, which ds_read_b64_tr_b16 hands out in that order; scattered to the other form it took twelve two-byte writes
+    // per four features.  us, those / transposing reads: 412 planes of 103, bias 13.4 / 12.4, 64 features 24.0 / 21.0, 824 of 256 79.0 / 76.1, 64
+    // features 160 / 131, 824 of 52 without bias 11.5 / 10.2.
+    static constexpr int V_HALF = 576, V_FRAG = 2 * V_HALF, V_CHUNK = 3 * V_FRAG;
+    static constexpr int VT_BYTES = IN_LD ? (DP / 32) * 2 * 3 * 1024 : NC * V_CHUNK;
     static constexpr size_t lds_bytes = static_cast<size_t>(CH / 32) * (KT_BYTES + VT_BYTES);
 };
 
@@ -68,7 +72,6 @@ struct AttnParams {
     float scale, eps;
     int head;            // keys of the reference's first block: min(Bc, keys of the row)
     int stage_rows;      // keys staged in LDS at a time: at most CH, L's tiles of 32 shared out evenly
-    int in_ld;           // Q, K, V are [B][h][d][L] (the graph's [L, D, h, B] tensors, not yet permuted)
     int out_ld;          // O is written as [B][h][d][L]
 };
 
@@ -80,10 +83,11 @@ __device__ __forceinline__ float lane_xor32(float x) {
 // PF: request each tile's bias one tile ahead.  It costs 16 registers, i.e. the fourth wave per SIMD, so only
 // the instance for short sequences uses it: there a work-group is a chain of memory latencies and the
 // machine is far from full anyway.
-template <int DP, int NW, bool PF>
+// IN_LD: Q, K, V are [B][h][d][L] (the graph's [L, D, h, B] tensors, not yet permuted).
+template <int DP, int NW, bool PF, bool IN_LD>
 // (the instance for long sequences is held to 128 registers: four waves per SIMD; the other one of narrow heads to three)
 __global__ __launch_bounds__(NW * 64, DP <= 32 ? (PF ? 3 : 4) : 1) void flash_attn_forward_kernel(const AttnParams p) {
-    using T = AttnTiling<DP, NW, PF>;
+    using T = AttnTiling<DP, NW, PF, IN_LD>;
     constexpr int NC = T::NC, KT_BYTES = T::KT_BYTES, VT_BYTES = T::VT_BYTES;
     constexpr int NB = DP / 32;                       // 32-row blocks of the transposed output
     extern __shared__ __attribute__((aligned(16))) float attn_lds[];
@@ -109,15 +113,15 @@ __global__ __launch_bounds__(NW * 64, DP <= 32 ? (PF ? 3 : 4) : 1) void flash_at
     const auto load1 = [](const __amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0)); };
     if (wave_active) {
         // the wave's rows, or the whole plane where a row is a feature
-        const int64_t q_bytes = p.in_ld ? static_cast<int64_t>(L) * d * 4 : (L - q0 < 32 ? L - q0 : 32) * d * 4;
-        const __amdgpu_buffer_rsrc_t rq = buffer_of(p.Q + plane_off + (p.in_ld ? 0 : static_cast<int64_t>(q0) * d), q_bytes < 0x7fffffff ? q_bytes : 0x7fffffff);
+        const int64_t q_bytes = IN_LD ? static_cast<int64_t>(L) * d * 4 : (L - q0 < 32 ? L - q0 : 32) * d * 4;
+        const __amdgpu_buffer_rsrc_t rq = buffer_of(p.Q + plane_off + (IN_LD ? 0 : static_cast<int64_t>(q0) * d), q_bytes < 0x7fffffff ? q_bytes : 0x7fffffff);
         v4f xq[NC][2];
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             const int e0 = 16 * c + 8 * half;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                if (p.in_ld) {
+                if (IN_LD) {
                     // [d][L]: one element per feature row, lanes along the queries (whole 128-byte runs)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
@@ -233,7 +237,9 @@ __global__ __launch_bounds__(NW * 64, DP <= 32 ? (PF ? 3 : 4) : 1) void flash_at
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc_o[b][r] *= alpha;
         }
-        const uint8_t* vfrag = lds_v + kt * VT_BYTES + lane * 16;
+        const int grp = lane & 15;
+        const uint8_t* vfrag = lds_v + kt * VT_BYTES + (IN_LD ? lane * 16 : ((lane >> 4) & 1) * T::V_CHUNK + ((grp >> 1) & 1) * T::V_HALF +
+                                                                            (4 * half + (grp >> 2)) * 16 + (grp & 1) * 8);
 #pragma unroll
         for (int ch = 0; ch < 2; ++ch) {
             // the probabilities of 16 keys as three bf16 parts: score registers 8 ch .. 8 ch + 7 of this lane
@@ -249,7 +255,9 @@ __global__ __launch_bounds__(NW * 64, DP <= 32 ? (PF ? 3 : 4) : 1) void flash_at
             for (int b = 0; b < NB; ++b) {
                 v8bf va[3];
 #pragma unroll
-                for (int part = 0; part < 3; ++part) va[part] = *reinterpret_cast<const v8bf*>(vfrag + ((b * 2 + ch) * 3 + part) * 1024);
+                for (int part = 0; part < 3; ++part)
+                    va[part] = IN_LD ? *reinterpret_cast<const v8bf*>(vfrag + ((b * 2 + ch) * 3 + part) * 1024)
+                                     : read_transposed(vfrag + b * 2 * T::V_CHUNK + part * T::V_FRAG + ch * 256, 128);
 #pragma unroll
                 for (int t = 0; t < 6; ++t)
                     acc_o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[SPLIT_TERMS[t][0]], pb[SPLIT_TERMS[t][1]], acc_o[b], 0, 0, 0);
@@ -280,7 +288,7 @@ __global__ __launch_bounds__(NW * 64, DP <= 32 ? (PF ? 3 : 4) : 1) void flash_at
         __syncthreads();
         const int ckeys = L - c0 < stage ? L - c0 : stage;
         const int rows = (ckeys + 31) / 32 * 32;
-        if (p.in_ld) {
+        if (IN_LD) {
             // source rows run along the keys: four keys of one feature per thread, scattered into the
             // key-major LDS tiles
             // (eight lanes read 128 contiguous bytes of one feature row; the LDS writes of a wave then
@@ -339,21 +347,10 @@ __global__ __launch_bounds__(NW * 64, DP <= 32 ? (PF ? 3 : 4) : 1) void flash_at
                 uint8_t* dst = lds_k + (key >> 5) * KT_BYTES + (c >> 4) * 3072 + ((c >> 3) & 1) * 512 + (key & 31) * 16 + ((c >> 2) & 1) * 8;
 #pragma unroll
                 for (int part = 0; part < 3; ++part) *reinterpret_cast<uint2*>(dst + part * 1024) = parts[part];
-                // V: features c .. c+3 of one key go to four lane slots of the fragments of V^T, two bytes each
                 split4(vx[it], parts);
-                {
-                    const int kc = key & 15;
-                    const int slot = 4 * (kc >> 3) + (kc & 3);
-                    uint8_t* vdst = lds_v + (key >> 5) * VT_BYTES + (((c >> 5) * 2 + ((key >> 4) & 1)) * 3) * 1024 +
-                                    (((kc >> 2) & 1) * 32 + (c & 31)) * 16 + slot * 2;
+                dst = lds_v + (key >> 5) * VT_BYTES + (c >> 4) * T::V_CHUNK + ((c >> 3) & 1) * T::V_HALF + (key & 31) * 16 + ((c >> 2) & 1) * 8;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int part = 0; part < 3; ++part) {
-                            const uint32_t w = (i < 2 ? parts[part].x : parts[part].y) >> (16 * (i & 1));
-                            *reinterpret_cast<uint16_t*>(vdst + part * 1024 + i * 16) = static_cast<uint16_t>(w);
-                        }
-                }
+                for (int part = 0; part < 3; ++part) *reinterpret_cast<uint2*>(dst + part * T::V_FRAG) = parts[part];
             }
         }
         __syncthreads();
@@ -406,10 +403,10 @@ __global__ __launch_bounds__(NW * 64, DP <= 32 ? (PF ? 3 : 4) : 1) void flash_at
     if (p.LSE && half == 0) p.LSE[static_cast<int64_t>(plane) * L + q] = live ? m_run * LN2 + __logf(l_run + p.eps) : -INFINITY;
 }
 
-template <int DP, int NW, bool PF>
-int launch_flash(AttnParams p, hipStream_t stream) {
-    using T = AttnTiling<DP, NW, PF>;
-    auto kernel = &flash_attn_forward_kernel<DP, NW, PF>;
+template <int DP, int NW, bool PF, bool IN_LD>
+int launch_flash_ld(AttnParams p, hipStream_t stream) {
+    using T = AttnTiling<DP, NW, PF, IN_LD>;
+    auto kernel = &flash_attn_forward_kernel<DP, NW, PF, IN_LD>;
     const int l32 = (p.L + 31) / 32 * 32;
     // stages of even size: eight waves take 160 keys as 96 + 64, not 128 + 32
     const int stages = (l32 + T::CH - 1) / T::CH;
@@ -423,6 +420,11 @@ int launch_flash(AttnParams p, hipStream_t stream) {
     const dim3 grid((p.L + 32 * NW - 1) / (32 * NW), p.planes), block(NW * 64);
     hipLaunchKernelGGL(kernel, grid, block, lds, stream, p);
     return check_launch("flash_attn_forward_kernel");
+}
+
+template <int DP, int NW, bool PF>
+int launch_flash(const AttnParams& p, bool in_ld, hipStream_t stream) {
+    return in_ld ? launch_flash_ld<DP, NW, PF, true>(p, stream) : launch_flash_ld<DP, NW, PF, false>(p, stream);
 }
 
 }  // namespace
@@ -460,7 +462,7 @@ extern "C" int flash_attn_forward_ex_hip(int B, int h, int L, int d, int causal,
     p.eps = softmax_eps;
     p.head = Bc > 0 ? Bc : 64;                        // FlashAttn.cpp:62
     p.stage_rows = 0;                                 // set per instance
-    p.in_ld = layout & 1;
+    const bool in_ld = (layout & 1) != 0;
     p.out_ld = (layout >> 1) & 1;
     StatsScope stat("hip/flash_attn", static_cast<int64_t>(planes) * L, d, L, static_cast<hipStream_t>(stream));
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -478,10 +480,10 @@ extern "C" int flash_attn_forward_ex_hip(int B, int h, int L, int d, int causal,
     const int64_t cus = device_cu_count(), rounds = (2 * planes + cus - 1) / cus;
     const bool whole = L > 128 && L <= 256 && 2 * planes > cus && (L <= 160 || (causal ? L > 192 || rounds % 2 == 0 : rounds != 3));
     if (d <= 32) {
-        if (short_rows) return launch_flash<32, 4, true>(p, s);
-        return whole ? launch_flash<32, 8, false>(p, s) : launch_flash<32, 4, false>(p, s);
+        if (short_rows) return launch_flash<32, 4, true>(p, in_ld, s);
+        return whole ? launch_flash<32, 8, false>(p, in_ld, s) : launch_flash<32, 4, false>(p, in_ld, s);
     }
-    return short_rows ? launch_flash<64, 4, true>(p, s) : launch_flash<64, 4, false>(p, s);
+    return short_rows ? launch_flash<64, 4, true>(p, in_ld, s) : launch_flash<64, 4, false>(p, in_ld, s);
 }
 
 extern "C" int flash_attn_forward_hip(int B, int h, int L, int d, int causal, float scale, float softmax_eps, int Bc,

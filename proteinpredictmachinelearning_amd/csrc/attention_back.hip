@@ -71,15 +71,6 @@ template <int DP> struct BackTiling {
     static constexpr int CH_COLS = DP <= 32 ? 96 : 32;
 };
 
-// eight 16-bit elements of this lane's column, four rows at `at` and four at `at + step`, each piece transposed on the
-// way (a group of sixteen lanes names four rows of sixteen columns, four columns per lane)
-typedef short v4s __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ v8bf read_transposed(const uint8_t* at, int step) {
-    typedef __attribute__((address_space(3))) v4s* lds_v4s;
-    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at));
-    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at + step));
-    return __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
 // this lane's place in a tile: its row's half chunk, and what it names of the transposed reads of 32 features
 template <int DP> __device__ __forceinline__ int row_place(int lane) { return (lane & 31) * 16 + (lane >> 5) * BackTiling<DP>::HALF; }
 template <int DP> __device__ __forceinline__ int column_place(int lane) {

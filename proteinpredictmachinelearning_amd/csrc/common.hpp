@@ -175,6 +175,20 @@ __device__ __forceinline__ void split8(const v4f (&x)[2], v8bf (&out)[3], SplitG
         out[s] = __builtin_bit_cast(v8bf, v4i{static_cast<int>(lo[s].x), static_cast<int>(lo[s].y), static_cast<int>(hi[s].x), static_cast<int>(hi[s].y)});
 }
 
+// eight 16-bit elements of this lane's column, four rows at `at` and four at `at + step`, each piece transposed on the
+// way (a group of sixteen lanes names four rows of sixteen columns, four columns per lane)
+typedef short v4s __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ v8bf read_transposed(const uint8_t* at, int step) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(3))) v4s* lds_v4s;
+    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at));
+    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(at + step));
+    return __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#else
+    return v8bf{};
+#endif
+}
+
 // op over all 64 lanes, with the partners of a butterfly over lane ^ 32, 16, 8, 4, 2, 1 -- and so its bits, for a commutative
 // op.  No step goes through LDS: the halves and the rows of sixteen lanes change places by v_permlane32_swap / 16_swap (both
 // operands the value: one comes back as the even halves or rows twice over, the other as the odd ones), within a row the
