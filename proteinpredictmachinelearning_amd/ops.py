@@ -9,6 +9,8 @@ reverse of the reference's ``dims[0]``-innermost notation.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import math
 import os
 
@@ -22,12 +24,50 @@ WTYPE_Q8_0, WTYPE_Q8_1, WTYPE_Q8_0R, WTYPE_Q8_0M = 0, 1, 2, 3
 
 # What a call asks of torch beside its kernel -- the current device, its stream, the addresses -- costs more than a small
 # kernel: a projection of 408 x 256 -> 256, whose kernel takes 3.7 us, took 10.3 through this module with torch's public
-# forms (a stream object alone 2.7 us, is_available and current_device 0.8) and 6.1 with the functions beneath them.
+# forms (a stream object alone 2.7 us, is_available and current_device 0.8) and 6.1 with the functions beneath them.  That is the
+# long way; ordinary calls go through native code (csrc/host_calls.cpp) in 4.2.
 _current_device = torch._C._cuda_getDevice if hasattr(torch._C, "_cuda_getDevice") else torch.cuda.current_device
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
 
+
+
+def _load_host_calls():
+    """The native host side of the operators below (csrc/host_calls.cpp), or None where it was not built for this torch: every
+    operator then does its call itself, as it does any call that is not ordinary."""
+    path = os.path.join(os.path.dirname(cabi.LIB_PATH), "_host_calls.so")
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_host_calls", path)
+        spec = importlib.util.spec_from_file_location("_host_calls", path, loader=loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        return module
+    except (ImportError, OSError):
+        return None
+
+
+def _not_taken(*_):
+    return None
+
+
+_host = _load_host_calls()
+# each takes a call of its operator if everything about it is ordinary and answers None otherwise
+(_host_mul_mat, _host_mul_mat_f16, _host_mul_mat_q8, _host_outer_product_mean, _host_outer_prod_mean_back, _host_tri_mul, _host_tri_mul_back,
+ _host_flash_attn_forward, _host_flash_attn_backward) = (
+    getattr(_host, name, _not_taken) for name in ("mul_mat", "mul_mat_f16", "mul_mat_q8", "outer_product_mean", "outer_prod_mean_back", "tri_mul",
+                                                   "tri_mul_back", "flash_attn_forward", "flash_attn_backward"))
+_HOST_LAUNCHERS = ("mul_mat_hip", "mul_mat_f16_hip", "mul_mat_q8_hip", "mul_mat_q8_ex_hip", "outer_prod_mean_hip", "outer_prod_mean_back_hip",
+                   "tri_mul_hip", "tri_mul_back_hip", "flash_attn_forward_ex_hip", "flash_attn_backward_hip")
+
 _initialised = set()                                  # devices ppml_hip_init has run on in this process
-os.register_at_fork(after_in_child=_initialised.clear)      # (torch refuses the GPU in a forked child: the long way round says so)
+
+
+def _forget_devices():
+    _initialised.clear()
+    if _host is not None:
+        _host.forget()
+
+
+os.register_at_fork(after_in_child=_forget_devices)      # (torch refuses the GPU in a forked child: the long way round says so)
 
 
 def _lib():
@@ -38,6 +78,10 @@ def _lib():
         raise RuntimeError("the gfx950 backend needs a GPU; there is no CPU path")
     dev = torch.cuda.current_device()
     cabi.check("ppml_hip_init", lib.ppml_hip_init(dev))
+    if _host is not None:
+        for name in _HOST_LAUNCHERS:
+            _host.bind(name, C.cast(getattr(lib, name), C.c_void_p).value)
+        _host.ready(dev)
     _initialised.add(dev)
     return lib
 
@@ -93,6 +137,9 @@ def set_f32_arithmetic(mode: str) -> str:
 
 def mul_mat(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """a [M,K], b [N,K] -> [M,N] = a @ b.T (+ bias[N]); src/core/ComputeGraphHelper.cpp:262-314."""
+    out = _host_mul_mat(a, b, bias)
+    if out is not None:
+        return out
     a, b = _dev_f32(a, "a"), _dev_f32(b, "b")
     if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[1]:
         raise ValueError(f"mul_mat: inner dimensions differ, a {tuple(a.shape)} b {tuple(b.shape)}")
@@ -111,6 +158,9 @@ def mul_mat(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = None) 
 def mul_mat_f16(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """F16 x F16 -> F32 mul_mat: a [M,K], b [N,K] float16 on the device, binary32 products and sum,
     bias (f32 [N]) added to the finished sum (src/backend/CPUKernels.cpp:646-672)."""
+    out = _host_mul_mat_f16(a, b, bias)
+    if out is not None:
+        return out
     for t, name in ((a, "a"), (b, "b")):
         if not t.is_cuda or t.dtype != torch.float16:
             raise TypeError(f"mul_mat_f16: {name} must be a float16 tensor on the device")
@@ -180,6 +230,9 @@ def attention_logits(k: torch.Tensor, q: torch.Tensor, head_dim: int | None = No
 def outer_product_mean(left: torch.Tensor, right: torch.Tensor, D: int, L: int, N: int, B: int) -> torch.Tensor:
     """Graph form (src/core/ComputeGraphHelper.cpp:1748-1764): flat buffers indexed as
     src/backend/CPUKernels.cpp:1006-1028; returns the flat [D*D*L*L*B] result."""
+    out = _host_outer_product_mean(left, right, D, L, N, B)
+    if out is not None:
+        return out
     left, right = _dev_f32(left, "left").reshape(-1), _dev_f32(right, "right").reshape(-1)
     if left.numel() != D * L * N * B or right.numel() != D * L * N * B:
         raise ValueError("outer_product_mean: operand size does not match D*L*N*B")
@@ -192,6 +245,10 @@ def outer_product_mean(left: torch.Tensor, right: torch.Tensor, D: int, L: int, 
 def outer_prod_mean_back(grad: torch.Tensor, left: torch.Tensor, right: torch.Tensor, D: int, L: int, N: int, B: int,
                          want_left: bool = True, want_right: bool = True):
     """Gradients of outer_prod_mean's operands (src/backend/CPUKernels.cpp:1034-1105); flat tensors."""
+    if want_left is True and want_right is True:
+        both = _host_outer_prod_mean_back(grad, left, right, D, L, N, B)
+        if both is not None:
+            return both
     grad, left, right = _dev_f32(grad, "grad"), _dev_f32(left, "left"), _dev_f32(right, "right")
     if grad.numel() != D * D * L * L * B or left.numel() != D * L * N * B or right.numel() != D * L * N * B:
         raise ValueError("outer_prod_mean_back: operand size does not match D, L, N, B")
@@ -224,6 +281,9 @@ def tri_mul(left: torch.Tensor, right: torch.Tensor, D: int, I: int, J: int, K: 
             outgoing: bool = True) -> torch.Tensor:
     """Triangle multiplication, graph form (src/backend/CPUKernels.cpp:907-968): flat operands indexed as the
     kernel does (d outermost, b innermost); returns the flat [D*I*J*B] result incl. the 1/L and the finite guard."""
+    out = _host_tri_mul(left, right, D, I, J, K, B, L, outgoing)
+    if out is not None:
+        return out
     left, right = _dev_f32(left, "left"), _dev_f32(right, "right")
     if L == 0:
         raise ValueError("tri_mul: L must not be zero")
@@ -238,6 +298,10 @@ def tri_mul(left: torch.Tensor, right: torch.Tensor, D: int, I: int, J: int, K: 
 def tri_mul_back(grad: torch.Tensor, left: torch.Tensor, right: torch.Tensor, D: int, I: int, J: int, K: int, B: int,
                  L: float, outgoing: bool = True, want_left: bool = True, want_right: bool = True):
     """Gradients of tri_mul's operands (src/backend/CPUKernels.cpp:1238-1367); flat tensors, same indexing."""
+    if want_left is True and want_right is True:
+        both = _host_tri_mul_back(grad, left, right, D, I, J, K, B, L, outgoing)
+        if both is not None:
+            return both
     grad, left, right = _dev_f32(grad, "grad"), _dev_f32(left, "left"), _dev_f32(right, "right")
     if L == 0 or not (want_left or want_right):
         raise ValueError("tri_mul_back: L must not be zero and at least one gradient must be wanted")
@@ -257,6 +321,10 @@ def flash_attn_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bias: 
     """Fused attention forward (include/ppml/FlashAttn.h:8-65): Q, K, V (B,h,L,d), bias (B,h,L,L) or None
     -> O (B,h,L,d) and LSE (B,h,L) (None when not wanted).  in_ld: Q, K, V are (B,h,d,L) instead (the graph
     tensors before their layout bridge); out_ld: O is returned as (B,h,d,L)."""
+    if not in_ld and not out_ld:
+        both = _host_flash_attn_forward(q, k, v, bias, causal, scale, eps, Bc, want_lse)
+        if both is not None:
+            return both
     q, k, v = _dev_f32(q, "q"), _dev_f32(k, "k"), _dev_f32(v, "v")
     if q.dim() != 4 or q.shape != k.shape or q.shape != v.shape:
         raise ValueError("flash_attn_forward: Q, K and V must be 4-D tensors of one shape (B,h,L,d)")
@@ -281,6 +349,10 @@ def flash_attn_backward(q, k, v, bias, o, do, lse, causal: bool = False, scale: 
                         want=("dq", "dk", "dv", "dbias")):
     """Fused attention backward (include/ppml/FlashAttn.h:67-101): returns (dQ, dK, dV, dbias), None for the
     gradients not named in `want`."""
+    grads = _host_flash_attn_backward(q, k, v, bias, o, do, lse, causal, scale,
+                                      ("dq" in want) | ("dk" in want) << 1 | ("dv" in want) << 2 | ("dbias" in want) << 3)
+    if grads is not None:
+        return grads
     q, k, v, o, do, lse = (_dev_f32(t, n) for t, n in ((q, "q"), (k, "k"), (v, "v"), (o, "o"), (do, "do"), (lse, "lse")))
     B, h, L, d = q.shape
     if bias is not None:
@@ -502,6 +574,10 @@ def mul_mat_q8(w: Q8Weight, x: torch.Tensor, c_trans: int = 1, relu: bool = Fals
     "weight-stationary-column-parts" / "-whole": that kernel with the columns shared out between work-groups
     wherever an instance exists / never); every choice gives the same bits.
     ``out``: a contiguous f32 device tensor of the result's shape to write into instead of a new one."""
+    if out is None and dump is False and act == "q8_0" and path == "auto":
+        y = _host_mul_mat_q8(w.data, x, w.M, w.K, w.wtype, c_trans, 1 if relu else 0)
+        if y is not None:
+            return y
     if act not in ("q8_0", "q8_1"):
         raise ValueError("mul_mat_q8: act must be 'q8_0' or 'q8_1'")
     x = _dev_f32(x, "x")
