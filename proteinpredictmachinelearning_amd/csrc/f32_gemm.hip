@@ -686,7 +686,7 @@ __global__ __launch_bounds__(256) void gemm_bf16x3_kernel(const GemmParams p) {
 // each other anyway and the two forms measure the same: the launcher takes this one up to one tile per CU.
 constexpr int PC_AHEAD = 3;                       // chunks a producer wave has in flight
 constexpr int PC_STAGE = 3 * SPLIT_PLANE;         // the three planes of one operand's chunk
-template <int MODE, bool STREAM_C, bool K4, int BMODE>
+template <int MODE, bool STREAM_C, bool K4, int BMODE, int C_FORM = C_DENSE>
 __device__ __forceinline__ void pc_tile(const GemmParams& p, uint8_t (&lds_ab)[2][2 * PC_STAGE], int group) {
     // (MODE: how A lies; BMODE: how B lies -- the backward of the triangle multiplication contracts a gradient that is
     // contiguous in k with an operand that is contiguous in its rows)
@@ -789,15 +789,22 @@ __device__ __forceinline__ void pc_tile(const GemmParams& p, uint8_t (&lds_ab)[2
         return;
     }
     if (!producer) {
-        const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(C, 0, static_cast<int>(p.M * p.c_mi * 4), 0x00020000);
-        store_acc_buffer<STREAM_C>(rsrc_c, static_cast<uint32_t>(p.c_mi) * 4u, p.N, p.alpha, acc, m0 + wm, n0 + wn, lane);
+        if (C_FORM == C_COMPOUND_BUFFER) {
+            store_acc_compound_buffer<STREAM_C, 2>(p, C, acc, m0 + wm, n0 + wn, lane);
+        } else if (C_FORM == C_COMPOUND) {
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti) store_tile_compound<2>(p, C, acc[ti], m0 + wm + ti * 32, n0 + wn, lane);
+        } else {
+            const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(C, 0, static_cast<int>(p.M * p.c_mi * 4), 0x00020000);
+            store_acc_buffer<STREAM_C>(rsrc_c, static_cast<uint32_t>(p.c_mi) * 4u, p.N, p.alpha, acc, m0 + wm, n0 + wn, lane);
+        }
     }
 }
 
-template <int MODE, bool STREAM_C, bool K4, int BMODE = MODE>
+template <int MODE, bool STREAM_C, bool K4, int BMODE = MODE, int C_FORM = C_DENSE>
 __global__ __launch_bounds__(512) void gemm_bf16x3_pc_kernel(const GemmParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t lds_ab[2][2 * PC_STAGE];
-    pc_tile<MODE, STREAM_C, K4, BMODE>(p, lds_ab, static_cast<int>(blockIdx.x));
+    pc_tile<MODE, STREAM_C, K4, BMODE, C_FORM>(p, lds_ab, static_cast<int>(blockIdx.x));
 }
 
 // The same on tiles of 64 x 64 with two chunks per barrier, for a LinearLayer's contraction that leaves most CUs without a
@@ -811,7 +818,8 @@ constexpr int PC64_PLANE = 64 * SPLIT_PITCH;      // one of the three planes of 
 constexpr int PC64_OPERAND = 2 * 3 * PC64_PLANE;  // [16 k][plane][row]
 // BMODE LOAD_ROW_CONTIG: B(n, k) = B[k * b_ks + n], a weight as it lies under a contraction over its rows (the gradient of a linear
 // layer's input): a thread then loads one column of the tile and eight k of the stage, and writes what the other form writes.
-template <bool STREAM_C, bool K4, int BMODE = LOAD_K_CONTIG>
+// C_FORM: an output with compound addressing too (a small outer-product-mean), stored as gemm_bf16x3_kernel does.
+template <bool STREAM_C, bool K4, int BMODE = LOAD_K_CONTIG, int C_FORM = C_DENSE>
 __global__ __launch_bounds__(512) void gemm_bf16x3_pc64_kernel(const GemmParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t lds_ab[2][2 * PC64_OPERAND];
     const int tid = threadIdx.x;
@@ -924,6 +932,14 @@ __global__ __launch_bounds__(512) void gemm_bf16x3_pc64_kernel(const GemmParams 
     // an operand of this tile that the split could not carry: the whole tile again, the reference's way
     if (__syncthreads_or(fired)) {
         if (tid < 256) plain_tile(p, p.A, p.B, p.C, m0, n0, 64, 64, tid);
+        return;
+    }
+    if (C_FORM != C_DENSE) {
+        if (wave < 4) {
+            const v16f one[1] = {acc};
+            if (C_FORM == C_COMPOUND_BUFFER) store_tile_compound_buffer<STREAM_C, 1>(p, p.C, one, m0 + wm, n0 + wn, lane);
+            else store_tile_compound<1>(p, p.C, one, m0 + wm, n0 + wn, lane);
+        }
         return;
     }
     if (wave < 4) {
@@ -2763,6 +2779,22 @@ int launch_gemm_sums(GemmParams p, hipStream_t stream, const char* what, uint8_t
         // below 2 GiB that are contiguous in k or in their rows: buffer-addressed loads, the generic store
         else if (split && p.a_lm == 0 && mode == LOAD_K_CONTIG && ((p.M - 1) * p.a_rs + p.K) * 4 < (1LL << 31) &&
                  ((p.N - 1) * p.b_rs + p.K) * 4 < (1LL << 31) && p.a_rs < (1 << 22) && p.b_rs < (1 << 22)) {
+            // a single plane of few tiles (an outer-product-mean of up to 2048 columns a side): 128 x 128 tiles of
+            // gemm_bf16x3_kernel leave CUs idle there and hide neither their loads nor their stores.  64 x 64 tiles of the
+            // loading / contracting form up to two per CU; 128 x 128 ones up to one where K is long enough to fill its ring.
+            // The same bits.  us, before / now, features x residues x sequences: 8 x 24 x 9 13.4 / 5.8, 16 x 24 x 64
+            // 16.5 / 5.9, 8 x 103 x 118 13.8 / 7.1, 32 x 40 x 256 21.8 / 12.2; in 128 x 128 tiles 32 x 51 x 256 23.2 / 19.8, x 97
+            // 15.5 / 14.2 (x 64 11.1 / 11.7).  64 x 64 tiles at three to four per CU: 32 x 64 x 9 7.6 / 9.5, x 118 15.6 / 17.2
+            const bool c64 = tiles64 <= 2 * device_cu_count();
+            if (p.np2 * p.np3 == 1 && !p.stream_c && (c64 || (p.K > 6 * BK && total <= device_cu_count()))) {
+                const dim3 g64(static_cast<unsigned>(tiles64));
+#define PPML_CPC(C_, K4_) do { if (c64) hipLaunchKernelGGL((gemm_bf16x3_pc64_kernel<false, K4_, LOAD_K_CONTIG, C_>), g64, dim3(512), 0, stream, p); \
+                               else hipLaunchKernelGGL((gemm_bf16x3_pc_kernel<LOAD_K_CONTIG, false, K4_, LOAD_K_CONTIG, C_>), grid, dim3(512), 0, stream, p); } while (0)
+                if (p.c_span) { if (p.K % 4 == 0) PPML_CPC(C_COMPOUND_BUFFER, true); else PPML_CPC(C_COMPOUND_BUFFER, false); }
+                else          { if (p.K % 4 == 0) PPML_CPC(C_COMPOUND, true); else PPML_CPC(C_COMPOUND, false); }
+#undef PPML_CPC
+                return check_launch(what);
+            }
 #define PPML_KFAST_SPLIT(C_, STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_kernel<LOAD_K_CONTIG, C_, STREAM_, true, K4_>), grid, block, 0, stream, p)
 #define PPML_KFAST_SPLIT_K4(C_, STREAM_) do { if (p.K % 4 == 0) PPML_KFAST_SPLIT(C_, STREAM_, 1); else PPML_KFAST_SPLIT(C_, STREAM_, 0); } while (0)
             if (p.c_span) { if (p.stream_c) PPML_KFAST_SPLIT_K4(C_COMPOUND_BUFFER, true); else PPML_KFAST_SPLIT_K4(C_COMPOUND_BUFFER, false); }

@@ -149,6 +149,22 @@ __device__ __forceinline__ void store_tile_compound_buffer(const GemmParams& p, 
     }
 }
 
+// Any compound output, 64-bit addresses
+template <int TJ>
+__device__ __forceinline__ void store_tile_compound(const GemmParams& p, float* __restrict__ C, const v16f (&acc)[TJ], int m_base, int n_base, int lane) {
+#pragma unroll
+    for (int tj = 0; tj < TJ; ++tj) {
+        const int n = n_base + tj * 32 + (lane & 31);
+        if (n >= p.N) continue;
+        float* const col = C + static_cast<int64_t>(n / p.c_ln) * p.c_no + static_cast<int64_t>(n % p.c_ln) * p.c_ni;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = m_base + mfma32_row(r, lane);
+            if (m < p.M) col[static_cast<int64_t>(m / p.c_lm) * p.c_mo + static_cast<int64_t>(m % p.c_lm) * p.c_mi] = acc[tj][r] * p.alpha;
+        }
+    }
+}
+
 template <bool STREAM_C, int TI>
 __device__ __forceinline__ void store_acc_compound_buffer(const GemmParams& p, float* __restrict__ C, const v16f (&acc)[TI][2],
                                                           int m_base, int n_base, int lane) {

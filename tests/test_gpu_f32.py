@@ -689,6 +689,27 @@ def test_outer_prod_mean_compound_store(ops, oracle, D, L, N, B):
     assert np.array_equal(got, oracle.outer_prod_mean(l, r, D, L, N, B))
 
 
+# one plane in 64 x 64 tiles: one tile, ragged ones, runs shorter than a row tile and longer, K of one step, in whole groups of
+# four or not, short of a stage, into the second chunk and over the ring; nearly two tiles per CU (22 x 22) and the
+# 128 x 128 ones behind them, from K = 97 on.  Whole numbers; then one value that the split cannot carry
+@pytest.mark.parametrize("D,L,N", [(1, 64, 4), (1, 5, 1), (3, 24, 9), (7, 19, 17), (2, 33, 47), (3, 65, 33), (4, 31, 64), (9, 47, 97), (5, 40, 258),
+                                   (45, 31, 20), (44, 32, 5), (13, 128, 100), (54, 31, 97)])
+def test_outer_prod_mean_of_few_tiles(ops, oracle, D, L, N):
+    rng = np.random.default_rng(D * L + N)
+    l, r = (rng.integers(-3, 4, size=D * L * N).astype(np.float32) for _ in range(2))
+    l *= N                                             # sums of at most 9 N * N < 2^24: exact, and so are the means
+    want = oracle.outer_prod_mean(l, r, D, L, N, 1)
+    exact = np.rint(want.astype(np.float64)).astype(np.float32)
+    got = ops.outer_product_mean(_dev(l), _dev(r), D, L, N, 1).cpu().numpy()
+    assert np.abs(got - exact).max() <= np.abs(exact).max() * 2.0 ** -23       # 1 / N and the product by it: two roundings
+    if D * L * N < 20000:
+        l[D * L * N // 2] = np.inf
+        got, want = ops.outer_product_mean(_dev(l), _dev(r), D, L, N, 1).cpu().numpy(), oracle.outer_prod_mean(l, r, D, L, N, 1)
+        fin = np.isfinite(want)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        assert np.abs(got[fin] - want[fin]).max() <= np.abs(want[fin]).max() * 2.0 ** -22
+
+
 def test_outer_product_mean_graph_form_large(ops, oracle):
     # D * L = 5888 rows a side: the graph form through the split-ahead path, compound output index
     D, L, N, B = 32, 184, 8, 1
