@@ -2488,6 +2488,16 @@ bool streams_output(const GemmParams& p) {
     return compound ? static_cast<int64_t>(p.M) * p.N * p.np2 * p.np3 * 4 >= (128LL << 20) : whole_lines;
 }
 
+// An index of one value may come with any stride (a pair tensor of one residue has 1 for several), but the forms that address
+// by buffers take an operand's or the output's extent from it: such a stride becomes a dense tensor's.
+void settle_unit_strides(GemmParams& p) {
+    if (p.K == 1 && p.a_lm == 0 && !(p.a_ks == 1 && p.b_ks == 1)) {
+        if (p.a_rs == 1) p.a_ks = std::max<int64_t>(p.a_ks, p.M);
+        if (p.b_rs == 1) p.b_ks = std::max<int64_t>(p.b_ks, p.N);
+    }
+    if (p.M == 1 && p.c_ni == 1) p.c_mi = std::max<int64_t>(p.c_mi, p.N);
+}
+
 // Both gradients of the triangle multiplication in one launch (gemm_bf16x3_pc_pair_kernel); -1 when one of the two is not
 // of the kind that launch_gemm gives to gemm_bf16x3_pc_kernel with at most one tile per CU (beyond that each fills the
 // chip by itself) or the two do not lie as one of the two instances has them, and the caller launches them one by one.
@@ -2496,6 +2506,7 @@ int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what
     if (f32_arithmetic() == 1) return -1;
     const auto kmode = [](int64_t rs, int64_t ks) { return ks == 1 ? LOAD_K_CONTIG : rs == 1 ? LOAD_ROW_CONTIG : LOAD_STRIDED; };
     for (GemmParams* p : {&a, &b}) {
+        settle_unit_strides(*p);
         p->tiles_m = (p->M + BM - 1) / BM;
         p->tiles_n = (p->N + BN - 1) / BN;
         p->stream_c = streams_output(*p);
@@ -2531,6 +2542,7 @@ int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what
 // is refused, any other runs, in the form that it takes without one where that fits.
 // sums_done: set where p.row_sums has been seen to.
 int launch_gemm_sums(GemmParams p, hipStream_t stream, const char* what, uint8_t* fixed_ws, size_t fixed_cap, bool& sums_done) {
+    settle_unit_strides(p);
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
     p.stream_c = streams_output(p);

@@ -761,6 +761,21 @@ def test_tri_mul_whole_k_kernel_gives_the_staged_kernel_bits(ops, outgoing):
         assert torch.equal(part, full[d0:d0 + 100]), f"planes {d0}..{d0 + 100}"
 
 
+# dimensions of one element, whose strides coincide with others'
+@pytest.mark.parametrize("D,I,J,K", [(1, 1, 1, 2), (3, 1, 5, 7), (3, 5, 1, 7), (2, 33, 1, 70), (2, 1, 70, 33), (3, 7, 5, 1), (1, 1, 2, 1), (2, 70, 1, 1), (1, 1, 1, 1)])
+@pytest.mark.parametrize("outgoing", [True, False])
+def test_tri_mul_back_of_single_rows(ops, oracle, D, I, J, K, outgoing):
+    rng = np.random.default_rng(D * I + J * K)
+    grad, left, right = (rng.integers(-9, 10, size=n).astype(np.float32) for n in (D * I * J, D * I * K, D * J * K))
+    args = (D, I, J, K, 1, 8.0, outgoing)              # whole numbers by 1/8: exact
+    want_l, want_r = oracle.tri_mul_back(grad, left, right, *args)
+    gl, gr = ops.tri_mul_back(_dev(grad), _dev(left), _dev(right), *args)
+    one_l, _ = ops.tri_mul_back(_dev(grad), _dev(left), _dev(right), *args, want_right=False)
+    _, one_r = ops.tri_mul_back(_dev(grad), _dev(left), _dev(right), *args, want_left=False)
+    for got, want in ((gl, want_l), (one_l, want_l), (gr, want_r), (one_r, want_r)):
+        assert np.array_equal(got.cpu().numpy().reshape(-1), want.reshape(-1))
+
+
 def test_tri_mul_finite_guard(ops, oracle):
     # src/backend/CPUKernels.cpp:957-962
     left = np.zeros((1, 4, 2, 1), dtype=np.float32)
