@@ -2499,8 +2499,11 @@ void settle_unit_strides(GemmParams& p) {
 }
 
 // Both gradients of the triangle multiplication in one launch (gemm_bf16x3_pc_pair_kernel); -1 when one of the two is not
-// of the kind that launch_gemm gives to gemm_bf16x3_pc_kernel with at most one tile per CU (beyond that each fills the
+// of a kind that gemm_bf16x3_pc_kernel takes with at most one tile per CU (beyond that each fills the
 // chip by itself) or the two do not lie as one of the two instances has them, and the caller launches them one by one.
+// K of up to three chunks and sides of up to 32 too, for which one contraction alone has kernels of its own: a second launch costs
+// more than those save, and the bits are the same.  us, two launches / one, outgoing: 128 planes of 19 x 19 x 19 11.7 / 6.2, of 47 13.6 / 7.2,
+// 256 of 47 14.2 / 9.2, 32 of 32 11.7 / 5.9; incoming the same within 0.3.
 // I, J, K: the statistics' row, which is that of the left gradient's contraction.
 int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what, int64_t I, int64_t J, int64_t K) {
     if (f32_arithmetic() == 1) return -1;
@@ -2511,7 +2514,7 @@ int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what
         p->tiles_n = (p->N + BN - 1) / BN;
         p->stream_c = streams_output(*p);
         if (static_cast<int64_t>(p->tiles_m) * p->tiles_n * p->np2 * p->np3 > device_cu_count()) return -1;
-        if (p->M <= 32 || p->N <= 32 || p->K <= 3 * BK || p->np2 * p->np3 == 1 || p->bias || p->clamp || p->f16_in || p->a_lm > 0) return -1;
+        if (p->np2 * p->np3 == 1 || p->bias || p->clamp || p->f16_in || p->a_lm > 0) return -1;
         if (p->c_ni != 1 || p->c_lm < p->M || p->c_ln < p->N) return -1;
         // buffer addressing: every plane below 2 GiB, and the launcher's bounds on the pitches
         const auto reach = [&](int64_t rs, int64_t ks, int64_t rows) {

@@ -776,6 +776,26 @@ def test_tri_mul_back_of_single_rows(ops, oracle, D, I, J, K, outgoing):
         assert np.array_equal(got.cpu().numpy().reshape(-1), want.reshape(-1))
 
 
+# both gradients in one launch: one chunk of K, three and the first size past them, a side of one row, of a tile row and one more
+@pytest.mark.parametrize("D,I,J,K", [(3, 1, 5, 7), (40, 19, 19, 19), (7, 48, 33, 16), (5, 32, 47, 49), (9, 64, 17, 130), (256, 47, 47, 47)])
+@pytest.mark.parametrize("outgoing", [True, False])
+def test_tri_mul_back_in_one_launch_has_the_bits_of_two(ops, oracle, D, I, J, K, outgoing):
+    rng = np.random.default_rng(D * I + J * K)
+    grad, left, right = (rng.standard_normal(n).astype(np.float32) for n in (D * I * J, D * I * K, D * J * K))
+    args = (D, I, J, K, 1, 8.0, outgoing)
+    gl, gr = ops.tri_mul_back(_dev(grad), _dev(left), _dev(right), *args)
+    one_l, _ = ops.tri_mul_back(_dev(grad), _dev(left), _dev(right), *args, want_right=False)
+    _, one_r = ops.tri_mul_back(_dev(grad), _dev(left), _dev(right), *args, want_left=False)
+    assert torch.equal(gl, one_l) and torch.equal(gr, one_r)
+    if D <= 9:
+        grad[1] = np.inf                               # (one that the split cannot carry)
+        gl, gr = ops.tri_mul_back(_dev(grad), _dev(left), _dev(right), *args)
+        for got, want in zip((gl, gr), oracle.tri_mul_back(grad, left, right, D, I, J, K, 1, 8.0, outgoing)):
+            got, fin = got.cpu().numpy(), np.isfinite(want)
+            assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+            _check(got[fin], want[fin])
+
+
 def test_tri_mul_finite_guard(ops, oracle):
     # src/backend/CPUKernels.cpp:957-962
     left = np.zeros((1, 4, 2, 1), dtype=np.float32)
