@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <functional>
 #include <new>
 #include <unordered_map>
 #include <unordered_set>
@@ -805,7 +806,18 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
             const bool two_outputs = m->op == OP_TRI_MUL_BACK || m->op == OP_OUTER_PROD_MEAN_BACK;
             const auto plan = plans.find(m);
             return meet(m, t) || ((two_outputs || m->op == OP_FLASH_ATTN_EXT) && meet(m->src[4], t)) || (two_outputs && meet(m->src[3], t)) ||
-                   (plan != plans.end() && meet(plan->second.bridge_out, t));
+                   (plan != plans.end() && (meet(plan->second.bridge_out, t) || meet(plan->second.bias_grad, t)));
+        };
+        // m reads memory of t's when it runs: where a source has been folded away, what that one would have read (a folded node whose
+        // result is written all the same, by another node, is `early`)
+        std::unordered_set<const Tensor*> early;
+        std::function<bool(const Tensor*, const Tensor*)> reads = [&](const Tensor* m, const Tensor* t) {
+            for (const Tensor* s : m->src) {
+                const Tensor* from = s;
+                for (int guard = 0; guard < 64 && from && (from->op == OP_VIEW || from->op == OP_RESHAPE); ++guard) from = from->view_src ? from->view_src : from->src[0];
+                if (from && skipped.count(from) && !early.count(from) ? reads(from, t) : meet(s, t)) return true;
+            }
+            return false;
         };
         // what `from` reads of t can be read by `n` instead (nodes folded away in between are in `skipped` already)
         const auto stands_until = [&](const Tensor* from, const Tensor* n, const Tensor* t) {
@@ -856,7 +868,7 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                 }
                 if (!b.bridges_in && !b.bridge_out) continue;
                 plans[n] = b;
-                if (b.bridge_out) skipped.insert(b.bridge_out);
+                if (b.bridge_out) { skipped.insert(b.bridge_out); early.insert(b.bridge_out); }
             }
         }
 
@@ -1028,8 +1040,8 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
             }
         }
         // (8) a LinearLayer's bias gradient behind its weight gradient (src/core/ComputeGraph.cpp:738, 742): the sums over the
-        // rows that the contraction reads, left beside it.  The sum then runs before its place, so nothing between the two may
-        // read or write its memory, or write the gradient's.
+        // rows that the contraction reads, left beside it.  The sum then runs before its place, so nothing that runs between the two
+        // may read its memory, for itself or for a node folded into it, or write it, or write the gradient's.
         if (fuse_permutes_into_mul_mat_) {
             for (Tensor* n : *graph) {
                 if (!n || n->op != OP_MUL_MAT || skipped.count(n)) continue;
@@ -1043,11 +1055,13 @@ Status HipBackend::graph_compute(ComputeGraph* graph) {
                     if (r->view_src || r->dims[0] != g->dims[0] || r->numel() != g->dims[0] || g->numel() != g->dims[0] * g->dims[1]) continue;
                     bool free = !meet(r, n) && !meet(r, g) && !meet(r, x) && !meet(n, g);
                     for (int i = position[n] + 1; i < at && free; ++i) {
-                        free = !overwrites(order[i], r) && !overwrites(order[i], g);
-                        for (int s = 0; s < 10 && free; ++s) free = !meet(order[i]->src[s], r);
+                        const Tensor* m = order[i];
+                        const bool runs = m->op != OP_NONE && m->op != OP_VIEW && m->op != OP_RESHAPE && !skipped.count(m);
+                        free = !overwrites(m, r) && !overwrites(m, g) && !(runs && reads(m, r));
                     }
                     if (!free) continue;
                     skipped.insert(r);
+                    early.insert(r);
                     planned->second.bias_grad = const_cast<Tensor*>(r);
                     break;
                 }

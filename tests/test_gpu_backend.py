@@ -632,6 +632,90 @@ def test_bias_gradient_beside_the_weight_gradient(be, T, K, N):
     assert np.all(np.abs(be.download(db).reshape(N) - 2 * want) <= 2 * bound)
 
 
+# what stands between a weight gradient and the bias gradient behind it, reading -- for a node folded into it -- the memory that an
+# allocator has given to the bias gradient because its last reader by the graph alone has run: another layer's gradient or activations,
+# a weight under its input's gradient, a softmax with its add, a scaled product, a product of transposed operands, a quantized linear
+# with its ReLU, and two of them
+@pytest.mark.parametrize("between", ["gradient", "activations", "weight", "added", "bias", "scaled", "transposed", "relu", "first"])
+def test_bias_gradient_keeps_off_memory_that_folded_readers_read(be, oracle, between):
+    import torch
+    T, K, N = 300, 64, 128
+    rng = np.random.default_rng(11)
+    X, G, X2, G2, W2 = (rng.standard_normal(s).astype(np.float32) for s in ((T, K), (T, N), (T, K), (T, N), (N, K)))
+    w1t, _ = _q8_leaf(be, oracle, (rng.standard_normal((256, N)) * 0.05).astype(np.float32), "Q8_0R")
+    w2t, _ = _q8_leaf(be, oracle, (rng.standard_normal((N, 256)) * 0.05).astype(np.float32), "Q8_0R")
+    homes = {}
+
+    def home(arr):
+        t = torch.from_numpy(np.ascontiguousarray(arr)).cuda()
+        leaf = B.Tensor(arr.shape[::-1]).bind(t.data_ptr())
+        homes[leaf] = t
+        return leaf
+
+    def swapped(t, dims, nd=2):
+        n = B.Tensor(dims, B.F32, B.OP_PERMUTE, [t])
+        for d, a in enumerate((1, 0, 2, 3)[:nd]):
+            n.set_param(d, a)
+        return n
+
+    def run(fused):
+        homes.clear()
+        x, g, x2, g2, w2 = (home(a) for a in (X, G, X2, G2, W2))
+        gt, xt = swapped(g, (T, N)), swapped(x, (T, K))
+        dW = B.Tensor((K, N), B.F32, B.OP_MUL_MAT, [gt, xt])
+        first, behind = [], []
+        if between in ("gradient", "activations"):
+            gt2, xt2 = swapped(g2, (T, N)), swapped(x2, (T, K))
+            out = B.Tensor((K, N), B.F32, B.OP_MUL_MAT, [gt2, xt2])
+            first, behind, victim = [gt2, xt2], [out], g2 if between == "gradient" else x2
+        elif between == "weight":
+            wt = swapped(w2, (N, K))
+            out = B.Tensor((K, T), B.F32, B.OP_MUL_MAT, [g2, wt])
+            first, behind, victim = [wt], [out], w2
+        elif between in ("added", "bias"):
+            full, b = home(G2), home(G)
+            add = B.Tensor((N, T), B.F32, B.OP_ADD, [full, b])
+            out = B.Tensor((N, T), B.F32, B.OP_SOFT_MAX, [add])
+            first, behind, victim = [add], [out], full if between == "added" else b
+        elif between == "scaled":
+            a, b = home(X2.reshape(1, 1, T, K)), home(G2.reshape(1, 1, T, N))
+            p = B.Tensor((K, N, 1, 1), B.F32, B.OP_OUT_PROD, [a, b])
+            out = B.Tensor((K, N, 1, 1), B.F32, B.OP_SCALE, [p]).set_param(0, 0.5)
+            first, behind, victim = [p], [out], b
+        elif between == "transposed":
+            a, b = home(X2.reshape(1, 1, T, K)), home(W2.reshape(1, 1, N, K))
+            pa, pb = swapped(a, (T, K, 1, 1), 4), swapped(b, (N, K, 1, 1), 4)
+            out = B.Tensor((T, N, 1, 1), B.F32, B.OP_OUT_PROD, [pa, pb])
+            first, behind, victim = [pa, pb], [out], a
+        elif between == "relu":
+            r = B.Tensor((N, T), B.F32, B.OP_UNARY, [g2]).set_param(0, B.UNARY_OP_RELU)
+            out = B.Tensor((256, T), B.F32, B.OP_MUL_MAT, [r, w1t])
+            first, behind, victim = [r], [out], g2
+        else:
+            h = B.Tensor((256, T), B.F32, B.OP_MUL_MAT, [g2, w1t])
+            r = B.Tensor((256, T), B.F32, B.OP_UNARY, [h]).set_param(0, B.UNARY_OP_RELU)
+            out = B.Tensor((N, T), B.F32, B.OP_MUL_MAT, [r, w2t])
+            first, behind, victim = [h], [r, out], g2
+        db = B.Tensor((N,), B.F32, B.OP_REPEAT_BACK, [g]).bind(homes[victim].data_ptr())
+        for switch in SWITCHES:
+            getattr(be, switch)(fused)
+        try:
+            assert be.graph_compute(first + [gt, xt, dW] + behind + [db]) == B.SUCCESS, be.last_error
+        finally:
+            for switch in SWITCHES:
+                getattr(be, switch)(True)
+        be.synchronize()
+        return be.download(out), be.download(dW), be.download(db)
+
+    SWITCHES = ("set_fuse_permutes_into_mul_mat", "set_fuse_add_into_soft_max", "set_fuse_scale_into_out_prod", "set_fuse_permutes_into_out_prod",
+                "set_fuse_relu_into_q8")
+    got, want = run(True), run(False)
+    for a, b in zip(got[:2], want[:2]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    bound = np.abs(G.astype(np.float64)).sum(axis=0) * 860 * 2.0 ** -24
+    assert np.all(np.abs(got[2].reshape(N) - G.astype(np.float64).sum(axis=0)) <= bound)
+
+
 def test_f32_arithmetic_is_a_field_of_the_backend(be, oracle):
     # two backends with different pipes do not disturb each other or the calling thread's own setting
     import torch
