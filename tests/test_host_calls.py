@@ -1,4 +1,7 @@
 """The native host side of the operators (csrc/host_calls.cpp): it takes ordinary calls only, and what it takes is what the long way gives."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 import torch
@@ -19,6 +22,19 @@ def test_it_is_built_and_answers_none_to_what_is_not_ordinary():
     assert ops._host.tri_mul(a, b, 1, 2, 3, 4, 5, 0.0, True) is None and ops._host.outer_product_mean(a, b, 1 << 40, 1 << 40, 1, 1) is None
     with pytest.raises(ValueError):
         ops._host.bind("no_such_launcher", 0)
+
+
+def test_the_library_is_built_without_it(tmp_path):
+    """C++ users need neither torch nor Python's headers: the build says that the module is left out, and goes on."""
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "proteinpredictmachinelearning_amd", "csrc")
+    no_torch = tmp_path / "python"
+    no_torch.write_text("#!/bin/sh\nexit 1\n")
+    no_torch.chmod(0o755)
+    for variables in (f"PYTHON={no_torch}", "CXX=false"):
+        out = tmp_path / "_host_calls.so"
+        done = subprocess.run(["make", "-C", csrc, f"HOST={out}", variables, str(out)], capture_output=True, text=True)
+        assert done.returncode == 0, done.stderr
+        assert "not built" in done.stdout and not out.exists()
 
 
 def _calls():
