@@ -304,4 +304,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods
 
 }  // namespace
 
+// whose class layouts this was compiled against: read before the module is imported
+#define TEXT_OF_(x_) #x_
+#define TEXT_OF(x_) TEXT_OF_(x_)
+extern "C" __attribute__((visibility("default"))) const char host_calls_built_for[] = TEXT_OF(BUILT_FOR);
+
 PyMODINIT_FUNC PyInit__host_calls() { return PyModule_Create(&module); }

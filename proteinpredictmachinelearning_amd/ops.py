@@ -13,6 +13,7 @@ import importlib.machinery
 import importlib.util
 import math
 import os
+import sys
 
 import torch
 
@@ -30,18 +31,20 @@ _current_device = torch._C._cuda_getDevice if hasattr(torch._C, "_cuda_getDevice
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
 
 
-
 def _load_host_calls():
-    """The native host side of the operators below (csrc/host_calls.cpp), or None where it was not built for this torch: every
-    operator then does its call itself, as it does any call that is not ordinary."""
+    """The native host side of the operators below (csrc/host_calls.cpp), or None where it was not built for this torch and Python
+    (another one's tensors may lie differently): every operator then does its call itself, as it does any call that is not ordinary."""
     path = os.path.join(os.path.dirname(cabi.LIB_PATH), "_host_calls.so")
     try:
+        built_for = C.string_at(C.addressof(C.c_char.in_dll(C.CDLL(path), "host_calls_built_for"))).decode()
+        if built_for != f"torch-{torch.__version__}-python-{sys.version_info[0]}.{sys.version_info[1]}":
+            return None
         loader = importlib.machinery.ExtensionFileLoader("_host_calls", path)
         spec = importlib.util.spec_from_file_location("_host_calls", path, loader=loader)
         module = importlib.util.module_from_spec(spec)
         loader.exec_module(module)
         return module
-    except (ImportError, OSError):
+    except (ImportError, OSError, ValueError):          # not there, other symbols, no such mark
         return None
 
 

@@ -37,6 +37,12 @@ def test_the_library_is_built_without_it(tmp_path):
         assert "not built" in done.stdout and not out.exists()
 
 
+def test_a_module_built_for_another_torch_is_not_loaded(monkeypatch):
+    assert ops._load_host_calls() is not None
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    assert ops._load_host_calls() is None
+
+
 def _calls():
     torch.manual_seed(3)
     r = lambda *s: torch.randn(*s, device="cuda")      # noqa: E731
