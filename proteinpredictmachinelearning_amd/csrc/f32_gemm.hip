@@ -2530,21 +2530,14 @@ int try_pc_pair(GemmParams a, GemmParams b, hipStream_t stream, const char* what
     const bool k4 = a.K % 4 == 0 && (outgoing || b.K % 4 == 0);      // (loads along k; the outgoing `b` has none)
     const int groups_a = a.tiles_m * a.tiles_n * a.np2 * a.np3, groups_b = b.tiles_m * b.tiles_n * b.np2 * b.np3;
     const dim3 grid(static_cast<unsigned>(groups_a + groups_b)), block(512);
-    // (small ones keep the two rows that they have in the statistics; the launch's time is in the left gradient's)
-    const bool small = a.K <= 3 * BK || b.K <= 3 * BK || std::min(std::min(a.M, a.N), std::min(b.M, b.N)) <= 32;
-    int rc;
-    {
-        StatsScope stat(small ? "hip/tri_mul_back" : "hip/tri_mul_back_pair", I, J, K, stream);
+    StatsScope stat("hip/tri_mul_back_pair", I, J, K, stream);
 #define PPML_PAIR(AB_, BM_, STREAM_, K4_) hipLaunchKernelGGL((gemm_bf16x3_pc_pair_kernel<LOAD_K_CONTIG, AB_, BM_, LOAD_ROW_CONTIG, STREAM_, K4_>), grid, block, 0, stream, a, b, groups_a)
 #define PPML_PAIR_K4(AB_, BM_, STREAM_) do { if (k4) PPML_PAIR(AB_, BM_, STREAM_, true); else PPML_PAIR(AB_, BM_, STREAM_, false); } while (0)
-        if (outgoing) { if (a.stream_c) PPML_PAIR_K4(LOAD_ROW_CONTIG, LOAD_ROW_CONTIG, true); else PPML_PAIR_K4(LOAD_ROW_CONTIG, LOAD_ROW_CONTIG, false); }
-        else          { if (a.stream_c) PPML_PAIR_K4(LOAD_K_CONTIG, LOAD_K_CONTIG, true); else PPML_PAIR_K4(LOAD_K_CONTIG, LOAD_K_CONTIG, false); }
+    if (outgoing) { if (a.stream_c) PPML_PAIR_K4(LOAD_ROW_CONTIG, LOAD_ROW_CONTIG, true); else PPML_PAIR_K4(LOAD_ROW_CONTIG, LOAD_ROW_CONTIG, false); }
+    else          { if (a.stream_c) PPML_PAIR_K4(LOAD_K_CONTIG, LOAD_K_CONTIG, true); else PPML_PAIR_K4(LOAD_K_CONTIG, LOAD_K_CONTIG, false); }
 #undef PPML_PAIR_K4
 #undef PPML_PAIR
-        rc = check_launch(what);
-    }
-    if (small && rc == RC_OK) StatsScope beside("hip/tri_mul_back", J, I, K, stream);
-    return rc;
+    return check_launch(what);
 }
 
 // `fixed_ws` / `fixed_cap`: a workspace the caller brings (the static array of the entry point that allocates

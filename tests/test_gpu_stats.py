@@ -68,7 +68,8 @@ def test_both_triangle_gradients_in_one_launch_are_one_row():
     before = ops.mulmat_stats_enable(True)
     try:
         for D, I, J, K, paths in ((4, 64, 96, 60, {("hip/tri_mul_back_pair", 64, 96, 60)}),                            # one launch
-                                  (4, 40, 40, 40, {("hip/tri_mul_back", 40, 40, 40)}),                                 # too short a contraction: two
+                                  # three chunks of K at most: launches of their own until contractions as short were given the shared one
+                                  (4, 40, 40, 40, {("hip/tri_mul_back_pair", 40, 40, 40)}), (5, 19, 33, 47, {("hip/tri_mul_back_pair", 19, 33, 47)}),
                                   (300, 60, 52, 56, {("hip/tri_mul_back", 60, 52, 56), ("hip/tri_mul_back", 52, 60, 56)})):     # more tiles than CUs: two
             lib.ppml_hip_mulmat_stats_reset()
             left, right, grad = (torch.randn(D * n, device="cuda", generator=g) for n in (I * K, J * K, I * J))
