@@ -352,18 +352,18 @@ def flash_attn_backward(q, k, v, bias, o, do, lse, causal: bool = False, scale: 
                         want=("dq", "dk", "dv", "dbias")):
     """Fused attention backward (include/ppml/FlashAttn.h:67-101): returns (dQ, dK, dV, dbias), None for the
     gradients not named in `want`."""
-    grads = _host_flash_attn_backward(q, k, v, bias, o, do, lse, causal, scale,
-                                      ("dq" in want) | ("dk" in want) << 1 | ("dv" in want) << 2 | ("dbias" in want) << 3)
+    want_dq, want_dk, want_dv, want_dbias = "dq" in want, "dk" in want, "dv" in want, "dbias" in want      # (once: it may be an iterator)
+    grads = _host_flash_attn_backward(q, k, v, bias, o, do, lse, causal, scale, want_dq | want_dk << 1 | want_dv << 2 | want_dbias << 3)
     if grads is not None:
         return grads
     q, k, v, o, do, lse = (_dev_f32(t, n) for t, n in ((q, "q"), (k, "k"), (v, "v"), (o, "o"), (do, "do"), (lse, "lse")))
     B, h, L, d = q.shape
     if bias is not None:
         bias = _dev_f32(bias, "bias")
-    dq = torch.empty_like(q) if "dq" in want else None
-    dk = torch.empty_like(q) if "dk" in want else None
-    dv = torch.empty_like(q) if "dv" in want else None
-    db = torch.empty((B, h, L, L), dtype=torch.float32, device=q.device) if "dbias" in want else None
+    dq = torch.empty_like(q) if want_dq else None
+    dk = torch.empty_like(q) if want_dk else None
+    dv = torch.empty_like(q) if want_dv else None
+    db = torch.empty((B, h, L, L), dtype=torch.float32, device=q.device) if want_dbias else None
     opt = lambda t: _ptr(t) if t is not None else None      # noqa: E731
     cabi.check("flash_attn_backward_hip",
                _lib().flash_attn_backward_hip(B, h, L, d, int(causal), scale, _ptr(q), _ptr(k), _ptr(v), opt(bias), _ptr(o),

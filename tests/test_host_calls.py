@@ -103,6 +103,17 @@ def test_calls_it_takes_are_the_long_ways(monkeypatch):
 
 
 @pytest.mark.gpu
+def test_gradients_named_by_an_iterator(monkeypatch):
+    q, k, v, do = (torch.randn(1, 2, 21, 8, device="cuda") for _ in range(4))
+    o, lse = ops.flash_attn_forward(q, k, v)
+    names = ("dq", "dk", "dv", "dbias")
+    want = ops.flash_attn_backward(q, k, v, None, o, do, lse, want=names)
+    for _ in range(2):                                 # the native way, then the long one
+        _same(ops.flash_attn_backward(q, k, v, None, o, do, lse, want=iter(names)), want)
+        monkeypatch.setattr(ops, "_host_flash_attn_backward", ops._not_taken)
+
+
+@pytest.mark.gpu
 def test_calls_that_are_not_ordinary_go_the_long_way():
     a, b = torch.randn(33, 20, device="cuda"), torch.randn(7, 20, device="cuda")
     want = ops.mul_mat(a, b)
