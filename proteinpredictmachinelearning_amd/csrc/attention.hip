@@ -45,9 +45,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const float* base, i
 }
 
 template <int DP, int NW, bool PF, bool IN_LD> struct AttnTiling {
-    // keys staged in LDS at a time: 36 KB per four-wave work-group (four of them share a CU and its
-    // 160 KB; 128 keys would leave room for three, measured 64.7 against 61.2 us at the MSA shape).  The form of short
-    // rows has the registers for three anyway, and with 128 its rows are one stage.
+    // keys staged in LDS at a time: 38.25 KB per four-wave work-group of narrow heads (36 where the source rows run along the keys): four
+    // of them share a CU and its 160 KB; 128 keys would leave room for three, measured 64.7 against 61.2 us at the MSA shape.  The form of
+    // short rows has the registers for three anyway, and with 128 keys, 51 KB, its rows are one stage.
     static constexpr int CH = DP <= 32 ? (NW == 4 && !PF ? 96 : 128) : (NW == 4 ? 64 : 128);
     static constexpr int NC = DP / 16;                // 16-feature chunks of the score contraction
     // a 32-key tile of K in LDS: one 1 KB MFMA operand fragment per (chunk, bf16 part), [half][key][8 bf16]
@@ -60,6 +60,7 @@ template <int DP, int NW, bool PF, bool IN_LD> struct AttnTiling {
     static constexpr int V_HALF = 576, V_FRAG = 2 * V_HALF, V_CHUNK = 3 * V_FRAG;
     static constexpr int VT_BYTES = IN_LD ? (DP / 32) * 2 * 3 * 1024 : NC * V_CHUNK;
     static constexpr size_t lds_bytes = static_cast<size_t>(CH / 32) * (KT_BYTES + VT_BYTES);
+    static_assert(DP > 32 || NW != 4 || (PF ? 3 : 4) * lds_bytes <= 160 * 1024, "the work-groups that the registers leave room for");
 };
 
 constexpr int MASKED = 0, PLAIN = 1, HEAD = 2;          // kinds of tiles (see where they are told apart)
