@@ -2365,7 +2365,10 @@ extern "C" int mul_mat_q8_ex_hip(const void* W, const float* X, float* C, int M,
     }
 }
 
-// K -> H -> K features with a ReLU between, both weights packed or both Q8_0R: q8_feed_forward_kernel's instances
+// K -> H -> K features with a ReLU between, both weights packed or both Q8_0R: q8_feed_forward_kernel's instances.  What the kernel can
+// take: K of blocks in pairs (a wave quantizes two at a time) up to eight (eight waves have the output tiles, and hold one hidden
+// tile's fragments of the first weight in registers), H of blocks in fours (the ring) up to what leaves LDS for two work-groups.  Of
+// these sizes the widenings by two and by four, which transitions use, have instances; others go as two linears.
 namespace ppmlhip {
 bool q8_feed_forward_fits(int64_t N, int64_t K, int64_t H, int wtype1, int wtype2) {
     if (wtype1 != wtype2 || (wtype1 != PPML_WTYPE_Q8_0M && wtype1 != PPML_WTYPE_Q8_0R)) return false;
@@ -2377,12 +2380,15 @@ int q8_feed_forward(const void* W1, const void* W2, const float* X, float* Y, in
     StatsScope stat("hip/q8-feed-forward", H, K, N, stream);
     set_q8_path(PPML_Q8_PATH_LOW_LATENCY);
     const dim3 grid((N + FF_TOK - 1) / FF_TOK), block(FF_WAVES * 64);
-    // Q8_0R planes are read in place or packed first, both in one launch (2.5 us).  A fragment of such a weight is 32 pieces one
-    // row apart: rows of 512 bytes or 1 KB put them in the same sets of the vector cache, whose lines are fetched again then.  us, in place / packed
-    // weights, without the packing: 128 -> 512, 361 tokens 11.5 / 7.9, 10609 18.6 / 11.6; 256 -> 1024, 10609 44.6 / 26.5;
-    // 128 -> 256, 10609 9.7 / 7.6, 25600 18.2 / 12.8; 192 -> 768, 361 13.6 / 11.8, 10609 22.4 / 18.9; 192 -> 384 8.8 / 7.8, 12.2 / 11.5.
+    // Q8_0R planes are read in place or packed first, both in one launch (1.4 to 2.5 us of a call).  A fragment of such a weight is 32
+    // pieces one row apart: rows of 512 bytes or 1 KB put them in the same sets of the vector cache, whose lines are fetched again
+    // then, at any number of tokens; from other rows the pieces cost less, and a launch more from some number of tokens on.  us a call, in
+    // place / packed first: 128 -> 512, 361 tokens 11.5 / 11.0, 10609 18.9 / 15.0; 256 -> 1024, 10609 44.8 / 29.1; 192 -> 768, 8100 15.0 / 16.3, 10609 22.7 / 21.4, 40000 51.6 / 46.5;
+    // 128 -> 256, 10609 10.2 / 10.9, 25600 18.2 / 15.9; 192 -> 384, 32400 22.6 / 23.2, 40000 29.3 / 28.6, 147456 98 / 88; 64 -> 256,
+    // 32400 11.6 / 12.3, 40000 14.9 / 14.2, 147456 47.6 / 38.8; 64 -> 128, 65536 13.5 / 14.2, 90000 18.2 / 18.0, 147456 31.1 / 29.0.
     Workspace held;
-    if (wtype == PPML_WTYPE_Q8_0R && (H == 512 || H == 1024 || (K == 128 && N >= 14000))) {
+    const int packed_from = H == 512 || H == 1024 ? 0 : H == 768 ? 9000 : K == 128 ? 14000 : H == 128 ? 90000 : 36000;
+    if (wtype == PPML_WTYPE_Q8_0R && N >= packed_from) {
         const size_t bytes1 = (q8_weight_packed_bytes_hip(H, K) + 255) / 256 * 256;
         held = workspace_take(bytes1 + q8_weight_packed_bytes_hip(K, H), stream);
         if (held.ptr) {
