@@ -537,6 +537,12 @@ def test_weight_gradient_reads_the_untransposed_matrices(be, T, K, N):
 @pytest.mark.parametrize("T,K,N", [(26368, 256, 256), (9040, 600, 333), (1058, 480, 395), (701, 64, 397), (408, 256, 256), (51, 33, 49),
                                    (22373, 368, 100), (10609, 21, 128), (26368, 24, 64), (2601, 132, 50), (97, 40, 48)])
 def test_input_gradient_reads_the_weight_as_it_lies(be, T, K, N):
+    import torch
+    tiles = 64 * torch.cuda.get_device_properties(0).multi_processor_count
+    _input_gradient(be, T, K, N, folded=N > 48 and (K > 32 or T <= tiles))      # (a narrow side of many tiles and a K of three chunks at most keep the copy)
+
+
+def _input_gradient(be, T, K, N, folded):
     """dX = mul_mat(grad, mat_transpose(w)) (src/core/ComputeGraph.cpp:735): the copy of the weight is not made when nobody else
     reads it, and the result has the bits of the two nodes run one by one."""
     rng = np.random.default_rng(T + N)
@@ -550,8 +556,7 @@ def test_input_gradient_reads_the_weight_as_it_lies(be, T, K, N):
             wt = B.Tensor((N, K), B.F32, B.OP_PERMUTE, [w]); wt.set_param(0, 1).set_param(1, 0)
             dX = B.Tensor((K, T), B.F32, B.OP_MUL_MAT, [g, wt])
             assert be.graph_compute([wt, dX]) == B.SUCCESS, be.last_error
-            # (a narrow side of many tiles and a K of three chunks at most keep the copy)
-            assert be.nodes_fused_away == (1 if fused and N > 48 and (K > 32 or T <= 64 * 256) else 0)
+            assert be.nodes_fused_away == (1 if fused and folded else 0)
             results[fused] = be.download(dX).reshape(T, K)
         finally:
             be.set_fuse_permutes_into_mul_mat(True)
