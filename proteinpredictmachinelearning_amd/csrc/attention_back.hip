@@ -60,8 +60,8 @@ template <int DP> struct BackTiling {
     static constexpr int NC = DP / 16;                // 16-feature chunks of a contraction over the features
     static constexpr int NB = DP / 32;                // 32-feature blocks of a transposed gradient
     // A 32-row tile of a streamed matrix in LDS, as MFMA operand fragments, one per (chunk, part): features 8 half .. + 7 of
-    // the chunk, sixteen bytes per row, the two halves 576 bytes apart (the transposing reads and the staging writes then touch every bank
-    // once).  The same fragments serve the contraction over the tile's rows: ds_read_b64_tr_b16 hands them out transposed
+    // the chunk, sixteen bytes per row, the two halves 576 bytes apart (the transposing reads and, of heads of up to 32, the staging writes then touch every bank
+    // once; of wider ones, chunks two apart share banks).  The same fragments serve the contraction over the tile's rows: ds_read_b64_tr_b16 hands them out transposed
     // (read_transposed), in the order in which the accumulator registers 8 ch .. 8 ch + 7 of a 32 x 32 product hold the rows.
     static constexpr int HALF = 576, FRAG = 2 * HALF, CHUNK = 3 * FRAG;
     static constexpr int TILE = NC * CHUNK;

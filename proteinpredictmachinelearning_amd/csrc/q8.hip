@@ -1658,10 +1658,11 @@ int try_q8_linear_ll(const void* W, const float* X, float* C, int M, int N, int 
 // they are -- from Q8_0R planes, which then need no packing launch.  Blocks ascend per output and every settlement is the same
 // fma as everywhere else: same bits.
 //
-// What bounds it: up to some 8000 tokens one work-group's chain; beyond, the vector pipe (settlements 0.5 of its time, quantization the
-// rest) and, from 256 KB of weights on, their way out of L2 for every 32 tokens.  us, two kernels / this one, packed weights: 128 -> 512
+// What bounds it: up to some 8000 tokens one work-group's chain; beyond, the vector pipe, which settles and quantizes (10609 tokens: 0.54 of its
+// cycles at 128 -> 512, 0.71 at 256 -> 1024, the matrix pipe 0.19 and 0.23), and, from 256 KB of weights on, their way out of L2 for every 32 tokens.  us, two kernels / this one, packed weights: 128 -> 512
 // 1600 tokens 8.5 / 7.7, 10609 20.2 / 11.5, 25600 30.9 / 19.9; 64 -> 256, 10609 11.4 / 5.6; 192 -> 768, 361 19.3 / 11.7, 10609 36 / 18.6;
-// 256 -> 1024, 10609 39 / 26, 25600 75 / 49; 192 -> 384, 1600 8.6 / 7.9, 10609 28 / 11.2.  No size between 361 and 25600 tokens was slower.
+// 256 -> 1024, 10609 39 / 26, 25600 75 / 49; 192 -> 384, 1600 8.6 / 7.9, 10609 28 / 11.2.  From 1 to 147456 tokens
+// none was slower (192 -> 384 of up to 144 tokens: even).
 // ------------------------------------------------------------------------------------------
 
 // ReLU and quantization of the 32 hidden features a lane and its neighbour 32 lanes on hold of one token: registers as
