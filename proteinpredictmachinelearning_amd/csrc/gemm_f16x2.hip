@@ -1050,7 +1050,7 @@ bool plan_f16x2(const GemmParams& p0, F16x2Plan& pl, int cu_share = 1) {
     const bool partial = slices > 1 || p.a_lm > 0 || p.c_ni != 1;     // (no direct instances for a compound A)
     const size_t part_bytes = partial ? static_cast<size_t>(slices) * ma_pad * nb_pad * 4 : 0;
     if (static_cast<size_t>(ma_pad) * nb_pad * 4 >= (1ull << 31) && partial) return false;
-    const int wgs = std::min<int64_t>((tiles * slices + 7) / 8 * 8, (tj == 1 ? 2 * cus : cus) / cu_share / 8 * 8);
+    const int wgs = std::min<int64_t>((tiles * slices + 7) / 8 * 8, std::max((tj == 1 ? 2 * cus : cus) / cu_share / 8 * 8, 8));
     const int most_items = static_cast<int>(((tiles * slices + 7) / 8 + wgs / 8 - 1) / (wgs / 8));
     pl.b_bytes = b_bytes;
     pl.e_bytes = e_bytes;
